@@ -1,8 +1,9 @@
-"""ctypes binding of ``libjvpfa.so`` (the C ABI declared in ``include/jvpfa.h``).
+"""Bindings of ``libjvpfa.so`` (the C ABI declared in ``include/jvpfa.h``).
 
-The library is loaded after ``import torch`` so that the HIP runtime torch already mapped is the
-one the kernels launch on.  There is no fallback: if the library is missing, or a tensor is not
-on a GPU, the call raises.
+Forward and backward go through ``_torch_binding.so`` (``csrc/torch_binding.cpp``: allocation, argument block, launch
+and the autograd node of an eager call in native code); the mask scans and everything else of the C ABI through ctypes.
+The libraries are loaded after ``import torch`` so that the HIP runtime torch already mapped is the one the kernels
+launch on.  There is no fallback: if a library is missing, or a tensor is not on a GPU, the call raises.
 """
 from __future__ import annotations
 
@@ -112,6 +113,22 @@ def load() -> C.CDLL:
             raise RuntimeError("libjvpfa.so ABI version mismatch; rebuild the library")
         _lib = lib
     return _lib
+
+
+_binding = None
+
+
+def binding():
+    """The native host path (``csrc/torch_binding.cpp``), loaded once; raises if it has not been built."""
+    global _binding
+    if _binding is None:
+        load()
+        try:
+            from . import _torch_binding
+        except ImportError as e:
+            raise RuntimeError("_torch_binding.so is missing: build it with `python -m jvp_flash_attention_amd.build`") from e
+        _binding = _torch_binding
+    return _binding
 
 
 def check(status: int) -> None:
@@ -311,18 +328,25 @@ def _stream(t) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
-# The reference admits a head dim of 16 (jvp_flash_attention/jvp_attention.py:2371-2374); the matrix instructions
-# here contract over 16 and produce 32 columns, so the kernels start at 32 and a head dim of 16 runs on them with
-# zero columns appended (one copy of each operand per call).
-PADDED_HEAD_DIM = 16
+def _wants_backward(q, k, v, level) -> bool:
+    """Whether a call on these tensors (dual tensors of ``level``, if that is not negative) may be differentiated."""
+    if not torch.is_grad_enabled():
+        return False
+    if q.requires_grad or k.requires_grad or v.requires_grad:
+        return True
+    tangents = (torch.autograd.forward_ad.unpack_dual(t).tangent for t in (q, k, v)) if level >= 0 else ()
+    return any(t is not None and t.requires_grad for t in tangents)
 
 
-def _pad_head_dim(t):
-    return None if t is None else torch.nn.functional.pad(t, (0, 32 - PADDED_HEAD_DIM))
-
-
-def _cut_head_dim(t):
-    return None if t is None else t[..., :PADDED_HEAD_DIM].contiguous()
+def mask_hints(q, mask, mask_kind, Lk, backward: bool):
+    """(key_limit, tiles_q, tiles_k, bits) for a call with this mask, each None where it does not apply; the last two
+    only for a backward."""
+    if mask_kind == MASK_NONE:
+        return None, None, None, None
+    with torch.cuda.device(q.device):
+        lim = key_limit_hint(mask, mask_kind, q.shape[0], Lk)
+        tq, tk = tile_lists(q, mask, mask_kind, backward, Lk)
+        return lim, tq, tk, mask_bits(q, mask, mask_kind, Lk) if backward else None
 
 
 class HipBackend:
@@ -353,74 +377,26 @@ class HipBackend:
                          want_tangent_grads, dropout_p, dropout_seed)
 
     def _fwd(self, q, k, v, qt, kt, vt, mask, mask_kind, causal, sm_scale, dropout_p=0.0, dropout_seed=0):
-        _require_gpu(q, k, v, qt, kt, vt, mask)
-        if q.shape[-1] == PADDED_HEAD_DIM:
-            # zero columns change neither Q K^T nor the columns of P V that are kept
-            o, ot, M, mu = self._fwd(*map(_pad_head_dim, (q, k, v, qt, kt, vt)), mask, mask_kind, causal, sm_scale,
-                                     dropout_p, dropout_seed)
-            return _cut_head_dim(o), _cut_head_dim(ot), M, mu
-        lib = load()
-        dual = qt is not None
-        o = torch.empty_like(q)
-        ot = torch.empty_like(q) if dual else None
-        Z, H, L, _ = q.shape
-        M = torch.empty((Z, H, L), device=q.device, dtype=torch.float32)
-        mu = torch.empty((Z, H, L), device=q.device, dtype=torch.float32) if dual else None
-        a = FwdArgs()
-        a.struct_size = C.sizeof(FwdArgs)
-        a.p = make_problem(q, mask, mask_kind, causal, sm_scale, dropout_p, dropout_seed)
-        a.q, a.k, a.v = _ptr(q), _ptr(k), _ptr(v)
-        a.qt, a.kt, a.vt = _ptr(qt), _ptr(kt), _ptr(vt)
-        a.o, a.ot, a.M, a.mu = _ptr(o), _ptr(ot), _ptr(M), _ptr(mu)
-        a.Hk, a.Lk = k.shape[1], k.shape[2]  # key/value heads and length (may differ from q's)
-        with torch.cuda.device(q.device):
-            lim = key_limit_hint(mask, mask_kind, Z, k.shape[2])
-            a.key_limit = _ptr(lim)
-            tq, _ = tile_lists(q, mask, mask_kind, False, k.shape[2])
-            a.tiles_q = _ptr(tq)
-            nsplit = lib.jvpfa_fwd_split_workspace_bytes(C.byref(a.p), a.Lk) if _split_enabled else 0
-            if nsplit:
-                split_ws = torch.empty(nsplit, device=q.device, dtype=torch.uint8)
-                a.split_workspace, a.split_workspace_bytes = split_ws.data_ptr(), nsplit
-            check(lib.jvpfa_fwd(C.byref(a), _stream(q)))
-        return o, ot, M, mu
+        _require_gpu(q, mask)
+        lim, tq, _, _ = mask_hints(q, mask, mask_kind, k.shape[2], False)
+        return binding().fwd(q, k, v, qt, kt, vt, float(sm_scale), bool(causal), float(dropout_p), int(dropout_seed) & (2**64 - 1),
+                             _split_enabled, mask, mask_kind, lim, tq)
 
     def _bwd(self, q, k, v, qt, kt, vt, o, ot, M, mu, go, gt, mask, mask_kind, causal, sm_scale,
              want_tangent_grads=False, dropout_p=0.0, dropout_seed=0):
-        _require_gpu(q, k, v, qt, kt, vt, o, ot, M, mu, go, gt, mask)
-        if q.shape[-1] == PADDED_HEAD_DIM:
-            q, k, v, qt, kt, vt, o, ot, go, gt = map(_pad_head_dim, (q, k, v, qt, kt, vt, o, ot, go, gt))
-            grads = self._bwd(q, k, v, qt, kt, vt, o, ot, M, mu, go, gt, mask, mask_kind, causal, sm_scale,
-                              want_tangent_grads, dropout_p, dropout_seed)
-            return tuple(map(_cut_head_dim, grads))
-        lib = load()
-        Z, H, L, _ = q.shape
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        dqt = dkt = dvt = None
-        if want_tangent_grads:
-            dqt, dkt, dvt = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        ws = torch.empty(lib.jvpfa_bwd_workspace_bytes(Z, H, L), device=q.device, dtype=torch.uint8)
-        a = BwdArgs()
-        a.struct_size = C.sizeof(BwdArgs)
-        a.p = make_problem(q, mask, mask_kind, causal, sm_scale, dropout_p, dropout_seed)
-        a.q, a.k, a.v = _ptr(q), _ptr(k), _ptr(v)
-        a.qt, a.kt, a.vt = _ptr(qt), _ptr(kt), _ptr(vt)
-        a.o, a.ot, a.M, a.mu = _ptr(o), _ptr(ot), _ptr(M), _ptr(mu)
-        a.go, a.gt = _ptr(go), _ptr(gt)
-        a.dq, a.dk, a.dv = _ptr(dq), _ptr(dk), _ptr(dv)
-        a.dqt, a.dkt, a.dvt = _ptr(dqt), _ptr(dkt), _ptr(dvt)
-        a.workspace = _ptr(ws)
-        a.Hk, a.Lk = k.shape[1], k.shape[2]
-        with torch.cuda.device(q.device):
-            lim = key_limit_hint(mask, mask_kind, Z, k.shape[2])
-            a.key_limit = _ptr(lim)
-            tq, tk = tile_lists(q, mask, mask_kind, True, k.shape[2])
-            a.tiles_q, a.tiles_k = _ptr(tq), _ptr(tk)
-            bits = mask_bits(q, mask, mask_kind, k.shape[2])
-            a.mask_bits = _ptr(bits)
-            check(lib.jvpfa_bwd(C.byref(a), _stream(q)))
-        return dq, dk, dv, dqt, dkt, dvt
+        _require_gpu(q, mask)
+        return tuple(binding().bwd(q, k, v, qt, kt, vt, o, ot, M, mu, go, gt, float(sm_scale), bool(causal),
+                                   bool(want_tangent_grads), float(dropout_p), int(dropout_seed) & (2**64 - 1), _split_enabled,
+                                   mask, mask_kind, *mask_hints(q, mask, mask_kind, k.shape[2], True)))
 
+    def attend(self, q, k, v, mask, mask_kind, causal, sm_scale, dropout_p, dropout_seed, level):
+        """The whole eager call, autograd included, on tensors that may be dual tensors of ``level``; None when the
+        shapes or types of q, k, v are not supported."""
+        hints = (None,) * 4
+        if mask_kind != MASK_NONE:
+            _require_gpu(q, mask)
+            hints = mask_hints(q, mask, mask_kind, k.shape[2], _wants_backward(q, k, v, level))
+        return binding().attend(q, k, v, level, sm_scale, causal, dropout_p, dropout_seed, _split_enabled, mask, mask_kind, *hints)
 
     def dropout_keep(self, q, Lk, dropout_p, dropout_seed):
         """The keep pattern (bool, shape (Z, H, L, Lk)) that a call with this dropout_p and seed applies."""

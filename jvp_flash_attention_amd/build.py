@@ -3,13 +3,14 @@
 ``python -m jvp_flash_attention_amd.build`` compiles every translation unit (one per element
 type x head dim for the forward and for the backward, plus the C ABI files) in parallel and
 links them into ``jvp_flash_attention_amd/libjvpfa.so``.  hipcc cross-compiles, so no GPU is
-needed to build.
+needed to build.  The host path above it, ``csrc/torch_binding.cpp``, becomes ``_torch_binding.so``.
 """
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -110,8 +111,33 @@ def build(jobs: int | None = None, verbose: bool = True, extra_flags=(), lib: st
     if verbose:
         print("asm lint: clean", flush=True)
     if lib == LIB:
+        build_binding(verbose)
         build_host_check(verbose)
     return lib
+
+
+BINDING_SRC = os.path.join(CSRC, "torch_binding.cpp")
+BINDING_LIB = os.path.join(HERE, "_torch_binding.so")
+
+
+def build_binding(verbose: bool = True) -> str:
+    """The native host path above the C ABI (``csrc/torch_binding.cpp``): host code only, linked with the library just
+    built and with torch."""
+    import torch
+    from torch.utils import cpp_extension
+
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
+    includes = [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-DTORCH_EXTENSION_NAME=_torch_binding", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{d}" for d in includes), BINDING_SRC, "-o", BINDING_LIB, *(f"-L{d}" for d in cpp_extension.library_paths()), f"-L{HERE}",
+           "-ljvpfa", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for the torch binding:\n{' '.join(cmd)}\n{r.stderr[-4000:]}")
+    if verbose:
+        print(f"built {BINDING_LIB}", flush=True)
+    return BINDING_LIB
 
 
 HOST_CHECK_SRC = os.path.join(os.path.dirname(HERE), "tests", "cabi_host", "host_check.cpp")

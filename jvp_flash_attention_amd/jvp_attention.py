@@ -346,56 +346,27 @@ class _AttachTangent(Function):
         return g, None, None, None, None
 
 
-# Twins of the three Functions above in the older style (``forward(ctx, ...)``, no ``setup_context``).
-# ``Function.apply`` binds the arguments of a ``setup_context`` Function through ``inspect.signature``
-# on every call, about 25 us each; that style is only needed under ``torch.func`` transforms and
-# while ``torch.compile`` traces, so ordinary eager calls take these.
-
-
-class _DualCoreEager(Function):
-    @staticmethod
-    def forward(ctx, q, k, v, q_t, k_t, v_t, mask_tensor, MASK_TYPE, causal, sm_scale, dropout_p=0.0, seed=0):
-        o, o_t, M, mu = _lib.backend().fwd(q, k, v, q_t, k_t, v_t, mask_tensor, MASK_TYPE, causal, sm_scale,
-                                           dropout_p, seed)
-        ctx.set_materialize_grads(False)
-        ctx.mark_non_differentiable(M, mu)
-        ctx.save_for_backward(q, k, v, q_t, k_t, v_t, o, o_t, M, mu)
-        ctx.mask_tensor, ctx.MASK_TYPE, ctx.causal, ctx.sm_scale = mask_tensor, MASK_TYPE, causal, sm_scale
-        ctx.dropout_p, ctx.philox_seed = dropout_p, seed
-        return o, o_t, M, mu
-
-    backward = _DualCore.backward
-
-
-class _PlainCoreEager(Function):
-    @staticmethod
-    def forward(ctx, q, k, v, mask_tensor, MASK_TYPE, causal, sm_scale, dropout_p=0.0, seed=0):
-        o, _o_t, M, _mu = _lib.backend().fwd(q, k, v, None, None, None, mask_tensor, MASK_TYPE, causal, sm_scale,
-                                             dropout_p, seed)
-        ctx.set_materialize_grads(False)
-        ctx.mark_non_differentiable(M)
-        ctx.save_for_backward(q, k, v, o, M)
-        ctx.mask_tensor, ctx.MASK_TYPE, ctx.causal, ctx.sm_scale = mask_tensor, MASK_TYPE, causal, sm_scale
-        ctx.dropout_p, ctx.philox_seed = dropout_p, seed
-        return o, M
-
-    backward = _PlainCore.backward
-
-
-class _AttachTangentEager(Function):
-    @staticmethod
-    def forward(ctx, o, o_t, q, k, v):
-        ctx.set_materialize_grads(False)
-        ctx.save_for_forward(o_t)
-        return o.view_as(o)
-
-    jvp = _AttachTangent.jvp
-    backward = _AttachTangent.backward
-
-
 def _transforms_active() -> bool:
     """A ``torch.func`` transform (jvp, vmap, grad ...) is running."""
     return torch._C._functorch.peek_interpreter_stack() is not None
+
+
+def _attend(q, k, v, attn_mask, dropout_p, causal, sm_scale, level):
+    """An eager call outside of ``torch.func`` transforms, on tensors that may be dual tensors of ``level``: natively
+    from here on (``csrc/torch_binding.cpp``), autograd included."""
+    mask, kind = None, _lib.MASK_NONE
+    if attn_mask is not None:
+        _validate(q, k, v, attn_mask, dropout_p, causal)
+        mask, kind = _classify_mask(attn_mask, q, True)
+    o = _lib.backend().attend(q, k, v, mask, kind, causal, sm_scale, dropout_p, _new_dropout_seed(dropout_p), level)
+    if o is None:
+        _validate(q, k, v, attn_mask, dropout_p, causal)  # says what is wrong
+        raise ValueError("unsupported arguments")
+    return o
+
+
+def _native() -> bool:
+    return hasattr(_lib.backend(), "attend") and not _transforms_active()
 
 
 class JVPAttn(Function):
@@ -542,12 +513,11 @@ class JVPAttn(Function):
         USE_TMA: bool = True,
     ) -> Tensor:
         """Plain attention forward, differentiable in q, k, v (JA:2700-2752)."""
-        if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
-            q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         if torch.compiler.is_compiling():
             # the same computation through a Function the tracer can follow (no custom jvp, no
             # data-dependent mask checks); the kernels appear in the graph as jvpfa::fwd / jvpfa::bwd, with
             # dropout as jvpfa::fwd_drop / jvpfa::bwd_drop, which draw and carry the seed themselves
+            q, k, v = _dense(q), _dense(k), _dense(v)
             _validate(q, k, v, attn_mask, dropout_p, causal)
             scale = q.shape[-1] ** -0.5 if sm_scale is None else sm_scale
             mask_tensor, MASK_TYPE = _classify_mask(attn_mask, q, False)
@@ -556,15 +526,9 @@ class JVPAttn(Function):
                 return o
             o, _M = _PlainCore.apply(q, k, v, mask_tensor, MASK_TYPE, causal, scale, 0.0, 0)
             return o
-        if fwAD._current_level < 0 and not _transforms_active():
-            # no forward-mode level anywhere: nothing can ask for a tangent, so the plain Function
-            # (same kernels, same backward) stands in for JVPAttn.apply and its per-call set-up
-            _validate(q, k, v, attn_mask, dropout_p, causal)
-            scale = q.shape[-1] ** -0.5 if sm_scale is None else sm_scale
-            mask_tensor, MASK_TYPE = _classify_mask(attn_mask, q, True)
-            o, _M = _PlainCoreEager.apply(q, k, v, mask_tensor, MASK_TYPE, causal, scale, dropout_p,
-                                          _new_dropout_seed(dropout_p))
-            return o
+        if fwAD._current_level < 0 and _native():
+            return _attend(q, k, v, attn_mask, dropout_p, causal, sm_scale, -1)
+        q, k, v = _dense(q), _dense(k), _dense(v)
         out: JVPAttn.FwdOut = JVPAttn.apply(
             q, k, v, None, None, None, attn_mask, dropout_p, causal, sm_scale, warp_specialize, USE_TMA
         )
@@ -612,8 +576,9 @@ class JVPAttn(Function):
                                                                 causal, scale, 0.0, 0)
                     return fwAD.make_dual(o, o_t)
             return JVPAttn.fwd(q, k, v, attn_mask, dropout_p, causal, sm_scale, warp_specialize, USE_TMA)
-        if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
-            q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        if _native():
+            return _attend(q, k, v, attn_mask, dropout_p, causal, sm_scale, fwAD._current_level)
+        q, k, v = _dense(q), _dense(k), _dense(v)
         q_p, q_t = fwAD.unpack_dual(q)
         k_p, k_t = fwAD.unpack_dual(k)
         v_p, v_t = fwAD.unpack_dual(v)
@@ -627,13 +592,12 @@ class JVPAttn(Function):
         q_t = torch.zeros_like(q_p) if q_t is None else _dense(q_t)
         k_t = torch.zeros_like(k_p) if k_t is None else _dense(k_t)
         v_t = torch.zeros_like(v_p) if v_t is None else _dense(v_t)
-        core, attach = (_DualCore, _AttachTangent) if _transforms_active() else (_DualCoreEager, _AttachTangentEager)
-        o, o_t, _M, _mu = core.apply(
+        o, o_t, _M, _mu = _DualCore.apply(
             _dense(q_p), _dense(k_p), _dense(v_p), q_t, k_t, v_t, mask_tensor, MASK_TYPE, causal, sm_scale,
             dropout_p, _new_dropout_seed(dropout_p),
         )
         # NOTE: q, k, v are passed as dual tensors so that autograd calls jvp(), which hands back O'.
-        return attach.apply(o, o_t, q, k, v)
+        return _AttachTangent.apply(o, o_t, q, k, v)
 
     @staticmethod
     def jvp(ctx: "JVPAttn.FnCtx", gq: Tensor, gk: Tensor, gv: Tensor, *_) -> "JVPAttn.JVPOut":

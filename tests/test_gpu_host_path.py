@@ -1,0 +1,55 @@
+"""The native path of eager calls (``csrc/torch_binding.cpp``): which gradients arrive, and what it refuses."""
+import numpy as np
+import pytest
+import torch
+import torch.autograd.forward_ad as fwAD
+
+from jvp_flash_attention_amd import JVPAttn, attention
+from oracle import dense
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(D, dtype, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(2, 3, 75, D, generator=g).to(dtype) for _ in range(8)]
+
+
+@pytest.mark.parametrize("D,dtype", [(16, torch.bfloat16), (64, torch.float16), (32, torch.float32)])
+@pytest.mark.parametrize("of", ["o", "ot", "both"])
+@pytest.mark.parametrize("six", [False, True])
+def test_gradients_of_either_output_or_both(D, dtype, of, six):
+    """A gradient that does not arrive counts as zero; without one for O' the tangent inputs get zeros."""
+    print("case", D, dtype, of, six, flush=True)
+    cpu = _inputs(D, dtype)
+    leaves = [x.cuda().requires_grad_(i < 3 or six) for i, x in enumerate(cpu[:6])]
+    go, gt = cpu[6].cuda(), cpu[7].cuda()
+    with fwAD.dual_level():
+        o, ot = fwAD.unpack_dual(JVPAttn.fwd_dual(*(fwAD.make_dual(p, t) for p, t in zip(leaves[:3], leaves[3:]))))
+        outs, gs = {"o": ((o,), (go,)), "ot": ((ot,), (gt,)), "both": ((o, ot), (go, gt))}[of]
+        grads = torch.autograd.grad(outs, leaves[: 6 if six else 3], gs)
+    f = [x.double().numpy() for x in cpu]
+    f[6] = f[6] if of != "ot" else np.zeros_like(f[6])
+    f[7] = f[7] if of != "o" else np.zeros_like(f[7])
+    want = dense.backward(*f)
+    for name, got in zip(("dq", "dk", "dv", "dqt", "dkt", "dvt"), grads):
+        w = want[name]
+        bar = 1e-4 if dtype == torch.float32 else 2e-2 * np.abs(w).max()
+        assert np.abs(got.double().cpu().numpy() - w).max() <= bar, name
+
+
+def test_a_second_derivative_is_refused():
+    q, k, v = (x.cuda().requires_grad_() for x in _inputs(64, torch.bfloat16)[:3])
+    (dq,) = torch.autograd.grad(attention(q, k, v).float().sum(), q, create_graph=True)
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        dq.float().sum().backward()
+
+
+def test_arguments_are_refused_with_the_reason():
+    q, k, v = (x.cuda() for x in _inputs(64, torch.bfloat16)[:3])
+    with pytest.raises(AssertionError, match="one dtype"):
+        attention(q, k.half(), v)
+    with pytest.raises(AssertionError, match="HEAD_DIM_K"):
+        attention(*(x[..., :48] for x in (q, k, v)))
+    with pytest.raises(AssertionError, match="dropout_p"):
+        attention(q, k, v, dropout_p=1.5)
