@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define JVPFA_ABI_VERSION 8
+#define JVPFA_ABI_VERSION 9
 
 enum jvpfa_dtype { JVPFA_BF16 = 0, JVPFA_FP16 = 1, JVPFA_FP32 = 2 };
 
@@ -152,11 +152,21 @@ typedef struct jvpfa_bwd_args {
                                tiles_q and tiles_k are both NULL or both set */
   int32_t Lk, Hk;           /* as in jvpfa_fwd_args; dk, dv, dkt, dvt have the shape of k */
   const uint32_t *mask_bits; /* optional, boolean masks only: the copy written by jvpfa_mask_bits(), or NULL */
+  /* optional workspace for grouped heads (Hk < p.H), or NULL: jvpfa_bwd_split_workspace_bytes() bytes of device
+   * memory, 16-byte aligned, contents don't-care.  Where one workgroup per 128 keys of a key/value head would leave
+   * compute units idle, the query heads of a group are then dealt to several workgroups that leave fp32 shares of the
+   * key and value gradients there, and a second kernel adds them up.  Results agree with the unsplit launch to rounding. */
+  void *split_workspace;
+  uint64_t split_workspace_bytes;
 } jvpfa_bwd_args;
 
 int jvpfa_bwd(const jvpfa_bwd_args *args, void *hip_stream);
 
 size_t jvpfa_bwd_workspace_bytes(int32_t Z, int32_t H, int32_t L);
+
+/* Bytes of split_workspace with which jvpfa_bwd would split this problem on the current device (tangent_grads: dqt,
+ * dkt, dvt are asked for too); 0 if it would not. */
+size_t jvpfa_bwd_split_workspace_bytes(const jvpfa_problem *p, int32_t Lk, int32_t Hk, int32_t tangent_grads);
 
 /*
  * jvpfa_bwd for callers that cannot hand over a workspace because they cannot allocate one: code

@@ -16,10 +16,10 @@ import torch
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libjvpfa.so")
 
-ABI_VERSION = 8
+ABI_VERSION = 9
 DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 MASK_NONE, MASK_BOOL, MASK_ADD = 0, 1, 2
-EXPORTS = ("jvpfa_fwd", "jvpfa_bwd", "jvpfa_fwd_split_workspace_bytes", "jvpfa_dropout_keep", "jvpfa_bwd_workspace_bytes", "jvpfa_bwd_static", "jvpfa_bwd_static_max_rows", "jvpfa_mask_tiles", "jvpfa_mask_tiles_bytes",
+EXPORTS = ("jvpfa_fwd", "jvpfa_bwd", "jvpfa_fwd_split_workspace_bytes", "jvpfa_dropout_keep", "jvpfa_bwd_workspace_bytes", "jvpfa_bwd_split_workspace_bytes", "jvpfa_bwd_static", "jvpfa_bwd_static_max_rows", "jvpfa_mask_tiles", "jvpfa_mask_tiles_bytes",
            "jvpfa_mask_bits", "jvpfa_mask_bits_bytes",
            "jvpfa_abi_version", "jvpfa_error_string")
 
@@ -67,6 +67,7 @@ class BwdArgs(C.Structure):
         ("tiles_q", C.c_void_p), ("tiles_k", C.c_void_p),
         ("Lk", C.c_int32), ("Hk", C.c_int32),
         ("mask_bits", C.c_void_p),
+        ("split_workspace", C.c_void_p), ("split_workspace_bytes", C.c_uint64),
     ]
 
 
@@ -89,6 +90,8 @@ def load() -> C.CDLL:
         lib.jvpfa_bwd.restype = C.c_int
         lib.jvpfa_bwd_workspace_bytes.argtypes = [C.c_int32, C.c_int32, C.c_int32]
         lib.jvpfa_bwd_workspace_bytes.restype = C.c_size_t
+        lib.jvpfa_bwd_split_workspace_bytes.argtypes = [C.POINTER(Problem), C.c_int32, C.c_int32, C.c_int32]
+        lib.jvpfa_bwd_split_workspace_bytes.restype = C.c_size_t
         lib.jvpfa_bwd_static.argtypes = [C.POINTER(BwdArgs), C.c_void_p]
         lib.jvpfa_bwd_static.restype = C.c_int
         lib.jvpfa_bwd_static_max_rows.argtypes = []
@@ -216,8 +219,8 @@ _split_enabled = True
 
 def set_split(enabled: bool) -> None:
     """Switch the split of small launches over several workgroups per block on or off (default on): with it a
-    launch that would leave most compute units idle (one sequence, few heads) hands the library a workspace for
-    partial results, see ``split_workspace`` in ``include/jvpfa.h``."""
+    launch that would leave most compute units idle (one sequence, few heads; few key/value heads in the backward)
+    hands the library a workspace for partial results, see ``split_workspace`` in ``include/jvpfa.h``."""
     global _split_enabled
     _split_enabled = bool(enabled)
 

@@ -7,6 +7,7 @@
 #include <mutex>
 
 #include "api_common.hpp"
+#include "split.hpp"
 
 namespace jvpfa {
 #define JVPFA_DECL(name) int name(const BwdParams &, int, bool, bool, hipStream_t);
@@ -27,6 +28,14 @@ using namespace jvpfa;
 extern "C" size_t jvpfa_bwd_workspace_bytes(int32_t Z, int32_t H, int32_t L) {
   if (Z < 1 || H < 1 || L < 1) return 0;
   return 3 * stat_floats(Z, H, L) * sizeof(float);
+}
+
+extern "C" size_t jvpfa_bwd_split_workspace_bytes(const jvpfa_problem *p, int32_t Lk, int32_t Hk, int32_t tangent_grads) {
+  if (!p || check_problem(*p) != JVPFA_OK || check_kv_shape(*p, Lk, Hk) != JVPFA_OK) return 0;
+  Lk = Lk > 0 ? Lk : p->L;
+  Hk = Hk > 0 ? Hk : p->H;
+  const int chunks = bwd_kv_chunks(*p, Lk, Hk);
+  return chunks > 1 ? bwd_part_floats(*p, Lk, Hk, chunks, tangent_grads != 0) * sizeof(float) : 0;
 }
 
 // Everything jvpfa_bwd does, with the row statistics of the pre-pass in `workspace`.
@@ -61,6 +70,14 @@ static int bwd_impl(const jvpfa_bwd_args *a, void *workspace, void *hip_stream) 
   p.go = a->go; p.gt = a->gt;
   p.dq = a->dq; p.dk = a->dk; p.dv = a->dv;
   p.dqt = a->dqt; p.dkt = a->dkt; p.dvt = a->dvt;
+  if (a->split_workspace) {  // few dk/dv workgroups: split the query heads of every group, if the workspace suffices
+    const int chunks = bwd_kv_chunks(a->p, p.pr.Lk, p.pr.Hk);
+    if (chunks > 1 && aligned16(a->split_workspace) &&
+        a->split_workspace_bytes >= bwd_part_floats(a->p, p.pr.Lk, p.pr.Hk, chunks, ntg == 3) * sizeof(float)) {
+      p.pr.chunks = chunks;
+      p.pr.part = static_cast<float *>(a->split_workspace);
+    }
+  }
   const size_t n = stat_floats(a->p.Z, a->p.H, a->p.L);
   p.d1 = static_cast<float *>(workspace);
   p.a = p.d1 + n;

@@ -72,6 +72,16 @@ static auto pick_dkdv_for(const BwdParams &p, bool no_go, bool grouped, bool fol
   return pick_dkdv<T, D, MODE, MASK>(no_go, grouped, fold_kv, drop);
 }
 
+// Adds up the shares of dk, dv (dk', dv' of the tangent mode; all four where the dual kernel folds them in) that a
+// launch over pr.chunks query heads groups left, see split.hpp.
+template <typename T, int D> static void launch_kv_merge(const BwdParams &p, bool tangent, bool four, hipStream_t stream) {
+  if (p.pr.chunks <= 1) return;
+  const size_t elems = (size_t)p.pr.Z * p.pr.Hk * p.pr.Lk * D;
+  T *dk = reinterpret_cast<T *>(p.dk), *dv = reinterpret_cast<T *>(p.dv), *dkt = reinterpret_cast<T *>(p.dkt), *dvt = reinterpret_cast<T *>(p.dvt);
+  hipLaunchKernelGGL((bwd_kv_merge_kernel<T>), dim3((unsigned)((elems / 8 + 255) / 256), four ? 4 : 2), dim3(256), 0, stream, p.pr.part,
+                     p.pr.chunks, elems, tangent ? dkt : dk, tangent ? dvt : dv, dkt, dvt);
+}
+
 // six: all six gradients were asked for.  The dual launch then also writes what BwdFold says, and the tangent
 // launch skips the kernels whose outputs exist already.
 template <typename T, int D, int MODE, int MASK>
@@ -82,7 +92,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
   if (blocks > 0x7fffffffLL) return -2;
   // the dk/dv kernels run one workgroup per 128 keys of a key/value head (the same count as for dq
   // when k, v have q's shape)
-  const long long kv_blocks = (long long)((p.pr.Lk + BWD_BLK - 1) / BWD_BLK) * p.pr.Z * p.pr.Hk;
+  const long long kv_blocks = (long long)((p.pr.Lk + BWD_BLK - 1) / BWD_BLK) * p.pr.Z * p.pr.Hk * p.pr.chunks;
   if (kv_blocks > 0x7fffffffLL) return -2;
   if (p.pr.drop_thr != 0) {
     // dropout: the direct-to-LDS kernels carry it for the 16-bit types, the register-staged ones for fp32
@@ -98,13 +108,14 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), kv_lds);
       if (rc != 0) return rc;
       hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(Cfg2::NT), kv_lds, stream, p);
+      launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
       hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(Cfg2::NT), Cfg2::DQ_LDS, stream, p);
       return hipGetLastError() == hipSuccess ? 0 : -6;
     } else if constexpr (sizeof(T) == 2 && D == 256 && MODE == BWD_DUAL) {
       using CfgP = BwdPairCfg<T, D>;
       const bool no_go = p.go == nullptr;
       const long long qblocks = (long long)((p.pr.L + CfgP::BLK - 1) / CfgP::BLK) * p.pr.Z * p.pr.H;
-      const long long kblocks = (long long)((p.pr.Lk + CfgP::BLK - 1) / CfgP::BLK) * p.pr.Z * p.pr.Hk;
+      const long long kblocks = (long long)((p.pr.Lk + CfgP::BLK - 1) / CfgP::BLK) * p.pr.Z * p.pr.Hk * p.pr.chunks;
       if (qblocks > 0x7fffffffLL || kblocks > 0x7fffffffLL) return -2;
       void (*kq)(const BwdParams) = no_go ? bwdp_dq_kernel<T, D, MASK, false, false, true> : bwdp_dq_kernel<T, D, MASK, true, false, true>;
       void (*kkv)(const BwdParams) = no_go ? bwdp_dkdv_kernel<T, D, MASK, false, true> : bwdp_dkdv_kernel<T, D, MASK, true, true>;
@@ -112,6 +123,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), CfgP::DKV_LDS);
       if (rc != 0) return rc;
       hipLaunchKernelGGL(kkv, dim3((unsigned)kblocks), dim3(CfgP::NT), CfgP::DKV_LDS, stream, p);
+      launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
       hipLaunchKernelGGL(kq, dim3((unsigned)qblocks), dim3(CfgP::NT), CfgP::DQ_LDS, stream, p);
       return hipGetLastError() == hipSuccess ? 0 : -6;
     } else if constexpr (sizeof(T) == 2 && D == 256) {
@@ -123,6 +135,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), CfgK::DKV_LDS);
       if (rc != 0) return rc;
       hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(CfgK::NT), CfgK::DKV_LDS, stream, p);
+      launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
       hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(CfgW::NT), CfgW::DQ_LDS, stream, p);
       return hipGetLastError() == hipSuccess ? 0 : -6;
     } else {
@@ -132,6 +145,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), Cfg::DKV_LDS);
       if (rc != 0) return rc;
       hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(BWD_NT), Cfg::DKV_LDS, stream, p);
+      launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
       hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(BWD_NT), Cfg::DQ_LDS, stream, p);
       return hipGetLastError() == hipSuccess ? 0 : -6;
     }
@@ -180,7 +194,10 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     int rc = allow_lds(reinterpret_cast<const void *>(kq), Cfg2::DQ_LDS);
     if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), kv_lds);
     if (rc != 0) return rc;
-    if (run_kv) hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(Cfg2::NT), kv_lds, stream, p);
+    if (run_kv) {
+      hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(Cfg2::NT), kv_lds, stream, p);
+      launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, MODE == BWD_DUAL && six && Fold::KV, stream);
+    }
     if (run_q) hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(Cfg2::NT), Cfg2::DQ_LDS, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -6;
    }
@@ -189,7 +206,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     using CfgP = BwdPairCfg<T, D>;
     const bool no_go = p.go == nullptr;
     const long long qblocks = (long long)((p.pr.L + CfgP::BLK - 1) / CfgP::BLK) * p.pr.Z * p.pr.H;
-    const long long kblocks = (long long)((p.pr.Lk + CfgP::BLK - 1) / CfgP::BLK) * p.pr.Z * p.pr.Hk;
+    const long long kblocks = (long long)((p.pr.Lk + CfgP::BLK - 1) / CfgP::BLK) * p.pr.Z * p.pr.Hk * p.pr.chunks;
     if (qblocks > 0x7fffffffLL || kblocks > 0x7fffffffLL) return -2;
     void (*kq)(const BwdParams) = no_go ? bwdp_dq_kernel<T, D, MASK, false> : bwdp_dq_kernel<T, D, MASK, true>;
     if (six) kq = no_go ? bwdp_dq_kernel<T, D, MASK, false, true> : bwdp_dq_kernel<T, D, MASK, true, true>;
@@ -198,6 +215,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), CfgP::DKV_LDS);
     if (rc != 0) return rc;
     hipLaunchKernelGGL(kkv, dim3((unsigned)kblocks), dim3(CfgP::NT), CfgP::DKV_LDS, stream, p);
+    launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
     hipLaunchKernelGGL(kq, dim3((unsigned)qblocks), dim3(CfgP::NT), CfgP::DQ_LDS, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -6;
   } else if constexpr (sizeof(T) == 2 && D == 256) {
@@ -210,6 +228,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), CfgK::DKV_LDS);
     if (rc != 0) return rc;
     hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(CfgK::NT), CfgK::DKV_LDS, stream, p);
+    launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
     // (six: the tangent launch of a six-gradient call, whose dq' the dual launch has written already)
     if (!(MODE == BWD_TANGENT && six)) hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(CfgW::NT), CfgW::DQ_LDS, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -6;
@@ -220,6 +239,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), Cfg::DKV_LDS);
     if (rc != 0) return rc;
     hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(BWD_NT), Cfg::DKV_LDS, stream, p);
+    launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
     hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(BWD_NT), Cfg::DQ_LDS, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -6;
   }

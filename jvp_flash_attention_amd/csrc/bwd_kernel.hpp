@@ -390,10 +390,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;  // queries, keys
   const int nkb = (Lk + BWD_BLK - 1) / BWD_BLK;
-  const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk);
-  const int zhk = id / nkb;
+  const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks);
+  const int zhk = id / nkb / pr.chunks, chunk = id / nkb % pr.chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nkb;  // causal: the first key blocks have the longest query loops
-  const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = pr.H / pr.Hk;
+  const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = pr.H / pr.Hk / pr.chunks;
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
   const int r = lane % 32, g = lane / 32, pr32 = perm32(r);
 
@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   const float sl2 = pr.scale * LOG2E;
   const int istart = pr.causal ? (k0 / BWD_T) * BWD_T : 0;
   for (int gi = 0; gi < group; ++gi) {
-  const int h = hk * group + gi;  // query head
+  const int h = (hk * pr.chunks + chunk) * group + gi;  // query head
   const size_t head = ((size_t)z * pr.H + h) * L * D;
   const size_t srow = ((size_t)z * pr.H + h) * L;
   const T *Qg = reinterpret_cast<const T *>(p.q) + head;
@@ -635,8 +635,9 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   }  // query heads of the group
 
   if (krow < Lk) {
-    T *outk = reinterpret_cast<T *>(TAN ? p.dkt : p.dk) + kvhead + (size_t)krow * D;
-    T *outv = reinterpret_cast<T *>(TAN ? p.dvt : p.dv) + kvhead + (size_t)krow * D;
+    T *outk = reinterpret_cast<T *>(TAN ? p.dkt : p.dk), *outv = reinterpret_cast<T *>(TAN ? p.dvt : p.dv);
+    float *partk = kv_part(pr, D, 2, 0, chunk), *partv = kv_part(pr, D, 2, 1, chunk);
+    const size_t off = kvhead + (size_t)krow * D + 8 * g;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
 #pragma unroll
@@ -647,8 +648,8 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
           xk[e] = dK[db][8 * hf + e] * pr.scale;
           xv[e] = dV[db][8 * hf + e];
         }
-        store8<T>(outk + 32 * db + 16 * hf + 8 * g, xk);
-        store8<T>(outv + 32 * db + 16 * hf + 8 * g, xv);
+        store8_or_part<T>(outk, partk, off + 32 * db + 16 * hf, xk);
+        store8_or_part<T>(outv, partv, off + 32 * db + 16 * hf, xv);
       }
     }
   }

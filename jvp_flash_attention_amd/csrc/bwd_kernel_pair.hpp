@@ -419,10 +419,11 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nblk = (Lk + Cfg::BLK - 1) / Cfg::BLK;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk);
-  const int zh = id / nblk;
+  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * pr.chunks);
+  const int zh = id / nblk / pr.chunks, chunk = id / nblk % pr.chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nblk;
-  const int z = zh / pr.Hk, hk = zh % pr.Hk, group = pr.H / pr.Hk;
+  const int z = zh / pr.Hk, hk = zh % pr.Hk, group = pr.H / pr.Hk / pr.chunks;
+  const int h0 = (hk * pr.chunks + chunk) * group;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int pairi = wave >> 1, role = wave & 1;
@@ -433,13 +434,15 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
   const int kld = krow < Lk ? krow : Lk - 1;
   const uint32_t drop_lane = DROP ? (uint32_t)kld * DROP_C_KEY + (uint32_t)(8 * g) * DROP_C_ROW : 0u;
   // role 0 writes dV, role 1 dK
-  T *out = reinterpret_cast<T *>(role ? p.dk : p.dv) + head + (size_t)krow * D;
+  T *out = reinterpret_cast<T *>(role ? p.dk : p.dv);
+  float *part = kv_part(pr, D, 2, 1 - role, chunk);
+  const size_t off = head + (size_t)krow * D;
   if constexpr (MASK != MASK_NONE) {
     if (pr.klimit && k0 >= pr.klimit[z]) {
       if (krow < Lk) {
         float zero8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int d0 = 8 * g; d0 < D; d0 += 16) store8<T>(out + d0, zero8);
+        for (int d0 = 8 * g; d0 < D; d0 += 16) store8_or_part<T>(out, part, off + d0, zero8);
       }
       return;
     }
@@ -511,7 +514,7 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
     mask_small = pr.ms[2] >= 0 && pr.ms[3] >= 0 && 8 * pr.ms[2] + (int64_t)Lk * pr.ms[3] < lim;
     mlane = (uint32_t)(8 * g * pr.ms[2] + (int64_t)kld * pr.ms[3]);
   }
-  int h = hk * group;
+  int h = h0;
   const char *Qb = nullptr, *gTb = nullptr, *Gb = nullptr, *Qtb = nullptr;
   const float *st_p[4] = {nullptr, nullptr, nullptr, nullptr};
   auto set_query_head = [&](int hq) {
@@ -751,8 +754,8 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
   const int t_end = mask_small ? max(t_diag, (L - istart) / BT) : t_diag;
   for (int gi = 0; gi < group; ++gi) {
     if (gi > 0) __syncthreads();
-    set_query_head(hk * group + gi);
-    set_list(hk * group + gi);
+    set_query_head(h0 + gi);
+    set_list(h0 + gi);
     icur = query_of(tlist ? tlist[1] : 0, 0);
     inext = query_of(tlist ? tlist[1 + (min(1, ntiles - 1) >> 1)] : 0, min(1, ntiles - 1));
     if constexpr (MASK != MASK_NONE) fetch_mask_tile(icur);
@@ -775,7 +778,7 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = acc[db][8 * hf + e] * os;
-        store8<T>(out + 32 * db + 16 * hf + 8 * g, x);
+        store8_or_part<T>(out, part, off + 32 * db + 16 * hf + 8 * g, x);
       }
     }
   }

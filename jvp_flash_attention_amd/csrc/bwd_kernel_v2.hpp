@@ -65,24 +65,24 @@ template <int N> __device__ __forceinline__ void lds_wait4(u32x4 &a, u32x4 &b, u
 // SLOTn are LDS tile slots inside a stage; a tile is BT rows, row-major, chunks swizzled by swz_u.
 // the loads of the next tile are spread over the first three quarters of a tile's steps
 constexpr int bwd_spread(int nstep) { return 3 * nstep / 4; }
-#define JVPFA_BWD2_COMMON(Cfg, STREAMED_ROWS, OWN_ROWS, OWN_HEADS)                                                                                      \
+#define JVPFA_BWD2_COMMON(Cfg, STREAMED_ROWS, OWN_ROWS, OWN_HEADS, CHUNKS)                                                                                      \
   constexpr int CH = Cfg::CH, ROWB = Cfg::ROWB, TILEB = Cfg::TILEB, IPW = Cfg::IPW, BT = Cfg::BT;                   \
   constexpr int KK = D / 16, DB = D / 32;                                                                           \
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];                                        \
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem_raw;                                                              \
   const Problem &pr = p.pr;                                                                                         \
   const int L = pr.L;                                                                                               \
-  /* a workgroup owns 128 of the OWN_ROWS rows of one (z, head out of OWN_HEADS) */                               \
+  /* a workgroup owns 128 of the OWN_ROWS rows of one (z, head out of OWN_HEADS), or one of CHUNKS shares of it */ \
   const int nblk = ((OWN_ROWS) + Cfg::BLK - 1) / Cfg::BLK;                                                          \
-  const int id = xcd_remap(bid, nblk, pr.Z * (OWN_HEADS));                                                   \
-  const int zh = id / nblk;                                                                                         \
+  const int id = xcd_remap(bid, nblk, pr.Z * (OWN_HEADS) * (CHUNKS));                                               \
+  const int zh = id / nblk / (CHUNKS), chunk = id / nblk % (CHUNKS);                                                \
   const int z = zh / (OWN_HEADS), h = zh % (OWN_HEADS);                                                             \
   const int tid = threadIdx.x;                                                                                      \
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;                                   \
   const int r = lane % 32, g = lane / 32, pr32 = perm32(r);                                                         \
   const size_t head = (size_t)zh * (OWN_ROWS) * D;                                                                  \
   const size_t srow = (size_t)zh * (OWN_ROWS);                                                                      \
-  (void)z; (void)h; (void)srow;                                                                                     \
+  (void)z; (void)h; (void)srow; (void)chunk;                                                                                     \
   /* direct loads: instruction i of this wave fills LDS chunks 64*(wave*IPW+i) .. +63 of a tile */                   \
   int ld_row[IPW];                                                                                                  \
   uint32_t ld_c[IPW];                                                                                               \
@@ -150,7 +150,7 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   static_assert(!SIX || DUAL, "dq' rides on the dual mode");
-  JVPFA_BWD2_COMMON(Cfg, pr.Lk, pr.L, pr.H)  // owns query rows, streams key tiles
+  JVPFA_BWD2_COMMON(Cfg, pr.Lk, pr.L, pr.H, 1)  // owns query rows, streams key tiles
   const int qb = pr.causal ? nblk - 1 - id % nblk : id % nblk;
   const int q0 = qb * Cfg::BLK;
   const int qrow = q0 + wave * 32 + r;
@@ -501,29 +501,34 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   static_assert(!SIX || (DUAL && D <= 64), "dk', dv' ride on the dual mode, where the accumulators fit");
-  JVPFA_BWD2_COMMON(Cfg, pr.L, pr.Lk, pr.Hk)  // owns key rows (h: key/value head), streams query tiles
+  JVPFA_BWD2_COMMON(Cfg, pr.L, pr.Lk, pr.Hk, GROUPED ? pr.chunks : 1)  // owns key rows (h: key/value head), streams query tiles
   const int kb = id % nblk;  // causal: the first key blocks have the longest query loops
   const int k0 = kb * Cfg::BLK;
   const int krow = k0 + wave * 32 + r;
   const int Lk = pr.Lk;  // keys; L counts queries
   const int kld = krow < Lk ? krow : Lk - 1;
   const uint32_t drop_lane = DROP ? (uint32_t)kld * DROP_C_KEY + (uint32_t)(8 * g) * DROP_C_ROW : 0u;
+  // 8 columns of this lane's row of dk, dv (dk', dv'); of a share of them where the group's query heads are split
+  auto store_grads = [&](int d0, const float *xk, const float *xv, const float *xkt, const float *xvt) {
+    constexpr int NT = SIX ? 4 : 2;
+    const size_t off = head + (size_t)krow * D + d0;
+    auto put = [&](void *dst, int t, const float *x) {
+      store8_or_part<T>(reinterpret_cast<T *>(dst), GROUPED ? kv_part(pr, D, NT, t, chunk) : nullptr, off, x);
+    };
+    put(TAN ? p.dkt : p.dk, 0, xk);
+    put(TAN ? p.dvt : p.dv, 1, xv);
+    if constexpr (SIX) {
+      put(p.dkt, 2, xkt);
+      put(p.dvt, 3, xvt);
+    }
+  };
   if constexpr (MASK != MASK_NONE) {
     // a key block that the caller's hint declares fully masked has zero gradients
     if (pr.klimit && k0 >= pr.klimit[z]) {
       if (krow < Lk) {
-        T *outk = reinterpret_cast<T *>(MODE == BWD_TANGENT ? p.dkt : p.dk) + head + (size_t)krow * D;
-        T *outv = reinterpret_cast<T *>(MODE == BWD_TANGENT ? p.dvt : p.dv) + head + (size_t)krow * D;
         float zero8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int d0 = 8 * g; d0 < D; d0 += 16) {
-          store8<T>(outk + d0, zero8);
-          store8<T>(outv + d0, zero8);
-          if constexpr (SIX) {
-            store8<T>(reinterpret_cast<T *>(p.dkt) + head + (size_t)krow * D + d0, zero8);
-            store8<T>(reinterpret_cast<T *>(p.dvt) + head + (size_t)krow * D + d0, zero8);
-          }
-        }
+        for (int d0 = 8 * g; d0 < D; d0 += 16) store_grads(d0, zero8, zero8, zero8, zero8);
       }
       return;
     }
@@ -598,8 +603,9 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   // the shapes the reference admits); hq is the current one, and what depends on it is set per head:
   // tile slots 0 Q, 1 G (gO; gT in TANGENT; gT again in DUAL without gO), 2 Q', 3 gT, and the
   // statistics slots PLAIN M, d1 | DUAL M, mu, a, d2 (= d1 + d2) | TANGENT M, a
-  const int group = GROUPED ? pr.H / pr.Hk : 1;
-  int hq = h * group;
+  const int group = GROUPED ? pr.H / pr.Hk / pr.chunks : 1;  // ... of this workgroup's share
+  const int hq0 = GROUPED ? h * (pr.H / pr.Hk) + chunk * group : h;
+  int hq = hq0;
   const char *Qb = nullptr, *gTb = nullptr, *Gb = nullptr, *Qtb = nullptr;
   const float *st_p[4] = {nullptr, nullptr, nullptr, nullptr};
   const uint32_t *bits_head = nullptr;  // MASK_BITS: the packed mask words of the current query head's plane
@@ -618,7 +624,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
     if constexpr (MASK == MASK_TILE)
       mt_head = reinterpret_cast<const char *>(pr.mask) + (z * pr.ms[0] + hq * pr.ms[1] + (int64_t)k0) * (int64_t)sizeof(T);
   };
-  set_query_head(h * group);
+  set_query_head(hq0);
 
   const int istart = pr.causal ? (k0 / BT) * BT : 0;
   // Query tiles visited, counted from istart: 0 .. ntiles-1, or the caller's list of the tiles of this
@@ -637,7 +643,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
       }
     }
   };
-  set_list(h * group);
+  set_list(hq0);
   // List elements are requested a tile ahead, unconditionally (from a harmless address when there is
   // no list: a branch around the read would split the tile loop's straight-line body).
   auto list_slot = [&](int i) { return tlist ? tlist + 1 + i : reinterpret_cast<const int *>(p.q); };
@@ -1007,8 +1013,8 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   for (int gi = 0; gi < group; ++gi) {
     if (gi > 0) {
       __syncthreads();  // every wave is done with the previous head's last tile: its stage may be refilled
-      set_query_head(h * group + gi);
-      if constexpr (GROUPED) set_list(h * group + gi);
+      set_query_head(hq0 + gi);
+      if constexpr (GROUPED) set_list(hq0 + gi);
     }
     tcur = tlist ? min(max(tlist[1], 0), tmax) : 0;
     tnext = tlist ? min(max(tlist[1 + min(1, ntiles - 1)], 0), tmax) : min(1, ntiles - 1);
@@ -1025,30 +1031,21 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   }
 
   if (krow < Lk) {
-    T *outk = reinterpret_cast<T *>(TAN ? p.dkt : p.dk) + head + (size_t)krow * D;
-    T *outv = reinterpret_cast<T *>(TAN ? p.dvt : p.dv) + head + (size_t)krow * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
-        float xk[8], xv[8];
+        float xk[8], xv[8], xkt[8], xvt[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           xk[e] = dK[db][8 * hf + e] * pr.scale;
           xv[e] = dV[db][8 * hf + e];
-        }
-        store8<T>(outk + 32 * db + 16 * hf + 8 * g, xk);
-        store8<T>(outv + 32 * db + 16 * hf + 8 * g, xv);
-        if constexpr (SIX) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            xk[e] = dKt[db][8 * hf + e] * pr.scale;
-            xv[e] = dVt[db][8 * hf + e];
+          if constexpr (SIX) {
+            xkt[e] = dKt[db][8 * hf + e] * pr.scale;
+            xvt[e] = dVt[db][8 * hf + e];
           }
-          const size_t o = head + (size_t)krow * D + 32 * db + 16 * hf + 8 * g;
-          store8<T>(reinterpret_cast<T *>(p.dkt) + o, xk);
-          store8<T>(reinterpret_cast<T *>(p.dvt) + o, xv);
         }
+        store_grads(32 * db + 16 * hf + 8 * g, xk, xv, xkt, xvt);
       }
     }
   }

@@ -337,10 +337,11 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;  // queries, keys
   const int nblk = (Lk + Cfg::BLK - 1) / Cfg::BLK;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk);
-  const int zh = id / nblk;
+  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * pr.chunks);
+  const int zh = id / nblk / pr.chunks, chunk = id / nblk % pr.chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nblk;  // causal: the first key blocks have the longest query loops
-  const int z = zh / pr.Hk, hk = zh % pr.Hk, group = pr.H / pr.Hk;
+  const int z = zh / pr.Hk, hk = zh % pr.Hk, group = pr.H / pr.Hk / pr.chunks;
+  const int h0 = (hk * pr.chunks + chunk) * group;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int r = lane % 32, g = lane / 32, pr32 = perm32(r);
@@ -349,8 +350,9 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   const int krow = k0 + wave * 32 + r;
   const int kld = krow < Lk ? krow : Lk - 1;
   const uint32_t drop_lane = DROP ? (uint32_t)kld * DROP_C_KEY + (uint32_t)(8 * g) * DROP_C_ROW : 0u;
-  T *outk = reinterpret_cast<T *>(TAN ? p.dkt : p.dk) + head + (size_t)krow * D;
-  T *outv = reinterpret_cast<T *>(TAN ? p.dvt : p.dv) + head + (size_t)krow * D;
+  T *outk = reinterpret_cast<T *>(TAN ? p.dkt : p.dk), *outv = reinterpret_cast<T *>(TAN ? p.dvt : p.dv);
+  float *partk = kv_part(pr, D, 2, 0, chunk), *partv = kv_part(pr, D, 2, 1, chunk);
+  const size_t off = head + (size_t)krow * D;
   if constexpr (MASK != MASK_NONE) {
     // a key block that the caller's hint declares fully masked has zero gradients
     if (pr.klimit && k0 >= pr.klimit[z]) {
@@ -358,8 +360,8 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
         float zero8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int d0 = 8 * g; d0 < D; d0 += 16) {
-          store8<T>(outk + d0, zero8);
-          store8<T>(outv + d0, zero8);
+          store8_or_part<T>(outk, partk, off + d0, zero8);
+          store8_or_part<T>(outv, partv, off + d0, zero8);
         }
       }
       return;
@@ -433,7 +435,7 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   }
   // tile slots 0 Q, 1 G (gO; gT in TANGENT), and the statistics slots PLAIN M, d1 | TANGENT M, a
   // h is the query head being visited; what depends on it is set per head
-  int h = hk * group;
+  int h = h0;
   const char *Qb = nullptr, *Gb = nullptr;
   const float *st_p[2] = {nullptr, nullptr};
   auto set_query_head = [&](int hq) {
@@ -644,8 +646,8 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   const int t_end = mask_small ? max(t_diag, (L - istart) / BT) : t_diag;
   for (int gi = 0; gi < group; ++gi) {
     if (gi > 0) __syncthreads();  // every wave is done with the previous head's last tile: its stage may be refilled
-    set_query_head(hk * group + gi);
-    set_list(hk * group + gi);
+    set_query_head(h0 + gi);
+    set_list(h0 + gi);
     icur = query_of(tlist ? tlist[1] : 0, 0);
     inext = query_of(tlist ? tlist[1 + (min(1, ntiles - 1) >> 1)] : 0, min(1, ntiles - 1));
     if constexpr (MASK != MASK_NONE) fetch_mask_tile(icur);
@@ -670,8 +672,8 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
           x[e] = dK[db][8 * hf + e] * pr.scale;
           y[e] = dV[db][8 * hf + e];
         }
-        store8<T>(outk + 32 * db + 16 * hf + 8 * g, x);
-        store8<T>(outv + 32 * db + 16 * hf + 8 * g, y);
+        store8_or_part<T>(outk, partk, off + 32 * db + 16 * hf + 8 * g, x);
+        store8_or_part<T>(outv, partv, off + 32 * db + 16 * hf + 8 * g, y);
       }
     }
   }

@@ -249,4 +249,10 @@ template <> __device__ __forceinline__ void store8<float>(float *dst, const floa
   *reinterpret_cast<f32x4 *>(dst + 4) = hi;
 }
 
+// ... at element `off` of dst, or in fp32 at the same place of a partial result, where there is one.
+template <typename T> __device__ __forceinline__ void store8_or_part(T *dst, float *part, size_t off, const float *x) {
+  if (part) store8<float>(part + off, x);
+  else store8<T>(dst + off, x);
+}
+
 }  // namespace jvpfa

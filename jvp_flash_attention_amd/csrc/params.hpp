@@ -32,6 +32,8 @@ struct Problem {
   // a launch would otherwise leave most compute units idle: workgroup c of a block takes the tiles
   // c * chunk_tiles .. (c + 1) * chunk_tiles - 1 and writes fp32 partial results to `part`, which a merge
   // kernel adds up.  Only the kernels for 16-bit element types, D = 128, without a mask.
+  // In the backward: the query heads of a key/value head's group are dealt to `chunks` dk/dv workgroups (see
+  // split.hpp), each of which leaves its share of the gradients in `part`.
   int chunks, chunk_tiles;
   float *part;
   // Dropout on the attention probabilities (0 in drop_thr: none).  Entry (z, h, query i, key j) is kept when
@@ -112,6 +114,11 @@ struct BwdParams {
   void *dq, *dk, *dv, *dqt, *dkt, *dvt;
   float *d1, *a, *d2;  // row statistics produced by the pre-pass, each (Z, H, L)
 };
+
+// Share `chunk` of gradient t out of nt in the backward's partial results, or null where nothing is split.
+__host__ __device__ inline float *kv_part(const Problem &pr, int D, int nt, int t, int chunk) {
+  return pr.chunks > 1 ? pr.part + ((size_t)chunk * nt + t) * ((size_t)pr.Z * pr.Hk * pr.Lk * D) : nullptr;
+}
 
 // What a backward launch computes.
 //   BWD_PLAIN    gradient of <gO,O> only (no tangents anywhere): dq / dk,dv

@@ -2,9 +2,9 @@
 // thousand tokens, a handful of heads), the kernels for 16-bit element types with D = 128 and no mask split
 // the streamed tiles of every block of owned rows over several workgroups ("chunks").  Each writes fp32
 // partial results to a workspace and a merge kernel combines them with the online-softmax merge (every running
-// quantity is linear in p once the reference points m and c are made common).  Forward only: the backward of
-// such a launch runs its dk/dv and dq workgroups side by side in one launch instead (bwd2_both_kernel).  The
-// reference has nothing like it (one program per 32 query rows, jvp_attention.py:2474).
+// quantity is linear in p once the reference points m and c are made common).  The backward of such a launch runs
+// its dk/dv and dq workgroups side by side in one launch instead (bwd2_both_kernel); what it splits is grouped heads
+// (bwd_kv_chunks below).  The reference has nothing like it (one program per 32 query rows, jvp_attention.py:2474).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -68,6 +68,26 @@ template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk) {
   return split_plan(blocks, (keys + 63) / 64, device_cus());
 }
 
+// Backward with grouped heads.  A dk/dv workgroup owns 128 keys of a key/value head and works through the query heads
+// of its group one after another: 4 key/value heads for 16 query heads make a quarter of the workgroups, each four
+// times as long.  Where they would leave the GPU idle, the group's query heads are dealt to `chunks` workgroups that
+// leave fp32 shares of dk, dv (and dk', dv'), which bwd_kv_merge_kernel adds up.  The line: enough workgroups for
+// two rounds on every compute unit (D <= 64: up to three share one, so four per unit).  bf16 B4 H16 over 4 key/value
+// heads, L1500 D64, causal, dropout: 192 workgroups 229 us -> 768 workgroups 95 us + merge 9 us.  Beyond the
+// line the shares (16 bytes per chunk and element, written and read) cost more than the idle tail.
+template <typename P> inline int bwd_kv_chunks(const P &p, int Lk, int Hk) {
+  const int group = p.H / Hk;
+  const long long blocks = (long long)((Lk + 127) / 128) * p.Z * Hk;
+  const long long want = (long long)device_cus() * (p.dtype != 2 && p.D <= 64 ? 4 : 2);
+  for (int c = 1; c < group; ++c)
+    if (group % c == 0 && blocks * c >= want) return c;
+  return blocks < want ? group : 1;
+}
+// ... floats of the shares: dk, dv, and dk', dv' where one kernel makes all four (tangent_grads)
+template <typename P> inline size_t bwd_part_floats(const P &p, int Lk, int Hk, int chunks, bool tangent_grads) {
+  return (size_t)chunks * (tangent_grads ? 4 : 2) * ((size_t)p.Z * Hk * Lk * p.D);
+}
+
 // ---- merge kernels -------------------------------------------------------------------------------
 // Forward.  part = [chunk][row][2][D] accumulators, then [chunk][row][4] statistics.  One thread per (row, 8
 // columns).  With m the largest reference point of the row's chunks and w_c = 2^(m_c - m):
@@ -125,6 +145,22 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const float *part, int c
     M[row] = dead ? __builtin_inff() : m + __builtin_amdgcn_logf(l);
     if constexpr (DUAL) mu[row] = dead ? 0.f : mu_n + cref;
   }
+}
+
+// Backward: gradient t = blockIdx.y out of gridDim.y is the sum of its shares part[chunk][t][elems].  One thread per 8
+// elements; bound by HBM (the shares are read once, 16 bytes per lane and load).
+template <typename T>
+__global__ __launch_bounds__(256) void bwd_kv_merge_kernel(const float *part, int chunks, size_t elems, T *g0, T *g1, T *g2, T *g3) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= elems) return;
+  const int t = blockIdx.y, nt = gridDim.y;
+  float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < chunks; ++c) {
+    const f32x8 x = ld8<float>(part + ((size_t)c * nt + t) * elems + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum[e] += x[e];
+  }
+  store8<T>((t == 0 ? g0 : t == 1 ? g1 : t == 2 ? g2 : g3) + i, sum);
 }
 
 }  // namespace jvpfa

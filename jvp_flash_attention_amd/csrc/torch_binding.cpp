@@ -149,6 +149,14 @@ std::vector<Tensor> backward(const Tensor &q, const Tensor &k, const Tensor &v, 
   a.key_limit = in<int32_t>(c.key_limit), a.tiles_q = in<int32_t>(c.tiles_q), a.tiles_k = in<int32_t>(c.tiles_k);
   a.mask_bits = in<uint32_t>(c.bits);
   a.Hk = static_cast<int32_t>(k.size(1)), a.Lk = static_cast<int32_t>(k.size(2));
+  Tensor shares;
+  if (c.split && a.Hk < a.p.H) {
+    a.split_workspace_bytes = jvpfa_bwd_split_workspace_bytes(&a.p, a.Lk, a.Hk, want_tangent_grads ? 1 : 0);
+    if (a.split_workspace_bytes) {
+      shares = at::empty({static_cast<int64_t>(a.split_workspace_bytes)}, q.options().dtype(at::kByte).requires_grad(false));
+      a.split_workspace = out(shares);
+    }
+  }
   check(jvpfa_bwd(&a, c10::hip::getCurrentHIPStream(q.device().index()).stream()));
   return g;
 }
@@ -169,7 +177,7 @@ struct Attention : public torch::autograd::Function<Attention> {
     // the mask and what was derived from it are kept as they are (no version check: as before, a mask may be refilled)
     auto &d = ctx->saved_data;
     d["c"] = c10::IValue(std::make_tuple(c.mask, c.key_limit, c.tiles_q, c.tiles_k, c.bits, c.mask_kind, c.causal, c.scale,
-                                         c.dropout_p, static_cast<int64_t>(c.seed)));
+                                         c.dropout_p, static_cast<int64_t>(c.seed), c.split));
     if (qt.defined()) return {o, ot};
     return {o};
   }
@@ -181,7 +189,7 @@ struct Attention : public torch::autograd::Function<Attention> {
     c.mask = e[0].toOptional<Tensor>(), c.key_limit = e[1].toOptional<Tensor>(), c.tiles_q = e[2].toOptional<Tensor>();
     c.tiles_k = e[3].toOptional<Tensor>(), c.bits = e[4].toOptional<Tensor>();
     c.mask_kind = e[5].toInt(), c.causal = e[6].toBool(), c.scale = e[7].toDouble(), c.dropout_p = e[8].toDouble();
-    c.seed = static_cast<uint64_t>(e[9].toInt());
+    c.seed = static_cast<uint64_t>(e[9].toInt()), c.split = e[10].toBool();
     const bool dual = s[3].defined();
     const Tensor go = dense(grads[0]), gt = dual ? dense(grads[1]) : Tensor();
     const bool want_t = dual && (ctx->needs_input_grad(3) || ctx->needs_input_grad(4) || ctx->needs_input_grad(5));
