@@ -3,6 +3,7 @@
 // and exporting  int JVPFA_NAME(const BwdParams&, int mask_kind, bool dual, bool tangent_grads,
 // hipStream_t): pre-pass, then the dq and dk/dv kernels of every requested mode.
 #include "bwd_kernel.hpp"
+#include "bwd_kernel_f32.hpp"
 #include "bwd_kernel_v2.hpp"
 #include "bwd_kernel_wide.hpp"
 #include "bwd_kernel_pair.hpp"
@@ -82,6 +83,23 @@ template <typename T, int D> static void launch_kv_merge(const BwdParams &p, boo
                      p.pr.chunks, elems, tangent ? dkt : dk, tangent ? dvt : dv, dkt, dvt);
 }
 
+// fp32 with D <= 128.
+template <int D, int MODE, int MASK, bool DROP>
+static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blocks, hipStream_t stream) {
+  constexpr bool NG = MODE != BWD_DUAL;  // gO may be absent only in the dual mode
+  const bool no_go = MODE == BWD_DUAL && p.go == nullptr;
+  void (*kq)(const BwdParams) = no_go ? bwd_f32_dq_kernel<D, MODE, MASK, NG, DROP> : bwd_f32_dq_kernel<D, MODE, MASK, true, DROP>;
+  void (*kkv)(const BwdParams) = no_go ? bwd_f32_dkdv_kernel<D, MODE, MASK, NG, DROP> : bwd_f32_dkdv_kernel<D, MODE, MASK, true, DROP>;
+  using Lds = BwdF32Lds<D, MODE>;
+  int rc = allow_lds(reinterpret_cast<const void *>(kq), Lds::DQ);
+  if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), Lds::DKV);
+  if (rc != 0) return rc;
+  hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(BWD_NT), Lds::DKV, stream, p);
+  launch_kv_merge<float, D>(p, MODE == BWD_TANGENT, false, stream);
+  hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(BWD_NT), Lds::DQ, stream, p);
+  return hipGetLastError() == hipSuccess ? 0 : -6;
+}
+
 // six: all six gradients were asked for.  The dual launch then also writes what BwdFold says, and the tangent
 // launch skips the kernels whose outputs exist already.
 template <typename T, int D, int MODE, int MASK>
@@ -138,6 +156,8 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
       hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(CfgW::NT), CfgW::DQ_LDS, stream, p);
       return hipGetLastError() == hipSuccess ? 0 : -6;
+    } else if constexpr (D <= 128) {
+      return launch_bwd_f32<D, MODE, MASK, true>(p, blocks, kv_blocks, stream);
     } else {
       auto kq = bwd_dq_kernel<T, D, MODE, MASK, true>;
       auto kkv = bwd_dkdv_kernel<T, D, MODE, MASK, true>;
@@ -232,6 +252,8 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     // (six: the tangent launch of a six-gradient call, whose dq' the dual launch has written already)
     if (!(MODE == BWD_TANGENT && six)) hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(CfgW::NT), CfgW::DQ_LDS, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -6;
+  } else if constexpr (D <= 128) {
+    return launch_bwd_f32<D, MODE, MASK, false>(p, blocks, kv_blocks, stream);
   } else {
     auto kq = bwd_dq_kernel<T, D, MODE, MASK>;
     auto kkv = bwd_dkdv_kernel<T, D, MODE, MASK>;

@@ -1,5 +1,5 @@
-// Backward kernels for  Loss = <gO, O> + <gT, O'>  with P recomputed from the saved
-// log-sum-exp M (and mu for the tangent path).
+// Backward for  Loss = <gO, O> + <gT, O'>  with P recomputed from the saved log-sum-exp M (and mu for the tangent
+// path): the pre-pass of every backward, and the dq, dk/dv kernels for fp32 at D = 256.
 //
 //   prepass   d1 = rowsum(gO*O), a = rowsum(gT*O), d2 = d1 + rowsum(gT*O') - a*mu
 //   dq        one workgroup per 128 query rows, loop over key tiles
@@ -69,49 +69,21 @@ template <typename T, int D, int MODE> struct BwdCfg {
   static constexpr int LDT = BWD_T + PAD;   // transposed streamed tiles (D x 32)
   static constexpr int N_ELEMS = BWD_T * LDN;
   static constexpr int T_ELEMS = D * LDT;
-  // dq:   PLAIN K,V,K^T | DUAL K,K',V,V',K^T,K'^T | TANGENT K,V,K^T
-  // dkdv: PLAIN Q,gO,Q^T,gO^T | DUAL Q,Q',gO,gT + 4 transposed | TANGENT Q,gT,Q^T,gT^T
-  // D = 256 (fp32: rows of 1024 bytes; 16-bit types come here with dropout only): a wave's own rows of four
-  // operands would be the whole register file (fp32: 4 x 128 registers, next to 128 - 256 of accumulators) and
-  // eight 32-row fp32 tiles twice the LDS, so there the own rows are read from global
-  // memory where they are used (the same 32 bytes per lane every tile: cache hits) and only the tiles whose
-  // fragments run along the streamed index are staged (dq: K, K' both ways; dk/dv: the four transposed ones);
-  // the other row-wise fragments also come straight from global memory.
-  static constexpr bool SB = D == 256;
-  static constexpr int DQ_NAT = SB ? (MODE == BWD_DUAL ? 2 : 1) : (MODE == BWD_DUAL ? 4 : 2);
+  // dq:   PLAIN K,K^T | DUAL K,K',K^T,K'^T | TANGENT K,K^T
+  // dkdv: PLAIN Q^T,gO^T | DUAL Q^T,Q'^T,gO^T,gT^T | TANGENT Q^T,gT^T
+  // Rows of 1024 bytes: a wave's own rows of four operands would be the whole register file (4 x 128 registers, next
+  // to 128 - 256 of accumulators) and eight 32-row tiles twice the LDS, so the own rows are read from global memory
+  // where they are used (the same 32 bytes per lane every tile: cache hits) and only the tiles whose fragments run
+  // along the streamed index are staged (dq: K, K' both ways; dk/dv: the four transposed ones); the other row-wise
+  // fragments also come straight from global memory.
+  static constexpr int DQ_NAT = MODE == BWD_DUAL ? 2 : 1;
   static constexpr int DQ_TR = MODE == BWD_DUAL ? 2 : 1;
-  static constexpr int DKV_NAT = SB ? 0 : (MODE == BWD_DUAL ? 4 : 2);
   static constexpr int DKV_TR = MODE == BWD_DUAL ? 4 : 2;
   static constexpr size_t DQ_LDS = (size_t)(DQ_NAT * N_ELEMS + DQ_TR * T_ELEMS) * sizeof(T);
-  static constexpr size_t DKV_LDS = (size_t)(DKV_NAT * N_ELEMS + DKV_TR * T_ELEMS) * sizeof(T) + 5 * BWD_T * sizeof(float);
+  static constexpr size_t DKV_LDS = (size_t)(DKV_TR * T_ELEMS) * sizeof(T) + 5 * BWD_T * sizeof(float);
 };
 
-// whether the dq / dk,dv kernels fetch the next tile into registers during the current one's
-// computation (needs up to 64 registers; see the forward kernel)
-template <typename T, int D> constexpr bool BWD_FETCH_AHEAD = D == 64 || (D == 32 && sizeof(T) == 4);
-// rows of 512 bytes: the resident operands of the dual backward fill the register file by themselves
-template <typename T, int D> constexpr bool BWD_WIDE_ROWS = D * sizeof(T) >= 512;
-
-template <int KK, typename T>
-__device__ __forceinline__ void load_row_frags(Frag<T> *f, const T *row, int g) {
-#pragma unroll
-  for (int kk = 0; kk < KK; ++kk) f[kk] = ld8<T>(row + 16 * kk + 8 * g);
-}
-
-template <int KK, typename T>
-__device__ __forceinline__ void gemm_tile(f32x16 &acc, const T *tile, int ld, int arow, int g, const Frag<T> *b) {
-#pragma unroll
-  for (int kk = 0; kk < KK; ++kk) {
-    mma(acc, lds_frag(tile + arow * ld + 16 * kk + 8 * g), b[kk]);
-    // rows of 512 bytes (fp32 D = 128): the register file is full of resident operands; keep the
-    // scheduler from hoisting more than four fragment reads above the products that consume them
-    if constexpr (KK * sizeof(Frag<T>) >= 256) {
-      if (kk % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-}
-
-// The same with the B fragments (the lane's own row) read from global memory where they are used; `tile` may
+// One 32 x 32 tile of a product over d, the B fragments (the lane's own row) read from global memory; `tile` may
 // be an LDS tile or rows of global memory (then `ld` is the row length and `arow` an index clamped by the caller).
 template <int KK, typename T>
 __device__ __forceinline__ void gemm_tile(f32x16 &acc, const T *tile, int ld, int arow, int g, const T *brow) {
@@ -138,13 +110,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(const BwdParams p) {
   constexpr float NEG_INF = -__builtin_inff();
 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  constexpr bool SB = Cfg::SB;    // V, V' are not staged (see BwdCfg)
   T *Kn = reinterpret_cast<T *>(smem_raw);
-  T *Vn = Kn + Cfg::N_ELEMS;
-  T *KT = SB ? Vn : Vn + Cfg::N_ELEMS;
+  T *KT = Kn + Cfg::N_ELEMS;
   T *Ktn = KT + Cfg::T_ELEMS;     // DUAL only from here on
-  T *Vtn = Ktn + Cfg::N_ELEMS;
-  T *KtT = SB ? Vtn : Vtn + Cfg::N_ELEMS;
+  T *KtT = Ktn + Cfg::N_ELEMS;
 
   const Problem &pr = p.pr;
   const int L = pr.L;
@@ -164,21 +133,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(const BwdParams p) {
   const int qld = qrow < L ? qrow : L - 1;
   const bool has_go = p.go != nullptr;
 
-  // this lane's own row of the tensors that are B operands: resident fragments, or (SB) pointers to read through
+  // this lane's own row of the tensors that are B operands
   const T *Qrow = reinterpret_cast<const T *>(p.q) + head + (size_t)qld * D;
   const T *gOrow = (!TAN && has_go) ? reinterpret_cast<const T *>(p.go) + head + (size_t)qld * D : nullptr;
   const T *Qtrow = DUAL ? reinterpret_cast<const T *>(p.qt) + head + (size_t)qld * D : nullptr;
   const T *gTrow = (DUAL || TAN) ? reinterpret_cast<const T *>(p.gt) + head + (size_t)qld * D : nullptr;
-  constexpr int KR = SB ? 1 : KK;
-  Frag<T> Qf[KR], gOf[TAN ? 1 : KR], Qtf[DUAL ? KR : 1], gTf[(DUAL || TAN) ? KR : 1];
-  if constexpr (!SB) {
-    load_row_frags<KK>(Qf, Qrow, g);
-    if constexpr (!TAN) {
-      if (has_go) load_row_frags<KK>(gOf, gOrow, g);
-    }
-    if constexpr (DUAL) load_row_frags<KK>(Qtf, Qtrow, g);
-    if constexpr (DUAL || TAN) load_row_frags<KK>(gTf, gTrow, g);
-  }
 
   const float Mq = qrow < L ? p.M[srow + qld] : __builtin_inff();
   const float d1 = (MODE == BWD_PLAIN) ? p.d1[srow + qld] : 0.f;  // BWD_DUAL: d2 already holds d1 + d2
@@ -211,89 +170,37 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(const BwdParams p) {
     }
     walk.init(tl, 0, kend, Lk);
   }
-  // The next tile is fetched into registers while this one is computed and written to LDS behind the
-  // barrier that follows; K (, K') is fetched once and written both ways.  (See the forward kernel for
-  // where this is left out.)
-  constexpr bool AHEAD = BWD_FETCH_AHEAD<T, D>;
-  QuadChunks<T, BWD_T, D, BWD_NT> rk, rkt;
-  RowChunks<T, BWD_T, D, BWD_NT> rv, rvt;
-  auto fetch_tile = [&](int j0) {
-    const int nvalid = Lk - j0;
-    fetch_quads(rk, Kg + (size_t)j0 * D, nvalid, tid);
-    fetch_rows(rv, Vg + (size_t)j0 * D, nvalid, tid);
-    if constexpr (DUAL) {
-      fetch_quads(rkt, Ktg + (size_t)j0 * D, nvalid, tid);
-      fetch_rows(rvt, Vtg + (size_t)j0 * D, nvalid, tid);
-    }
-  };
-  if constexpr (AHEAD) {
-    if (walk.n > 0) fetch_tile(walk.at(0));
-  }
   for (int it = 0; it < walk.n; ++it) {
     const int j0 = walk.at(it);
     __syncthreads();
-    if constexpr (AHEAD) {
-      put_quads_rows(Kn, Cfg::LDN, rk, tid);
-      put_quads_transposed(KT, Cfg::LDT, rk, tid);
-      put_rows(Vn, Cfg::LDN, rv, tid);
-      if constexpr (DUAL) {
-        put_quads_rows(Ktn, Cfg::LDN, rkt, tid);
-        put_quads_transposed(KtT, Cfg::LDT, rkt, tid);
-        put_rows(Vtn, Cfg::LDN, rvt, tid);
-      }
-    } else {
-      const int nvalid = Lk - j0;
-      copy_rows<T, BWD_T, D, BWD_NT>(Kn, Cfg::LDN, Kg + (size_t)j0 * D, nvalid, tid);
-      if constexpr (!SB) copy_rows<T, BWD_T, D, BWD_NT>(Vn, Cfg::LDN, Vg + (size_t)j0 * D, nvalid, tid);
-      copy_rows_transposed<T, BWD_T, D, BWD_NT>(KT, Cfg::LDT, Kg + (size_t)j0 * D, nvalid, tid);
-      if constexpr (DUAL) {
-        copy_rows<T, BWD_T, D, BWD_NT>(Ktn, Cfg::LDN, Ktg + (size_t)j0 * D, nvalid, tid);
-        if constexpr (!SB) copy_rows<T, BWD_T, D, BWD_NT>(Vtn, Cfg::LDN, Vtg + (size_t)j0 * D, nvalid, tid);
-        copy_rows_transposed<T, BWD_T, D, BWD_NT>(KtT, Cfg::LDT, Ktg + (size_t)j0 * D, nvalid, tid);
-      }
+    const int nvalid = Lk - j0;
+    copy_rows<T, BWD_T, D, BWD_NT>(Kn, Cfg::LDN, Kg + (size_t)j0 * D, nvalid, tid);
+    copy_rows_transposed<T, BWD_T, D, BWD_NT>(KT, Cfg::LDT, Kg + (size_t)j0 * D, nvalid, tid);
+    if constexpr (DUAL) {
+      copy_rows<T, BWD_T, D, BWD_NT>(Ktn, Cfg::LDN, Ktg + (size_t)j0 * D, nvalid, tid);
+      copy_rows_transposed<T, BWD_T, D, BWD_NT>(KtT, Cfg::LDT, Ktg + (size_t)j0 * D, nvalid, tid);
     }
     __syncthreads();
-    if constexpr (AHEAD) {
-      if (it + 1 < walk.n) fetch_tile(walk.at(it + 1));
-    }
 
     f32x16 S, dP, Sp, At;  // DUAL: dP also collects gT V'^T (the B term)
     zero16(S);
-    if constexpr (SB) {
-      // V, V' fragments from global memory: this lane's key row, clamped (a key past the end has p = 0 and
-      // must meet finite values)
-      const int vrow = min(j0 + pr32, Lk - 1);
-      gemm_tile<KK>(S, Kn, Cfg::LDN, pr32, g, Qrow);
-      if constexpr (!TAN) {
-        zero16(dP);
-        if (has_go) gemm_tile<KK>(dP, Vg, D, vrow, g, gOrow);
-      }
-      if constexpr (DUAL) {
-        zero16(Sp);
-        gemm_tile<KK>(Sp, Kn, Cfg::LDN, pr32, g, Qtrow);
-        gemm_tile<KK>(Sp, Ktn, Cfg::LDN, pr32, g, Qrow);
-        gemm_tile<KK>(dP, Vtg, D, vrow, g, gTrow);
-      }
-      if constexpr (DUAL || TAN) {
-        zero16(At);
-        gemm_tile<KK>(At, Vg, D, vrow, g, gTrow);
-      }
-    } else {
-    gemm_tile<KK>(S, Kn, Cfg::LDN, pr32, g, Qf);
+    // V, V' fragments from global memory: this lane's key row, clamped (a key past the end has p = 0 and
+    // must meet finite values)
+    const int vrow = min(j0 + pr32, Lk - 1);
+    gemm_tile<KK>(S, Kn, Cfg::LDN, pr32, g, Qrow);
     if constexpr (!TAN) {
       zero16(dP);
-      if (has_go) gemm_tile<KK>(dP, Vn, Cfg::LDN, pr32, g, gOf);
+      if (has_go) gemm_tile<KK>(dP, Vg, D, vrow, g, gOrow);
     }
     if constexpr (DUAL) {
       zero16(Sp);
-      gemm_tile<KK>(Sp, Kn, Cfg::LDN, pr32, g, Qtf);
-      gemm_tile<KK>(Sp, Ktn, Cfg::LDN, pr32, g, Qf);
-      gemm_tile<KK>(dP, Vtn, Cfg::LDN, pr32, g, gTf);
+      gemm_tile<KK>(Sp, Kn, Cfg::LDN, pr32, g, Qtrow);
+      gemm_tile<KK>(Sp, Ktn, Cfg::LDN, pr32, g, Qrow);
+      gemm_tile<KK>(dP, Vtg, D, vrow, g, gTrow);
     }
     if constexpr (DUAL || TAN) {
       zero16(At);
-      gemm_tile<KK>(At, Vn, Cfg::LDN, pr32, g, gTf);
-    }
+      gemm_tile<KK>(At, Vg, D, vrow, g, gTrow);
     }
 
     const bool diag = pr.causal && (j0 + BWD_T - 1 > q0 + wave * 32);
@@ -340,9 +247,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(const BwdParams p) {
       for (int db = 0; db < DB; ++db) {
         mma(acc[db], lds_frag(KT + (32 * db + pr32) * Cfg::LDT + 16 * c + 8 * g), dsf);
         if constexpr (DUAL) mma(acc[db], lds_frag(KtT + (32 * db + pr32) * Cfg::LDT + 16 * c + 8 * g), dspf);
-        if constexpr (BWD_WIDE_ROWS<T, D>) {  // as in gemm_tile, bound the fragment reads in flight
-          if (db % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-        }
+        if (db % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // as in gemm_tile, bound the fragment reads in flight
       }
     }
   }
@@ -372,17 +277,12 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  // row-major tiles first, then transposed ones, then the row statistics
-  T *Qn = reinterpret_cast<T *>(smem_raw);
-  T *Gn = Qn + Cfg::N_ELEMS;                         // gO (PLAIN, DUAL) or gT (TANGENT)
-  T *Qtn = Gn + Cfg::N_ELEMS;                        // DUAL: Q'
-  T *GTn = Qtn + Cfg::N_ELEMS;                       // DUAL: gT
-  T *trbase = Qn + Cfg::DKV_NAT * Cfg::N_ELEMS;
-  T *QT = trbase;
-  T *GT = QT + Cfg::T_ELEMS;
+  // transposed tiles, then the row statistics
+  T *QT = reinterpret_cast<T *>(smem_raw);
+  T *GT = QT + Cfg::T_ELEMS;                         // gO (PLAIN, DUAL) or gT (TANGENT)
   T *QtT = GT + Cfg::T_ELEMS;                        // DUAL
   T *GTT = QtT + Cfg::T_ELEMS;                       // DUAL
-  float *stats = reinterpret_cast<float *>(trbase + Cfg::DKV_TR * Cfg::T_ELEMS);
+  float *stats = reinterpret_cast<float *>(QT + Cfg::DKV_TR * Cfg::T_ELEMS);
   float *sM = stats, *sd1 = stats + BWD_T, *smu = stats + 2 * BWD_T, *sa = stats + 3 * BWD_T, *sd2 = stats + 4 * BWD_T;
 
   // One workgroup per (batch entry, key/value head, block of 128 keys).  With grouped heads the query
@@ -403,22 +303,11 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   const int kld = krow < Lk ? krow : Lk - 1;
   const bool has_go = p.go != nullptr;
 
-  // this lane's own key row of K, V (, K', V'): resident fragments, or (SB, see BwdCfg) pointers to read through
-  constexpr bool SB = Cfg::SB;
+  // this lane's own key row of K, V (, K', V')
   const T *Krow = reinterpret_cast<const T *>(p.k) + kvhead + (size_t)kld * D;
   const T *Vrow = reinterpret_cast<const T *>(p.v) + kvhead + (size_t)kld * D;
   const T *Ktrow = DUAL ? reinterpret_cast<const T *>(p.kt) + kvhead + (size_t)kld * D : nullptr;
   const T *Vtrow = DUAL ? reinterpret_cast<const T *>(p.vt) + kvhead + (size_t)kld * D : nullptr;
-  constexpr int KR = SB ? 1 : KK;
-  Frag<T> Kf[KR], Vf[KR], Ktf[DUAL ? KR : 1], Vtf[DUAL ? KR : 1];
-  if constexpr (!SB) {
-    load_row_frags<KK>(Kf, Krow, g);
-    load_row_frags<KK>(Vf, Vrow, g);
-    if constexpr (DUAL) {
-      load_row_frags<KK>(Ktf, Ktrow, g);
-      load_row_frags<KK>(Vtf, Vtrow, g);
-    }
-  }
 
   f32x16 dK[DB], dV[DB];
 #pragma unroll
@@ -438,10 +327,6 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   const T *gOg = (!TAN && has_go) ? reinterpret_cast<const T *>(p.go) + head : nullptr;
   const T *gTg = (DUAL || TAN) ? reinterpret_cast<const T *>(p.gt) + head : nullptr;
   const T *Gg = TAN ? gTg : gOg;  // tensor staged in Gn / GT
-  // The next tile (each tensor once, written to LDS both ways) and its row statistics are fetched
-  // into registers while this tile is computed, as in the dq kernel.
-  constexpr bool AHEAD = BWD_FETCH_AHEAD<T, D>;
-  QuadChunks<T, BWD_T, D, BWD_NT> rq, rg, rqt, rgt;
   float rs[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // M, d1, mu, a, d2 of query row i0 + tid
   auto fetch_stats = [&](int i0) {
     if (tid < BWD_T) {
@@ -459,16 +344,6 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
       sM[tid] = rs[0], sd1[tid] = rs[1], smu[tid] = rs[2], sa[tid] = rs[3], sd2[tid] = rs[4];
     }
   };
-  auto fetch_tile = [&](int i0) {
-    const int nvalid = L - i0;
-    fetch_quads(rq, Qg + (size_t)i0 * D, nvalid, tid);
-    if (Gg) fetch_quads(rg, Gg + (size_t)i0 * D, nvalid, tid);
-    if constexpr (DUAL) {
-      fetch_quads(rqt, Qtg + (size_t)i0 * D, nvalid, tid);
-      fetch_quads(rgt, gTg + (size_t)i0 * D, nvalid, tid);
-    }
-    fetch_stats(i0);
-  };
   // query tiles visited: all from istart on, or the caller's list of the tiles of this key block (and this
   // query head's mask plane) that hold an attended entry
   TileWalk<BWD_T> walk;
@@ -482,88 +357,41 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
       if (pr.klimit && k0 >= pr.klimit[z]) walk.n = 0;  // a key block the caller's hint declares fully masked: zeros
     }
   }
-  if constexpr (AHEAD) {
-    if (walk.n > 0) fetch_tile(walk.at(0));
-  }
   for (int it = 0; it < walk.n; ++it) {
     const int i0 = walk.at(it);
     __syncthreads();
-    if constexpr (AHEAD) {
-      put_quads_rows(Qn, Cfg::LDN, rq, tid);
-      put_quads_transposed(QT, Cfg::LDT, rq, tid);
-      if (Gg) {
-        put_quads_rows(Gn, Cfg::LDN, rg, tid);
-        put_quads_transposed(GT, Cfg::LDT, rg, tid);
-      }
-      if constexpr (DUAL) {
-        put_quads_rows(Qtn, Cfg::LDN, rqt, tid);
-        put_quads_transposed(QtT, Cfg::LDT, rqt, tid);
-        put_quads_rows(GTn, Cfg::LDN, rgt, tid);
-        put_quads_transposed(GTT, Cfg::LDT, rgt, tid);
-      }
-    } else {
-      const int nvalid = L - i0;
-      if constexpr (!SB) copy_rows<T, BWD_T, D, BWD_NT>(Qn, Cfg::LDN, Qg + (size_t)i0 * D, nvalid, tid);
-      copy_rows_transposed<T, BWD_T, D, BWD_NT>(QT, Cfg::LDT, Qg + (size_t)i0 * D, nvalid, tid);
-      if (Gg) {
-        if constexpr (!SB) copy_rows<T, BWD_T, D, BWD_NT>(Gn, Cfg::LDN, Gg + (size_t)i0 * D, nvalid, tid);
-        copy_rows_transposed<T, BWD_T, D, BWD_NT>(GT, Cfg::LDT, Gg + (size_t)i0 * D, nvalid, tid);
-      }
-      if constexpr (DUAL) {
-        if constexpr (!SB) copy_rows<T, BWD_T, D, BWD_NT>(Qtn, Cfg::LDN, Qtg + (size_t)i0 * D, nvalid, tid);
-        copy_rows_transposed<T, BWD_T, D, BWD_NT>(QtT, Cfg::LDT, Qtg + (size_t)i0 * D, nvalid, tid);
-        if constexpr (!SB) copy_rows<T, BWD_T, D, BWD_NT>(GTn, Cfg::LDN, gTg + (size_t)i0 * D, nvalid, tid);
-        copy_rows_transposed<T, BWD_T, D, BWD_NT>(GTT, Cfg::LDT, gTg + (size_t)i0 * D, nvalid, tid);
-      }
-      fetch_stats(i0);
+    const int nvalid = L - i0;
+    copy_rows_transposed<T, BWD_T, D, BWD_NT>(QT, Cfg::LDT, Qg + (size_t)i0 * D, nvalid, tid);
+    if (Gg) copy_rows_transposed<T, BWD_T, D, BWD_NT>(GT, Cfg::LDT, Gg + (size_t)i0 * D, nvalid, tid);
+    if constexpr (DUAL) {
+      copy_rows_transposed<T, BWD_T, D, BWD_NT>(QtT, Cfg::LDT, Qtg + (size_t)i0 * D, nvalid, tid);
+      copy_rows_transposed<T, BWD_T, D, BWD_NT>(GTT, Cfg::LDT, gTg + (size_t)i0 * D, nvalid, tid);
     }
+    fetch_stats(i0);
     put_stats();
     __syncthreads();
-    if constexpr (AHEAD) {
-      if (it + 1 < walk.n) fetch_tile(walk.at(it + 1));
-    }
 
     f32x16 S, dP, Sp, At;  // DUAL: dP also collects V' gT^T (the B term)
     zero16(S);
-    if constexpr (SB) {
-      // row-wise fragments of Q, G (, Q', gT) from global memory: this lane's query row, clamped (a query past
-      // the end has p = 0 and must meet finite values)
-      const int qr = min(i0 + pr32, L - 1);
-      gemm_tile<KK>(S, Qg, D, qr, g, Krow);
-      if constexpr (!TAN) {
-        zero16(dP);
-        if (has_go) gemm_tile<KK>(dP, Gg, D, qr, g, Vrow);
-      }
-      if constexpr (DUAL) {
-        zero16(Sp);
-        gemm_tile<KK>(Sp, Qtg, D, qr, g, Krow);
-        gemm_tile<KK>(Sp, Qg, D, qr, g, Ktrow);
-        zero16(At);
-        gemm_tile<KK>(At, gTg, D, qr, g, Vrow);
-        gemm_tile<KK>(dP, gTg, D, qr, g, Vtrow);
-      }
-      if constexpr (TAN) {
-        zero16(At);
-        gemm_tile<KK>(At, Gg, D, qr, g, Vrow);
-      }
-    } else {
-    gemm_tile<KK>(S, Qn, Cfg::LDN, pr32, g, Kf);
+    // row-wise fragments of Q, G (, Q', gT) from global memory: this lane's query row, clamped (a query past
+    // the end has p = 0 and must meet finite values)
+    const int qr = min(i0 + pr32, L - 1);
+    gemm_tile<KK>(S, Qg, D, qr, g, Krow);
     if constexpr (!TAN) {
       zero16(dP);
-      if (has_go) gemm_tile<KK>(dP, Gn, Cfg::LDN, pr32, g, Vf);
+      if (has_go) gemm_tile<KK>(dP, Gg, D, qr, g, Vrow);
     }
     if constexpr (DUAL) {
       zero16(Sp);
-      gemm_tile<KK>(Sp, Qtn, Cfg::LDN, pr32, g, Kf);
-      gemm_tile<KK>(Sp, Qn, Cfg::LDN, pr32, g, Ktf);
+      gemm_tile<KK>(Sp, Qtg, D, qr, g, Krow);
+      gemm_tile<KK>(Sp, Qg, D, qr, g, Ktrow);
       zero16(At);
-      gemm_tile<KK>(At, GTn, Cfg::LDN, pr32, g, Vf);
-      gemm_tile<KK>(dP, GTn, Cfg::LDN, pr32, g, Vtf);
+      gemm_tile<KK>(At, gTg, D, qr, g, Vrow);
+      gemm_tile<KK>(dP, gTg, D, qr, g, Vtrow);
     }
     if constexpr (TAN) {
       zero16(At);
-      gemm_tile<KK>(At, Gn, Cfg::LDN, pr32, g, Vf);
-    }
+      gemm_tile<KK>(At, Gg, D, qr, g, Vrow);
     }
 
     const bool diag = pr.causal && (i0 < k0 + wave * 32 + 31);  // some query may precede a key
@@ -626,9 +454,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
           mma(dK[db], lds_frag(QT + off), dspf);
           mma(dV[db], lds_frag(GT + off), pf);
         }
-        if constexpr (BWD_WIDE_ROWS<T, D>) {  // as in gemm_tile, bound the fragment reads in flight
-          if (db % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-        }
+        if (db % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // as in gemm_tile, bound the fragment reads in flight
       }
     }
   }

@@ -2,6 +2,7 @@
 //   -DJVPFA_T=<__bf16|_Float16|float> -DJVPFA_D=<32|64|128|256> -DJVPFA_NAME=<symbol>
 // and exporting  int JVPFA_NAME(const FwdParams&, bool dual, int mask_kind, hipStream_t).
 #include "fwd_kernel.hpp"
+#include "fwd_kernel_f32.hpp"
 #include "fwd_kernel_v2.hpp"
 #include "fwd_kernel_v3.hpp"
 #include "fwd_kernel_wide.hpp"
@@ -20,6 +21,20 @@ static int launch_fwd_one(const FwdParams &p, hipStream_t stream) {
   const long long blocks = (long long)nqb * p.pr.Z * p.pr.H;
   if (blocks > 0x7fffffffLL) return -2;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, p);
+  return hipGetLastError() == hipSuccess ? 0 : -6;
+}
+
+// fp32 with D <= 128: direct-to-LDS as well.
+template <int D, bool DUAL, int MASK, bool DROP = false>
+static int launch_fwd_f32_one(const FwdParams &p, hipStream_t stream) {
+  using C = F32Cfg<D>;
+  constexpr size_t LDS = 2 * (DUAL ? 4 : 2) * (size_t)C::TILEB;
+  auto kern = fwd_f32_kernel<D, DUAL, MASK, DROP>;
+  int rc = allow_lds(reinterpret_cast<const void *>(kern), LDS);
+  if (rc != 0) return rc;
+  const long long blocks = (long long)((p.pr.L + C::BLK - 1) / C::BLK) * p.pr.Z * p.pr.H;
+  if (blocks > 0x7fffffffLL) return -2;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NT), LDS, stream, p);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
@@ -113,12 +128,17 @@ static int launch_fwd_mask(const FwdParams &p, int mask, hipStream_t stream) {
         case MASK_BOOL: return launch_fwd2_one<T, D, DUAL, MASK_BOOL, true>(p, stream);
         case MASK_ADD: return launch_fwd2_one<T, D, DUAL, MASK_ADD, true>(p, stream);
       }
-    } else {
-      constexpr int BNG = (sizeof(T) == 4 || D > 128) ? 32 : 64;
+    } else if constexpr (D <= 128) {
       switch (mask) {
-        case MASK_NONE: return launch_fwd_one<T, D, BNG, DUAL, MASK_NONE, true>(p, stream);
-        case MASK_BOOL: return launch_fwd_one<T, D, BNG, DUAL, MASK_BOOL, true>(p, stream);
-        case MASK_ADD: return launch_fwd_one<T, D, BNG, DUAL, MASK_ADD, true>(p, stream);
+        case MASK_NONE: return launch_fwd_f32_one<D, DUAL, MASK_NONE, true>(p, stream);
+        case MASK_BOOL: return launch_fwd_f32_one<D, DUAL, MASK_BOOL, true>(p, stream);
+        case MASK_ADD: return launch_fwd_f32_one<D, DUAL, MASK_ADD, true>(p, stream);
+      }
+    } else {
+      switch (mask) {
+        case MASK_NONE: return launch_fwd_one<T, D, BN, DUAL, MASK_NONE, true>(p, stream);
+        case MASK_BOOL: return launch_fwd_one<T, D, BN, DUAL, MASK_BOOL, true>(p, stream);
+        case MASK_ADD: return launch_fwd_one<T, D, BN, DUAL, MASK_ADD, true>(p, stream);
       }
     }
     return -3;
@@ -143,6 +163,13 @@ static int launch_fwd_mask(const FwdParams &p, int mask, hipStream_t stream) {
       case MASK_NONE: return launch_fwd2_one<T, D, DUAL, MASK_NONE>(p, stream);
       case MASK_BOOL: return launch_fwd2_one<T, D, DUAL, MASK_BOOL>(p, stream);
       case MASK_ADD: return launch_fwd2_one<T, D, DUAL, MASK_ADD>(p, stream);
+    }
+    return -3;
+  } else if constexpr (D <= 128) {
+    switch (mask) {
+      case MASK_NONE: return launch_fwd_f32_one<D, DUAL, MASK_NONE>(p, stream);
+      case MASK_BOOL: return launch_fwd_f32_one<D, DUAL, MASK_BOOL>(p, stream);
+      case MASK_ADD: return launch_fwd_f32_one<D, DUAL, MASK_ADD>(p, stream);
     }
     return -3;
   } else {

@@ -1,4 +1,5 @@
-// Fused dual forward: O, O', M, mu in one pass over LDS-staged K/K'/V/V' tiles.
+// Fused dual forward: O, O', M, mu in one pass over LDS-staged K/K'/V/V' tiles.  Launched for fp32 at D = 256, whose
+// rows and accumulators leave no registers for the pipeline of the other kernels (fwd_kernel_f32.hpp, fwd_kernel_v2.hpp).
 //
 // Work split: one workgroup of 4 waves owns 128 query rows of one (z, h); each wave owns 32
 // of them and keeps Q, Q' (B operands) and the accumulators O^T, T^T (D x 32 each) in
@@ -75,19 +76,9 @@ __global__ __launch_bounds__(256, 1) void fwd_kernel(const FwdParams p) {
   const int qrow = q0 + wave * 32 + r; // this lane's query row
   const int qld = qrow < L ? qrow : L - 1;
 
-  // D = 256 (fp32 only: the 16-bit types have kernels of their own at this head dim, fwd_kernel_wide.hpp): Q, Q'
-  // resident would be up to 256 registers next to 256 of accumulators, so there the lane's fragments are read
-  // from global memory where they are used (the same 32 bytes per lane on every tile: cache hits)
-  constexpr bool SB = D == 256;
+  // Q, Q' resident would be up to 256 registers next to 256 of accumulators: the lane's fragments are read from
+  // global memory where they are used (the same 32 bytes per lane on every tile: cache hits)
   const T *Qrow = Qg + (size_t)qld * D + 8 * g, *Qtrow = DUAL ? Qtg + (size_t)qld * D + 8 * g : nullptr;
-  Frag<T> Qf[SB ? 1 : KK], Qtf[(DUAL && !SB) ? KK : 1];
-  if constexpr (!SB) {
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      Qf[kk] = ld8<T>(Qrow + 16 * kk);
-      if constexpr (DUAL) Qtf[kk] = ld8<T>(Qtrow + 16 * kk);
-    }
-  }
 
   f32x16 Oacc[DB], Tacc[DUAL ? DB : 1];
 #pragma unroll
@@ -117,48 +108,17 @@ __global__ __launch_bounds__(256, 1) void fwd_kernel(const FwdParams p) {
     walk.init(tl, 0, kend, Lk);
   }
 
-  // The next tile is fetched into registers while this one is computed and written to LDS behind the
-  // barrier that follows.  Not for D >= 128 (no registers to spare) and not for 16-bit D = 32, where
-  // the registers would cost the second and third workgroup per compute unit that hide the latency
-  // better (403 vs 327 TFLOP/s measured).
-  constexpr bool AHEAD = D == 64 || (D == 32 && sizeof(T) == 4);
-  RowChunks<T, BN, D, Cfg::NT> rk, rkt;
-  QuadChunks<T, BN, D, Cfg::NT> rv, rvt;
-  auto fetch_tile = [&](int j0) {
-    const int nvalid = Lk - j0;  // rows >= nvalid are zero-filled
-    fetch_rows(rk, Kg + (size_t)j0 * D, nvalid, tid);
-    fetch_quads(rv, Vg + (size_t)j0 * D, nvalid, tid);
-    if constexpr (DUAL) {
-      fetch_rows(rkt, Ktg + (size_t)j0 * D, nvalid, tid);
-      fetch_quads(rvt, Vtg + (size_t)j0 * D, nvalid, tid);
-    }
-  };
-  if constexpr (AHEAD) {
-    if (walk.n > 0) fetch_tile(walk.at(0));
-  }
   for (int it = 0; it < walk.n; ++it) {
     const int j0 = walk.at(it);
     __syncthreads();
-    if constexpr (AHEAD) {
-      put_rows(Ks, Cfg::LDK, rk, tid);
-      put_quads_transposed(Vs, Cfg::LDV, rv, tid);
-      if constexpr (DUAL) {
-        put_rows(Kts, Cfg::LDK, rkt, tid);
-        put_quads_transposed(Vts, Cfg::LDV, rvt, tid);
-      }
-    } else {
-      const int nvalid = Lk - j0;  // rows >= nvalid are zero-filled
-      copy_rows<T, BN, D, Cfg::NT>(Ks, Cfg::LDK, Kg + (size_t)j0 * D, nvalid, tid);
-      copy_rows_transposed<T, BN, D, Cfg::NT>(Vs, Cfg::LDV, Vg + (size_t)j0 * D, nvalid, tid);
-      if constexpr (DUAL) {
-        copy_rows<T, BN, D, Cfg::NT>(Kts, Cfg::LDK, Ktg + (size_t)j0 * D, nvalid, tid);
-        copy_rows_transposed<T, BN, D, Cfg::NT>(Vts, Cfg::LDV, Vtg + (size_t)j0 * D, nvalid, tid);
-      }
+    const int nvalid = Lk - j0;  // rows >= nvalid are zero-filled
+    copy_rows<T, BN, D, Cfg::NT>(Ks, Cfg::LDK, Kg + (size_t)j0 * D, nvalid, tid);
+    copy_rows_transposed<T, BN, D, Cfg::NT>(Vs, Cfg::LDV, Vg + (size_t)j0 * D, nvalid, tid);
+    if constexpr (DUAL) {
+      copy_rows<T, BN, D, Cfg::NT>(Kts, Cfg::LDK, Ktg + (size_t)j0 * D, nvalid, tid);
+      copy_rows_transposed<T, BN, D, Cfg::NT>(Vts, Cfg::LDV, Vtg + (size_t)j0 * D, nvalid, tid);
     }
     __syncthreads();
-    if constexpr (AHEAD) {
-      if (it + 1 < walk.n) fetch_tile(walk.at(it + 1));
-    }
 
     // ---- S^T = K Q^T and S'^T = K Q'^T + K' Q^T -------------------------------------------
     f32x16 S[NB], Sp[DUAL ? NB : 1];
@@ -172,23 +132,14 @@ __global__ __launch_bounds__(256, 1) void fwd_kernel(const FwdParams p) {
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
         Frag<T> a = lds_frag(Ks + (32 * nb + pr32) * Cfg::LDK + 16 * kk + 8 * g);
-        if constexpr (SB) {
-          const Frag<T> qf = ld8<T>(Qrow + 16 * kk);
-          mma(S[nb], a, qf);
-          if constexpr (DUAL) {
-            mma(Sp[nb], a, ld8<T>(Qtrow + 16 * kk));
-            Frag<T> a2 = lds_frag(Kts + (32 * nb + pr32) * Cfg::LDK + 16 * kk + 8 * g);
-            mma(Sp[nb], a2, qf);
-          }
-          if (kk % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // bound the fragment reads in flight
-        } else {
-        mma(S[nb], a, Qf[kk]);
+        const Frag<T> qf = ld8<T>(Qrow + 16 * kk);
+        mma(S[nb], a, qf);
         if constexpr (DUAL) {
-          mma(Sp[nb], a, Qtf[kk]);
+          mma(Sp[nb], a, ld8<T>(Qtrow + 16 * kk));
           Frag<T> a2 = lds_frag(Kts + (32 * nb + pr32) * Cfg::LDK + 16 * kk + 8 * g);
-          mma(Sp[nb], a2, Qf[kk]);
+          mma(Sp[nb], a2, qf);
         }
-        }
+        if (kk % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // bound the fragment reads in flight
       }
     }
 

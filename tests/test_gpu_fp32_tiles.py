@@ -1,0 +1,36 @@
+"""fp32 kernels at the edges of their 32-row tiles and 128-row blocks, against the dense oracle."""
+import numpy as np
+import pytest
+import torch
+
+from jvp_flash_attention_amd import _lib
+from oracle import dense
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("L,Lk", [(1, 1), (31, 33), (32, 32), (33, 31), (127, 129), (128, 64), (129, 96), (160, 255)])
+@pytest.mark.parametrize("mask", ["none", "causal", "bool", "bias"])
+def test_tile_edges(D, L, Lk, mask):
+    print("case", D, L, Lk, mask, flush=True)
+    g = torch.Generator().manual_seed(1000 * D + L)
+    rand = lambda n: torch.randn(1, 2, n, D, generator=g)  # noqa: E731
+    cpu = [rand(L), rand(Lk), rand(Lk), rand(L), rand(Lk), rand(Lk), rand(L), rand(L)]
+    m, kind = None, _lib.MASK_NONE
+    if mask == "bool":
+        m, kind = torch.rand(1, 2, L, Lk, generator=g) < 0.7, _lib.MASK_BOOL
+        m[..., 0] = True
+    elif mask == "bias":
+        m, kind = torch.randn(1, 1, L, Lk, generator=g), _lib.MASK_ADD
+    f = [x.double().numpy() for x in cpu]
+    opts = dict(mask=None if m is None else (m.numpy() if kind == _lib.MASK_BOOL else m.double().numpy()), causal=mask == "causal")
+    fwd, bwd = dense.forward(*f[:6], **opts), dense.backward(*f, **opts)
+    q, k, v, qt, kt, vt, go, gt = (x.cuda() for x in cpu)
+    md = None if m is None else m.cuda()
+    be = _lib.backend()
+    o, ot, M, mu = be.fwd(q, k, v, qt, kt, vt, md, kind, mask == "causal", D**-0.5)
+    six = be.bwd(q, k, v, qt, kt, vt, o, ot, M, mu, go, gt, md, kind, mask == "causal", D**-0.5, True)
+    for name, got, want in (("O", o, fwd["O"]), ("Ot", ot, fwd["Ot"]), *zip(("dq", "dk", "dv", "dqt", "dkt", "dvt"), six, (bwd[n] for n in ("dq", "dk", "dv", "dqt", "dkt", "dvt")))):
+        # the repository's fp32 bar, relative where the quantity is larger than one
+        assert np.abs(got.double().cpu().numpy() - want).max() <= 1e-4 * max(1.0, np.abs(want).max()), name

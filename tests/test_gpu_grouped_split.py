@@ -39,9 +39,10 @@ def test_split_groups_agree_with_whole_ones(dtype, D, H, Hk, L, Lk, mode):
         _lib.set_split(True)
     got = grads()
     # both add the same fp32 products in another order and round once, so an entry may round to the neighbouring value:
-    # a spacing of at most 2^-7 of the entry in bf16 and 2^-10 in fp16 (7 and 10 fraction bits); in fp32 what is left is
-    # the error of sums over at most 6 heads x 300 queries
-    bar = {torch.bfloat16: 2**-7, torch.float16: 2**-10, torch.float32: 2e-6}[dtype]
+    # a spacing of at most 2^-7 of the entry in bf16 and 2^-10 in fp16 (7 and 10 fraction bits).  In fp32 the order itself
+    # is what is left: up to n = 2 x 4 heads x 200 queries additions round partial sums of the result's size, an error of
+    # sqrt(n) 2^-24 = 2.4e-6 on either side, 3.4e-6 for the difference; three times that is allowed.
+    bar = {torch.bfloat16: 2**-7, torch.float16: 2**-10, torch.float32: 1e-5}[dtype]
     for name, a, b in zip(("dq", "dk", "dv", "dqt", "dkt", "dvt"), got, want):
         if b is None:
             continue
