@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(const BwdParams p) {
   const int L = pr.L;
   const int nqb = (L + BWD_BLK - 1) / BWD_BLK;
   const int total = nqb * pr.Z * pr.H;
-  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H);
+  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nqb;
   const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
   const int z = zh / pr.H, h = zh % pr.H;
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;  // queries, keys
   const int nkb = (Lk + BWD_BLK - 1) / BWD_BLK;
-  const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks);
+  const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zhk = id / nkb / pr.chunks, chunk = id / nkb % pr.chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nkb;  // causal: the first key blocks have the longest query loops
   const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = pr.H / pr.Hk / pr.chunks;

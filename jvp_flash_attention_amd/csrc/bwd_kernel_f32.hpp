@@ -54,7 +54,7 @@ __device__ __forceinline__ void bwd_f32_dq_body(const BwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nqb = (L + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H);
+  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nqb;
   const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
   const int z = zh / pr.H, h = zh % pr.H;
@@ -261,7 +261,7 @@ __device__ __forceinline__ void bwd_f32_dkdv_body(const BwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nkb = (Lk + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks);
+  const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zhk = id / nkb / pr.chunks, chunk = id / nkb % pr.chunks;
   const int kb = id % nkb;  // causal: the first key blocks have the longest query loops
   const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = pr.H / pr.Hk / pr.chunks;

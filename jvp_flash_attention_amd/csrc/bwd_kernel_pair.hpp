@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L;
   const int nblk = (L + Cfg::BLK - 1) / Cfg::BLK;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.H);
+  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nblk;
   const int rem = id % nblk;
   const int qb = pr.causal ? nblk - 1 - rem : rem;
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nblk = (Lk + Cfg::BLK - 1) / Cfg::BLK;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * pr.chunks);
+  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zh = id / nblk / pr.chunks, chunk = id / nblk % pr.chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nblk;
   const int z = zh / pr.Hk, hk = zh % pr.Hk, group = pr.H / pr.Hk / pr.chunks;

@@ -74,7 +74,7 @@ constexpr int bwd_spread(int nstep) { return 3 * nstep / 4; }
   const int L = pr.L;                                                                                               \
   /* a workgroup owns 128 of the OWN_ROWS rows of one (z, head out of OWN_HEADS), or one of CHUNKS shares of it */ \
   const int nblk = ((OWN_ROWS) + Cfg::BLK - 1) / Cfg::BLK;                                                          \
-  const int id = xcd_remap(bid, nblk, pr.Z * (OWN_HEADS) * (CHUNKS));                                               \
+  const int id = xcd_remap(bid, nblk, pr.Z * (OWN_HEADS) * (CHUNKS), pr.causal != 0);                                               \
   const int zh = id / nblk / (CHUNKS), chunk = id / nblk % (CHUNKS);                                                \
   const int z = zh / (OWN_HEADS), h = zh % (OWN_HEADS);                                                             \
   const int tid = threadIdx.x;                                                                                      \

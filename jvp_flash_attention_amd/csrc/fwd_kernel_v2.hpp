@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256, 1) void fwd2_kernel(const FwdParams p) {
   const int L = pr.L;
   const int nqb = (L + Cfg::BM - 1) / Cfg::BM;
   const int total = nqb * pr.Z * pr.H;
-  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H);
+  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nqb;
   const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
   const int z = zh / pr.H, h = zh % pr.H;

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
   // small grids: the key tiles of a query block are split over pr.chunks workgroups (see split.hpp)
   const int chunks = pr.chunks;
   const int chunk = chunks > 1 ? (int)(blockIdx.x % chunks) : 0;
-  const int id = xcd_remap(chunks > 1 ? blockIdx.x / chunks : blockIdx.x, nqb, pr.Z * pr.H);
+  const int id = xcd_remap(chunks > 1 ? blockIdx.x / chunks : blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nqb;
   const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
 

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256, 1) void fwd_wide_kernel(const FwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L;
   const int nqb = (L + Cfg::BM - 1) / Cfg::BM;
-  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H);
+  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nqb;
   const int rem = id % nqb;
   const int qb = pr.causal ? nqb - 1 - rem : rem;
