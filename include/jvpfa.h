@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define JVPFA_ABI_VERSION 9
+#define JVPFA_ABI_VERSION 10
 
 enum jvpfa_dtype { JVPFA_BF16 = 0, JVPFA_FP16 = 1, JVPFA_FP32 = 2 };
 
@@ -112,6 +112,9 @@ typedef struct jvpfa_fwd_args {
    * No counterpart in the reference (one program per 32 query rows whatever the grid, JA:2474-2476). */
   void *split_workspace;
   uint64_t split_workspace_bytes;
+  /* optional, boolean masks only: the copy packed along the key axis that jvpfa_mask_scan() writes, or NULL.  Changes no
+   * result; the kernels for 16-bit element types at D <= 128 read it (without dropout), the others the mask itself. */
+  const uint32_t *mask_bits_q;
 } jvpfa_fwd_args;
 
 int jvpfa_fwd(const jvpfa_fwd_args *args, void *hip_stream);
@@ -158,6 +161,7 @@ typedef struct jvpfa_bwd_args {
    * key and value gradients there, and a second kernel adds them up.  Results agree with the unsplit launch to rounding. */
   void *split_workspace;
   uint64_t split_workspace_bytes;
+  const uint32_t *mask_bits_q; /* as in jvpfa_fwd_args (dq kernels) */
 } jvpfa_bwd_args;
 
 int jvpfa_bwd(const jvpfa_bwd_args *args, void *hip_stream);
@@ -220,6 +224,22 @@ int jvpfa_mask_tiles(const jvpfa_problem *p, int32_t Lk, int32_t *tiles_q, int32
  */
 size_t jvpfa_mask_bits_bytes(const jvpfa_problem *p, int32_t Lk);
 int jvpfa_mask_bits(const jvpfa_problem *p, int32_t Lk, uint32_t *bits, void *hip_stream);
+
+/*
+ * Everything the kernels can use about a boolean mask with a row per query, from one pass over it: both tile lists (as
+ * jvpfa_mask_tiles writes them), both packed copies (bits_k as jvpfa_mask_bits writes it; bits_q the same with the axes
+ * exchanged: word [((plane * ceil(Lk/64) + t) * L + i) * 2 + hf], bit j, is the entry of (query i, key 64 t + 32 hf + j);
+ * either may be NULL) and per mask plane whether it attends to anything (0 / 1).  bits_q takes
+ * planes * ceil(Lk/64) * L * 8 bytes; scratch jvpfa_mask_scan_bytes() bytes, contents don't-care.  Device memory throughout.
+ */
+typedef struct jvpfa_mask_scan_out {
+  int32_t *tiles_q, *tiles_k;
+  uint32_t *bits_q, *bits_k;
+  int32_t *attends;
+  void *scratch;
+} jvpfa_mask_scan_out;
+size_t jvpfa_mask_scan_bytes(const jvpfa_problem *p, int32_t Lk);
+int jvpfa_mask_scan(const jvpfa_problem *p, int32_t Lk, const jvpfa_mask_scan_out *out, void *hip_stream);
 
 /*
  * The keep pattern of dropout for this problem (only Z, H, L, dropout_p, dropout_seed are read) and Lk keys

@@ -9,18 +9,18 @@ from __future__ import annotations
 
 import ctypes as C
 import os
-from typing import Optional, Tuple
+from typing import NamedTuple, Optional, Tuple
 
 import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libjvpfa.so")
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 MASK_NONE, MASK_BOOL, MASK_ADD = 0, 1, 2
 EXPORTS = ("jvpfa_fwd", "jvpfa_bwd", "jvpfa_fwd_split_workspace_bytes", "jvpfa_dropout_keep", "jvpfa_bwd_workspace_bytes", "jvpfa_bwd_split_workspace_bytes", "jvpfa_bwd_static", "jvpfa_bwd_static_max_rows", "jvpfa_mask_tiles", "jvpfa_mask_tiles_bytes",
-           "jvpfa_mask_bits", "jvpfa_mask_bits_bytes",
+           "jvpfa_mask_bits", "jvpfa_mask_bits_bytes", "jvpfa_mask_scan", "jvpfa_mask_scan_bytes",
            "jvpfa_abi_version", "jvpfa_error_string")
 
 
@@ -48,6 +48,7 @@ class FwdArgs(C.Structure):
         ("tiles_q", C.c_void_p),
         ("Lk", C.c_int32), ("Hk", C.c_int32),
         ("split_workspace", C.c_void_p), ("split_workspace_bytes", C.c_uint64),
+        ("mask_bits_q", C.c_void_p),
     ]
 
 
@@ -68,7 +69,12 @@ class BwdArgs(C.Structure):
         ("Lk", C.c_int32), ("Hk", C.c_int32),
         ("mask_bits", C.c_void_p),
         ("split_workspace", C.c_void_p), ("split_workspace_bytes", C.c_uint64),
+        ("mask_bits_q", C.c_void_p),
     ]
+
+
+class MaskScanOut(C.Structure):
+    _fields_ = [(name, C.c_void_p) for name in ("tiles_q", "tiles_k", "bits_q", "bits_k", "attends", "scratch")]
 
 
 _lib = None
@@ -108,6 +114,10 @@ def load() -> C.CDLL:
         lib.jvpfa_mask_bits_bytes.restype = C.c_size_t
         lib.jvpfa_mask_bits.argtypes = [C.POINTER(Problem), C.c_int32, C.c_void_p, C.c_void_p]
         lib.jvpfa_mask_bits.restype = C.c_int
+        lib.jvpfa_mask_scan_bytes.argtypes = [C.POINTER(Problem), C.c_int32]
+        lib.jvpfa_mask_scan_bytes.restype = C.c_size_t
+        lib.jvpfa_mask_scan.argtypes = [C.POINTER(Problem), C.c_int32, C.POINTER(MaskScanOut), C.c_void_p]
+        lib.jvpfa_mask_scan.restype = C.c_int
         lib.jvpfa_abi_version.argtypes = []
         lib.jvpfa_abi_version.restype = C.c_int
         lib.jvpfa_error_string.argtypes = [C.c_int]
@@ -178,7 +188,7 @@ def forget_mask(mask) -> None:
     are keyed by the tensor's version counter, which ordinary in-place operations bump; writes that bypass it
     (``mask.data``, a custom kernel writing through ``data_ptr()``, a dlpack / numpy alias) do not, and after
     such a write this must be called before the mask is used again."""
-    for name in ("_jvpfa_verified", "_jvpfa_key_limit", "_jvpfa_tiles", "_jvpfa_bits"):
+    for name in ("_jvpfa_verified", "_jvpfa_key_limit", "_jvpfa_tiles", "_jvpfa_bits", "_jvpfa_scan"):
         try:
             delattr(mask, name)
         except AttributeError:
@@ -341,15 +351,68 @@ def _wants_backward(q, k, v, level) -> bool:
     return any(t is not None and t.requires_grad for t in tangents)
 
 
+class MaskScan(NamedTuple):
+    """What ``jvpfa_mask_scan`` found out about a boolean mask; the packed copies only where kernels read them."""
+
+    version: int | None
+    tiles_q: torch.Tensor
+    tiles_k: torch.Tensor
+    bits_q: torch.Tensor | None
+    bits_k: torch.Tensor | None
+    attends: torch.Tensor  # per mask plane: 1 where it attends to anything
+
+
+def mask_scan(q, mask, mask_kind, Lk):
+    """The ``MaskScan`` of a boolean mask with a row per query (shape [*, *, L, Lk]), from one pass over it, or None for
+    other masks, short sequences, and with the tile lists or the packed copies switched off.  Cached on the mask tensor,
+    keyed by its version counter, where ``tile_lists`` and ``mask_bits`` look as well."""
+    Z, H, L, D = q.shape
+    if not (_tile_lists_enabled and _mask_bits_enabled) or mask is None or mask_kind != MASK_BOOL or max(L, Lk) < TILE_LISTS_MIN_L:
+        return None
+    if mask.dim() != 4 or mask.shape[2] != L or mask.shape[3] != Lk or not mask.is_cuda:
+        return None
+    packed = q.element_size() == 2 and D <= 128
+    version = mask_version(mask)
+    cached = getattr(mask, "_jvpfa_scan", None)
+    if cached is not None and version is not None and cached.version == version and (cached.bits_q is not None or not packed):
+        return cached
+    lib = load()
+    prob = make_problem(q, mask, mask_kind, False, 1.0)
+    planes = (Z if prob.mask_stride[0] else 1) * (H if prob.mask_stride[1] else 1)
+
+    def ints(n):
+        return torch.empty(n, device=mask.device, dtype=torch.int32)
+
+    scan = MaskScan(version, ints(lib.jvpfa_mask_tiles_bytes(C.byref(prob), Lk, 0) // 4), ints(lib.jvpfa_mask_tiles_bytes(C.byref(prob), Lk, 1) // 4),
+                    ints(planes * ((Lk + 63) // 64) * L * 2) if packed else None,
+                    ints(lib.jvpfa_mask_bits_bytes(C.byref(prob), Lk) // 4) if packed else None, ints(planes))
+    scratch = torch.empty(lib.jvpfa_mask_scan_bytes(C.byref(prob), Lk), device=mask.device, dtype=torch.uint8)
+    out = MaskScanOut(_ptr(scan.tiles_q), _ptr(scan.tiles_k), _ptr(scan.bits_q), _ptr(scan.bits_k), _ptr(scan.attends), _ptr(scratch))
+    with torch.cuda.device(mask.device):
+        check(lib.jvpfa_mask_scan(C.byref(prob), Lk, C.byref(out), _stream(mask)))
+    if version is not None:
+        try:
+            mask._jvpfa_scan = scan
+            mask._jvpfa_tiles = [version, scan.tiles_q, scan.tiles_k]
+            if packed:
+                mask._jvpfa_bits = (version, scan.bits_k)
+        except (AttributeError, RuntimeError):
+            pass
+    return scan
+
+
 def mask_hints(q, mask, mask_kind, Lk, backward: bool):
-    """(key_limit, tiles_q, tiles_k, bits) for a call with this mask, each None where it does not apply; the last two
-    only for a backward."""
+    """(key_limit, tiles_q, tiles_k, bits_k, bits_q) for a call with this mask, each None where it does not apply; tiles_k and
+    bits_k only for a backward."""
     if mask_kind == MASK_NONE:
-        return None, None, None, None
+        return (None,) * 5
+    scan = mask_scan(q, mask, mask_kind, Lk)
+    if scan is not None:
+        return None, scan.tiles_q, scan.tiles_k if backward else None, scan.bits_k if backward else None, scan.bits_q
     with torch.cuda.device(q.device):
         lim = key_limit_hint(mask, mask_kind, q.shape[0], Lk)
         tq, tk = tile_lists(q, mask, mask_kind, backward, Lk)
-        return lim, tq, tk, mask_bits(q, mask, mask_kind, Lk) if backward else None
+        return lim, tq, tk, mask_bits(q, mask, mask_kind, Lk) if backward else None, None
 
 
 class HipBackend:
@@ -381,9 +444,9 @@ class HipBackend:
 
     def _fwd(self, q, k, v, qt, kt, vt, mask, mask_kind, causal, sm_scale, dropout_p=0.0, dropout_seed=0):
         _require_gpu(q, mask)
-        lim, tq, _, _ = mask_hints(q, mask, mask_kind, k.shape[2], False)
+        lim, tq, _, _, bits_q = mask_hints(q, mask, mask_kind, k.shape[2], False)
         return binding().fwd(q, k, v, qt, kt, vt, float(sm_scale), bool(causal), float(dropout_p), int(dropout_seed) & (2**64 - 1),
-                             _split_enabled, mask, mask_kind, lim, tq)
+                             _split_enabled, mask, mask_kind, lim, tq, bits_q)
 
     def _bwd(self, q, k, v, qt, kt, vt, o, ot, M, mu, go, gt, mask, mask_kind, causal, sm_scale,
              want_tangent_grads=False, dropout_p=0.0, dropout_seed=0):
@@ -395,7 +458,7 @@ class HipBackend:
     def attend(self, q, k, v, mask, mask_kind, causal, sm_scale, dropout_p, dropout_seed, level):
         """The whole eager call, autograd included, on tensors that may be dual tensors of ``level``; None when the
         shapes or types of q, k, v are not supported."""
-        hints = (None,) * 4
+        hints = (None,) * 5
         if mask_kind != MASK_NONE:
             _require_gpu(q, mask)
             hints = mask_hints(q, mask, mask_kind, k.shape[2], _wants_backward(q, k, v, level))

@@ -34,7 +34,8 @@ extern "C" int jvpfa_fwd(const jvpfa_fwd_args *a, void *hip_stream) {
     if (ptr && !aligned16(ptr)) return JVPFA_E_ALIGN;
 
   FwdParams p;
-  p.pr = to_problem(a->p, a->key_limit, a->tiles_q, nullptr, a->Lk, a->Hk);
+  if (reinterpret_cast<uintptr_t>(a->mask_bits_q) & 7u) return JVPFA_E_ALIGN;
+  p.pr = to_problem(a->p, a->key_limit, a->tiles_q, nullptr, a->Lk, a->Hk, nullptr, a->mask_bits_q);
   p.q = a->q; p.k = a->k; p.v = a->v;
   p.qt = a->qt; p.kt = a->kt; p.vt = a->vt;
   p.o = a->o; p.ot = a->ot; p.M = a->M; p.mu = a->mu;

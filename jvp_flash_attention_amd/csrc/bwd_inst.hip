@@ -23,6 +23,24 @@ template <typename T, int D> struct BwdFold {
   static constexpr bool KV = sizeof(T) == 2 && D <= 64;
 };
 
+// The dq kernel of the direct-to-LDS family for one launch.  MK is MASK, or MASK_BITS for a boolean mask whose packed copy
+// the caller handed over.  six: the dual variant that also writes dq'.
+template <typename T, int D, int MODE, int MK> static auto pick_dq(bool no_go, bool six) -> void (*)(const BwdParams) {
+  constexpr bool NG = MODE != BWD_DUAL;  // the GO template argument of the kernels without gO
+  if constexpr (MODE == BWD_DUAL) {
+    if (six) {
+      // (without gO the register cap of the two-workgroup twin makes the allocator copy LDS fragments out of
+      // their registers before they have arrived, which the build's lint refuses: that variant runs uncapped)
+      if constexpr (D == 64) return no_go ? bwd2_dq_kernel<T, D, MODE, MK, false, true> : bwd2_dq_kernel_2wg<T, D, MODE, MK, true, true>;
+      else return no_go ? bwd2_dq_kernel<T, D, MODE, MK, false, true> : bwd2_dq_kernel<T, D, MODE, MK, true, true>;
+    }
+  }
+  if constexpr (D == 128 && MODE == BWD_PLAIN) return bwd2_dq_kernel_2wg_plain<T, D, MODE, MK>;
+  // D = 64: the register-capped twins, two workgroups per compute unit (D = 32 needs no cap for that)
+  else if constexpr (D == 64) return no_go ? bwd2_dq_kernel_2wg<T, D, MODE, MK, NG> : bwd2_dq_kernel_2wg<T, D, MODE, MK, true>;
+  else return no_go ? bwd2_dq_kernel<T, D, MODE, MK, NG> : bwd2_dq_kernel<T, D, MODE, MK, true>;
+}
+
 // The dk/dv kernel of the direct-to-LDS family for one launch.  MK is MASK, or MASK_BITS for a boolean mask
 // whose bit-packed copy the caller handed over.  fold_kv: the dual variant that also writes dk', dv'.
 template <typename T, int D, int MODE, int MK>
@@ -184,20 +202,9 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       run_q = !(six && Fold::DQ);
       run_kv = !(six && Fold::KV);
     }
-    if constexpr (MODE == BWD_DUAL) {
-      if (six) {  // the variants that also write dq' (and dk', dv')
-        // (without gO the register cap of the two-workgroup twin makes the allocator copy LDS fragments out of
-        // their registers before they have arrived, which the build's lint refuses: that variant runs uncapped)
-        if constexpr (D == 64) kq = no_go ? bwd2_dq_kernel<T, D, MODE, MASK, false, true> : bwd2_dq_kernel_2wg<T, D, MODE, MASK, true, true>;
-        else kq = no_go ? bwd2_dq_kernel<T, D, MODE, MASK, false, true> : bwd2_dq_kernel<T, D, MODE, MASK, true, true>;
-      }
-    }
-    const bool plain_q = !(MODE == BWD_DUAL && six);
-    if constexpr (D == 64) {  // the register-capped twins: two workgroups per compute unit (D = 32 needs no cap for that)
-      if (plain_q) kq = no_go ? bwd2_dq_kernel_2wg<T, D, MODE, MASK, NG> : bwd2_dq_kernel_2wg<T, D, MODE, MASK, true>;
-    } else {
-      if (plain_q) kq = no_go ? bwd2_dq_kernel<T, D, MODE, MASK, NG> : bwd2_dq_kernel<T, D, MODE, MASK, true>;
-      if constexpr (D == 128 && MODE == BWD_PLAIN) kq = bwd2_dq_kernel_2wg_plain<T, D, MODE, MASK>;
+    kq = pick_dq<T, D, MODE, MASK>(no_go, MODE == BWD_DUAL && six);
+    if constexpr (MASK == MASK_BOOL) {
+      if (p.pr.bits_q) kq = pick_dq<T, D, MODE, MASK_BITS>(no_go, MODE == BWD_DUAL && six);
     }
     size_t kv_lds = 0;
     kkv = pick_dkdv_for<T, D, MODE, MASK>(p, no_go, grouped, MODE == BWD_DUAL && six, false, &kv_lds);

@@ -192,7 +192,9 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
   const float sl2 = pr.scale * LOG2E;
   const int64_t mrow = MASK != MASK_NONE ? z * pr.ms[0] + h * pr.ms[1] + (int64_t)qld * pr.ms[2] : 0;
   bool mask_al = false;  // mask rows can be fetched with aligned vector loads
-  if constexpr (MASK != MASK_NONE) mask_al = mask_rows_aligned<T, MASK>(pr);
+  if constexpr (MASK == MASK_BOOL || MASK == MASK_ADD) mask_al = mask_rows_aligned<T, MASK>(pr);
+  const uint32_t *bits_row = nullptr;
+  if constexpr (MASK == MASK_BITS) bits_row = pr.bits_q + mask_bits_q_offset(pr, z, h) + (size_t)qld * 2;
   // keys: Lk of them, in head h / (H / Hk) of the key/value tensors (L and h themselves for the
   // shapes the reference admits)
   const int Lk = pr.Lk;
@@ -297,12 +299,20 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
 
     // ---- P and the score gradients -------------------------------------------------------------
     const int klim = min(pr.causal ? qrow : 0x7fffffff, Lk - 1);  // keys above this index are masked
+    float spread[MASK == MASK_BITS ? 16 : 1];  // MASK_BITS: all ones for an attended entry, all zeros for a masked one
+    if constexpr (MASK == MASK_BITS) {
+      const uint32_t w = mah[0].w >> (8 * g);
+      static_for<16>([&](auto ec) {
+        constexpr int e = decltype(ec)::value;
+        spread[e] = __uint_as_float(mask_spread<mask_bit_of(e)>(w));
+      });
+    }
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
       const int key0 = jh + 16 * hf + 8 * g;
       float bias[8];
       bool keep[8];
-      if constexpr (MASK != MASK_NONE) {
+      if constexpr (MASK == MASK_BOOL || MASK == MASK_ADD) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           // the mask value and the row's reference point in one term: the exponent is then one fused multiply-add
@@ -318,6 +328,7 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
         if constexpr (MASK == MASK_ADD) pv = fast_exp2(fmaf(S[i], sl2, bias[e]));
         else pv = fast_exp2(S[i] * sl2 - Mq);
         if constexpr (MASK == MASK_BOOL) pv = keep[e] ? pv : 0.f;
+        if constexpr (MASK == MASK_BITS) pv = __uint_as_float(__float_as_uint(pv) & __float_as_uint(spread[i]));
         if constexpr (EDGE) pv = (key0 + e <= klim) ? pv : 0.f;
         if constexpr (DROP) {
           const float ks = drop_scale_of(pr, xb + (uint32_t)e * DROP_C_KEY);
@@ -388,7 +399,10 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
   // Mask values travel from HBM or the far caches, further than one phase of matrix products hides:
   // those of tile t+1 are requested at the top of tile t.
   auto fetch_masks = [&](int tn) {
-    if constexpr (MASK != MASK_NONE) {
+    if constexpr (MASK == MASK_BITS) {
+      mnext[0][0] = mask_fetch_bits<T>(pr, bits_row, tn * BT);
+      mnext[1][0] = mask_fetch_bits<T>(pr, bits_row, tn * BT + 32);
+    } else if constexpr (MASK != MASK_NONE) {
       const int jn = tn * BT;
       if (mask_al && jn + BT <= Lk) {  // aligned rows, all 64 keys exist: one vector load per 8 keys
 #pragma unroll
@@ -434,7 +448,7 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
   // own so that the common tile carries no limit tests.  (q0 is a multiple of the tile size.)
   int t_edge = Lk / BT;
   if (pr.causal) t_edge = min(t_edge, q0 / BT);
-  if (MASK != MASK_NONE && !mask_al) t_edge = 0;  // interior tiles fetch mask rows with aligned vector loads
+  if ((MASK == MASK_BOOL || MASK == MASK_ADD) && !mask_al) t_edge = 0;  // interior tiles fetch mask rows with aligned vector loads
   int t = 0;
   if constexpr (!LEAN) {
     for (; t < ntiles && tcur < t_edge; ++t) tile(t, std::false_type{});
@@ -900,10 +914,9 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
           else pv = fast_exp2(s - stat(0, e));
           if constexpr (MASK == MASK_BOOL) pv = keep ? pv : 0.f;
           if constexpr (MASK == MASK_BITS) {
-            // the entry's bit spread over a word (0 or all ones), and-ed onto P: two instructions (written as
-            // asm: from the builtin the compiler makes a bit test, a compare and a select)
+            // (written as asm: from the builtin the compiler makes a bit test, a compare and a select)
             uint32_t spread;
-            asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(spread) : "v"(mraw_w), "n"(16 * (e / 8) + (e % 8)));
+            asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(spread) : "v"(mraw_w), "n"(mask_bit_of(e)));
             pv = __uint_as_float(__float_as_uint(pv) & spread);
           }
           if constexpr (EDGE) pv = (qi >= qmin && qi < L) ? pv : 0.f;

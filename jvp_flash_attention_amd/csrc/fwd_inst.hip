@@ -154,14 +154,14 @@ static int launch_fwd_mask(const FwdParams &p, int mask, hipStream_t stream) {
     // the pipelined kernel pays off where a slot has enough matrix work to hide the softmax behind
     switch (mask) {
       case MASK_NONE: return launch_fwd3_one<T, D, DUAL>(p, stream);
-      case MASK_BOOL: return launch_fwd3_one<T, D, DUAL, MASK_BOOL>(p, stream);
+      case MASK_BOOL: return p.pr.bits_q ? launch_fwd3_one<T, D, DUAL, MASK_BITS>(p, stream) : launch_fwd3_one<T, D, DUAL, MASK_BOOL>(p, stream);
       case MASK_ADD: return launch_fwd3_one<T, D, DUAL, MASK_ADD>(p, stream);
     }
     return -3;
   } else if constexpr (sizeof(T) == 2 && D < 128) {
     switch (mask) {
       case MASK_NONE: return launch_fwd2_one<T, D, DUAL, MASK_NONE>(p, stream);
-      case MASK_BOOL: return launch_fwd2_one<T, D, DUAL, MASK_BOOL>(p, stream);
+      case MASK_BOOL: return p.pr.bits_q ? launch_fwd2_one<T, D, DUAL, MASK_BITS>(p, stream) : launch_fwd2_one<T, D, DUAL, MASK_BOOL>(p, stream);
       case MASK_ADD: return launch_fwd2_one<T, D, DUAL, MASK_ADD>(p, stream);
     }
     return -3;

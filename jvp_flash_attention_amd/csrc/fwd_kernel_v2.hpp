@@ -186,7 +186,9 @@ __global__ __launch_bounds__(256, 1) void fwd2_kernel(const FwdParams p) {
   const int64_t mrow = MASK != MASK_NONE ? z * pr.ms[0] + h * pr.ms[1] + (int64_t)qld * pr.ms[2] : 0;
   const uint32_t drop_row = DROP ? drop_row_word(pr, zh, qld) : 0u;  // dropout: this lane's query row, see params.hpp
   bool mask_al = false;  // mask rows can be fetched with aligned vector loads
-  if constexpr (MASK != MASK_NONE) mask_al = mask_rows_aligned<T, MASK>(pr);
+  if constexpr (MASK == MASK_BOOL || MASK == MASK_ADD) mask_al = mask_rows_aligned<T, MASK>(pr);
+  const uint32_t *bits_row = nullptr;
+  if constexpr (MASK == MASK_BITS) bits_row = pr.bits_q + mask_bits_q_offset(pr, z, h) + (size_t)qld * 2;
 
   int kend = Lk;
   // padded batches: the caller's hint says the mask hides every key from klimit[z] on, so those tiles
@@ -325,7 +327,15 @@ __global__ __launch_bounds__(256, 1) void fwd2_kernel(const FwdParams p) {
         const int key0 = jh + 16 * hf + 8 * g;
         float bias[8];
         bool keep[8];
-        if constexpr (MASK != MASK_NONE) {
+        if constexpr (MASK == MASK_BITS) {
+          if (hf == 0) {
+            const uint32_t w = mah[0].w >> (8 * g);
+            static_for<16>([&](auto ec) {
+              constexpr int e = decltype(ec)::value;
+              S[e] = mask_logit_of_bit<mask_bit_of(e)>(w, S[e] * sl2, 0xff800000u);
+            });
+          }
+        } else if constexpr (MASK != MASK_NONE) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             if constexpr (MASK == MASK_ADD) bias[e] = mask_bias_of<T, MASK>(mah[hf], e);
@@ -334,7 +344,7 @@ __global__ __launch_bounds__(256, 1) void fwd2_kernel(const FwdParams p) {
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          float s = S[8 * hf + e] * sl2;
+          float s = MASK == MASK_BITS ? S[8 * hf + e] : S[8 * hf + e] * sl2;
           if constexpr (MASK == MASK_ADD) s += bias[e];
           if constexpr (MASK == MASK_BOOL) s = keep[e] ? s : NEG_INF;
           if constexpr (EDGE) s = (key0 + e <= klim) ? s : NEG_INF;
@@ -453,7 +463,10 @@ __global__ __launch_bounds__(256, 1) void fwd2_kernel(const FwdParams p) {
   // Mask values travel from HBM or the far caches, further than one phase of matrix products hides:
   // those of tile t+1 are requested at the top of tile t.  [half tile][16-key group] of a tile.
   auto fetch_masks = [&](int tn) {
-    if constexpr (MASK != MASK_NONE) {
+    if constexpr (MASK == MASK_BITS) {
+      mnext[0][0] = mask_fetch_bits<T>(pr, bits_row, tn * BN);
+      mnext[1][0] = mask_fetch_bits<T>(pr, bits_row, tn * BN + 32);
+    } else if constexpr (MASK != MASK_NONE) {
       const int jn = tn * BN;
       if (mask_al && jn + BN <= Lk) {  // aligned rows, all 64 keys exist: one vector load per 8 keys
 #pragma unroll
@@ -498,7 +511,7 @@ __global__ __launch_bounds__(256, 1) void fwd2_kernel(const FwdParams p) {
   // common tile carries no limit tests.  (q0 is a multiple of the tile size.)
   int t_edge = Lk / BN;
   if (pr.causal) t_edge = min(t_edge, q0 / BN);
-  if (!(sl2 > 0.f) || (MASK != MASK_NONE && !mask_al)) t_edge = 0;
+  if (!(sl2 > 0.f) || ((MASK == MASK_BOOL || MASK == MASK_ADD) && !mask_al)) t_edge = 0;
   int t = 0;
   for (; t < ntiles && tcur < t_edge; ++t) tile(t, std::false_type{});
   for (; t < ntiles; ++t) tile(t, std::true_type{});

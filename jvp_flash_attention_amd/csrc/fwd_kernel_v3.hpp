@@ -186,7 +186,9 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
   const int qlim = pr.causal ? qrow - k0 : 0x7fffffff;  // keys above this index are masked
   const int64_t mrow = MASK != MASK_NONE ? (zh / pr.H) * pr.ms[0] + (zh % pr.H) * pr.ms[1] + (int64_t)qld * pr.ms[2] : 0;
   bool mask_al = false;  // mask rows can be fetched with aligned vector loads
-  if constexpr (MASK != MASK_NONE) mask_al = mask_rows_aligned<T, MASK>(pr);
+  if constexpr (MASK == MASK_BOOL || MASK == MASK_ADD) mask_al = mask_rows_aligned<T, MASK>(pr);
+  const uint32_t *bits_row = nullptr;
+  if constexpr (MASK == MASK_BITS) bits_row = pr.bits_q + mask_bits_q_offset(pr, zh / pr.H, zh % pr.H) + (size_t)qld * 2;
   const uint32_t drop_row = DROP ? drop_row_word(pr, zh, qld) : 0u;  // dropout: this lane's query row, see params.hpp
   // List elements are requested an iteration ahead, unconditionally (from a harmless address when there is no
   // list: a branch around the read would split the loop's straight-line body).
@@ -270,7 +272,7 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
   // One slot.  QK: scores of a half tile (K rows at LDS address kaddr) into Sn, Spn.  PV: accumulate
   // the half tile whose V rows are at vaddr, with fragments pfp, psfp.  SM: softmax of Sc, Spc (first
   // key jh) into pfn, psfn.  GEN: 0 the softmax takes the scores as they are; 1 it adds the mask terms madd
-  // (0 or -inf for a boolean mask, the bias in log2 units for an additive one) to the scaled scores; 2 it
+  // (0 or -inf for a boolean mask, from its bytes or its packed copy; the bias in log2 units for an additive one) to the scaled scores; 2 it
   // applies the causal / sequence-end limits (kernels without a mask).  With a mask, a slot that forms scores
   // also forms the mask terms that go with them, in its gaps: madd is read by the front of the softmax and
   // refilled behind it from the mask words mah of the half tile whose scores the slot forms (keys
@@ -288,7 +290,9 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
     constexpr bool PREC = MASK != MASK_NONE && QK;  // mask terms for the scores this slot forms
     constexpr int NPRE = PREC ? 8 : 0;              // ... as this many vector units of two entries
     uint32_t vzero = 0u, vninf = 0xff800000u;
-    if constexpr (PREC && MASK == MASK_BOOL) asm volatile("" : "+v"(vzero), "+v"(vninf));  // vector registers that hold 0 and -inf
+    if constexpr (PREC && (MASK == MASK_BOOL || MASK == MASK_BITS)) asm volatile("" : "+v"(vzero), "+v"(vninf));  // vector registers that hold 0 and -inf
+    uint32_t mword = 0u;  // MASK_BITS: the word the mask terms of this slot come from
+    if constexpr (PREC && MASK == MASK_BITS) mword = mah[0].w >> (8 * g);
     // dropout: register e holds key jh + 16(e/8) + 8g + e%8 of this lane's query
     const uint32_t xb = DROP ? drop_row + (uint32_t)(jh + 8 * g) * DROP_C_KEY : 0u;
     constexpr int LB = decltype(LBc)::value;
@@ -408,6 +412,7 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
               const uint32_t word = (e % 8) < 4 ? (uint32_t)mah[e / 8].w : (uint32_t)(mah[e / 8].w >> 32);
               madd[e] = mask_term_of_byte<e % 4>(word, vzero, vninf);
             }
+            if constexpr (MASK == MASK_BITS) madd[e] = mask_term_of_bit<mask_bit_of(e)>(mword, vninf);
             if constexpr (MASK == MASK_ADD) madd[e] = (float)mah[e / 8].f[e % 8] * LOG2E;
           });
           anchor(madd[2 * (k - NUS)]);
@@ -572,7 +577,9 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
   MaskAhead<T, MASK> mcur[2][2], mnext[2][2];
   float madd[16];  // mask terms of the scores in flight, see slot()
   auto fetch_half = [&](MaskAhead<T, MASK>(&dst)[2], int jh) {
-    if constexpr (MASKED) {
+    if constexpr (MASK == MASK_BITS) {
+      dst[0] = mask_fetch_bits<T>(pr, bits_row, jh);
+    } else if constexpr (MASKED) {
       if (mask_al && jh + 32 <= pr.Lk) {  // aligned rows, all 32 keys exist: one vector load per 8 keys
 #pragma unroll
         for (int c = 0; c < 2; ++c) dst[c] = mask_fetch8<T, MASK>(pr, mrow, jh + 16 * c + 8 * g);

@@ -1,4 +1,5 @@
-// C ABI: jvpfa_mask_tiles -- lists of the 64-wide tiles of a mask that hold an attended entry.
+// C ABI: jvpfa_mask_tiles, jvpfa_mask_bits, jvpfa_mask_scan -- lists of the 64-wide tiles of a mask that hold an attended
+// entry, and bit-packed copies.
 //
 // The forward and dq kernels own 128 query rows and stream 64-key tiles; the dk/dv kernels own 128
 // keys and stream 64-query tiles.  One workgroup here walks the strip of one such owner and writes
@@ -10,6 +11,7 @@
 #include <algorithm>
 
 #include "api_common.hpp"
+#include "common.hpp"
 
 namespace jvpfa {
 
@@ -140,6 +142,96 @@ __global__ __launch_bounds__(256) void mask_bits_kernel(const uint8_t *mask, int
   uint32_t *dst = out + (((size_t)plane * (nqb / 2) + qb / 2) * (size_t)Lk + key0) * 2 + (qb & 1);
   for (int j = 0; j < min(4, Lk - key0); ++j) dst[2 * j] = w[j];
 }
+
+// ---- everything about a boolean mask from one pass over it ------------------------------------------------------
+// A wave takes 64 query rows x 64 keys: lane = key reads one byte per row (16 rows in flight; the four waves of a
+// workgroup take neighbouring keys, so lines are read whole), the ballot of a row is its 64 bits, and lane r keeps row
+// r's.  From those registers: the copy packed along the key axis, the copy packed along the query axis (64 ballots, lane
+// = key), and whether the tile holds an attended entry.  Bound by HBM for large masks ((Z,H,L,L) at B4 H16 L4096: 1.07 GB
+// read, a quarter of it written), by latency for small ones.  Before, two list kernels and the packing kernel each read
+// the mask, with one workgroup walking a whole strip: packed documents B2 L2077, 337 -> 26 us; (Z,H,L,L) 721 -> 469 us.
+__global__ __launch_bounds__(256) void mask_scan_kernel(const uint8_t *mask, int64_t s0, int64_t s1, int64_t s2, int64_t s3, int hm,
+                                                        int Lq, int Lk, uint32_t *bits_q, uint32_t *bits_k, uint8_t *flags) {
+  const int nqt = (Lq + 63) / 64, nkt = (Lk + 63) / 64, kgroups = (nkt + 3) / 4;
+  const int lane = threadIdx.x % WAVE, kt = (blockIdx.x % kgroups) * 4 + threadIdx.x / WAVE;
+  const int qt = blockIdx.x / kgroups % nqt, plane = blockIdx.x / kgroups / nqt;
+  if (kt >= nkt) return;
+  const int row0 = qt * 64, key = kt * 64 + lane, rows = min(64, Lq - row0);
+  const uint8_t *base = mask + (int64_t)(plane / hm) * s0 + (int64_t)(plane % hm) * s1 + (int64_t)min(key, Lk - 1) * s3;
+  const bool exists = key < Lk;
+  uint32_t lo = 0u, hi = 0u;  // this lane's row: keys 0..31 and 32..63 of the tile
+#pragma unroll
+  for (int r0 = 0; r0 < 64; r0 += 16) {
+    uint32_t x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = base[(int64_t)(row0 + min(r0 + i, rows - 1)) * s2];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const uint64_t b = __ballot(exists && r0 + i < rows && x[i] != 0);
+      lo = lane == r0 + i ? (uint32_t)b : lo;
+      hi = lane == r0 + i ? (uint32_t)(b >> 32) : hi;
+    }
+  }
+  if (bits_q && lane < rows) {
+    uint32_t *dst = bits_q + (((size_t)plane * nkt + kt) * (size_t)Lq + row0 + lane) * 2;
+    dst[0] = lo;
+    dst[1] = hi;
+  }
+  const bool any = __ballot((lo | hi) != 0) != 0;
+  if (lane == 0) flags[((size_t)plane * nkt + kt) * nqt + qt] = any ? 1 : 0;
+  if (bits_k) {
+    uint32_t klo = 0u, khi = 0u;  // this lane's key: queries 0..31 and 32..63 of the tile
+    if (any) {
+#pragma unroll
+      for (int k = 0; k < 64; ++k) {
+        const uint64_t b = __ballot(((k < 32 ? lo : hi) >> (k % 32)) & 1u);
+        klo = lane == k ? (uint32_t)b : klo;
+        khi = lane == k ? (uint32_t)(b >> 32) : khi;
+      }
+    }
+    if (exists) {
+      uint32_t *dst = bits_k + (((size_t)plane * nqt + qt) * (size_t)Lk + key) * 2;
+      dst[0] = klo;
+      dst[1] = khi;
+    }
+  }
+}
+
+// The tile lists from the tiles' flags (flags[plane][key tile][query tile]), a wave per list: the nqb lists of a plane's
+// query blocks, then the nkb lists of its key blocks, then one wave that says whether the plane attends to anything.
+__global__ __launch_bounds__(64) void mask_lists_kernel(const uint8_t *flags, int Lq, int Lk, int *tiles_q, int *tiles_k, int *attends) {
+  const int nqt = (Lq + 63) / 64, nkt = (Lk + 63) / 64;
+  const int nqb = (Lq + TILE_BLOCK - 1) / TILE_BLOCK, nkb = (Lk + TILE_BLOCK - 1) / TILE_BLOCK;
+  const int plane = blockIdx.x / (nqb + nkb + 1), what = blockIdx.x % (nqb + nkb + 1), lane = threadIdx.x;
+  const uint8_t *f = flags + (size_t)plane * nkt * nqt;
+  if (what == nqb + nkb) {
+    bool any = false;
+    for (int i = lane; i < nkt * nqt; i += WAVE) any |= f[i] != 0;
+    any = __ballot(any) != 0;
+    if (lane == 0) attends[plane] = any ? 1 : 0;
+    return;
+  }
+  const bool keys = what >= nqb;
+  const int b = keys ? what - nqb : what, nt = keys ? nqt : nkt, owned = keys ? nkt : nqt;
+  int *list = (keys ? tiles_k + ((size_t)plane * nkb + b) * (size_t)(nt + 1) : tiles_q + ((size_t)plane * nqb + b) * (size_t)(nt + 1));
+  const bool two = 2 * b + 1 < owned;
+  int count = 0;
+  for (int t0 = 0; t0 < nt; t0 += WAVE) {
+    const int t = t0 + lane;
+    bool on = false;
+    if (t < nt) {
+      if (keys) on = f[(size_t)(2 * b) * nqt + t] || (two && f[(size_t)(2 * b + 1) * nqt + t]);
+      else on = f[(size_t)t * nqt + 2 * b] || (two && f[(size_t)t * nqt + 2 * b + 1]);
+    }
+    const uint64_t m = __ballot(on);
+    if (on) list[1 + count + __popcll(m & (((uint64_t)1 << lane) - 1))] = t;
+    count += __popcll(m);
+  }
+  if (lane == 0) {
+    if (count == 0) list[1] = 0;  // one (fully masked) tile is visited all the same, see above
+    list[0] = count == 0 ? 1 : count;
+  }
+}
 }  // namespace jvpfa
 
 using namespace jvpfa;
@@ -218,5 +310,33 @@ extern "C" int jvpfa_mask_bits(const jvpfa_problem *p, int32_t Lk, uint32_t *bit
   const int64_t *s = p->mask_stride;
   hipLaunchKernelGGL(mask_bits_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(hip_stream),
                      static_cast<const uint8_t *>(p->mask), s[0], s[1], s[2], s[3], hm, p->L, lk, kchunks, bits);
+  return hipGetLastError() == hipSuccess ? JVPFA_OK : JVPFA_E_LAUNCH;
+}
+
+extern "C" size_t jvpfa_mask_scan_bytes(const jvpfa_problem *p, int32_t Lk) {
+  if (!p || p->Z < 1 || p->H < 1 || p->L < 1 || Lk < 0) return 0;
+  const size_t lk = Lk > 0 ? Lk : p->L;
+  return mask_planes(p) * (((size_t)p->L + 63) / 64) * ((lk + 63) / 64);
+}
+
+extern "C" int jvpfa_mask_scan(const jvpfa_problem *p, int32_t Lk, const jvpfa_mask_scan_out *out, void *hip_stream) {
+  if (!p || !out || !out->scratch || !out->tiles_q || !out->tiles_k || !out->attends) return JVPFA_E_NULL;
+  if (p->Z < 1 || p->H < 1 || p->L < 1 || Lk < 0) return JVPFA_E_SHAPE;
+  if (p->mask_kind != JVPFA_MASK_BOOL) return JVPFA_E_DTYPE;
+  if (!p->mask) return JVPFA_E_NULL;
+  for (int i = 0; i < 4; ++i)
+    if (p->mask_stride[i] < 0) return JVPFA_E_SHAPE;
+  if ((reinterpret_cast<uintptr_t>(out->bits_q) | reinterpret_cast<uintptr_t>(out->bits_k)) & 7u) return JVPFA_E_ALIGN;
+  const int lk = Lk > 0 ? Lk : p->L, hm = p->mask_stride[1] ? p->H : 1;
+  const long long planes = (long long)mask_planes(p);
+  const long long blocks = planes * ((p->L + 63) / 64) * (((lk + 63) / 64 + 3) / 4);
+  const long long lists = planes * ((p->L + TILE_BLOCK - 1) / TILE_BLOCK + (lk + TILE_BLOCK - 1) / TILE_BLOCK + 1);
+  if (blocks > 0x7fffffffLL || lists > 0x7fffffffLL) return JVPFA_E_SHAPE;
+  const int64_t *s = p->mask_stride;
+  hipStream_t stream = static_cast<hipStream_t>(hip_stream);
+  hipLaunchKernelGGL(mask_scan_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, static_cast<const uint8_t *>(p->mask), s[0], s[1],
+                     s[2], s[3], hm, p->L, lk, out->bits_q, out->bits_k, static_cast<uint8_t *>(out->scratch));
+  hipLaunchKernelGGL(mask_lists_kernel, dim3((unsigned)lists), dim3(64), 0, stream, static_cast<const uint8_t *>(out->scratch), p->L, lk,
+                     out->tiles_q, out->tiles_k, out->attends);
   return hipGetLastError() == hipSuccess ? JVPFA_OK : JVPFA_E_LAUNCH;
 }

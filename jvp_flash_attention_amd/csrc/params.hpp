@@ -4,9 +4,9 @@
 
 namespace jvpfa {
 
-// MASK_BITS is a boolean mask read by the dk/dv kernels from its bit-packed transposed copy (Problem::bits_k),
-// MASK_TILE an additive mask whose 64-query x 128-key tiles those kernels stream through LDS like the operand
-// tiles (rows of 16-byte aligned, contiguous keys); both exist as template arguments of those kernels only.
+// MASK_BITS is a boolean mask read from a bit-packed copy (Problem::bits_q by the forward and dq kernels, bits_k by the
+// dk/dv kernels), MASK_TILE an additive mask whose 64-query x 128-key tiles those kernels stream through LDS like the operand
+// tiles (rows of 16-byte aligned, contiguous keys); both exist as template arguments of the 16-bit kernels only.
 enum MaskKind { MASK_NONE = 0, MASK_BOOL = 1, MASK_ADD = 2, MASK_BITS = 3, MASK_TILE = 4 };
 
 struct Problem {
@@ -28,6 +28,10 @@ struct Problem {
   // zero bits.  The dk/dv kernels, whose lanes own a key, read one pair per 64 queries instead of 64 bytes a
   // mask row apart.
   const uint32_t *bits_k;
+  // The same packed along the key axis, or null: per mask plane, tile of 64 keys and query row a pair of words, bit i
+  // of word hf being the entry of (query, key 64 * tile + 32 * hf + i); keys past Lk are zero bits.  For the forward and
+  // dq kernels, whose lanes own a query.
+  const uint32_t *bits_q;
   // Split of the streamed tiles of one block of owned rows over `chunks` workgroups (1 = no split), used when
   // a launch would otherwise leave most compute units idle: workgroup c of a block takes the tiles
   // c * chunk_tiles .. (c + 1) * chunk_tiles - 1 and writes fp32 partial results to `part`, which a merge
@@ -94,7 +98,10 @@ __host__ __device__ inline size_t tile_list_offset_k(const Problem &pr, int z, i
   return (tile_list_plane(pr, z, h) * nblk + block) * (size_t)(nt + 1);
 }
 
-// first word of the plane of (z, h) in the bit-packed mask
+// first word of the plane of (z, h) in either bit-packed mask
+__host__ __device__ inline size_t mask_bits_q_offset(const Problem &pr, int z, int h) {
+  return tile_list_plane(pr, z, h) * (size_t)((pr.Lk + 63) / 64) * (size_t)pr.L * 2;
+}
 __host__ __device__ inline size_t mask_bits_offset(const Problem &pr, int z, int h) {
   return tile_list_plane(pr, z, h) * (size_t)((pr.L + 63) / 64) * (size_t)pr.Lk * 2;
 }

@@ -31,7 +31,7 @@ using torch::autograd::variable_list;
 
 // What a call is besides its tensors; the same in the forward and the backward.
 struct Call {
-  OptTensor mask, key_limit, tiles_q, tiles_k, bits;
+  OptTensor mask, key_limit, tiles_q, tiles_k, bits_k, bits_q;
   int64_t mask_kind = JVPFA_MASK_NONE;
   bool causal = false;
   double scale = 1.0, dropout_p = 0.0;
@@ -106,7 +106,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> forward(const Tensor &q, const Tensor
   a.qt = in(qt), a.kt = in(kt), a.vt = in(vt);
   a.o = out(o), a.ot = out(ot);
   a.M = static_cast<float *>(out(M)), a.mu = static_cast<float *>(out(mu));
-  a.key_limit = in<int32_t>(c.key_limit), a.tiles_q = in<int32_t>(c.tiles_q);
+  a.key_limit = in<int32_t>(c.key_limit), a.tiles_q = in<int32_t>(c.tiles_q), a.mask_bits_q = in<uint32_t>(c.bits_q);
   a.Hk = static_cast<int32_t>(k.size(1)), a.Lk = static_cast<int32_t>(k.size(2));  // may differ from q's
   Tensor workspace;
   if (c.split) {
@@ -147,7 +147,7 @@ std::vector<Tensor> backward(const Tensor &q, const Tensor &k, const Tensor &v, 
   Tensor workspace = at::empty({bytes}, q.options().dtype(at::kByte).requires_grad(false));
   a.workspace = out(workspace);
   a.key_limit = in<int32_t>(c.key_limit), a.tiles_q = in<int32_t>(c.tiles_q), a.tiles_k = in<int32_t>(c.tiles_k);
-  a.mask_bits = in<uint32_t>(c.bits);
+  a.mask_bits = in<uint32_t>(c.bits_k), a.mask_bits_q = in<uint32_t>(c.bits_q);
   a.Hk = static_cast<int32_t>(k.size(1)), a.Lk = static_cast<int32_t>(k.size(2));
   Tensor shares;
   if (c.split && a.Hk < a.p.H) {
@@ -176,7 +176,7 @@ struct Attention : public torch::autograd::Function<Attention> {
     ctx->save_for_backward({q, k, v, qt, kt, vt, o, ot, M, mu});
     // the mask and what was derived from it are kept as they are (no version check: as before, a mask may be refilled)
     auto &d = ctx->saved_data;
-    d["c"] = c10::IValue(std::make_tuple(c.mask, c.key_limit, c.tiles_q, c.tiles_k, c.bits, c.mask_kind, c.causal, c.scale,
+    d["c"] = c10::IValue(std::make_tuple(c.mask, c.key_limit, c.tiles_q, c.tiles_k, c.bits_k, c.bits_q, c.mask_kind, c.causal, c.scale,
                                          c.dropout_p, static_cast<int64_t>(c.seed), c.split));
     if (qt.defined()) return {o, ot};
     return {o};
@@ -187,9 +187,9 @@ struct Attention : public torch::autograd::Function<Attention> {
     Call c;
     const auto e = ctx->saved_data["c"].toTuple()->elements();
     c.mask = e[0].toOptional<Tensor>(), c.key_limit = e[1].toOptional<Tensor>(), c.tiles_q = e[2].toOptional<Tensor>();
-    c.tiles_k = e[3].toOptional<Tensor>(), c.bits = e[4].toOptional<Tensor>();
-    c.mask_kind = e[5].toInt(), c.causal = e[6].toBool(), c.scale = e[7].toDouble(), c.dropout_p = e[8].toDouble();
-    c.seed = static_cast<uint64_t>(e[9].toInt()), c.split = e[10].toBool();
+    c.tiles_k = e[3].toOptional<Tensor>(), c.bits_k = e[4].toOptional<Tensor>(), c.bits_q = e[5].toOptional<Tensor>();
+    c.mask_kind = e[6].toInt(), c.causal = e[7].toBool(), c.scale = e[8].toDouble(), c.dropout_p = e[9].toDouble();
+    c.seed = static_cast<uint64_t>(e[10].toInt()), c.split = e[11].toBool();
     const bool dual = s[3].defined();
     const Tensor go = dense(grads[0]), gt = dual ? dense(grads[1]) : Tensor();
     const bool want_t = dual && (ctx->needs_input_grad(3) || ctx->needs_input_grad(4) || ctx->needs_input_grad(5));
@@ -266,11 +266,12 @@ OptTensor attend(const Tensor &q, const Tensor &k, const Tensor &v, int64_t leve
 }
 
 Call make_call(OptTensor mask, int64_t mask_kind, bool causal, double dropout_p, uint64_t seed, OptTensor key_limit,
-               OptTensor tiles_q, OptTensor tiles_k, OptTensor bits, bool split) {
+               OptTensor tiles_q, OptTensor tiles_k, OptTensor bits_k, OptTensor bits_q, bool split) {
   Call c;
   if (mask_kind != JVPFA_MASK_NONE) c.mask = std::move(mask);
   c.mask_kind = mask_kind, c.causal = causal, c.dropout_p = dropout_p, c.seed = seed;
-  c.key_limit = std::move(key_limit), c.tiles_q = std::move(tiles_q), c.tiles_k = std::move(tiles_k), c.bits = std::move(bits);
+  c.key_limit = std::move(key_limit), c.tiles_q = std::move(tiles_q), c.tiles_k = std::move(tiles_k);
+  c.bits_k = std::move(bits_k), c.bits_q = std::move(bits_q);
   c.split = split;
   return c;
 }
@@ -280,14 +281,14 @@ Call make_call(OptTensor mask, int64_t mask_kind, bool causal, double dropout_p,
 PYBIND11_MODULE(_torch_binding, m) {
   m.def("attend", [](const Tensor &q, const Tensor &k, const Tensor &v, int64_t level, std::optional<double> scale, bool causal,
                      double dropout_p, uint64_t seed, bool split, OptTensor mask, int64_t mask_kind, OptTensor key_limit,
-                     OptTensor tiles_q, OptTensor tiles_k, OptTensor bits) {
+                     OptTensor tiles_q, OptTensor tiles_k, OptTensor bits_k, OptTensor bits_q) {
     const py::gil_scoped_release released;
-    return attend(q, k, v, level, scale, make_call(mask, mask_kind, causal, dropout_p, seed, key_limit, tiles_q, tiles_k, bits, split));
+    return attend(q, k, v, level, scale, make_call(mask, mask_kind, causal, dropout_p, seed, key_limit, tiles_q, tiles_k, bits_k, bits_q, split));
   });
   m.def("fwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &qt, const OptTensor &kt, const OptTensor &vt,
                   double scale, bool causal, double dropout_p, uint64_t seed, bool split, OptTensor mask, int64_t mask_kind,
-                  OptTensor key_limit, OptTensor tiles_q) {
-    Call c = make_call(mask, mask_kind, causal, dropout_p, seed, key_limit, tiles_q, {}, {}, split);
+                  OptTensor key_limit, OptTensor tiles_q, OptTensor bits_q) {
+    Call c = make_call(mask, mask_kind, causal, dropout_p, seed, key_limit, tiles_q, {}, {}, bits_q, split);
     c.scale = scale;
     auto [o, ot, M, mu] = forward(q, k, v, given(qt), given(kt), given(vt), c);
     return std::make_tuple(o, maybe(ot), M, maybe(mu));
@@ -295,8 +296,8 @@ PYBIND11_MODULE(_torch_binding, m) {
   m.def("bwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &qt, const OptTensor &kt, const OptTensor &vt,
                   const Tensor &o, const OptTensor &ot, const Tensor &M, const OptTensor &mu, const OptTensor &go, const OptTensor &gt,
                   double scale, bool causal, bool want_tangent_grads, double dropout_p, uint64_t seed, bool split, OptTensor mask,
-                  int64_t mask_kind, OptTensor key_limit, OptTensor tiles_q, OptTensor tiles_k, OptTensor bits) {
-    Call c = make_call(mask, mask_kind, causal, dropout_p, seed, key_limit, tiles_q, tiles_k, bits, split);
+                  int64_t mask_kind, OptTensor key_limit, OptTensor tiles_q, OptTensor tiles_k, OptTensor bits_k, OptTensor bits_q) {
+    Call c = make_call(mask, mask_kind, causal, dropout_p, seed, key_limit, tiles_q, tiles_k, bits_k, bits_q, split);
     c.scale = scale;
     std::vector<OptTensor> r;
     for (const Tensor &t : backward(q, k, v, given(qt), given(kt), given(vt), o, given(ot), M, given(mu), given(go), given(gt), c, want_tangent_grads))

@@ -135,9 +135,10 @@ def _classify_mask(attn_mask: Tensor | None, q: Tensor, verify_attn_mask: bool):
     if attn_mask.dtype == torch.bool:
         mask_tensor = attn_mask
         if verify_attn_mask and not _already_verified(attn_mask):
-            assert mask_tensor.any(dim=-1).any(dim=-1).all(), (
-                "The attention mask cannot be all False for any head."
-            )
+            # (large masks: from the pass over the mask that its tile lists and packed copies need anyway)
+            scan = _lib.mask_scan(q, mask_tensor, _lib.MASK_BOOL, mask_tensor.shape[3]) if _native() else None
+            attends = mask_tensor.any(dim=-1).any(dim=-1) if scan is None else scan.attends
+            assert attends.all(), "The attention mask cannot be all False for any head."
             _remember_verified(attn_mask)
         return mask_tensor, _lib.MASK_BOOL
     mask_tensor = attn_mask.to(q.dtype)
