@@ -79,9 +79,9 @@ static int bwd_impl(const jvpfa_bwd_args *a, void *workspace, void *hip_stream) 
     }
   }
   const size_t n = stat_floats(a->p.Z, a->p.H, a->p.L);
-  p.d1 = static_cast<float *>(workspace);
-  p.a = p.d1 + n;
-  p.d2 = p.a + n;
+  p.neg_d1 = static_cast<float *>(workspace);
+  p.neg_a = p.neg_d1 + n;
+  p.neg_d2 = p.neg_a + n;
   return kBwd[slot(a->p)](p, a->p.mask_kind, dual, ntg == 3, static_cast<hipStream_t>(hip_stream));
 }
 

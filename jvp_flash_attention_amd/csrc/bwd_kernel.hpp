@@ -1,13 +1,13 @@
 // Backward for  Loss = <gO, O> + <gT, O'>  with P recomputed from the saved log-sum-exp M (and mu for the tangent
 // path): the pre-pass of every backward, and the dq, dk/dv kernels for fp32 at D = 256.
 //
-//   prepass   d1 = rowsum(gO*O), a = rowsum(gT*O), d2 = d1 + rowsum(gT*O') - a*mu
+//   prepass   d1 = rowsum(gO*O), a = rowsum(gT*O), d2 = rowsum(gT*O')
 //   dq        one workgroup per 128 query rows, loop over key tiles
 //   dkdv      one workgroup per 128 key rows, loop over query tiles
 //
 // Replaces the reference's _attn_bwd_preprocess (jvp_attention.py:1384-1411), _attn_bwd_dq
 // (:1567-1707) and _attn_bwd_dkdv (:1415-1563), which handle gO only; the gT terms follow
-//   dS' = P*(A - a),  dS = P*(gO V^T - d1 + B + A*(S' - mu) - a*S' - d2),  P' = P*(S' - mu)
+//   dS' = P*(A - a),  dS = P*(gO V^T + B + (A - a)*(S' - mu) - (d1 + d2)),  P' = P*(S' - mu)
 //   A = gT V^T,  B = gT V'^T
 //   dQ = s(dS K + dS' K'), dK = s(dS^T Q + dS'^T Q'), dV = P^T gO + P'^T gT
 //   dQ' = s dS' K,         dK' = s dS'^T Q,           dV' = P^T gT          (s = sm_scale)
@@ -55,10 +55,10 @@ __global__ __launch_bounds__(256) void bwd_prepass_kernel(const BwdParams p, lon
     s2 += __shfl_xor(s2, w, 64);
   }
   if (row < rows && part == 0) {
-    p.d1[row] = s1;
+    p.neg_d1[row] = -s1;
     if (dual) {
-      p.a[row] = sa;
-      p.d2[row] = s1 + s2 - sa * p.mu[row];  // BWD_DUAL uses d1 + d2 only, kept in one statistic
+      p.neg_a[row] = -sa;
+      p.neg_d2[row] = -(s1 + s2);  // BWD_DUAL uses d1 + d2 only, kept in one statistic
     }
   }
 }
@@ -140,10 +140,10 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(const BwdParams p) {
   const T *gTrow = (DUAL || TAN) ? reinterpret_cast<const T *>(p.gt) + head + (size_t)qld * D : nullptr;
 
   const float Mq = qrow < L ? p.M[srow + qld] : __builtin_inff();
-  const float d1 = (MODE == BWD_PLAIN) ? p.d1[srow + qld] : 0.f;  // BWD_DUAL: d2 already holds d1 + d2
+  const float nd1 = (MODE == BWD_PLAIN) ? p.neg_d1[srow + qld] : 0.f;
   const float mu = (DUAL) ? p.mu[srow + qld] : 0.f;
-  const float av = (DUAL || TAN) ? p.a[srow + qld] : 0.f;
-  const float d2 = (DUAL) ? p.d2[srow + qld] : 0.f;
+  const float na = (DUAL || TAN) ? p.neg_a[srow + qld] : 0.f;
+  const float nd2 = (DUAL) ? p.neg_d2[srow + qld] : 0.f;
 
   f32x16 acc[DB];
 #pragma unroll
@@ -227,13 +227,13 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_kernel(const BwdParams p) {
           if constexpr (DUAL || TAN) At[i] *= ks;
         }
         if constexpr (MODE == BWD_PLAIN) {
-          S[i] = pv * (dP[i] - d1);
+          S[i] = pv * (dP[i] + nd1);
         } else if constexpr (DUAL) {
-          const float sp = Sp[i] * pr.scale;
-          Sp[i] = pv * (At[i] - av);
-          S[i] = pv * (dP[i] - d1 + At[i] * (sp - mu) - av * sp - d2);
+          const float u = fmaf(Sp[i], pr.scale, -mu), am = At[i] + na;
+          Sp[i] = pv * am;
+          S[i] = pv * fmaf(am, u, dP[i] + nd2);
         } else {
-          S[i] = pv * (At[i] - av);
+          S[i] = pv * (At[i] + na);
         }
       }
     }
@@ -327,16 +327,16 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   const T *gOg = (!TAN && has_go) ? reinterpret_cast<const T *>(p.go) + head : nullptr;
   const T *gTg = (DUAL || TAN) ? reinterpret_cast<const T *>(p.gt) + head : nullptr;
   const T *Gg = TAN ? gTg : gOg;  // tensor staged in Gn / GT
-  float rs[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // M, d1, mu, a, d2 of query row i0 + tid
+  float rs[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // M, -d1, mu, -a, -(d1 + d2) of query row i0 + tid
   auto fetch_stats = [&](int i0) {
     if (tid < BWD_T) {
       const bool ok = i0 + tid < L;
       const size_t si = srow + (ok ? i0 + tid : 0);
       rs[0] = ok ? p.M[si] : __builtin_inff();
-      rs[1] = (ok && MODE == BWD_PLAIN) ? p.d1[si] : 0.f;  // BWD_DUAL: d2 already holds d1 + d2
+      rs[1] = (ok && MODE == BWD_PLAIN) ? p.neg_d1[si] : 0.f;
       rs[2] = (ok && DUAL) ? p.mu[si] : 0.f;
-      rs[3] = (ok && (DUAL || TAN)) ? p.a[si] : 0.f;
-      rs[4] = (ok && DUAL) ? p.d2[si] : 0.f;
+      rs[3] = (ok && (DUAL || TAN)) ? p.neg_a[si] : 0.f;
+      rs[4] = (ok && DUAL) ? p.neg_d2[si] : 0.f;
     }
   };
   auto put_stats = [&]() {
@@ -419,16 +419,16 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
       }
       if constexpr (MODE == BWD_PLAIN) {
         S[e] = pv * ks;
-        dP[e] = pv * (dP[e] - sd1[ql]);
+        dP[e] = pv * (dP[e] + sd1[ql]);
       } else if constexpr (DUAL) {
-        const float sp = Sp[e] * pr.scale, m_ = smu[ql], a_ = sa[ql];
+        const float u = fmaf(Sp[e], pr.scale, -smu[ql]), am = At[e] + sa[ql];
         S[e] = pv * ks;
-        Pp[e] = pv * (sp - m_) * ks;
-        Sp[e] = pv * (At[e] - a_);
-        dP[e] = pv * (dP[e] - sd1[ql] + At[e] * (sp - m_) - a_ * sp - sd2[ql]);
+        Pp[e] = pv * u * ks;
+        Sp[e] = pv * am;
+        dP[e] = pv * fmaf(am, u, dP[e] + sd2[ql]);
       } else {
         S[e] = pv * ks;
-        Sp[e] = pv * (At[e] - sa[ql]);
+        Sp[e] = pv * (At[e] + sa[ql]);
       }
     }
 

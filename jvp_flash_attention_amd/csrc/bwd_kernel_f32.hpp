@@ -1,6 +1,6 @@
 // Backward kernels for fp32, D in {32, 64, 128}, on the forward's direct-to-LDS pipeline (fwd_kernel_f32.hpp: row-major tiles
 // of 32 rows, two stages, one barrier per tile, both reads from the one copy, contraction order chosen for them).
-// Mathematics and modes: bwd_kernel.hpp; d2 already contains d1.  What bounds them: the fp32 matrix rate, 8 (dq) and 10
+// Mathematics and modes: bwd_kernel.hpp; statistics arrive negated.  What bounds them: the fp32 matrix rate, 8 (dq) and 10
 // (dk/dv) executed products of which the register-staged kernels these replace reached 60 - 65 %.
 // Measured, B4 H8 L1024 D64 dual with an additive bias per head: dq 325 -> 257 us, dk/dv 432 -> 333 us (87 and 84 % of
 // the rate of a large fp32 matrix product); whole backward B4 H16 L2048 D64 5.56 -> 4.47 ms, D128 17.0 -> 9.4 ms.
@@ -76,10 +76,10 @@ __device__ __forceinline__ void bwd_f32_dq_body(const BwdParams &p) {
   if constexpr (DUAL) load_own_row(Qtf, p.qt, own, g);
   if constexpr (DUAL || TAN) load_own_row(gTf, p.gt, own, g);
   const float Mq = qrow < L ? p.M[srow + qld] : __builtin_inff();
-  const float d1 = MODE == BWD_PLAIN ? p.d1[srow + qld] : 0.f;
+  const float nd1 = MODE == BWD_PLAIN ? p.neg_d1[srow + qld] : 0.f;
   const float mu = DUAL ? p.mu[srow + qld] : 0.f;
-  const float av = (DUAL || TAN) ? p.a[srow + qld] : 0.f;
-  const float d2 = DUAL ? p.d2[srow + qld] : 0.f;
+  const float na = (DUAL || TAN) ? p.neg_a[srow + qld] : 0.f;
+  const float nd2 = DUAL ? p.neg_d2[srow + qld] : 0.f;
   f32x16 acc[DB];
   zero_accs(acc);
 
@@ -209,13 +209,13 @@ __device__ __forceinline__ void bwd_f32_dq_body(const BwdParams &p) {
         if constexpr (DUAL || TAN) At[e] *= ks;
       }
       if constexpr (MODE == BWD_PLAIN) {
-        S[e] = pv[e] * (dP[e] - d1);
+        S[e] = pv[e] * (dP[e] + nd1);
       } else if constexpr (DUAL) {
-        const float sp = Sp[e] * pr.scale;
-        Sp[e] = pv[e] * (At[e] - av);
-        S[e] = pv[e] * (dP[e] + At[e] * (sp - mu) - av * sp - d2);
+        const float u = __builtin_fmaf(Sp[e], pr.scale, -mu), am = At[e] + na;
+        Sp[e] = pv[e] * am;
+        S[e] = pv[e] * __builtin_fmaf(am, u, dP[e] + nd2);
       } else {
-        S[e] = pv[e] * (At[e] - av);
+        S[e] = pv[e] * (At[e] + na);
       }
     }
     if constexpr (DUAL) asm volatile("s_nop 1" : "+v"(S), "+v"(Sp));
@@ -297,7 +297,7 @@ __device__ __forceinline__ void bwd_f32_dkdv_body(const BwdParams &p) {
     const float *Qtg = DUAL ? reinterpret_cast<const float *>(p.qt) + head : nullptr;
     const float *gTg = (DUAL || TAN) ? reinterpret_cast<const float *>(p.gt) + head : nullptr;
     const float *Gg = TAN ? gTg : (GO ? reinterpret_cast<const float *>(p.go) + head : Qg);
-    const float *st_p[4] = {p.M + srow, (MODE == BWD_PLAIN ? p.d1 : DUAL ? p.mu : p.a) + srow, DUAL ? p.a + srow : nullptr, DUAL ? p.d2 + srow : nullptr};
+    const float *st_p[4] = {p.M + srow, (MODE == BWD_PLAIN ? p.neg_d1 : DUAL ? p.mu : p.neg_a) + srow, DUAL ? p.neg_a + srow : nullptr, DUAL ? p.neg_d2 + srow : nullptr};
     TileWalk<BT> walk;  // query tiles visited: all from istart on, or those of the caller's list
     {
       const int *tl = nullptr;
@@ -456,14 +456,14 @@ __device__ __forceinline__ void bwd_f32_dkdv_body(const BwdParams &p) {
           }
           S[e] = DROP ? pv[i] * ks : pv[i];
           if constexpr (MODE == BWD_PLAIN) {
-            dP[e] = pv[i] * (dP[e] - s_[1][i]);
+            dP[e] = pv[i] * (dP[e] + s_[1][i]);
           } else if constexpr (DUAL) {
-            const float sp = Sp[e] * pr.scale, m_ = s_[1][i], a_ = s_[2][i];
-            Pp[e] = DROP ? pv[i] * (sp - m_) * ks : pv[i] * (sp - m_);
-            Sp[e] = pv[i] * (At[e] - a_);
-            dP[e] = pv[i] * (dP[e] + At[e] * (sp - m_) - a_ * sp - s_[3][i]);
+            const float u = __builtin_fmaf(Sp[e], pr.scale, -s_[1][i]), am = At[e] + s_[2][i];
+            Pp[e] = DROP ? pv[i] * u * ks : pv[i] * u;
+            Sp[e] = pv[i] * am;
+            dP[e] = pv[i] * __builtin_fmaf(am, u, dP[e] + s_[3][i]);
           } else {
-            Sp[e] = pv[i] * (At[e] - s_[1][i]);
+            Sp[e] = pv[i] * (At[e] + s_[1][i]);
           }
         }
       });

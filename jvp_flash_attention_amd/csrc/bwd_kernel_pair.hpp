@@ -170,8 +170,8 @@ __global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {
 
   const float Mq = qrow < L ? p.M[srow + qld] : __builtin_inff();
   const float mu = p.mu[srow + qld];
-  const float av = p.a[srow + qld];
-  const float dsum = p.d2[srow + qld];
+  const float na = p.neg_a[srow + qld];
+  const float nd2 = p.neg_d2[srow + qld];
   const uint32_t drop_row = DROP ? drop_row_word(pr, zh, qld) : 0u;  // dropout: this lane's query row, see params.hpp
 
   f32x16 acc[DB], accT[SIX ? DB : 1];
@@ -298,9 +298,9 @@ __global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {
           dpv *= ks;
           atv *= ks;
         }
-        const float sp = Sp[i] * pr.scale, am = atv - av;
+        const float u = fmaf(Sp[i], pr.scale, -mu), am = atv + na;
         Sp[i] = pv * am;
-        S[i] = pv * (dpv + am * sp - atv * mu - dsum);
+        S[i] = pv * fmaf(am, u, dpv + nd2);
       }
     }
     Frag<T> dsf[2], dspf[2];
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {
 }
 
 // dk, dv of the dual mode: workgroup = 64 keys of a key/value head (two pairs), loop over 32-query tiles.
-// Tile slots of a stage: 0 Q, 1 gT, 2 Q', 3 gO; statistics slots M, mu, a, d2 (= d1 + d2).
+// Tile slots of a stage: 0 Q, 1 gT, 2 Q', 3 gO; statistics slots M, mu, -a, -(d1 + d2).
 template <typename T, int D, int MASK, bool GO, bool DROP = false>
 __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
   using Cfg = BwdPairCfg<T, D>;
@@ -526,8 +526,8 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
     Qtb = reinterpret_cast<const char *>(p.qt) + qhead;
     st_p[0] = p.M + srow;
     st_p[1] = p.mu + srow;
-    st_p[2] = p.a + srow;
-    st_p[3] = p.d2 + srow;
+    st_p[2] = p.neg_a + srow;
+    st_p[3] = p.neg_d2 + srow;
   };
 
   const int istart = pr.causal ? (k0 / BT) * BT : 0;
@@ -683,7 +683,7 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
         constexpr int younger = (c4 + 1 < 4) ? 4 : 0;
         lds_wait4<younger>(stq[sl][0], stq[sl][1], stq[sl][2], stq[sl][3]);
         auto stat = [&](int s_, int e) { return __uint_as_float(stq[sl][s_][e % 4]); };
-        float pv4[4], sp4[4], ks4[4];
+        float pv4[4], u4[4], ks4[4];  // u = S' - mu
 #pragma unroll
         for (int e = 4 * c4; e < 4 * c4 + 4; ++e) {
           const int qi = ih + 16 * (e / 8) + 8 * g + (e % 8);
@@ -695,22 +695,22 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
           if constexpr (MASK == MASK_BOOL) pv = keep ? pv : 0.f;
           if constexpr (EDGE) pv = (qi >= qmin && qi < L) ? pv : 0.f;
           pv4[e % 4] = pv;
-          sp4[e % 4] = Sp[e] * pr.scale;
+          u4[e % 4] = fmaf(Sp[e], pr.scale, -stat(1, e));
           ks4[e % 4] = DROP ? drop_scale_of(pr, drop_tile + (uint32_t)(16 * (e / 8) + (e % 8)) * DROP_C_ROW) : 1.f;
         }
         if (role) {  // X = A, Y = dP
 #pragma unroll
           for (int e = 4 * c4; e < 4 * c4 + 4; ++e) {
             const float at = DROP ? X[e] * ks4[e % 4] : X[e], dp = DROP ? Y[e] * ks4[e % 4] : Y[e];
-            const float pv = pv4[e % 4], m_ = stat(1, e), am = at - stat(2, e);
-            Fa[e - 8 * c] = pv * (dp + am * sp4[e % 4] - at * m_ - stat(3, e));
+            const float pv = pv4[e % 4], am = at + stat(2, e);
+            Fa[e - 8 * c] = pv * fmaf(am, u4[e % 4], dp + stat(3, e));
             Fb[e - 8 * c] = pv * am;
           }
         } else {
 #pragma unroll
           for (int e = 4 * c4; e < 4 * c4 + 4; ++e) {
             const float pw = DROP ? pv4[e % 4] * ks4[e % 4] : pv4[e % 4];
-            Fa[e - 8 * c] = pw * (sp4[e % 4] - stat(1, e));
+            Fa[e - 8 * c] = pw * u4[e % 4];
             Fb[e - 8 * c] = pw;
           }
         }

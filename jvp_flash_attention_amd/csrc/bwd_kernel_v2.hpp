@@ -6,8 +6,7 @@
 // ds_read_b64_tr_b16 gives the operand of the gradient accumulations (contraction over the
 // streamed index).  LDS reads are issued one step ahead of their matrix products.
 //
-// Mathematics, modes and the reference lines it replaces: see bwd_kernel.hpp.  In BWD_DUAL the
-// pre-pass statistic d2 already contains d1 (d2 := d1 + rowsum(gT*O') - a*mu).
+// Mathematics, modes and the reference lines it replaces: see bwd_kernel.hpp.
 #pragma once
 #include "common.hpp"
 #include "mask.hpp"
@@ -56,6 +55,14 @@ template <int N> __device__ __forceinline__ void lds_wait(FragT &a, FragT &b, Fr
   asm volatile("s_waitcnt lgkmcnt(%8)"
                : "+v"(a.lo), "+v"(a.hi), "+v"(b.lo), "+v"(b.hi), "+v"(c.lo), "+v"(c.hi), "+v"(d.lo), "+v"(d.hi)
                : "n"(N));
+}
+// A score-sized tile from four quads that a wait already passed covers: tied behind it, register e = quad e / 4, entry e % 4.
+__device__ __forceinline__ f32x16 tile_of(u32x4 (&q)[4]) {
+  asm volatile("" : "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3]));
+  f32x16 t;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) t[e] = __uint_as_float(q[e / 4][e % 4]);
+  return t;
 }
 template <int N> __device__ __forceinline__ void lds_wait4(u32x4 &a, u32x4 &b, u32x4 &c, u32x4 &d) {
   asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) : "n"(N));
@@ -143,6 +150,15 @@ __device__ __forceinline__ void zero_acc(f32x16 &x) {
 // SIX (dual mode only): dq' = scale dS' K as well, from the K fragments and the dS' tiles that dq already has.
 // DROP: dropout (see bwd_kernel.hpp): gO V^T, gT V^T and gT V'^T reach the logits through the kept, rescaled
 // entries only.
+// Where the dq kernels keep the tiles of constants that A and dP start from (16 registers each): at D = 128 with the dual
+// mode's one wave per SIMD, and without tangents or masks, where they fit the 256 registers of two; at D = 64 in the one
+// dual variant that still fits 256 with them.  The other variants would spill (9 - 75 registers) or lose a workgroup of
+// the two or three that share a compute unit; with dropout the products are scaled before anything is added.
+constexpr bool dq_init(int d, int mode, int mask, bool go, bool six, bool drop) {
+  if (six || drop) return false;
+  if (d == 128) return mode == BWD_DUAL || (mode == BWD_PLAIN && mask == MASK_NONE);
+  return d == 64 && mode == BWD_DUAL && mask == MASK_NONE && go;
+}
 // LEAN: one tile loop (every tile takes the limit tests) instead of an interior loop and an edge loop: less for
 // the compiler to keep in registers, for the variant that must stay within 256 of them.
 template <typename T, int D, int MODE, int MASK, bool GO, bool SIX, bool DROP = false, bool LEAN = false>
@@ -177,10 +193,24 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
 
   const float Mq = qrow < L ? p.M[srow + qld] : __builtin_inff();
   const uint32_t drop_row = DROP ? drop_row_word(pr, zh, qld) : 0u;  // dropout: this lane's query row
-  const float d1 = (MODE == BWD_PLAIN) ? p.d1[srow + qld] : 0.f;
+  const float nd1 = (MODE == BWD_PLAIN) ? p.neg_d1[srow + qld] : 0.f;
   const float mu = DUAL ? p.mu[srow + qld] : 0.f;
-  const float av = (DUAL || TAN) ? p.a[srow + qld] : 0.f;
-  const float dsum = DUAL ? p.d2[srow + qld] : 0.f;
+  const float na = (DUAL || TAN) ? p.neg_a[srow + qld] : 0.f;
+  const float nd2 = DUAL ? p.neg_d2[srow + qld] : 0.f;
+
+  // INIT: A and dP start from -a and -(d1 + d2) (PLAIN -d1, TANGENT -a), which saves an addition per entry each.  A lane
+  // owns one query, so a tile of either holds one number; the two tiles stay resident.
+  constexpr bool INIT = dq_init(D, MODE, MASK, GO, SIX, DROP);
+  f32x16 from_a, from_d;
+  if constexpr (INIT) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      if constexpr (DUAL || TAN) from_a[e] = na;
+      if constexpr (DUAL || MODE == BWD_PLAIN) from_d[e] = DUAL ? nd2 : nd1;
+    }
+    if constexpr (DUAL || TAN) asm volatile("" : "+v"(from_a));
+    if constexpr (DUAL || MODE == BWD_PLAIN) asm volatile("" : "+v"(from_d));
+  }
 
   f32x16 acc[DB], accT[SIX ? DB : 1];
 #pragma unroll
@@ -281,16 +311,21 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
       else lds_wait<(kk + 1 < KK) ? NRN : 0>(fk[sl], fv[sl]);
       load_step(std::integral_constant<int, HB * KK + kk>{});
       const Frag<T> k_ = as_frag<T>(fk[sl]), v_ = as_frag<T>(fv[sl]);
+      auto score = [&](f32x16 &tile, const Frag<T> &a, const Frag<T> &b, const f32x16 &from) {
+        if constexpr (F && INIT) mma_vra_from(tile, a, b, from);
+        else mma_vra<F>(tile, a, b);
+      };
       mma_vra<F>(S, k_, Qf[kk]);
-      if constexpr (MODE == BWD_PLAIN) mma_vra<F>(dP, v_, gOf[kk]);
-      if constexpr (TAN) mma_vra<F>(At, v_, gTf[kk]);
+      if constexpr (MODE == BWD_PLAIN) score(dP, v_, gOf[kk], from_d);
+      if constexpr (TAN) score(At, v_, gTf[kk], from_a);
       if constexpr (DUAL) {
         if constexpr (has_go && GO_V) mma_vrv<F>(dP, v_, gOf[kk]);
-        else if constexpr (has_go) mma_vra<F>(dP, v_, gOf[kk]);
+        else if constexpr (has_go) score(dP, v_, gOf[kk], from_d);
         mma_vra<F>(Sp, k_, Qtf[kk]);
-        mma_vra<F>(At, v_, gTf[kk]);
+        score(At, v_, gTf[kk], from_a);
         mma_vra<false>(Sp, as_frag<T>(fkt[sl]), Qf[kk]);
-        mma_vra<F && !has_go>(dP, as_frag<T>(fvt[sl]), gTf[kk]);
+        if constexpr (has_go) mma_vra<false>(dP, as_frag<T>(fvt[sl]), gTf[kk]);
+        else score(dP, as_frag<T>(fvt[sl]), gTf[kk], from_d);
       }
     });
     if constexpr (DUAL) tiles_ready(S, dP, Sp, At);
@@ -298,7 +333,10 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
     else tiles_ready(S, dP);
 
     // ---- P and the score gradients -------------------------------------------------------------
-    const int klim = min(pr.causal ? qrow : 0x7fffffff, Lk - 1);  // keys above this index are masked
+    // keys above this index are masked; counted from the lane's first key of the half tile it is compared with constants
+    // (not with dropout or an additive mask, where variants would take a register or two too many for their workgroups)
+    constexpr bool FAR = DROP || MASK == MASK_ADD;
+    const int klim = min(pr.causal ? qrow : 0x7fffffff, Lk - 1) - (FAR ? 0 : jh + 8 * g);
     float spread[MASK == MASK_BITS ? 16 : 1];  // MASK_BITS: all ones for an attended entry, all zeros for a masked one
     if constexpr (MASK == MASK_BITS) {
       const uint32_t w = mah[0].w >> (8 * g);
@@ -329,20 +367,20 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
         else pv = fast_exp2(S[i] * sl2 - Mq);
         if constexpr (MASK == MASK_BOOL) pv = keep[e] ? pv : 0.f;
         if constexpr (MASK == MASK_BITS) pv = __uint_as_float(__float_as_uint(pv) & __float_as_uint(spread[i]));
-        if constexpr (EDGE) pv = (key0 + e <= klim) ? pv : 0.f;
+        if constexpr (EDGE) pv = ((FAR ? key0 : 16 * hf) + e <= klim) ? pv : 0.f;
         if constexpr (DROP) {
           const float ks = drop_scale_of(pr, xb + (uint32_t)e * DROP_C_KEY);
           if constexpr (!TAN) dP[i] *= ks;
           if constexpr (DUAL || TAN) At[i] *= ks;
         }
         if constexpr (MODE == BWD_PLAIN) {
-          S[i] = pv * (dP[i] - d1);
+          S[i] = pv * (INIT ? dP[i] : dP[i] + nd1);
         } else if constexpr (DUAL) {
-          const float sp = Sp[i] * pr.scale, am = At[i] - av;
+          const float u = fmaf(Sp[i], pr.scale, -mu), am = INIT ? At[i] : At[i] + na;
           Sp[i] = pv * am;
-          S[i] = pv * (dP[i] + am * sp - At[i] * mu - dsum);
+          S[i] = pv * fmaf(am, u, INIT ? dP[i] : dP[i] + nd2);
         } else {
-          S[i] = pv * (At[i] - av);
+          S[i] = pv * (INIT ? At[i] : At[i] + na);
         }
       }
     }
@@ -616,7 +654,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   // The query heads that read this key/value head are visited one after another (one, h itself, for
   // the shapes the reference admits); hq is the current one, and what depends on it is set per head:
   // tile slots 0 Q, 1 G (gO; gT in TANGENT; gT again in DUAL without gO), 2 Q', 3 gT, and the
-  // statistics slots PLAIN M, d1 | DUAL M, mu, a, d2 (= d1 + d2) | TANGENT M, a
+  // statistics slots PLAIN M, -d1 | DUAL M, mu, -a, -(d1 + d2) | TANGENT M, -a
   const int group = GROUPED ? pr.H / pr.Hk / pr.chunks : 1;  // ... of this workgroup's share
   const int hq0 = GROUPED ? h * (pr.H / pr.Hk) + chunk * group : h;
   int hq = hq0;
@@ -631,9 +669,9 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
     Gb = TAN ? gTb : (has_go ? reinterpret_cast<const char *>(p.go) + qhead : gTb);
     Qtb = DUAL ? reinterpret_cast<const char *>(p.qt) + qhead : nullptr;
     st_p[0] = p.M + qrow0;
-    st_p[1] = MODE == BWD_PLAIN ? p.d1 + qrow0 : (DUAL ? p.mu + qrow0 : p.a + qrow0);
-    st_p[2] = DUAL ? p.a + qrow0 : nullptr;
-    st_p[3] = DUAL ? p.d2 + qrow0 : nullptr;
+    st_p[1] = MODE == BWD_PLAIN ? p.neg_d1 + qrow0 : (DUAL ? p.mu + qrow0 : p.neg_a + qrow0);
+    st_p[2] = DUAL ? p.neg_a + qrow0 : nullptr;
+    st_p[3] = DUAL ? p.neg_d2 + qrow0 : nullptr;
     if constexpr (MASK == MASK_BITS) bits_head = pr.bits_k + mask_bits_offset(pr, z, hq);
     if constexpr (MASK == MASK_TILE)
       mt_head = reinterpret_cast<const char *>(pr.mask) + (z * pr.ms[0] + hq * pr.ms[1] + (int64_t)k0) * (int64_t)sizeof(T);
@@ -809,6 +847,25 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
     }
     // tiles in ordinary vector registers; in DUAL, dP also collects gT V'^T (the B term)
     f32x16 S, dP, Sp, At;
+    // INIT: -a and -(d1 + d2) (PLAIN -d1, TANGENT -a) are what A and dP start from, read from LDS straight into the tiles'
+    // registers, instead of two additions per entry behind the products (not with dropout, which scales the products
+    // first; at D = 64 without gO two variants would need 258 and 260 registers and lose their second workgroup).  A lone
+    // wave per SIMD pays four cycles for every vector instruction, and with S' - mu shared by dS and P' a tile of the dual
+    // kernel at D = 128 has 306 of them where it had 434 (dq 240 for 336).  dk/dv and dq, bf16: B4 H16 L2048 D64 335 -> 321
+    // and 250 -> 242 us, packed documents B2 H16 L2077 D128 151 -> 143 us, both in one launch at B1 H16 L1024 D128, causal,
+    // gradients of O' alone, 68.1 -> 65.6 us.
+    constexpr bool INIT = !DROP && !(D == 64 && DUAL && !has_go && (GROUPED || MASK == MASK_TILE));
+    u32x4 ia[4], idp[4];
+    if constexpr (INIT) {
+      const uint32_t sad = sstat + (HB * 32 + 8 * g) * 4;
+      static_for<4>([&](auto cc) {
+        constexpr int c4 = decltype(cc)::value, O = (c4 / 2) * 64 + (c4 % 2) * 16;
+        if constexpr (DUAL) ia[c4] = lds_b128<2 * BT * 4 + O>(sad);
+        if constexpr (TAN) ia[c4] = lds_b128<BT * 4 + O>(sad);
+        if constexpr (DUAL) idp[c4] = lds_b128<3 * BT * 4 + O>(sad);
+        if constexpr (MODE == BWD_PLAIN) idp[c4] = lds_b128<BT * 4 + O>(sad);
+      });
+    }
     if constexpr (SAHEAD) issue_n(std::integral_constant<int, 0>{});
     static_for<KK>([&](auto kkc) {
       constexpr int kk = decltype(kkc)::value, sl = SAHEAD ? kk % 2 : 0;
@@ -818,18 +875,23 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
       constexpr int younger_n = (SAHEAD && kk + 1 < KK) ? NRN : 0;
       if constexpr (DUAL) lds_wait<younger_n>(fq[sl], fg[sl], fqt[sl], fgt[sl]);
       else lds_wait<younger_n>(fq[sl], fg[sl]);
+      if constexpr (INIT && F) {  // (older than the fragments just waited for)
+        if constexpr (DUAL || TAN) At = tile_of(ia);
+        if constexpr (DUAL || MODE == BWD_PLAIN) dP = tile_of(idp);
+      }
       load_step(std::integral_constant<int, HB * KK + kk>{});
       const Frag<T> q_ = as_frag<T>(fq[sl]), g_ = as_frag<T>(fg[sl]);
       mma_vra<F>(S, q_, Kf[kk]);
-      if constexpr (MODE == BWD_PLAIN) mma_vra<F>(dP, g_, Vf[kk]);
-      if constexpr (TAN) mma_vra<F>(At, g_, Vf[kk]);
+      constexpr bool FI = F && !INIT;
+      if constexpr (MODE == BWD_PLAIN) mma_vra<FI>(dP, g_, Vf[kk]);
+      if constexpr (TAN) mma_vra<FI>(At, g_, Vf[kk]);
       if constexpr (DUAL) {
         const Frag<T> gt_ = as_frag<T>(fgt[sl]);
-        if constexpr (has_go) mma_vra<F>(dP, g_, Vf[kk]);
+        if constexpr (has_go) mma_vra<FI>(dP, g_, Vf[kk]);
         mma_vra<F>(Sp, as_frag<T>(fqt[sl]), Kf[kk]);
-        mma_vra<F>(At, gt_, Vf[kk]);
+        mma_vra<FI>(At, gt_, Vf[kk]);
         mma_vra<false>(Sp, q_, Ktf[kk]);
-        mma_vrv<F && !has_go>(dP, gt_, Vtf[kk]);
+        mma_vrv<FI && !has_go>(dP, gt_, Vtf[kk]);
       }
     });
     if constexpr (DUAL) tiles_ready(S, dP, Sp, At);
@@ -838,19 +900,35 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
 
     // ---- row statistics of the 32 queries: register e belongs to query 16(e/8) + 8g + e%8 ------
     // read one quad of registers at a time (quad c4 = registers 4*c4 .. 4*c4+3), one quad ahead
-    u32x4 stq[2][Cfg::NSTAT];
     const uint32_t sad = sstat + (HB * 32 + 8 * g) * 4;
+    constexpr int NSTAT_Q = INIT ? (DUAL ? 2 : 1) : Cfg::NSTAT;  // statistics still to be read: M, mu first
+    u32x4 stq[2][NSTAT_Q];
     auto issue_s = [&](auto c4c) {
       constexpr int c4 = decltype(c4c)::value;
-      static_for<Cfg::NSTAT>([&](auto sc) {
+      static_for<NSTAT_Q>([&](auto sc) {
         constexpr int s_ = decltype(sc)::value;
         stq[c4 % 2][s_] = lds_b128<s_ * BT * 4 + (c4 / 2) * 64 + (c4 % 2) * 16>(sad);
       });
     };
     const int qmin = pr.causal ? krow : 0;  // queries below this index do not see this key
+    // EDGE: bit i = query ih + 8g + i exists and, in causal calls, sees this key (two instructions per entry, where
+    // comparing an index with both limits takes five; with dropout and mask tiles those stay: there the word's register is
+    // one too many)
+    constexpr bool SEEN = EDGE && !DROP && MASK != MASK_TILE;
+    uint32_t seen = ~0u;
+    if constexpr (SEEN) {
+      const int lo = qmin - (ih + 8 * g), n = L - (ih + 8 * g);
+      seen = lo >= 32 ? 0u : ~0u << max(lo, 0);
+      seen &= n >= 32 ? ~0u : n <= 0 ? 0u : ~(~0u << n);
+    }
     // The 32 queries are handled as two chunks of 16 (registers 8c .. 8c+7): score gradients of a
     // chunk, then its share of dK^T += Q^T dS (+ Q'^T dS'), dV^T += G^T P (+ gT^T P'), one step per
     // d-block; the transposed fragments of a step are read one step ahead.
+    auto spread = [](uint32_t w, int e) {  // the bit of register e over a word (from the builtin: a test, a compare and a select)
+      uint32_t t;
+      asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(t) : "v"(w), "n"(mask_bit_of(e)));
+      return t;
+    };
     FragT tq[2], tg[2], tqt[2], tgt[2];
     auto issue_t = [&](auto ic) {
       constexpr int i = decltype(ic)::value, c = i / DB, db = i % DB, sl = (D > 64) ? i % 2 : 0;
@@ -874,7 +952,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
       mfr[0] = as_frag<T>(FragT{mt_all[HB][0][0], mt_all[HB][0][1]});
       mfr[1] = as_frag<T>(FragT{mt_all[HB][1][0], mt_all[HB][1][1]});
     } else if constexpr (MASK == MASK_TILE) {
-      lds_wait<SAHEAD ? Cfg::NSTAT : 0>(mtv[0][0], mtv[0][1], mtv[1][0], mtv[1][1]);  // long since there
+      lds_wait<SAHEAD ? NSTAT_Q : 0>(mtv[0][0], mtv[0][1], mtv[1][0], mtv[1][1]);  // long since there
       mfr[0] = as_frag<T>(FragT{mtv[0][0], mtv[0][1]});
       mfr[1] = as_frag<T>(FragT{mtv[1][0], mtv[1][1]});
     }
@@ -886,14 +964,14 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
         if constexpr (!SAHEAD) issue_s(std::integral_constant<int, c4>{});
         else if constexpr (c4 + 1 < 4) issue_s(std::integral_constant<int, c4 + 1>{});
         // waits also cover the transposed fragments issued before (LDS reads complete in order)
-        constexpr int younger = (SAHEAD && c4 + 1 < 4) ? Cfg::NSTAT : 0;
-        if constexpr (Cfg::NSTAT == 4) lds_wait4<younger>(stq[sl][0], stq[sl][1], stq[sl][2], stq[sl][3]);
-        else lds_wait<younger>(stq[sl][0], stq[sl][1]);
+        constexpr int younger = (SAHEAD && c4 + 1 < 4) ? NSTAT_Q : 0;
+        if constexpr (NSTAT_Q == 4) lds_wait4<younger>(stq[sl][0], stq[sl][1], stq[sl][2], stq[sl][3]);
+        else if constexpr (NSTAT_Q == 2) lds_wait<younger>(stq[sl][0], stq[sl][1]);
+        else lds_wait<younger>(stq[sl][0]);
         auto stat = [&](int s_, int e) { return __uint_as_float(stq[sl][s_][e % 4]); };
 #pragma unroll
         for (int e = 4 * c4; e < 4 * c4 + 4; ++e) {
           const int qi = ih + 16 * (e / 8) + 8 * g + (e % 8);
-          float s = S[e] * sl2;
           bool keep = true;
           if constexpr (MBYTES && !MAHEAD) {
             if constexpr (!EDGE) {  // uniform row pointer + 32-bit lane offset, as above
@@ -911,15 +989,13 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
           float pv;
           if constexpr (MASK == MASK_ADD) pv = fast_exp2(fmaf(S[e], sl2, fmaf((float)mraw_a[MAHEAD ? e : 0], LOG2E, -stat(0, e))));
           else if constexpr (MASK == MASK_TILE) pv = fast_exp2(fmaf(S[e], sl2, fmaf((float)mfr[e / 8][e % 8], LOG2E, -stat(0, e))));
-          else pv = fast_exp2(s - stat(0, e));
+          else pv = fast_exp2(S[e] * sl2 - stat(0, e));
           if constexpr (MASK == MASK_BOOL) pv = keep ? pv : 0.f;
           if constexpr (MASK == MASK_BITS) {
-            // (written as asm: from the builtin the compiler makes a bit test, a compare and a select)
-            uint32_t spread;
-            asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(spread) : "v"(mraw_w), "n"(mask_bit_of(e)));
-            pv = __uint_as_float(__float_as_uint(pv) & spread);
+            pv = __uint_as_float(__float_as_uint(pv) & spread(SEEN ? mraw_w & seen : mraw_w, e));
           }
-          if constexpr (EDGE) pv = (qi >= qmin && qi < L) ? pv : 0.f;
+          if constexpr (EDGE && !SEEN) pv = (qi >= qmin && qi < L) ? pv : 0.f;
+          if constexpr (SEEN && MASK != MASK_BITS) pv = __uint_as_float(__float_as_uint(pv) & spread(seen, e));
           float ks = 1.f;  // dropout: 1 / (1 - p) for a kept entry, 0 for a dropped one
           if constexpr (DROP) {
             ks = drop_scale_of(pr, drop_half + (uint32_t)(16 * (e / 8) + (e % 8)) * DROP_C_ROW);
@@ -928,14 +1004,14 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
           }
           S[e] = pv * ks;
           if constexpr (MODE == BWD_PLAIN) {
-            dP[e] = pv * (dP[e] - stat(1, e));
+            dP[e] = pv * (INIT ? dP[e] : dP[e] + stat(1, e));
           } else if constexpr (DUAL) {
-            const float sp = Sp[e] * pr.scale, m_ = stat(1, e), am = At[e] - stat(2, e);
-            Pp[e - 8 * c] = pv * (sp - m_) * ks;
+            const float u = fmaf(Sp[e], pr.scale, -stat(1, e)), am = INIT ? At[e] : At[e] + stat(2, e);
+            Pp[e - 8 * c] = pv * u * ks;
             Sp[e] = pv * am;
-            dP[e] = pv * (dP[e] + am * sp - At[e] * m_ - stat(3, e));
+            dP[e] = pv * fmaf(am, u, INIT ? dP[e] : dP[e] + stat(3, e));
           } else {
-            Sp[e] = pv * (At[e] - stat(1, e));
+            Sp[e] = pv * (INIT ? At[e] : At[e] + stat(1, e));
           }
         }
       });

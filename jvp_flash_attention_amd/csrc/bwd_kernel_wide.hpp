@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256, 1) void bwdw_dq_kernel(const BwdParams p) {
   }
 
   const float Mq = qrow < L ? p.M[srow + qld] : __builtin_inff();
-  const float sub = TAN ? p.a[srow + qld] : p.d1[srow + qld];  // what the row takes off dP (PLAIN) or A (TANGENT)
+  const float shift = TAN ? p.neg_a[srow + qld] : p.neg_d1[srow + qld];  // what the row adds to dP (PLAIN) or A (TANGENT)
   const uint32_t drop_row = DROP ? drop_row_word(pr, zh, qld) : 0u;  // dropout: this lane's query row, see params.hpp
 
   f32x16 acc[DB];
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256, 1) void bwdw_dq_kernel(const BwdParams p) {
         if constexpr (EDGE) pv = (key0 + e <= klim) ? pv : 0.f;
         float gv = G[i];
         if constexpr (DROP) gv *= drop_scale_of(pr, drop_row + (uint32_t)(key0 + e) * DROP_C_KEY);
-        S[i] = pv * (gv - sub);
+        S[i] = pv * (gv + shift);
       }
     }
     Frag<T> dsf[2];
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
     Qb = reinterpret_cast<const char *>(p.q) + qhead;
     Gb = reinterpret_cast<const char *>(TAN ? p.gt : p.go) + qhead;
     st_p[0] = p.M + srow;
-    st_p[1] = (TAN ? p.a : p.d1) + srow;
+    st_p[1] = (TAN ? p.neg_a : p.neg_d1) + srow;
   };
 
   const int istart = pr.causal ? (k0 / BT) * BT : 0;
@@ -604,10 +604,10 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
           if constexpr (DROP) {
             const float ks = drop_scale_of(pr, drop_tile + (uint32_t)(16 * (e / 8) + (e % 8)) * DROP_C_ROW);
             S[e] = pv * ks;
-            G[e] = pv * (G[e] * ks - stat(1, e));
+            G[e] = pv * (G[e] * ks + stat(1, e));
           } else {
             S[e] = pv;
-            G[e] = pv * (G[e] - stat(1, e));
+            G[e] = pv * (G[e] + stat(1, e));
           }
         }
       });

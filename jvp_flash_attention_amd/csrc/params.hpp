@@ -119,7 +119,9 @@ struct BwdParams {
   const float *M, *mu;
   const void *go, *gt;
   void *dq, *dk, *dv, *dqt, *dkt, *dvt;
-  float *d1, *a, *d2;  // row statistics produced by the pre-pass, each (Z, H, L)
+  // Row statistics produced by the pre-pass, each (Z, H, L), with the sign with which the kernels add them (the 16-bit
+  // dk/dv kernels start their score-sized accumulators at them): -d1, -a and, dual mode only, -(d1 + d2).
+  float *neg_d1, *neg_a, *neg_d2;
 };
 
 // Share `chunk` of gradient t out of nt in the backward's partial results, or null where nothing is split.

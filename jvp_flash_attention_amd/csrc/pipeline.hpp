@@ -108,6 +108,13 @@ template <bool FIRST, bool GUARD = false> __device__ __forceinline__ void mma_vr
     else asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(b));
   }
 }
+// The first product of a tile that starts from `init` instead of zero (a tile of constants that stays resident).
+__device__ __forceinline__ void mma_vra_from(f32x16 &c, const bf16x8 &a, const bf16x8 &b, const f32x16 &init) {
+  asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(c) : "v"(a), "a"(b), "v"(init));
+}
+__device__ __forceinline__ void mma_vra_from(f32x16 &c, const f16x8 &a, const f16x8 &b, const f32x16 &init) {
+  asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(c) : "v"(a), "a"(b), "v"(init));
+}
 // The same with the B operand in ordinary vector registers.  Under register pressure the compiler may
 // park such a long-lived operand in the accumulation file and copy it back just before its use; a
 // matrix instruction must not read a register within two issue slots of a vector-ALU write to it, and
