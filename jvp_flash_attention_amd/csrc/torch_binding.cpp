@@ -165,8 +165,6 @@ std::vector<Tensor> backward(const Tensor &q, const Tensor &k, const Tensor &v, 
 // (q, k, v[, q', k', v']) -> (O[, O']), differentiable in every tensor input.  A gradient that does not arrive stays
 // absent: without one for O' the first-order backward runs (the tangent inputs then have zero gradients).
 struct Attention : public torch::autograd::Function<Attention> {
-  static constexpr bool is_traceable = true;
-
   // (the tangents as optionals: the node takes no undefined tensors)
   static variable_list forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &qt_,
                                const OptTensor &kt_, const OptTensor &vt_, const Call &c) {

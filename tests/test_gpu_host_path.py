@@ -53,3 +53,16 @@ def test_arguments_are_refused_with_the_reason():
         attention(*(x[..., :48] for x in (q, k, v)))
     with pytest.raises(AssertionError, match="dropout_p"):
         attention(q, k, v, dropout_p=1.5)
+
+
+def test_the_backward_under_compiled_autograd():
+    """The node's backward reads device pointers: compiled autograd has to call it as it is, not to trace it."""
+    from torch._dynamo import compiled_autograd
+
+    q, k, v = (x.cuda().requires_grad_() for x in _inputs(64, torch.bfloat16)[:3])
+    go = torch.ones_like(q)
+    want = torch.autograd.grad(attention(q, k, v, causal=True), (q, k, v), go)
+    o = attention(q, k, v, causal=True)
+    with compiled_autograd._enable(torch.compile(backend="eager")):
+        o.backward(go)
+    assert all(torch.equal(t.grad, w) for t, w in zip((q, k, v), want))
