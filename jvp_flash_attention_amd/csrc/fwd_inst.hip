@@ -112,7 +112,7 @@ static int launch_fwd_wide_one(const FwdParams &p, hipStream_t stream) {
 template <typename T, int D, int BN, bool DUAL>
 static int launch_fwd_mask(const FwdParams &p, int mask, hipStream_t stream) {
   if (p.pr.drop_thr != 0) {
-    // dropout: the direct-to-LDS kernels carry it for the 16-bit types, the register-staged one for fp32
+    // dropout: the direct-to-LDS kernels carry it, the register-staged one for fp32 at D = 256
     if constexpr (sizeof(T) == 2 && D == 256) {
       switch (mask) {
         case MASK_NONE: return launch_fwd_wide_one<T, D, DUAL, MASK_NONE, true>(p, stream);
