@@ -161,6 +161,13 @@ std::vector<Tensor> backward(const Tensor &q, const Tensor &k, const Tensor &v, 
   return g;
 }
 
+bool any_requires_grad(std::initializer_list<const Tensor *> tensors) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor *t : tensors)
+    if (t->defined() && t->requires_grad()) return true;
+  return false;
+}
+
 // ---- autograd ------------------------------------------------------------------------------------
 // (q, k, v[, q', k', v']) -> (O[, O']), differentiable in every tensor input.  A gradient that does not arrive stays
 // absent: without one for O' the first-order backward runs (the tangent inputs then have zero gradients).
@@ -202,7 +209,9 @@ struct Attention : public torch::autograd::Function<Attention> {
         if (want_t) g[3] = at::zeros_like(s[0]), g[4] = at::zeros_like(s[1]), g[5] = at::zeros_like(s[2]);
       }
     }
-    if (at::GradMode::is_enabled()) {  // create_graph: the gradients carry a node that says what is missing
+    // create_graph, and an arriving gradient that depends on something: the gradients carry a node that says what is
+    // missing (as behind torch's once_differentiable; gradients of constants are constants)
+    if (any_requires_grad({&go, &gt})) {
       for (Tensor &t : g) {
         if (!t.defined()) continue;
         auto error = std::make_shared<torch::autograd::DelayedError>(
@@ -214,13 +223,6 @@ struct Attention : public torch::autograd::Function<Attention> {
     return g;
   }
 };
-
-bool any_requires_grad(std::initializer_list<const Tensor *> tensors) {
-  if (!at::GradMode::is_enabled()) return false;
-  for (const Tensor *t : tensors)
-    if (t->defined() && t->requires_grad()) return true;
-  return false;
-}
 
 // The argument checks of a call without a mask, as one yes or no; the caller words the error.
 bool acceptable(const Tensor &q, const Tensor &k, const Tensor &v, double dropout_p) {

@@ -40,9 +40,30 @@ def test_gradients_of_either_output_or_both(D, dtype, of, six):
 
 def test_a_second_derivative_is_refused():
     q, k, v = (x.cuda().requires_grad_() for x in _inputs(64, torch.bfloat16)[:3])
-    (dq,) = torch.autograd.grad(attention(q, k, v).float().sum(), q, create_graph=True)
+    o = attention(q, k, v)
+    go = torch.ones_like(o, requires_grad=True)
+    (dq,) = torch.autograd.grad(o, q, go, create_graph=True)
     with pytest.raises(RuntimeError, match="once_differentiable"):
         dq.float().sum().backward()
+
+
+@pytest.mark.parametrize("dual", [False, True])
+def test_gradients_of_constants_are_constants_under_create_graph(dual):
+    """Where no arriving gradient requires grad, create_graph gives plain tensors that go on being used."""
+    q, k, v, *t = (x.cuda() for x in _inputs(64, torch.bfloat16)[:6])
+    q.requires_grad_()
+    w = torch.randn_like(q).requires_grad_()
+    with fwAD.dual_level():
+        if dual:
+            out = JVPAttn.fwd_dual(*(fwAD.make_dual(a, b) for a, b in zip((q, k, v), t)))
+            o, ot = fwAD.unpack_dual(out)
+            loss = o.float().sum() + ot.float().sum()
+        else:
+            loss = attention(q, k, v).float().sum()
+        (dq,) = torch.autograd.grad(loss, q, create_graph=True)
+    assert not dq.requires_grad
+    (dq * w).sum().backward()
+    assert torch.equal(w.grad, dq)
 
 
 def test_arguments_are_refused_with_the_reason():
