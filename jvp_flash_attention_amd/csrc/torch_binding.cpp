@@ -168,6 +168,15 @@ bool any_requires_grad(std::initializer_list<const Tensor *> tensors) {
   return false;
 }
 
+// What the kernels of a backward may use about the mask as it now is: one Python call, which finds what the
+// forward derived unless the mask has changed since.
+void look_up_hints(Call &c, const Tensor &q, int64_t Lk) {
+  if (c.mask_kind == JVPFA_MASK_NONE) return;
+  const py::gil_scoped_acquire gil;
+  const py::object hints = py::module_::import("jvp_flash_attention_amd._lib").attr("mask_hints")(q, *c.mask, c.mask_kind, Lk, true);
+  std::tie(c.key_limit, c.tiles_q, c.tiles_k, c.bits_k, c.bits_q) = hints.cast<std::tuple<OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>>();
+}
+
 // ---- autograd ------------------------------------------------------------------------------------
 // (q, k, v[, q', k', v']) -> (O[, O']), differentiable in every tensor input.  A gradient that does not arrive stays
 // absent: without one for O' the first-order backward runs (the tangent inputs then have zero gradients).
@@ -179,10 +188,8 @@ struct Attention : public torch::autograd::Function<Attention> {
     auto [o, ot, M, mu] = ::forward(q, k, v, qt, kt, vt, c);
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({q, k, v, qt, kt, vt, o, ot, M, mu});
-    // the mask and what was derived from it are kept as they are (no version check: as before, a mask may be refilled)
-    auto &d = ctx->saved_data;
-    d["c"] = c10::IValue(std::make_tuple(c.mask, c.key_limit, c.tiles_q, c.tiles_k, c.bits_k, c.bits_q, c.mask_kind, c.causal, c.scale,
-                                         c.dropout_p, static_cast<int64_t>(c.seed), c.split));
+    // the mask as it is: it may be refilled, and what was derived from it is looked up again by the backward
+    ctx->saved_data["c"] = c10::IValue(std::make_tuple(c.mask, c.mask_kind, c.causal, c.scale, c.dropout_p, static_cast<int64_t>(c.seed), c.split));
     if (qt.defined()) return {o, ot};
     return {o};
   }
@@ -191,16 +198,15 @@ struct Attention : public torch::autograd::Function<Attention> {
     const auto s = ctx->get_saved_variables();
     Call c;
     const auto e = ctx->saved_data["c"].toTuple()->elements();
-    c.mask = e[0].toOptional<Tensor>(), c.key_limit = e[1].toOptional<Tensor>(), c.tiles_q = e[2].toOptional<Tensor>();
-    c.tiles_k = e[3].toOptional<Tensor>(), c.bits_k = e[4].toOptional<Tensor>(), c.bits_q = e[5].toOptional<Tensor>();
-    c.mask_kind = e[6].toInt(), c.causal = e[7].toBool(), c.scale = e[8].toDouble(), c.dropout_p = e[9].toDouble();
-    c.seed = static_cast<uint64_t>(e[10].toInt()), c.split = e[11].toBool();
+    c.mask = e[0].toOptional<Tensor>(), c.mask_kind = e[1].toInt(), c.causal = e[2].toBool(), c.scale = e[3].toDouble();
+    c.dropout_p = e[4].toDouble(), c.seed = static_cast<uint64_t>(e[5].toInt()), c.split = e[6].toBool();
     const bool dual = s[3].defined();
     const Tensor go = dense(grads[0]), gt = dual ? dense(grads[1]) : Tensor();
     const bool want_t = dual && (ctx->needs_input_grad(3) || ctx->needs_input_grad(4) || ctx->needs_input_grad(5));
     variable_list g;
     {
       const at::AutoGradMode off(false);
+      if (go.defined() || gt.defined()) look_up_hints(c, s[0], s[1].size(2));
       if (gt.defined()) {
         g = ::backward(s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8], s[9], go, gt, c, want_t);
       } else {

@@ -1,10 +1,10 @@
-"""The native path of eager calls (``csrc/torch_binding.cpp``): which gradients arrive, and what it refuses."""
+"""The native path of eager calls (``csrc/torch_binding.cpp``): which gradients arrive, what it refuses, and masks that change."""
 import numpy as np
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
 
-from jvp_flash_attention_amd import JVPAttn, attention
+from jvp_flash_attention_amd import JVPAttn, _lib, attention
 from oracle import dense
 
 pytestmark = pytest.mark.gpu
@@ -87,3 +87,37 @@ def test_the_backward_under_compiled_autograd():
     with compiled_autograd._enable(torch.compile(backend="eager")):
         o.backward(go)
     assert all(torch.equal(t.grad, w) for t, w in zip((q, k, v), want))
+
+
+@pytest.mark.parametrize("dtype,D,H,L", [(torch.bfloat16, 64, 2, 520), (torch.bfloat16, 64, 32, 577), (torch.bfloat16, 256, 2, 520),
+                                         (torch.float32, 64, 2, 520)])
+@pytest.mark.parametrize("kind", ["rows", "keys"])
+@pytest.mark.parametrize("dropout", [0.0, 0.25])
+def test_a_backward_reads_the_mask_as_it_then_is(dtype, D, H, L, kind, dropout):
+    """A mask refilled between forward and backward: every kernel of the backward sees the new one, as one backward() of the
+    backend with that mask does.  (The new mask attends to no tile that the old one attends to, and to the keys past the old
+    one's last.)"""
+    print("case", dtype, D, H, L, kind, dropout, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(L)
+    Z = 4
+    q, k, v, go = (torch.randn(Z, H, L, D, generator=g, device="cuda").to(dtype) for _ in range(4))
+    q, k, v = (x.requires_grad_() for x in (q, k, v))
+    shape = (Z, 1, L if kind == "rows" else 1, L)
+    first = (torch.arange(L, device="cuda") < 200).expand(shape).contiguous()
+    second = ~first
+    be, scale = _lib.backend(), D**-0.5
+    mask = first.clone()
+    torch.manual_seed(3)
+    o = attention(q, k, v, attn_mask=mask, dropout_p=dropout)
+    mask.copy_(second)
+    got = torch.autograd.grad(o, (q, k, v), go)
+    torch.manual_seed(3)
+    drop = dict(dropout_p=dropout, dropout_seed=int(torch.randint(0, 2**62, (1,)).item()) if dropout else 0)
+    plain = [x.detach() for x in (q, k, v)]
+    none = (None,) * 3
+    o2, _, M, _ = be.fwd(*plain, *none, first, _lib.MASK_BOOL, False, scale, *drop.values())
+    assert torch.equal(o2, o)
+    want = be.bwd(*plain, *none, o2, None, M, None, go, None, second, _lib.MASK_BOOL, False, scale, **drop)
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        assert torch.equal(a, b), name
+    assert torch.count_nonzero(got[1][:, :, :192]) == 0 and torch.count_nonzero(got[1][:, :, 256:]) > 0
