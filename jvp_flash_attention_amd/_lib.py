@@ -195,7 +195,47 @@ def forget_mask(mask) -> None:
             pass
 
 
+# What is derived from a mask is kept on the mask tensor together with where it was made.  Kernels of another stream wait for
+# the event.  What a graph capture made exists only once the graph has run, and again after every replay, so it is used
+# within that capture alone; and a capture uses nothing made outside of it, so that every replay looks at the mask afresh.
+class Origin(NamedTuple):
+    stream: int
+    capture: int  # id of the capture under way on the stream, 0 for none
+    event: torch.cuda.Event | None
+
+
+def _here(t) -> Tuple[int, int]:
+    """The current stream of a tensor's device and the id of the capture under way on it (0, 0 on the CPU)."""
+    return binding().stream_state(t.device.index) if t.is_cuda else (0, 0)
+
+
+def _origin(t) -> Origin:
+    """The origin of what has just been launched on the current stream of a tensor's device."""
+    event = None
+    if t.is_cuda:
+        event = torch.cuda.Event()
+        event.record(torch.cuda.current_stream(t.device))
+    return Origin(*_here(t), event)
+
+
+def _usable(origin: Origin, mask, *tensors) -> bool:
+    """Whether work on the current stream may use these tensors made at ``origin``; it then comes after their making."""
+    stream, capture = _here(mask)
+    if capture != origin.capture:
+        return False
+    if stream != origin.stream:
+        current = torch.cuda.current_stream(mask.device)
+        current.wait_event(origin.event)
+        for t in tensors:
+            if t is not None:
+                t.record_stream(current)
+    return True
+
+
 KEY_LIMIT_MIN_L = 512  # below this the two small reductions cost more than the skipped tiles save
+# Longer rows are reduced in pieces: torch splits one long reduction over workgroups, with a memset of their counters in
+# front, and memset nodes of a captured graph have given wrong results on replays after the first.
+KEY_LIMIT_PIECE = 8192
 
 
 def key_limit_hint(mask, mask_kind, Z, L):
@@ -209,15 +249,18 @@ def key_limit_hint(mask, mask_kind, Z, L):
         return None
     version = mask_version(mask)
     cached = getattr(mask, "_jvpfa_key_limit", None)
-    if cached is not None and version is not None and cached[0] == version:
+    if cached is not None and version is not None and cached[0] == version and _usable(cached[2], mask, cached[1]):
         lim = cached[1]
     else:
         alive = mask if mask.dtype == torch.bool else mask > float("-inf")
         idx = torch.arange(1, L + 1, device=mask.device, dtype=torch.int32)
-        lim = (alive.view(mask.shape[0], L) * idx).amax(dim=1).to(torch.int32)  # one value per row of the mask
+        marks = alive.view(mask.shape[0], L) * idx
+        while marks.shape[1] > KEY_LIMIT_PIECE:
+            marks = torch.nn.functional.pad(marks, (0, -marks.shape[1] % KEY_LIMIT_PIECE)).view(mask.shape[0], -1, KEY_LIMIT_PIECE).amax(dim=2)
+        lim = marks.amax(dim=1).to(torch.int32)  # one value per row of the mask
         if version is not None:
             try:
-                mask._jvpfa_key_limit = (version, lim)
+                mask._jvpfa_key_limit = (version, lim, _origin(mask))
             except (AttributeError, RuntimeError):
                 pass
     # the kernels index the limits by batch entry: a mask shared by the batch ([1,1,1,L]) is spread over Z
@@ -268,9 +311,9 @@ def tile_lists(q, mask, mask_kind, want_k, Lk=None):
         return None, None
     version = mask_version(mask)
     cached = getattr(mask, "_jvpfa_tiles", None)
-    if cached is None or version is None or cached[0] != version:
-        cached = [version, None, None]
-    tq, tk = cached[1], cached[2]
+    tq = tk = None
+    if cached is not None and version is not None and cached[0] == version and _usable(cached[3], mask, cached[1], cached[2]):
+        tq, tk = cached[1], cached[2]
     if tq is None or (want_k and tk is None):
         lib = load()
         prob = make_problem(q, mask, mask_kind, False, 1.0)
@@ -282,10 +325,9 @@ def tile_lists(q, mask, mask_kind, want_k, Lk=None):
         check(lib.jvpfa_mask_tiles(C.byref(prob), Lk, _ptr(new_q), _ptr(new_k), _stream(q)))
         tq = new_q if tq is None else tq
         tk = new_k if new_k is not None else tk
-        cached[1], cached[2] = tq, tk
         if version is not None:
             try:
-                mask._jvpfa_tiles = cached
+                mask._jvpfa_tiles = (version, tq, tk, _origin(mask))
             except (AttributeError, RuntimeError):
                 pass
     return tq, (tk if want_k else None)
@@ -314,7 +356,7 @@ def mask_bits(q, mask, mask_kind, Lk=None):
         return None
     version = mask_version(mask)
     cached = getattr(mask, "_jvpfa_bits", None)
-    if cached is not None and version is not None and cached[0] == version:
+    if cached is not None and version is not None and cached[0] == version and _usable(cached[2], mask, cached[1]):
         return cached[1]
     lib = load()
     prob = make_problem(q, mask, mask_kind, False, 1.0)
@@ -322,7 +364,7 @@ def mask_bits(q, mask, mask_kind, Lk=None):
     check(lib.jvpfa_mask_bits(C.byref(prob), Lk, _ptr(bits), _stream(q)))
     if version is not None:
         try:
-            mask._jvpfa_bits = (version, bits)
+            mask._jvpfa_bits = (version, bits, _origin(mask))
         except (AttributeError, RuntimeError):
             pass
     return bits
@@ -360,6 +402,7 @@ class MaskScan(NamedTuple):
     bits_q: torch.Tensor | None
     bits_k: torch.Tensor | None
     attends: torch.Tensor  # per mask plane: 1 where it attends to anything
+    origin: Origin | None = None
 
 
 def mask_scan(q, mask, mask_kind, Lk):
@@ -375,7 +418,8 @@ def mask_scan(q, mask, mask_kind, Lk):
     version = mask_version(mask)
     cached = getattr(mask, "_jvpfa_scan", None)
     if cached is not None and version is not None and cached.version == version and (cached.bits_q is not None or not packed):
-        return cached
+        if _usable(cached.origin, mask, *cached[1:6]):
+            return cached
     lib = load()
     prob = make_problem(q, mask, mask_kind, False, 1.0)
     planes = (Z if prob.mask_stride[0] else 1) * (H if prob.mask_stride[1] else 1)
@@ -391,11 +435,12 @@ def mask_scan(q, mask, mask_kind, Lk):
     with torch.cuda.device(mask.device):
         check(lib.jvpfa_mask_scan(C.byref(prob), Lk, C.byref(out), _stream(mask)))
     if version is not None:
+        scan = scan._replace(origin=_origin(mask))
         try:
             mask._jvpfa_scan = scan
-            mask._jvpfa_tiles = [version, scan.tiles_q, scan.tiles_k]
+            mask._jvpfa_tiles = (version, scan.tiles_q, scan.tiles_k, scan.origin)
             if packed:
-                mask._jvpfa_bits = (version, scan.bits_k)
+                mask._jvpfa_bits = (version, scan.bits_k, scan.origin)
         except (AttributeError, RuntimeError):
             pass
     return scan

@@ -9,6 +9,7 @@
 #include <ATen/ATen.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPException.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
@@ -282,6 +283,15 @@ Call make_call(OptTensor mask, int64_t mask_kind, bool causal, double dropout_p,
   return c;
 }
 
+// The current stream of a device, and the id of the graph capture under way on it (0: none).
+std::pair<uintptr_t, uint64_t> stream_state(int64_t device) {
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (stream) C10_HIP_CHECK(hipStreamGetCaptureInfo(stream, &status, &id));  // (the default stream cannot be captured)
+  return {reinterpret_cast<uintptr_t>(stream), status == hipStreamCaptureStatusActive ? id : 0};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_torch_binding, m) {
@@ -291,6 +301,7 @@ PYBIND11_MODULE(_torch_binding, m) {
     const py::gil_scoped_release released;
     return attend(q, k, v, level, scale, make_call(mask, mask_kind, causal, dropout_p, seed, key_limit, tiles_q, tiles_k, bits_k, bits_q, split));
   });
+  m.def("stream_state", &stream_state);
   m.def("fwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &qt, const OptTensor &kt, const OptTensor &vt,
                   double scale, bool causal, double dropout_p, uint64_t seed, bool split, OptTensor mask, int64_t mask_kind,
                   OptTensor key_limit, OptTensor tiles_q, OptTensor bits_q) {

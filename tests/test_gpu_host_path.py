@@ -121,3 +121,59 @@ def test_a_backward_reads_the_mask_as_it_then_is(dtype, D, H, L, kind, dropout):
     for name, a, b in zip(("dq", "dk", "dv"), got, want):
         assert torch.equal(a, b), name
     assert torch.count_nonzero(got[1][:, :, :192]) == 0 and torch.count_nonzero(got[1][:, :, 256:]) > 0
+
+
+@pytest.mark.parametrize("dtype,D,Lq,Lk,kind", [(torch.bfloat16, 64, 577, 577, "rows"), (torch.float16, 128, 600, 520, "rows"),
+                                                (torch.float32, 32, 520, 520, "rows"), (torch.bfloat16, 256, 520, 520, "rows"),
+                                                (torch.bfloat16, 64, 70, 1000, "keys"), (torch.bfloat16, 128, 65, 17000, "keys")])
+def test_a_graph_replays_with_refilled_masks(dtype, D, Lq, Lk, kind):
+    """A captured forward and backward looks at the mask on every replay, whatever eager calls on the same mask leave behind
+    in between."""
+    print("case", dtype, D, Lq, Lk, kind, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(D + Lk)
+    rand = lambda n: torch.randn(2, 2, n, D, generator=g, device="cuda").to(dtype)  # noqa: E731
+    q, k, v, qt, kt, vt, go, gt = rand(Lq), rand(Lk), rand(Lk), rand(Lq), rand(Lk), rand(Lk), rand(Lq), rand(Lq)
+    leaves = [x.requires_grad_() for x in (q, k, v)]
+
+    def fresh():
+        if kind == "keys":
+            return torch.arange(Lk, device="cuda") < torch.randint(1, Lk + 1, (2, 1, 1, 1), generator=g, device="cuda")
+        m = torch.rand(2, 1, Lq, Lk, generator=g, device="cuda") < 0.5
+        cut = int(torch.randint(1, Lk, (1,), generator=g, device="cuda"))
+        m[0, :, : Lq // 2, cut:] = False  # tiles come and go
+        m[1, :, Lq // 2:, :cut] = False
+        return m
+
+    mask = fresh()
+
+    def step():
+        with fwAD.dual_level():
+            out = JVPAttn.fwd_dual(*(fwAD.make_dual(a, b) for a, b in zip(leaves, (qt, kt, vt))), attn_mask=mask)
+            o, ot = fwAD.unpack_dual(out)
+            return [o.detach(), ot.detach(), *torch.autograd.grad((o, ot), leaves, (go, gt))]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for rep in range(4):
+        if rep:
+            mask.copy_(fresh())
+        if rep % 2:  # an eager call first, which leaves its own lists and copies behind, and memory that is used again
+            want = step()
+            junk = [torch.full((1 << 16,), -1, dtype=torch.int32, device="cuda") for _ in range(8)]
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [x.clone() for x in captured]
+        if not rep % 2:
+            want = step()
+            junk = None
+        torch.cuda.synchronize()
+        for i, (a, b) in enumerate(zip(got, want)):
+            assert torch.equal(a, b), (rep, i)
+    del junk

@@ -377,3 +377,37 @@ def test_validation_report_figures_from_synthetic_rows(tmp_path):
             head = f.read(8)
         assert head == b"\x89PNG\r\n\x1a\n"
     assert validate.plot_report(rows[:3], "float32", str(tmp_path), masks=False)[0].endswith("float32_jvp_attention_perf.png")
+
+
+def test_what_is_kept_on_a_mask_is_not_shared_with_a_graph_capture(monkeypatch):
+    """Contents made during a capture exist after a replay only, and a graph must look at the mask on every replay: a capture
+    uses what it made itself, eager calls what eager calls made."""
+    L = _lib.KEY_LIMIT_MIN_L
+    mask = torch.ones(2, 1, 1, L, dtype=torch.bool)
+    at = [(5, 0)]  # stream, capture
+    monkeypatch.setattr(_lib, "_here", lambda t: at[0])
+
+    def limit(place):
+        at[0] = place
+        return _lib.key_limit_hint(mask, _lib.MASK_BOOL, 2, L)
+
+    eager = limit((5, 0))
+    assert limit((5, 0)) is eager
+    first = limit((5, 71))
+    assert first is not eager and limit((5, 71)) is first
+    second = limit((5, 72))
+    assert second is not first
+    after = limit((5, 0))
+    assert after is not second and limit((5, 0)) is after
+    mask[1, ..., 9:] = False
+    assert limit((5, 0)).tolist() == [L, 9]
+
+
+def test_key_limit_of_rows_reduced_in_pieces(monkeypatch):
+    monkeypatch.setattr(_lib, "KEY_LIMIT_PIECE", 16)
+    g = torch.Generator().manual_seed(0)
+    for L in (512, 513, 4111):
+        mask = torch.rand(3, 1, 1, L, generator=g) < 3 / L
+        mask[1] = False
+        want = [max([0, *(i + 1 for i in range(L) if row[i])]) for row in mask.view(3, L).tolist()]
+        assert _lib.key_limit_hint(mask, _lib.MASK_BOOL, 3, L).tolist() == want
