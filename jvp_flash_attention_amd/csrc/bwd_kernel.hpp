@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zhk = id / nkb / pr.chunks, chunk = id / nkb % pr.chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nkb;  // causal: the first key blocks have the longest query loops
-  const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = pr.H / pr.Hk / pr.chunks;
+  const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = group_share(pr, chunk + 1) - group_share(pr, chunk);
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
   const int r = lane % 32, g = lane / 32, pr32 = perm32(r);
 
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_kernel(const BwdParams p) {
   const float sl2 = pr.scale * LOG2E;
   const int istart = pr.causal ? (k0 / BWD_T) * BWD_T : 0;
   for (int gi = 0; gi < group; ++gi) {
-  const int h = (hk * pr.chunks + chunk) * group + gi;  // query head
+  const int h = hk * (pr.H / pr.Hk) + group_share(pr, chunk) + gi;  // query head
   const size_t head = ((size_t)z * pr.H + h) * L * D;
   const size_t srow = ((size_t)z * pr.H + h) * L;
   const T *Qg = reinterpret_cast<const T *>(p.q) + head;

@@ -264,7 +264,7 @@ __device__ __forceinline__ void bwd_f32_dkdv_body(const BwdParams &p) {
   const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zhk = id / nkb / pr.chunks, chunk = id / nkb % pr.chunks;
   const int kb = id % nkb;  // causal: the first key blocks have the longest query loops
-  const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = pr.H / pr.Hk / pr.chunks;
+  const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = group_share(pr, chunk + 1) - group_share(pr, chunk);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int r = lane % 32, g = lane / 32;
@@ -291,7 +291,7 @@ __device__ __forceinline__ void bwd_f32_dkdv_body(const BwdParams &p) {
   constexpr int NLOAD = C::IPW * NTILE;
 
   for (int gi = 0; gi < group; ++gi) {
-    const int h = (hk * pr.chunks + chunk) * group + gi;  // query head
+    const int h = hk * (pr.H / pr.Hk) + group_share(pr, chunk) + gi;  // query head
     const size_t head = ((size_t)z * pr.H + h) * L * D, srow = ((size_t)z * pr.H + h) * L;
     const float *Qg = reinterpret_cast<const float *>(p.q) + head;
     const float *Qtg = DUAL ? reinterpret_cast<const float *>(p.qt) + head : nullptr;

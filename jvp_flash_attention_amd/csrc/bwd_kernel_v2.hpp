@@ -655,8 +655,8 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   // the shapes the reference admits); hq is the current one, and what depends on it is set per head:
   // tile slots 0 Q, 1 G (gO; gT in TANGENT; gT again in DUAL without gO), 2 Q', 3 gT, and the
   // statistics slots PLAIN M, -d1 | DUAL M, mu, -a, -(d1 + d2) | TANGENT M, -a
-  const int group = GROUPED ? pr.H / pr.Hk / pr.chunks : 1;  // ... of this workgroup's share
-  const int hq0 = GROUPED ? h * (pr.H / pr.Hk) + chunk * group : h;
+  const int group = GROUPED ? group_share(pr, chunk + 1) - group_share(pr, chunk) : 1;  // ... of this workgroup's share
+  const int hq0 = GROUPED ? h * (pr.H / pr.Hk) + group_share(pr, chunk) : h;
   int hq = hq0;
   const char *Qb = nullptr, *gTb = nullptr, *Gb = nullptr, *Qtb = nullptr;
   const float *st_p[4] = {nullptr, nullptr, nullptr, nullptr};

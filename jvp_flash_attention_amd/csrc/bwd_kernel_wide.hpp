@@ -340,8 +340,8 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zh = id / nblk / pr.chunks, chunk = id / nblk % pr.chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nblk;  // causal: the first key blocks have the longest query loops
-  const int z = zh / pr.Hk, hk = zh % pr.Hk, group = pr.H / pr.Hk / pr.chunks;
-  const int h0 = (hk * pr.chunks + chunk) * group;
+  const int z = zh / pr.Hk, hk = zh % pr.Hk, group = group_share(pr, chunk + 1) - group_share(pr, chunk);
+  const int h0 = hk * (pr.H / pr.Hk) + group_share(pr, chunk);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int r = lane % 32, g = lane / 32, pr32 = perm32(r);

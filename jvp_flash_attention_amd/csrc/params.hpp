@@ -124,6 +124,8 @@ struct BwdParams {
   float *neg_d1, *neg_a, *neg_d2;
 };
 
+// The query heads of a key/value head's group that come before share `chunk` (0 .. pr.chunks).
+__host__ __device__ inline int group_share(const Problem &pr, int chunk) { return chunk * (pr.H / pr.Hk) / pr.chunks; }
 // Share `chunk` of gradient t out of nt in the backward's partial results, or null where nothing is split.
 __host__ __device__ inline float *kv_part(const Problem &pr, int D, int nt, int t, int chunk) {
   return pr.chunks > 1 ? pr.part + ((size_t)chunk * nt + t) * ((size_t)pr.Z * pr.Hk * pr.Lk * D) : nullptr;

@@ -10,6 +10,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "common.hpp"
@@ -70,18 +71,36 @@ template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk) {
 
 // Backward with grouped heads.  A dk/dv workgroup owns 128 keys of a key/value head and works through the query heads
 // of its group one after another: 4 key/value heads for 16 query heads make a quarter of the workgroups, each four
-// times as long.  Where they would leave the GPU idle, the group's query heads are dealt to `chunks` workgroups that
-// leave fp32 shares of dk, dv (and dk', dv'), which bwd_kv_merge_kernel adds up.  The line: enough workgroups for
-// two rounds on every compute unit (D <= 64: up to three share one, so four per unit).  bf16 B4 H16 over 4 key/value
-// heads, L1500 D64, causal, dropout: 192 workgroups 229 us -> 768 workgroups 95 us + merge 9 us.  Beyond the
-// line the shares (16 bytes per chunk and element, written and read) cost more than the idle tail.
+// times as long.  Where that leaves compute units idle, the group's query heads are dealt to `chunks` workgroups that
+// leave fp32 shares of dk, dv (and dk', dv'), which bwd_kv_merge_kernel adds up (group_share: they may differ by a head).
+// The number is the one with the least time by this account, in passes of one workgroup over one query head:
+//   * a compute unit gets ceil(workgroups / units) of them, and waits for 5 % of one; causal, whose work falls from block to
+//     block and is dealt longest first, half the work and a quarter of the longest share, but no less than that share;
+//   * at 16 bits and D <= 64, where two or three workgroups share a unit, one alone runs at 0.6 of their joint rate (causal:
+//     half of the longest share);
+//   * a share costs about 4 tiles of 64 queries (its first loads, and 16 bytes per element written and read; in fp32, where
+//     the products take 16 times as long, a sixteenth of that).
+// At most 10 workgroups per unit, so that the shares take no more than 10 * units * 128 * D * 8 bytes (twice that with tangent
+// gradients), whatever the group.  Measured, forward + backward, bf16, one share -> this rule (in brackets: with as many
+// shares as the group has heads): B4 H16 over 4, L1500 D64, causal, dropout 363 -> 184 us; B8 H71 over 1, L2048 D64 5.51 ->
+// 2.78 ms (2.79, and 595 MB of shares); B2 H28 over 4, D128, L4096 1.98 -> one share (2.02), L4800 3.57 -> 2.92, causal L4096
+// 3.48 -> 2.64; fp16 B4 H16 over 8, L1024 D256 0.35 -> one share (0.40); fp32 B2 H16 over 4, L2048 D64 2.17 -> 1.15.
 template <typename P> inline int bwd_kv_chunks(const P &p, int Lk, int Hk) {
-  const int group = p.H / Hk;
+  const int group = p.H / Hk, cus = device_cus();
   const long long blocks = (long long)((Lk + 127) / 128) * p.Z * Hk;
-  const long long want = (long long)device_cus() * (p.dtype != 2 && p.D <= 64 ? 4 : 2);
-  for (int c = 1; c < group; ++c)
-    if (group % c == 0 && blocks * c >= want) return c;
-  return blocks < want ? group : 1;
+  if (cus <= 0 || group == 1) return 1;
+  const bool shared = p.dtype != 2 && p.D <= 64;
+  const double share_cost = (p.dtype == 2 ? 0.25 : 4.0) / ((p.L + 63) / 64);
+  int best = 1;
+  double least = 0.0;
+  for (int c = 1; c <= group && (c == 1 || blocks * c <= 10LL * cus); ++c) {
+    const double heads = (group + c - 1) / c, per_cu = (double)((blocks * c + cus - 1) / cus);
+    double time = p.causal ? std::max(heads, 0.5 * group * blocks / cus + (shared ? 0.5 : 0.25) * heads) : (per_cu + 0.05) * heads;
+    if (shared && per_cu < 2.0) time /= 0.6;
+    if (c > 1) time += per_cu * share_cost;
+    if (c == 1 || time < least) best = c, least = time;
+  }
+  return best;
 }
 // ... floats of the shares: dk, dv, and dk', dv' where one kernel makes all four (tangent_grads)
 template <typename P> inline size_t bwd_part_floats(const P &p, int Lk, int Hk, int chunks, bool tangent_grads) {

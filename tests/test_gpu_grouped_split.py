@@ -1,5 +1,7 @@
 """Grouped heads in the backward: a group's query heads dealt to several dk/dv workgroups (fp32 shares, then a merge)
 against one workgroup visiting them all."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -7,9 +9,36 @@ from jvp_flash_attention_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
+KERNELS = [(torch.bfloat16, 32), (torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 256), (torch.float32, 64), (torch.float32, 256)]
 
-@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 32), (torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 256),
-                                     (torch.float32, 64), (torch.float32, 256)])
+
+def _share_bytes(H, Hk, L, Lk, D, dtype, Z=2, six=False):
+    prob = _lib.make_problem(torch.empty(Z, H, L, D, dtype=dtype, device="meta"), None, _lib.MASK_NONE, False, 1.0)
+    return _lib.load().jvpfa_bwd_split_workspace_bytes(C.byref(prob), Lk, Hk, int(six))
+
+
+@pytest.mark.parametrize("dtype,D", KERNELS)
+@pytest.mark.parametrize("H", [5, 7])
+@pytest.mark.parametrize("mode", ["plain", "six", "padding"])
+def test_uneven_shares_agree_with_whole_groups(dtype, D, H, mode):
+    """A prime group in shares that differ by a head: 64 key blocks, of which three (four) times as many fill the GPU once."""
+    shares = {5: 3, 7: 4}[H]
+    assert _share_bytes(H, 1, 70, 4096, D, dtype) == shares * 2 * (2 * 4096 * D) * 4
+    test_split_groups_agree_with_whole_ones(dtype, D, H, 1, 70, 4096, mode)
+
+
+@pytest.mark.parametrize("dtype,D", KERNELS)
+def test_shares_are_bounded(dtype, D):
+    """Whatever the group: dk and dv of at most 10 workgroups of 128 keys per compute unit, and none where the blocks alone
+    fill it."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for H, Hk, Lk, Z in [(71, 1, 2048, 8), (71, 1, 2048, 31), (28, 4, 4096, 2), (64, 1, 128, 1), (13, 1, 100000, 1), (12, 4, 1111, 3)]:
+        got = _share_bytes(H, Hk, 1024, Lk, D, dtype, Z)
+        assert got <= 10 * cus * 128 * D * 8 and got % (2 * Z * Hk * Lk * D * 4) == 0, (H, Hk, Lk, Z, got)
+    assert _share_bytes(28, 4, 1024, 128 * cus, D, dtype) == 0
+
+
+@pytest.mark.parametrize("dtype,D", KERNELS)
 @pytest.mark.parametrize("H,Hk,L,Lk", [(6, 2, 65, 65), (4, 1, 200, 129), (12, 2, 33, 300)])
 @pytest.mark.parametrize("mode", ["plain", "dual", "six", "padding", "dropout"])
 def test_split_groups_agree_with_whole_ones(dtype, D, H, Hk, L, Lk, mode):
