@@ -560,12 +560,15 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   const int Lk = pr.Lk;  // keys; L counts queries
   const int kld = krow < Lk ? krow : Lk - 1;
   const uint32_t drop_lane = DROP ? (uint32_t)kld * DROP_C_KEY + (uint32_t)(8 * g) * DROP_C_ROW : 0u;
-  // 8 columns of this lane's row of dk, dv (dk', dv'); of a share of them where the group's query heads are split
+  // 8 columns of this lane's row of dk, dv (dk', dv'); of a share of them where the group's query heads are split.  The choice
+  // is compiled in only where it can arise: with it the ungrouped kernels at D = 64 without tangents took 172 registers and
+  // two waves per SIMD instead of 168 and three.
   auto store_grads = [&](int d0, const float *xk, const float *xv, const float *xkt, const float *xvt) {
     constexpr int NT = SIX ? 4 : 2;
-    const size_t off = head + (size_t)krow * D + d0;
     auto put = [&](void *dst, int t, const float *x) {
-      store8_or_part<T>(reinterpret_cast<T *>(dst), GROUPED ? kv_part(pr, D, NT, t, chunk) : nullptr, off, x);
+      const size_t off = head + (size_t)krow * D + d0;
+      if constexpr (GROUPED) store8_or_part<T>(reinterpret_cast<T *>(dst), kv_part(pr, D, NT, t, chunk), off, x);
+      else store8<T>(reinterpret_cast<T *>(dst) + off, x);
     };
     put(TAN ? p.dkt : p.dk, 0, xk);
     put(TAN ? p.dvt : p.dv, 1, xv);
