@@ -91,6 +91,14 @@ static auto pick_dkdv_for(const BwdParams &p, bool no_go, bool grouped, bool fol
   return pick_dkdv<T, D, MODE, MASK>(no_go, grouped, fold_kv, drop);
 }
 
+// The dk/dv kernel for D = 256 without tangents in the launch: without masks one kernel whether the heads are split or not.
+template <typename T, int D, int MODE, int MASK, bool DROP> static auto pick_wide_dkdv(const BwdParams &p) -> void (*)(const BwdParams) {
+  if constexpr (MASK != MASK_NONE) {
+    if (p.pr.chunks <= 1) return bwdw_dkdv_kernel<T, D, MODE, MASK, DROP>;
+  }
+  return bwdw_dkdv_kernel<T, D, MODE, MASK, DROP, true>;
+}
+
 // Adds up the shares of dk, dv (dk', dv' of the tangent mode; all four where the dual kernel folds them in) that a
 // launch over pr.chunks query heads groups left, see split.hpp.
 template <typename T, int D> static void launch_kv_merge(const BwdParams &p, bool tangent, bool four, hipStream_t stream) {
@@ -166,7 +174,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       using CfgW = BwdWideCfg<T, D, MODE>;
       using CfgK = BwdWideKvCfg<T, D, MODE>;
       auto kq = bwdw_dq_kernel<T, D, MODE, MASK, true>;
-      auto kkv = bwdw_dkdv_kernel<T, D, MODE, MASK, true>;
+      auto kkv = pick_wide_dkdv<T, D, MODE, MASK, true>(p);
       int rc = allow_lds(reinterpret_cast<const void *>(kq), CfgW::DQ_LDS);
       if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), CfgK::DKV_LDS);
       if (rc != 0) return rc;
@@ -250,7 +258,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     using CfgW = BwdWideCfg<T, D, MODE>;
     using CfgK = BwdWideKvCfg<T, D, MODE>;
     auto kq = bwdw_dq_kernel<T, D, MODE, MASK>;
-    auto kkv = bwdw_dkdv_kernel<T, D, MODE, MASK>;
+    auto kkv = pick_wide_dkdv<T, D, MODE, MASK, false>(p);
     int rc = allow_lds(reinterpret_cast<const void *>(kq), CfgW::DQ_LDS);
     if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), CfgK::DKV_LDS);
     if (rc != 0) return rc;

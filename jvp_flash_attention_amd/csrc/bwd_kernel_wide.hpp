@@ -325,8 +325,11 @@ template <typename T, int D, int MODE> struct BwdWideKvCfg : BwdWideCfg<T, D, MO
   static constexpr size_t DKV_LDS = 2 * (size_t)BwdWideCfg<T, D, MODE>::STAGEB + 2 * (size_t)STATB;
 };
 
+// SPLIT: the query heads of a group may be dealt to several workgroups, which store shares of the gradients (split.hpp).
+// Compiled apart for masks, whose registers are full: with the shares' pointers 112 bytes are spilled, without them 80 - 96
+// (without a mask 0 and 12).
 #if defined(__HIP_DEVICE_COMPILE__)
-template <typename T, int D, int MODE, int MASK, bool DROP = false>
+template <typename T, int D, int MODE, int MASK, bool DROP = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   using Cfg = BwdWideKvCfg<T, D, MODE>;
   constexpr bool TAN = MODE == BWD_TANGENT;
@@ -337,11 +340,12 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;  // queries, keys
   const int nblk = (Lk + Cfg::BLK - 1) / Cfg::BLK;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
-  const int zh = id / nblk / pr.chunks, chunk = id / nblk % pr.chunks;  // chunk: this workgroup's share of the query heads
+  const int chunks = SPLIT ? pr.chunks : 1;
+  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * chunks, pr.causal != 0);
+  const int zh = id / nblk / chunks, chunk = id / nblk % chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nblk;  // causal: the first key blocks have the longest query loops
-  const int z = zh / pr.Hk, hk = zh % pr.Hk, group = group_share(pr, chunk + 1) - group_share(pr, chunk);
-  const int h0 = hk * (pr.H / pr.Hk) + group_share(pr, chunk);
+  const int z = zh / pr.Hk, hk = zh % pr.Hk, group = SPLIT ? group_share(pr, chunk + 1) - group_share(pr, chunk) : pr.H / pr.Hk;
+  const int h0 = hk * (pr.H / pr.Hk) + (SPLIT ? group_share(pr, chunk) : 0);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
   const int r = lane % 32, g = lane / 32, pr32 = perm32(r);
@@ -351,7 +355,7 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   const int kld = krow < Lk ? krow : Lk - 1;
   const uint32_t drop_lane = DROP ? (uint32_t)kld * DROP_C_KEY + (uint32_t)(8 * g) * DROP_C_ROW : 0u;
   T *outk = reinterpret_cast<T *>(TAN ? p.dkt : p.dk), *outv = reinterpret_cast<T *>(TAN ? p.dvt : p.dv);
-  float *partk = kv_part(pr, D, 2, 0, chunk), *partv = kv_part(pr, D, 2, 1, chunk);
+  float *partk = SPLIT ? kv_part(pr, D, 2, 0, chunk) : nullptr, *partv = SPLIT ? kv_part(pr, D, 2, 1, chunk) : nullptr;
   const size_t off = head + (size_t)krow * D;
   if constexpr (MASK != MASK_NONE) {
     // a key block that the caller's hint declares fully masked has zero gradients
@@ -679,7 +683,7 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   }
 }
 #else
-template <typename T, int D, int MODE, int MASK, bool DROP = false>
+template <typename T, int D, int MODE, int MASK, bool DROP = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {}
 #endif
 

@@ -1,4 +1,5 @@
-"""Registers of kernels whose number decides how many workgroups share a compute unit, from the compiler's own figures."""
+"""Registers of kernels whose number decides how many workgroups share a compute unit or what is spilled, from the compiler's
+own figures."""
 import os
 import re
 import subprocess
@@ -7,11 +8,14 @@ import pytest
 
 from jvp_flash_attention_amd import build
 
-# kernel, most vector registers (512 per lane and SIMD: 168 for three waves, 256 for two)
+# kernel, most vector registers (512 per lane and SIMD: 168 for three waves, 256 for two), most bytes spilled
 KERNELS = [
-    ("bwd2_dkdv_kernel_2wg<__bf16, 64, BWD_PLAIN, MASK_NONE, true, false>", 168),
-    ("bwd2_dkdv_kernel_2wg<_Float16, 64, BWD_TANGENT, MASK_NONE, true, false>", 168),
-    ("bwd2_dkdv_kernel<__bf16, 64, BWD_PLAIN, MASK_NONE, true, false, false, true>", 168),
+    ("bwd2_dkdv_kernel_2wg<__bf16, 64, BWD_PLAIN, MASK_NONE, true, false>", 168, 0),
+    ("bwd2_dkdv_kernel_2wg<_Float16, 64, BWD_TANGENT, MASK_NONE, true, false>", 168, 0),
+    ("bwd2_dkdv_kernel<__bf16, 64, BWD_PLAIN, MASK_NONE, true, false, false, true>", 168, 0),
+    ("bwdw_dkdv_kernel<__bf16, 256, BWD_PLAIN, MASK_NONE, false, true>", 512, 0),
+    ("bwdw_dkdv_kernel<_Float16, 256, BWD_PLAIN, MASK_BOOL>", 512, 80),
+    ("bwdw_dkdv_kernel<__bf16, 256, BWD_TANGENT, MASK_ADD, true>", 512, 96),
 ]
 
 
@@ -20,7 +24,7 @@ def figures(tmp_path_factory):
     """{kernel: (vector registers, scratch bytes)}, compiled on their own (a few seconds)."""
     src = tmp_path_factory.mktemp("registers") / "kernels.hip"
     kinds = "".join(f'#include "{h}.hpp"\n' for h in ("bwd_kernel", "bwd_kernel_v2", "bwd_kernel_wide"))
-    src.write_text(kinds + "namespace jvpfa {\n" + "".join(f"template __global__ void {k}(const BwdParams);\n" for k, _ in KERNELS) + "}\n")
+    src.write_text(kinds + "namespace jvpfa {\n" + "".join(f"template __global__ void {k}(const BwdParams);\n" for k, _, _ in KERNELS) + "}\n")
     asm = str(src) + ".s"
     subprocess.run([build.HIPCC, *build.FLAGS, "-Wno-pass-failed", "-I", build.CSRC, "--cuda-device-only", "-S", str(src), "-o", asm],
                    check=True, capture_output=True)
@@ -28,10 +32,10 @@ def figures(tmp_path_factory):
         blocks = re.split(r"\n  - \.agpr_count:", f.read())[1:]
     found = [tuple(int(re.search(rf"\.{k}:\s+(\d+)", b).group(1)) for k in ("vgpr_count", "private_segment_fixed_size")) for b in blocks]
     assert len(found) == len(KERNELS)  # in the order of the text
-    return dict(zip((k for k, _ in KERNELS), found))
+    return dict(zip((k for k, _, _ in KERNELS), found))
 
 
 @pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
-@pytest.mark.parametrize("kernel,most", KERNELS)
-def test_registers(figures, kernel, most):
-    assert figures[kernel][0] <= most
+@pytest.mark.parametrize("kernel,registers,spilled", KERNELS)
+def test_registers(figures, kernel, registers, spilled):
+    assert figures[kernel][0] <= registers and figures[kernel][1] <= spilled
