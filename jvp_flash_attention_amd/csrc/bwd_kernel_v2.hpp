@@ -852,12 +852,13 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
     f32x16 S, dP, Sp, At;
     // INIT: -a and -(d1 + d2) (PLAIN -d1, TANGENT -a) are what A and dP start from, read from LDS straight into the tiles'
     // registers, instead of two additions per entry behind the products (not with dropout, which scales the products
-    // first; at D = 64 without gO two variants would need 258 and 260 registers and lose their second workgroup).  A lone
+    // first, nor at D = 64 without gO for grouped heads without a mask, which would take 258 registers instead of 256 and
+    // lose their second workgroup; with a packed mask they take 248 with it and 260 without).  A lone
     // wave per SIMD pays four cycles for every vector instruction, and with S' - mu shared by dS and P' a tile of the dual
     // kernel at D = 128 has 306 of them where it had 434 (dq 240 for 336).  dk/dv and dq, bf16: B4 H16 L2048 D64 335 -> 321
     // and 250 -> 242 us, packed documents B2 H16 L2077 D128 151 -> 143 us, both in one launch at B1 H16 L1024 D128, causal,
     // gradients of O' alone, 68.1 -> 65.6 us.
-    constexpr bool INIT = !DROP && !(D == 64 && DUAL && !has_go && (GROUPED || MASK == MASK_TILE));
+    constexpr bool INIT = !DROP && !(D == 64 && DUAL && !has_go && GROUPED && MASK == MASK_NONE);
     u32x4 ia[4], idp[4];
     if constexpr (INIT) {
       const uint32_t sad = sstat + (HB * 32 + 8 * g) * 4;

@@ -13,6 +13,8 @@ KERNELS = [
     ("bwd2_dkdv_kernel_2wg<__bf16, 64, BWD_PLAIN, MASK_NONE, true, false>", 168, 0),
     ("bwd2_dkdv_kernel_2wg<_Float16, 64, BWD_TANGENT, MASK_NONE, true, false>", 168, 0),
     ("bwd2_dkdv_kernel<__bf16, 64, BWD_PLAIN, MASK_NONE, true, false, false, true>", 168, 0),
+    ("bwd2_dkdv_kernel_2wg<__bf16, 64, BWD_DUAL, MASK_NONE, false, true>", 256, 0),
+    ("bwd2_dkdv_kernel<__bf16, 64, BWD_DUAL, MASK_BITS, false, true, false>", 256, 0),
     ("bwdw_dkdv_kernel<__bf16, 256, BWD_PLAIN, MASK_NONE, false, true>", 512, 0),
     ("bwdw_dkdv_kernel<_Float16, 256, BWD_PLAIN, MASK_BOOL>", 512, 80),
     ("bwdw_dkdv_kernel<__bf16, 256, BWD_TANGENT, MASK_ADD, true>", 512, 96),
