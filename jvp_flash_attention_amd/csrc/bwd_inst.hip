@@ -220,6 +220,9 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     const int cus = device_cus();
     if (!grouped && !six && blocks < cus && kv_blocks < cus) {
       void (*kb)(const BwdParams, int) = no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG> : bwd2_both_kernel<T, D, MODE, MASK, true>;
+      if constexpr (MASK == MASK_BOOL) {
+        if (p.pr.bits_q && p.pr.bits_k) kb = no_go ? bwd2_both_kernel<T, D, MODE, MASK_BITS, NG> : bwd2_both_kernel<T, D, MODE, MASK_BITS, true>;
+      }
       constexpr size_t LDS = Cfg2::DKV_LDS > Cfg2::DQ_LDS ? Cfg2::DKV_LDS : Cfg2::DQ_LDS;
       const int rcb = allow_lds(reinterpret_cast<const void *>(kb), LDS);
       if (rcb != 0) return rcb;

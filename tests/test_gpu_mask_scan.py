@@ -48,22 +48,19 @@ def test_scan_matches_numpy(Lq, Lk, planes, strided):
                 assert got[p, b, 0] == len(want) and np.array_equal(got[p, b, 1: 1 + len(want)], want)
 
 
-@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 32), (torch.float16, 64), (torch.bfloat16, 128)])
-@pytest.mark.parametrize("Lq,Lk,Hk", [(513, 513, 4), (128, 577, 2), (600, 70, 4)])
-@pytest.mark.parametrize("dual", [False, True])
-def test_packed_copy_changes_no_bit(dtype, D, Lq, Lk, Hk, dual):
-    print("case", dtype, D, Lq, Lk, Hk, dual, flush=True)
+def _compare(dtype, D, Z, H, Hk, Lq, Lk, dual, with_go=True, six=None):
+    """Every output of a step, from the packed copies and from the mask's bytes."""
     g = torch.Generator(device="cuda").manual_seed(D + Lq)
-    rand = lambda h, n: torch.randn(2, h, n, D, generator=g, device="cuda").to(dtype)  # noqa: E731
-    q, k, v, qt, kt, vt, go, gt = rand(4, Lq), rand(Hk, Lk), rand(Hk, Lk), rand(4, Lq), rand(Hk, Lk), rand(Hk, Lk), rand(4, Lq), rand(4, Lq)
-    mask = torch.rand(2, 4, Lq, Lk, generator=g, device="cuda") < 0.7
+    rand = lambda h, n: torch.randn(Z, h, n, D, generator=g, device="cuda").to(dtype)  # noqa: E731
+    q, k, v, qt, kt, vt, go, gt = rand(H, Lq), rand(Hk, Lk), rand(Hk, Lk), rand(H, Lq), rand(Hk, Lk), rand(Hk, Lk), rand(H, Lq), rand(H, Lq)
+    mask = torch.rand(Z, H, Lq, Lk, generator=g, device="cuda") < 0.7
     be = _lib.backend()
 
     def step(m):
         t = (qt, kt, vt) if dual else (None,) * 3
         o, ot, M, mu = be.fwd(q, k, v, *t, m, _lib.MASK_BOOL, False, -0.3 if Lk == 70 else D**-0.5)
-        return (o, ot, M, mu, *be.bwd(q, k, v, *t, o, ot, M, mu, go, gt if dual else None, m, _lib.MASK_BOOL, False,
-                                      -0.3 if Lk == 70 else D**-0.5, want_tangent_grads=dual))
+        return (o, ot, M, mu, *be.bwd(q, k, v, *t, o, ot, M, mu, go if with_go else None, gt if dual else None, m, _lib.MASK_BOOL, False,
+                                      -0.3 if Lk == 70 else D**-0.5, want_tangent_grads=dual if six is None else six))
 
     packed = step(mask)
     _lib.set_mask_bits(False)
@@ -73,3 +70,19 @@ def test_packed_copy_changes_no_bit(dtype, D, Lq, Lk, Hk, dual):
         _lib.set_mask_bits(True)
     for name, a, b in zip(("O", "Ot", "M", "mu", "dq", "dk", "dv", "dqt", "dkt", "dvt"), packed, from_bytes):
         assert (a is None and b is None) or torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 32), (torch.float16, 64), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("Lq,Lk,Hk", [(513, 513, 4), (128, 577, 2), (600, 70, 4)])
+@pytest.mark.parametrize("dual", [False, True])
+def test_packed_copy_changes_no_bit(dtype, D, Lq, Lk, Hk, dual):
+    print("case", dtype, D, Lq, Lk, Hk, dual, flush=True)
+    _compare(dtype, D, 2, 4, Hk, Lq, Lk, dual)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 32), (torch.float16, 64), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("Z,H", [(1, 4), (4, 16)])  # both roles in one launch; a grid that fills the GPU
+@pytest.mark.parametrize("grads", ["o", "tangent", "both"])
+def test_packed_copy_changes_no_bit_of_three_gradients(dtype, D, Z, H, grads):
+    print("case", dtype, D, Z, H, grads, flush=True)
+    _compare(dtype, D, Z, H, H, 577, 577, grads != "o", grads != "tangent", False)
