@@ -193,6 +193,8 @@ def forget_mask(mask) -> None:
             delattr(mask, name)
         except AttributeError:
             pass
+    if mask.is_cuda:
+        binding().forget_masks()  # backwards of forwards already done look again, too
 
 
 # What is derived from a mask is kept on the mask tensor together with where it was made.  Kernels of another stream wait for

@@ -15,10 +15,12 @@
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
+#include <atomic>
 #include <cmath>
 #include <optional>
 #include <string>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "../../include/jvpfa.h"
@@ -169,10 +171,34 @@ bool any_requires_grad(std::initializer_list<const Tensor *> tensors) {
   return false;
 }
 
-// What the kernels of a backward may use about the mask as it now is: one Python call, which finds what the
-// forward derived unless the mask has changed since.
-void look_up_hints(Call &c, const Tensor &q, int64_t Lk) {
-  if (c.mask_kind == JVPFA_MASK_NONE) return;
+// The current stream of a device, and the id of the graph capture under way on it (0: none).
+std::pair<uintptr_t, uint64_t> stream_state(int64_t device) {
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (stream) C10_HIP_CHECK(hipStreamGetCaptureInfo(stream, &status, &id));  // (the default stream cannot be captured)
+  return {reinterpret_cast<uintptr_t>(stream), status == hipStreamCaptureStatusActive ? id : 0};
+}
+
+std::atomic<int64_t> masks_forgotten{0};  // calls of forget_mask, which stand for writes that no version counter shows
+
+// What a call derived from its mask holds for another call if nothing here has changed; a mask without a version counter
+// never compares equal.
+struct MaskState {
+  int64_t version = -1, forgotten = 0, stream = 0, capture = 0;
+  bool holds_for(const MaskState &o) const {
+    return version >= 0 && version == o.version && forgotten == o.forgotten && stream == o.stream && capture == o.capture;
+  }
+};
+MaskState mask_state(const Tensor &mask, const Tensor &q) {
+  const auto [stream, capture] = stream_state(q.device().index());
+  return {mask.is_inference() ? -1 : static_cast<int64_t>(mask._version()), masks_forgotten.load(), static_cast<int64_t>(stream),
+          static_cast<int64_t>(capture)};
+}
+
+// A backward uses what its forward derived from the mask, or looks it up again where the mask may have changed.
+void renew_hints(Call &c, const MaskState &then, const Tensor &q, int64_t Lk) {
+  if (c.mask_kind == JVPFA_MASK_NONE || then.holds_for(mask_state(*c.mask, q))) return;
   const py::gil_scoped_acquire gil;
   const py::object hints = py::module_::import("jvp_flash_attention_amd._lib").attr("mask_hints")(q, *c.mask, c.mask_kind, Lk, true);
   std::tie(c.key_limit, c.tiles_q, c.tiles_k, c.bits_k, c.bits_q) = hints.cast<std::tuple<OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>>();
@@ -189,8 +215,13 @@ struct Attention : public torch::autograd::Function<Attention> {
     auto [o, ot, M, mu] = ::forward(q, k, v, qt, kt, vt, c);
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({q, k, v, qt, kt, vt, o, ot, M, mu});
-    // the mask as it is: it may be refilled, and what was derived from it is looked up again by the backward
+    // (the mask is kept as it is and may be refilled: see renew_hints)
     ctx->saved_data["c"] = c10::IValue(std::make_tuple(c.mask, c.mask_kind, c.causal, c.scale, c.dropout_p, static_cast<int64_t>(c.seed), c.split));
+    if (c.mask) {
+      const MaskState m = mask_state(*c.mask, q);
+      ctx->saved_data["hints"] = c10::IValue(std::make_tuple(c.key_limit, c.tiles_q, c.tiles_k, c.bits_k, c.bits_q, m.version, m.forgotten,
+                                                             m.stream, m.capture));
+    }
     if (qt.defined()) return {o, ot};
     return {o};
   }
@@ -207,7 +238,12 @@ struct Attention : public torch::autograd::Function<Attention> {
     variable_list g;
     {
       const at::AutoGradMode off(false);
-      if (go.defined() || gt.defined()) look_up_hints(c, s[0], s[1].size(2));
+      if (c.mask) {
+        const auto h = ctx->saved_data["hints"].toTuple()->elements();
+        c.key_limit = h[0].toOptional<Tensor>(), c.tiles_q = h[1].toOptional<Tensor>(), c.tiles_k = h[2].toOptional<Tensor>();
+        c.bits_k = h[3].toOptional<Tensor>(), c.bits_q = h[4].toOptional<Tensor>();
+        renew_hints(c, {h[5].toInt(), h[6].toInt(), h[7].toInt(), h[8].toInt()}, s[0], s[1].size(2));
+      }
       if (gt.defined()) {
         g = ::backward(s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8], s[9], go, gt, c, want_t);
       } else {
@@ -283,15 +319,6 @@ Call make_call(OptTensor mask, int64_t mask_kind, bool causal, double dropout_p,
   return c;
 }
 
-// The current stream of a device, and the id of the graph capture under way on it (0: none).
-std::pair<uintptr_t, uint64_t> stream_state(int64_t device) {
-  const hipStream_t stream = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  unsigned long long id = 0;
-  if (stream) C10_HIP_CHECK(hipStreamGetCaptureInfo(stream, &status, &id));  // (the default stream cannot be captured)
-  return {reinterpret_cast<uintptr_t>(stream), status == hipStreamCaptureStatusActive ? id : 0};
-}
-
 }  // namespace
 
 PYBIND11_MODULE(_torch_binding, m) {
@@ -302,6 +329,7 @@ PYBIND11_MODULE(_torch_binding, m) {
     return attend(q, k, v, level, scale, make_call(mask, mask_kind, causal, dropout_p, seed, key_limit, tiles_q, tiles_k, bits_k, bits_q, split));
   });
   m.def("stream_state", &stream_state);
+  m.def("forget_masks", [] { ++masks_forgotten; });
   m.def("fwd", [](const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &qt, const OptTensor &kt, const OptTensor &vt,
                   double scale, bool causal, double dropout_p, uint64_t seed, bool split, OptTensor mask, int64_t mask_kind,
                   OptTensor key_limit, OptTensor tiles_q, OptTensor bits_q) {

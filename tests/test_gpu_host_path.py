@@ -123,6 +123,28 @@ def test_a_backward_reads_the_mask_as_it_then_is(dtype, D, H, L, kind, dropout):
     assert torch.count_nonzero(got[1][:, :, :192]) == 0 and torch.count_nonzero(got[1][:, :, 256:]) > 0
 
 
+def test_a_backward_looks_at_a_forgotten_mask_again():
+    """A write that no version counter shows, then forget_mask, between forward and backward."""
+    L = 520
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v, go = (torch.randn(1, 2, L, 64, generator=g, device="cuda").to(torch.bfloat16) for _ in range(4))
+    q, k, v = (x.requires_grad_() for x in (q, k, v))
+    mask = (torch.arange(L, device="cuda") < 200).expand(1, 1, L, L).contiguous()
+    second = ~mask
+    o = attention(q, k, v, attn_mask=mask)
+    version = mask._version
+    mask.data.copy_(second)
+    assert mask._version == version
+    _lib.forget_mask(mask)
+    got = torch.autograd.grad(o, (q, k, v), go)
+    mask.data.copy_(~second)
+    o = attention(q, k, v, attn_mask=mask.clone())
+    other = ~second
+    want_o = attention(q, k, v, attn_mask=other)
+    other.copy_(second)
+    assert all(torch.equal(a, b) for a, b in zip(got, torch.autograd.grad(want_o, (q, k, v), go)))
+
+
 @pytest.mark.parametrize("dtype,D,Lq,Lk,kind", [(torch.bfloat16, 64, 577, 577, "rows"), (torch.float16, 128, 600, 520, "rows"),
                                                 (torch.float32, 32, 520, 520, "rows"), (torch.bfloat16, 256, 520, 520, "rows"),
                                                 (torch.bfloat16, 64, 70, 1000, "keys"), (torch.bfloat16, 128, 65, 17000, "keys")])
