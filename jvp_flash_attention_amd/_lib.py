@@ -385,7 +385,7 @@ def _stream(t) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
-def _wants_backward(q, k, v, level) -> bool:
+def wants_backward(q, k, v, level) -> bool:
     """Whether a call on these tensors (dual tensors of ``level``, if that is not negative) may be differentiated."""
     if not torch.is_grad_enabled():
         return False
@@ -407,19 +407,22 @@ class MaskScan(NamedTuple):
     origin: Origin | None = None
 
 
-def mask_scan(q, mask, mask_kind, Lk):
+def mask_scan(q, mask, mask_kind, Lk, backward=None, dropout=False):
     """The ``MaskScan`` of a boolean mask with a row per query (shape [*, *, L, Lk]), from one pass over it, or None for
     other masks, short sequences, and with the tile lists or the packed copies switched off.  Cached on the mask tensor,
-    keyed by its version counter, where ``tile_lists`` and ``mask_bits`` look as well."""
+    keyed by its version counter, where ``tile_lists`` and ``mask_bits`` look as well.  A packed copy is made (16-bit element
+    types at D <= 128) if kernels of the call read it: along the keys without dropout, along the queries unless it is known
+    that no backward follows (``backward`` False, not None)."""
     Z, H, L, D = q.shape
     if not (_tile_lists_enabled and _mask_bits_enabled) or mask is None or mask_kind != MASK_BOOL or max(L, Lk) < TILE_LISTS_MIN_L:
         return None
     if mask.dim() != 4 or mask.shape[2] != L or mask.shape[3] != Lk or not mask.is_cuda:
         return None
     packed = q.element_size() == 2 and D <= 128
+    want_q, want_k = packed and not dropout, packed and backward is not False
     version = mask_version(mask)
     cached = getattr(mask, "_jvpfa_scan", None)
-    if cached is not None and version is not None and cached.version == version and (cached.bits_q is not None or not packed):
+    if cached is not None and version is not None and cached.version == version and (cached.bits_q is not None or not want_q):
         if _usable(cached.origin, mask, *cached[1:6]):
             return cached
     lib = load()
@@ -430,8 +433,8 @@ def mask_scan(q, mask, mask_kind, Lk):
         return torch.empty(n, device=mask.device, dtype=torch.int32)
 
     scan = MaskScan(version, ints(lib.jvpfa_mask_tiles_bytes(C.byref(prob), Lk, 0) // 4), ints(lib.jvpfa_mask_tiles_bytes(C.byref(prob), Lk, 1) // 4),
-                    ints(planes * ((Lk + 63) // 64) * L * 2) if packed else None,
-                    ints(lib.jvpfa_mask_bits_bytes(C.byref(prob), Lk) // 4) if packed else None, ints(planes))
+                    ints(planes * ((Lk + 63) // 64) * L * 2) if want_q else None,
+                    ints(lib.jvpfa_mask_bits_bytes(C.byref(prob), Lk) // 4) if want_k else None, ints(planes))
     scratch = torch.empty(lib.jvpfa_mask_scan_bytes(C.byref(prob), Lk), device=mask.device, dtype=torch.uint8)
     out = MaskScanOut(_ptr(scan.tiles_q), _ptr(scan.tiles_k), _ptr(scan.bits_q), _ptr(scan.bits_k), _ptr(scan.attends), _ptr(scratch))
     with torch.cuda.device(mask.device):
@@ -441,24 +444,29 @@ def mask_scan(q, mask, mask_kind, Lk):
         try:
             mask._jvpfa_scan = scan
             mask._jvpfa_tiles = (version, scan.tiles_q, scan.tiles_k, scan.origin)
-            if packed:
+            if want_k:
                 mask._jvpfa_bits = (version, scan.bits_k, scan.origin)
         except (AttributeError, RuntimeError):
             pass
     return scan
 
 
-def mask_hints(q, mask, mask_kind, Lk, backward: bool):
+def mask_hints(q, mask, mask_kind, Lk, backward, dropout=False):
     """(key_limit, tiles_q, tiles_k, bits_k, bits_q) for a call with this mask, each None where it does not apply; tiles_k and
-    bits_k only for a backward."""
+    bits_k only for a backward (None: a forward that may be followed by one)."""
     if mask_kind == MASK_NONE:
         return (None,) * 5
-    scan = mask_scan(q, mask, mask_kind, Lk)
+    scan = mask_scan(q, mask, mask_kind, Lk, backward, dropout)
     if scan is not None:
-        return None, scan.tiles_q, scan.tiles_k if backward else None, scan.bits_k if backward else None, scan.bits_q
+        if not backward:
+            return None, scan.tiles_q, None, None, scan.bits_q
+        if scan.bits_k is None:  # the mask was first met where no backward was to follow, or by kernels that read its bytes
+            with torch.cuda.device(q.device):
+                return None, scan.tiles_q, scan.tiles_k, mask_bits(q, mask, mask_kind, Lk), scan.bits_q
+        return None, scan.tiles_q, scan.tiles_k, scan.bits_k, scan.bits_q
     with torch.cuda.device(q.device):
         lim = key_limit_hint(mask, mask_kind, q.shape[0], Lk)
-        tq, tk = tile_lists(q, mask, mask_kind, backward, Lk)
+        tq, tk = tile_lists(q, mask, mask_kind, bool(backward), Lk)
         return lim, tq, tk, mask_bits(q, mask, mask_kind, Lk) if backward else None, None
 
 
@@ -491,7 +499,7 @@ class HipBackend:
 
     def _fwd(self, q, k, v, qt, kt, vt, mask, mask_kind, causal, sm_scale, dropout_p=0.0, dropout_seed=0):
         _require_gpu(q, mask)
-        lim, tq, _, _, bits_q = mask_hints(q, mask, mask_kind, k.shape[2], False)
+        lim, tq, _, _, bits_q = mask_hints(q, mask, mask_kind, k.shape[2], None, dropout_p > 0)
         return binding().fwd(q, k, v, qt, kt, vt, float(sm_scale), bool(causal), float(dropout_p), int(dropout_seed) & (2**64 - 1),
                              _split_enabled, mask, mask_kind, lim, tq, bits_q)
 
@@ -500,15 +508,15 @@ class HipBackend:
         _require_gpu(q, mask)
         return tuple(binding().bwd(q, k, v, qt, kt, vt, o, ot, M, mu, go, gt, float(sm_scale), bool(causal),
                                    bool(want_tangent_grads), float(dropout_p), int(dropout_seed) & (2**64 - 1), _split_enabled,
-                                   mask, mask_kind, *mask_hints(q, mask, mask_kind, k.shape[2], True)))
+                                   mask, mask_kind, *mask_hints(q, mask, mask_kind, k.shape[2], True, dropout_p > 0)))
 
-    def attend(self, q, k, v, mask, mask_kind, causal, sm_scale, dropout_p, dropout_seed, level):
+    def attend(self, q, k, v, mask, mask_kind, causal, sm_scale, dropout_p, dropout_seed, level, backward=None):
         """The whole eager call, autograd included, on tensors that may be dual tensors of ``level``; None when the
-        shapes or types of q, k, v are not supported."""
+        shapes or types of q, k, v are not supported.  ``backward``: what ``wants_backward`` says, for calls with a mask."""
         hints = (None,) * 5
         if mask_kind != MASK_NONE:
             _require_gpu(q, mask)
-            hints = mask_hints(q, mask, mask_kind, k.shape[2], _wants_backward(q, k, v, level))
+            hints = mask_hints(q, mask, mask_kind, k.shape[2], backward, dropout_p > 0)
         return binding().attend(q, k, v, level, sm_scale, causal, dropout_p, dropout_seed, _split_enabled, mask, mask_kind, *hints)
 
     def dropout_keep(self, q, Lk, dropout_p, dropout_seed):

@@ -200,7 +200,7 @@ MaskState mask_state(const Tensor &mask, const Tensor &q) {
 void renew_hints(Call &c, const MaskState &then, const Tensor &q, int64_t Lk) {
   if (c.mask_kind == JVPFA_MASK_NONE || then.holds_for(mask_state(*c.mask, q))) return;
   const py::gil_scoped_acquire gil;
-  const py::object hints = py::module_::import("jvp_flash_attention_amd._lib").attr("mask_hints")(q, *c.mask, c.mask_kind, Lk, true);
+  const py::object hints = py::module_::import("jvp_flash_attention_amd._lib").attr("mask_hints")(q, *c.mask, c.mask_kind, Lk, true, c.dropout_p > 0.0);
   std::tie(c.key_limit, c.tiles_q, c.tiles_k, c.bits_k, c.bits_q) = hints.cast<std::tuple<OptTensor, OptTensor, OptTensor, OptTensor, OptTensor>>();
 }
 

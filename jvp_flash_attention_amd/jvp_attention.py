@@ -128,15 +128,16 @@ def _remember_verified(mask: Tensor) -> None:
         pass
 
 
-def _classify_mask(attn_mask: Tensor | None, q: Tensor, verify_attn_mask: bool):
-    """Mask kind and the tensor the kernels read (JA:2429-2462)."""
+def _classify_mask(attn_mask: Tensor | None, q: Tensor, verify_attn_mask: bool, backward: bool | None = None, dropout: bool = False):
+    """Mask kind and the tensor the kernels read (JA:2429-2462).  ``backward``, ``dropout``: what of the call is known, see
+    ``_lib.mask_scan``."""
     if attn_mask is None:
         return torch.empty(0, device=q.device, dtype=q.dtype), _lib.MASK_NONE
     if attn_mask.dtype == torch.bool:
         mask_tensor = attn_mask
         if verify_attn_mask and not _already_verified(attn_mask):
             # (large masks: from the pass over the mask that its tile lists and packed copies need anyway)
-            scan = _lib.mask_scan(q, mask_tensor, _lib.MASK_BOOL, mask_tensor.shape[3]) if _native() else None
+            scan = _lib.mask_scan(q, mask_tensor, _lib.MASK_BOOL, mask_tensor.shape[3], backward, dropout) if _native() else None
             attends = mask_tensor.any(dim=-1).any(dim=-1) if scan is None else scan.attends
             assert attends.all(), "The attention mask cannot be all False for any head."
             _remember_verified(attn_mask)
@@ -355,11 +356,12 @@ def _transforms_active() -> bool:
 def _attend(q, k, v, attn_mask, dropout_p, causal, sm_scale, level):
     """An eager call outside of ``torch.func`` transforms, on tensors that may be dual tensors of ``level``: natively
     from here on (``csrc/torch_binding.cpp``), autograd included."""
-    mask, kind = None, _lib.MASK_NONE
+    mask, kind, backward = None, _lib.MASK_NONE, None
     if attn_mask is not None:
         _validate(q, k, v, attn_mask, dropout_p, causal)
-        mask, kind = _classify_mask(attn_mask, q, True)
-    o = _lib.backend().attend(q, k, v, mask, kind, causal, sm_scale, dropout_p, _new_dropout_seed(dropout_p), level)
+        backward = _lib.wants_backward(q, k, v, level)
+        mask, kind = _classify_mask(attn_mask, q, True, backward, dropout_p > 0)
+    o = _lib.backend().attend(q, k, v, mask, kind, causal, sm_scale, dropout_p, _new_dropout_seed(dropout_p), level, backward)
     if o is None:
         _validate(q, k, v, attn_mask, dropout_p, causal)  # says what is wrong
         raise ValueError("unsupported arguments")

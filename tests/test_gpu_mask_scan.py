@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from jvp_flash_attention_amd import _lib
+from jvp_flash_attention_amd import _lib, attention
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +86,28 @@ def test_packed_copy_changes_no_bit(dtype, D, Lq, Lk, Hk, dual):
 def test_packed_copy_changes_no_bit_of_three_gradients(dtype, D, Z, H, grads):
     print("case", dtype, D, Z, H, grads, flush=True)
     _compare(dtype, D, Z, H, H, 577, 577, grads != "o", grads != "tangent", False)
+
+
+def test_packed_copies_are_made_where_kernels_of_the_call_read_them():
+    q = torch.randn(1, 2, 513, 64, device="cuda").to(torch.bfloat16)
+    leaf = q.clone().requires_grad_()
+    wide = torch.randn(1, 2, 513, 256, device="cuda").to(torch.bfloat16).requires_grad_()
+    mask = torch.rand(1, 1, 513, 513, device="cuda") < 0.9
+
+    def made(x, p=0.0, m=None):
+        m = mask.clone() if m is None else m
+        o = attention(x, x, x, attn_mask=m, dropout_p=p)
+        return m, o, m._jvpfa_scan.bits_q is not None, hasattr(m, "_jvpfa_bits")
+
+    assert made(q)[2:] == (True, False)
+    assert made(leaf)[2:] == (True, True)
+    assert made(leaf, 0.25)[2:] == (False, True)
+    assert made(q, 0.25)[2:] == (False, False)
+    assert made(wide)[2:] == (False, False)
+    # what is missing is made when a later call asks for it
+    m = made(q, 0.25)[0]
+    assert made(q, m=m)[2:] == (True, False)
+    want, got = made(leaf)[1], made(leaf, m=m)
+    assert got[2:] == (True, True) and torch.equal(got[1], want)
+    grads = [torch.autograd.grad(o, leaf, torch.ones_like(o))[0] for o in (got[1], want)]
+    assert torch.equal(*grads)
