@@ -1,7 +1,7 @@
 // Fused dual forward for fp32, D in {32, 64, 128}, on the direct-to-LDS pipeline.
 //
 // Mathematics and work split as in fwd_kernel.hpp (4 waves = 128 query rows, scores transposed, lane = query).  An fp32
-// matrix instruction (32x32x2) takes 64 cycles for what the bf16 one does in 2, so a wave has time for everything else
+// matrix instruction (32x32x2) takes 64 cycles for what is 4 of the bf16 one's 32, so a wave has time for everything else
 // as long as it never waits: the register-staged kernel this replaces copied every tile through registers behind two
 // barriers, wrote V transposed, fetched mask values where they were used and rescaled the accumulators on every tile,
 // and kept the matrix cores busy 58 % of the time at B4 H8 L1024 D64 (one workgroup per compute unit, one wave per
@@ -96,9 +96,11 @@ template <int D, int NTILE> struct F32Tiles {
       col[e] = row * C::ROWB + (((byte / 16) ^ swz_f32<C::CH>(row)) * 16) + byte % 16;
     }
   }
-  // rows: those that exist from this tile's first on (rows past them, and tiles that do not exist, read as zeros)
+  // rows: those that exist from this tile's first on (rows past them, and tiles that do not exist, read as zeros).  The
+  // bytes of all that follow, 512 a row at D = 128, pass the descriptor's 32 bits at 2^23 rows: it then covers the next 2 GB.
+  // (Cut to the tile instead, the compiler finds other schedules, which take a wave or 16 - 60 bytes of spill from 17 kernels.)
   __device__ __forceinline__ void aim(int t, const float *base, int first, int rows) {
-    rs[t] = __builtin_amdgcn_make_buffer_rsrc((void *)(base + (size_t)first * D), 0, max(rows, 0) * C::ROWB, 0x00020000);
+    rs[t] = __builtin_amdgcn_make_buffer_rsrc((void *)(base + (size_t)first * D), 0, (int)min((long long)max(rows, 0) * C::ROWB, 0x7fffffffLL), 0x00020000);
   }
   template <int P> __device__ __forceinline__ void load() {
     constexpr int i = P / NTILE, t = P % NTILE;

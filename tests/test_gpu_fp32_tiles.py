@@ -34,3 +34,27 @@ def test_tile_edges(D, L, Lk, mask):
     for name, got, want in (("O", o, fwd["O"]), ("Ot", ot, fwd["Ot"]), *zip(("dq", "dk", "dv", "dqt", "dkt", "dvt"), six, (bwd[n] for n in ("dq", "dk", "dv", "dqt", "dkt", "dvt")))):
         # the repository's fp32 bar, relative where the quantity is larger than one
         assert np.abs(got.double().cpu().numpy() - want).max() <= 1e-4 * max(1.0, np.abs(want).max()), name
+
+
+def test_key_rows_past_32_bits_of_bytes():
+    """One query over 2^23 + 70 keys of 512 bytes: one of the first keys, then the last, has a logit of 64, all others 0, and so
+    all the weight but e^-64 each.  The exponent 64 log2(e) = 92 is rounded to 92 * 2^-24 on either side of its difference
+    with the row's log-sum-exp, so the weight is 1 within 2 * 92 * 2^-24 * ln 2 < 1e-5."""
+    D, Lk = 128, 2**23 + 70
+    q = torch.zeros(1, 1, 1, D, device="cuda")
+    q[..., 0] = 8.0
+    k = torch.zeros(1, 1, Lk, D, device="cuda")
+    v = torch.zeros_like(k)
+    be = _lib.backend()
+    for at in (84, Lk - 1):  # 84: in the tile from whose start 2^23 + 6 rows follow
+        k[0, 0, at, 0] = 8.0
+        v[0, 0, at] = 1.0 + torch.arange(D, device="cuda") / D
+        o, _, M, _ = be.fwd(q, k, v, None, None, None, None, _lib.MASK_NONE, False, 1.0)
+        assert (o[0, 0, 0] / v[0, 0, at] - 1).abs().max() <= 1e-5
+        go = torch.ones_like(q)
+        dq, _, dv = be.bwd(q, k, v, None, None, None, o, None, M, None, go, None, None, _lib.MASK_NONE, False, 1.0)[:3]
+        assert (dv[0, 0, at] - 1).abs().max() <= 1e-5
+        assert dq.abs().max() <= 1e-5 * 8 * 192  # P (gO V - rowsum gO O) K: both of the difference are 192 times the weight
+        dv[0, 0, at] = 0
+        assert dv.abs().max() <= 1e-20
+        k[0, 0, at], v[0, 0, at] = 0, 0
