@@ -1,8 +1,12 @@
 """The native path of eager calls (``csrc/torch_binding.cpp``): which gradients arrive, what it refuses, and masks that change."""
+import contextlib
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
+import torch.utils.checkpoint
 
 from jvp_flash_attention_amd import JVPAttn, _lib, attention
 from oracle import dense
@@ -199,3 +203,55 @@ def test_a_graph_replays_with_refilled_masks(dtype, D, Lq, Lk, kind):
         for i, (a, b) in enumerate(zip(got, want)):
             assert torch.equal(a, b), (rep, i)
     del junk
+
+
+def test_saved_tensor_hooks_and_checkpointing_change_nothing():
+    q, k, v, qt, kt, vt, go, gt = (x.cuda() for x in _inputs(64, torch.bfloat16))
+    mask = torch.rand(2, 1, 75, 75, device="cuda") < 0.5
+    leaves = [x.requires_grad_() for x in (q, k, v)]
+    packed = []
+
+    def step(hooks):
+        with fwAD.dual_level():
+            with hooks:
+                o, ot = fwAD.unpack_dual(JVPAttn.fwd_dual(*(fwAD.make_dual(a, b) for a, b in zip(leaves, (qt, kt, vt))), attn_mask=mask))
+            return [o.detach(), ot.detach(), *torch.autograd.grad((o, ot), leaves, (go, gt))]
+
+    def pack(t):
+        packed.append(t.shape)
+        return t.cpu()
+
+    want = step(contextlib.nullcontext())
+    hooked = step(torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()))
+    assert len(packed) >= 10  # q, k, v, their tangents, O, O', M, mu
+    assert all(torch.equal(a, b) for a, b in zip(hooked, want))
+    want = torch.autograd.grad(attention(q, k, v, causal=True), leaves, go)
+    o = torch.utils.checkpoint.checkpoint(attention, q, k, v, None, 0.0, True, use_reentrant=False)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o, leaves, go), want))
+
+
+def test_threads_on_streams_of_their_own_share_a_mask():
+    """(First-order steps: torch keeps one forward-mode level for all threads.)"""
+    mask = torch.rand(2, 1, 530, 530, generator=torch.Generator(device="cuda").manual_seed(9), device="cuda") < 0.5
+
+    def step(seed, mask):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        q, k, v, go = (torch.randn(2, 3, 530, 64, generator=g, device="cuda").to(torch.bfloat16) for _ in range(4))
+        q, k, v = (x.requires_grad_() for x in (q, k, v))
+        o = attention(q, k, v, attn_mask=mask)
+        return [o.detach(), *torch.autograd.grad(o, (q, k, v), go)]
+
+    want = [step(seed, mask) for seed in range(4)]
+    for shared in (mask, mask.clone()):  # scanned by the calls above; scanned by whichever thread comes first
+        torch.cuda.synchronize()
+
+        def work(seed, shared=shared):
+            with torch.cuda.stream(torch.cuda.Stream()):
+                got = [step(seed, shared) for _ in range(3)]
+                torch.cuda.current_stream().synchronize()
+                return got
+
+        with ThreadPoolExecutor(4) as pool:
+            for steps, w in zip(pool.map(work, range(4)), want):
+                for got in steps:
+                    assert all(torch.equal(a, b) for a, b in zip(got, w))
