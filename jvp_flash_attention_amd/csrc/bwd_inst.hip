@@ -139,7 +139,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
   const long long kv_blocks = (long long)((p.pr.Lk + BWD_BLK - 1) / BWD_BLK) * p.pr.Z * p.pr.Hk * p.pr.chunks;
   if (kv_blocks > 0x7fffffffLL) return -2;
   if (p.pr.drop_thr != 0) {
-    // dropout: the direct-to-LDS kernels carry it for the 16-bit types, the register-staged ones for fp32
+    // dropout: the direct-to-LDS kernels carry it, the register-staged ones for fp32 at D = 256
     if constexpr (sizeof(T) == 2 && D <= 128) {
       using Cfg2 = Bwd2Cfg<T, D, MODE>;
       const bool no_go = MODE == BWD_DUAL && p.go == nullptr;
