@@ -3,6 +3,7 @@
 // and exporting  int JVPFA_NAME(const FwdParams&, bool dual, int mask_kind, hipStream_t).
 #include "fwd_kernel.hpp"
 #include "fwd_kernel_f32.hpp"
+#include "fwd_kernel_f32x3.hpp"
 #include "fwd_kernel_v2.hpp"
 #include "fwd_kernel_v3.hpp"
 #include "fwd_kernel_wide.hpp"
@@ -24,12 +25,15 @@ static int launch_fwd_one(const FwdParams &p, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
-// fp32 with D <= 128: direct-to-LDS as well.
+// fp32 with D <= 128: direct-to-LDS as well; up to D = 64 as three bf16 parts.
 template <int D, bool DUAL, int MASK, bool DROP = false>
 static int launch_fwd_f32_one(const FwdParams &p, hipStream_t stream) {
   using C = F32Cfg<D>;
-  constexpr size_t LDS = 2 * (DUAL ? 4 : 2) * (size_t)C::TILEB;
-  auto kern = fwd_f32_kernel<D, DUAL, MASK, DROP>;
+  constexpr bool X3 = D <= 64;
+  constexpr size_t LDS = X3 ? X3Lds<D, DUAL>::FWD : 2 * (DUAL ? 4 : 2) * (size_t)C::TILEB;
+  void (*kern)(const FwdParams);
+  if constexpr (X3) kern = fwd_f32x3_kernel<D, DUAL, MASK, DROP>;
+  else kern = fwd_f32_kernel<D, DUAL, MASK, DROP>;
   int rc = allow_lds(reinterpret_cast<const void *>(kern), LDS);
   if (rc != 0) return rc;
   const long long blocks = (long long)((p.pr.L + C::BLK - 1) / C::BLK) * p.pr.Z * p.pr.H;

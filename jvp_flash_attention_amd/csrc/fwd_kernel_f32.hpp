@@ -73,6 +73,9 @@ __device__ __forceinline__ void mma_f32_acc(f32x16 &c, float a, float b) {
   asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 __device__ __forceinline__ void pin_acc(f32x4 &f) { asm volatile("" : "+a"(f)); }
+// A tile of zeros in the accumulation file by one product of zeros.  (Zeroed by element the compiler copies one register to
+// all others; where this is the second body of a kernel the build's lint cannot tell those copies from a tile moved.)
+__device__ __forceinline__ void zero_tile(f32x16 &c) { asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %1, 0" : "=a"(c) : "v"(0.f)); }
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // Direct loads of the tiles of up to four tensors into stage `stage`, and the addresses of both reads.
@@ -150,13 +153,8 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
   f32x16 Oacc[DB], Tacc[DUAL ? DB : 1];
 #pragma unroll
   for (int db = 0; db < DB; ++db) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      Oacc[db][e] = 0.f;
-      if constexpr (DUAL) Tacc[db][e] = 0.f;
-    }
-    pin_acc(Oacc[db]);
-    if constexpr (DUAL) pin_acc(Tacc[db]);
+    zero_tile(Oacc[db]);
+    if constexpr (DUAL) zero_tile(Tacc[db]);
   }
   float m_i = NEG_INF, l_i = 0.f, mu_i = 0.f;  // l_i, mu_i: this lane's keys
 
