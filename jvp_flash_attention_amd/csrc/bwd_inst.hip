@@ -4,6 +4,7 @@
 // hipStream_t): pre-pass, then the dq and dk/dv kernels of every requested mode.
 #include "bwd_kernel.hpp"
 #include "bwd_kernel_f32.hpp"
+#include "bwd_kernel_f32x3.hpp"
 #include "bwd_kernel_v2.hpp"
 #include "bwd_kernel_wide.hpp"
 #include "bwd_kernel_pair.hpp"
@@ -109,14 +110,22 @@ template <typename T, int D> static void launch_kv_merge(const BwdParams &p, boo
                      p.pr.chunks, elems, tangent ? dkt : dk, tangent ? dvt : dv, dkt, dvt);
 }
 
-// fp32 with D <= 128.
+// The dq and dk/dv kernels for fp32 with D <= 128: up to D = 64 as three bf16 parts.
+template <int D, int MODE, int MASK, bool GO, bool DROP> static auto pick_f32_dq() -> void (*)(const BwdParams) {
+  if constexpr (D <= 64) return bwd_f32x3_dq_kernel<D, MODE, MASK, GO, DROP>;
+  else return bwd_f32_dq_kernel<D, MODE, MASK, GO, DROP>;
+}
+template <int D, int MODE, int MASK, bool GO, bool DROP> static auto pick_f32_dkdv() -> void (*)(const BwdParams) {
+  if constexpr (D <= 64) return bwd_f32x3_dkdv_kernel<D, MODE, MASK, GO, DROP>;
+  else return bwd_f32_dkdv_kernel<D, MODE, MASK, GO, DROP>;
+}
 template <int D, int MODE, int MASK, bool DROP>
 static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blocks, hipStream_t stream) {
   constexpr bool NG = MODE != BWD_DUAL;  // gO may be absent only in the dual mode
   const bool no_go = MODE == BWD_DUAL && p.go == nullptr;
-  void (*kq)(const BwdParams) = no_go ? bwd_f32_dq_kernel<D, MODE, MASK, NG, DROP> : bwd_f32_dq_kernel<D, MODE, MASK, true, DROP>;
-  void (*kkv)(const BwdParams) = no_go ? bwd_f32_dkdv_kernel<D, MODE, MASK, NG, DROP> : bwd_f32_dkdv_kernel<D, MODE, MASK, true, DROP>;
-  using Lds = BwdF32Lds<D, MODE>;
+  void (*kq)(const BwdParams) = no_go ? pick_f32_dq<D, MODE, MASK, NG, DROP>() : pick_f32_dq<D, MODE, MASK, true, DROP>();
+  void (*kkv)(const BwdParams) = no_go ? pick_f32_dkdv<D, MODE, MASK, NG, DROP>() : pick_f32_dkdv<D, MODE, MASK, true, DROP>();
+  using Lds = std::conditional_t<D <= 64, BwdX3Lds<D, MODE>, BwdF32Lds<D, MODE>>;
   int rc = allow_lds(reinterpret_cast<const void *>(kq), Lds::DQ);
   if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), Lds::DKV);
   if (rc != 0) return rc;

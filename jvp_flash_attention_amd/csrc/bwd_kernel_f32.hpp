@@ -1,5 +1,6 @@
 // Backward kernels for fp32, D in {32, 64, 128}, on the forward's direct-to-LDS pipeline (fwd_kernel_f32.hpp: row-major tiles
-// of 32 rows, two stages, one barrier per tile, both reads from the one copy, contraction order chosen for them).
+// of 32 rows, two stages, one barrier per tile, both reads from the one copy, contraction order chosen for them).  Up to D = 64 what
+// bwd_kernel_f32x3.hpp falls back on for gradients that are not finite.
 // Mathematics and modes: bwd_kernel.hpp; statistics arrive negated.  What bounds them: the fp32 matrix rate, 8 (dq) and 10
 // (dk/dv) executed products of which the register-staged kernels these replace reached 60 - 65 %.
 // Measured, B4 H8 L1024 D64 dual with an additive bias per head: dq 325 -> 257 us, dk/dv 432 -> 333 us (87 and 84 % of

@@ -1,4 +1,5 @@
-// Fused dual forward for fp32, D in {32, 64, 128}, on the direct-to-LDS pipeline.
+// Fused dual forward for fp32, D in {32, 64, 128}, on the direct-to-LDS pipeline.  (Up to D = 64 it is what
+// fwd_kernel_f32x3.hpp, faster there, falls back on for outputs that are not finite.)
 //
 // Mathematics and work split as in fwd_kernel.hpp (4 waves = 128 query rows, scores transposed, lane = query).  An fp32
 // matrix instruction (32x32x2) takes 64 cycles for what is 4 of the bf16 one's 32, so a wave has time for everything else

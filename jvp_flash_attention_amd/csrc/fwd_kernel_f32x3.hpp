@@ -16,7 +16,8 @@
 // its workgroup start over with the fp32 instructions, so that every result that is not finite is theirs.
 //
 // Work split and softmax as in fwd_kernel_f32.hpp (4 waves = 128 query rows, 32-key tiles, scores transposed, lane = query).
-// Q, Q' stay resident as parts.  K, V, K', V' tiles go global -> registers (a tile ahead) -> three bf16 planes each in
+// Measured, dual forward at B4 H8 L1024 D64, kernel alone: key padding 201 -> 122 us, bias per head 206 -> 132 us (6 x 25.8
+// GFLOP in 16 bits: 1.2 PFLOP/s).  Q, Q' stay resident as parts.  K, V, K', V' tiles go global -> registers (a tile ahead) -> three bf16 planes each in
 // LDS; splitting there costs a tile's share of every lane once, not every wave once.  One wave per SIMD: a wave hides its
 // vector work itself, one unit of it behind each matrix instruction, in two phases per tile t with one barrier:
 //     A: scores of tile t + 1          with   exponentials, row sums and splitting of P, P S' of tile t
@@ -550,8 +551,8 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
 template <int D, bool DUAL> struct X3Lds {
   static constexpr size_t FWD = 2 * (size_t)(DUAL ? 4 : 2) * X3Cfg<D>::OPB;  // (more than the fp32 tiles take)
 };
-template <int D, bool DUAL, int MASK, bool DROP>
-__global__ __launch_bounds__(256, 1) void fwd_f32x3_kernel(const FwdParams p) {
+template <int D, bool DUAL, int MASK, bool DROP, int WGS = DUAL ? 1 : 2>
+__global__ __launch_bounds__(256, WGS) void fwd_f32x3_kernel(const FwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   if (!fwd_f32x3_body<D, DUAL, MASK, DROP>(p)) fwd_f32_body<D, DUAL, MASK, DROP>(p);
 #endif
