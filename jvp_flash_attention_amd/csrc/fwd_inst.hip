@@ -60,7 +60,9 @@ static int launch_fwd2_one(const FwdParams &p, hipStream_t stream) {
 template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false>
 static int launch_fwd3_one(const FwdParams &p, hipStream_t stream) {
   using Cfg = Fwd2Cfg<T, D, DUAL>;
-  auto kern = fwd3_kernel<T, D, DUAL, MASK, DROP>;
+  void (*kern)(const FwdParams);
+  if constexpr (D == 64 && DUAL) kern = fwd3_kernel_2wg<T, D, DUAL, MASK, DROP>;
+  else kern = fwd3_kernel<T, D, DUAL, MASK, DROP>;
   int rc = allow_lds(reinterpret_cast<const void *>(kern), Cfg::LDS_BYTES);
   if (rc != 0) return rc;
   const int nqb = (p.pr.L + Cfg::BM - 1) / Cfg::BM;
@@ -164,7 +166,13 @@ static int launch_fwd_mask(const FwdParams &p, int mask, hipStream_t stream) {
     return -3;
   } else if constexpr (sizeof(T) == 2 && D < 128) {
     switch (mask) {
-      case MASK_NONE: return launch_fwd2_one<T, D, DUAL, MASK_NONE>(p, stream);
+      case MASK_NONE:
+        // D = 64: the pipelined kernel with tangents, from 8 key tiles on (filling and draining it costs two of them), and
+        // wherever the keys are split, which it alone can.  Two workgroups of either share a compute unit.
+        if constexpr (D == 64) {
+          if (p.pr.chunks > 1 || (DUAL && p.pr.Lk >= 512)) return launch_fwd3_one<T, D, DUAL, MASK_NONE>(p, stream);
+        }
+        return launch_fwd2_one<T, D, DUAL, MASK_NONE>(p, stream);
       case MASK_BOOL: return p.pr.bits_q ? launch_fwd2_one<T, D, DUAL, MASK_BITS>(p, stream) : launch_fwd2_one<T, D, DUAL, MASK_BOOL>(p, stream);
       case MASK_ADD: return launch_fwd2_one<T, D, DUAL, MASK_ADD>(p, stream);
     }

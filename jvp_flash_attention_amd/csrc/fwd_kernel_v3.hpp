@@ -1,5 +1,5 @@
-// Software-pipelined fused dual forward for 16-bit element types at D = 128 (and the forward without tangents
-// at D = 256): causal, boolean and additive masks (with the key limit and the tile lists), ragged sequence ends, dropout.  Same tiles,
+// Software-pipelined fused dual forward for 16-bit element types at D = 128 (the forward without tangents at D = 256 as well,
+// and at D = 64 the dual forward of longer rows and both forwards of split launches): causal, boolean and additive masks (with the key limit and the tile lists), ragged sequence ends, dropout.  Same tiles,
 // swizzles, fragment layouts and mathematics as fwd_kernel_v2.hpp; what changes is the order of work
 // inside a wave.
 //
@@ -49,10 +49,12 @@ template <int N> __device__ __forceinline__ void lds_wait3(u32x4 &a, u32x2 &c, u
 // WGS: workgroups meant to share a compute unit.  Without tangents at D = 128, Q and the accumulator are 96
 // registers and a stage pair 64 KB, so two fit; the unmasked kernel stays within 256 registers by itself, the
 // masked ones are told to.
-template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false,
-          int WGS = (!DUAL && D <= 128 && (MASK != MASK_NONE || DROP)) ? 2 : 1>
-__global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
-#if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub (and has no buffer descriptor type)
+#if defined(__HIP_DEVICE_COMPILE__)
+// TIGHT: a third fewer registers for fragments.  Score fragments are read one super-step ahead instead of three, V fragments at
+// the top of their own super-step, behind whose score products they arrive.  For two workgroups on a compute unit, each of
+// which covers the other's waits.
+template <typename T, int D, bool DUAL, int MASK, bool DROP, bool TIGHT>
+__device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   using Cfg = Fwd2Cfg<T, D, DUAL>;
   constexpr int BN = Cfg::BN, CH = Cfg::CH, ROWB = Cfg::ROWB, TILEB = Cfg::TILEB, IPW = Cfg::IPW;
   constexpr int KK = D / 16, DB = D / 32;
@@ -267,7 +269,7 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
   constexpr int NRS = DUAL ? 2 : 1, NRV = DUAL ? 4 : 2;  // LDS reads per super-step
   constexpr int NU = 38;                                 // vector units of one softmax
   constexpr int NU0 = 5;                                 // ... of which this many form its front
-  constexpr int RD = 4, PD = RD - 1;           // fragment ring slots; reads run PD super-steps ahead
+  constexpr int RD = TIGHT ? 2 : 4, PD = RD - 1;           // fragment ring slots; reads run PD super-steps ahead
 
   // One slot.  QK: scores of a half tile (K rows at LDS address kaddr) into Sn, Spn.  PV: accumulate
   // the half tile whose V rows are at vaddr, with fragments pfp, psfp.  SM: softmax of Sc, Spc (first
@@ -279,7 +281,8 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
   // 16 c + 8 g .. + 7 in mah[c]; keys past the end come masked from the fetch).
   // LB: index of the first load step of this slot, or -1.
   u32x4 ka[RD], kb[RD];
-  u32x2 va[RD][2], vb[RD][2];
+  constexpr int RDV = TIGHT ? 1 : RD;  // TIGHT: V fragments are read behind the score products of their own super-step
+  u32x2 va[RDV][2], vb[RDV][2];
   auto slot = [&](auto QKc, auto PVc, auto SMc, auto GENc, auto LBc, auto PREc, auto NEXTc, uint32_t kaddr, uint32_t vaddr, f32x16 &Sc,
                   f32x16 &Spc, f32x16 &Sn, f32x16 &Spn, Frag<T>(&pfp)[2], Frag<T>(&psfp)[2], Frag<T>(&pfn)[2],
                   Frag<T>(&psfn)[2], int jh, const MaskAhead<T, MASK>(&mah)[2], float (&madd)[16]) {
@@ -424,7 +427,7 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
 
     // ---- fragment reads --------------------------------------------------------------------------
     // step NSS + j is step j of the next slot (rows 32 further down in the same tiles)
-    auto issue = [&](auto ic) {
+    auto issue_k = [&](auto ic) {
       constexpr int i = decltype(ic)::value % NSS, sl = i % RD;
       constexpr int HO = (decltype(ic)::value / NSS) * 32 * ROWB;
       if constexpr (QK) {
@@ -432,6 +435,10 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
         ka[sl] = lds_b128<HO>(ad);
         if constexpr (DUAL) kb[sl] = lds_b128<HO + 2 * TILEB>(ad);
       }
+    };
+    auto issue_v = [&](auto ic) {
+      constexpr int i = decltype(ic)::value % NSS, sl = i % RDV;
+      constexpr int HO = (decltype(ic)::value / NSS) * 32 * ROWB;
       if constexpr (PV) {
         constexpr int c = i / DB, db = i % DB;
         constexpr int VO = HO + TILEB + c * 16 * ROWB;
@@ -445,6 +452,10 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
         }
       }
     };
+    auto issue = [&](auto ic) {
+      issue_k(ic);
+      if constexpr (!TIGHT) issue_v(ic);
+    };
 
     if constexpr (SM) {
       if constexpr (DUAL) tiles_ready(Sc, Spc);
@@ -456,7 +467,13 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
     static_for<NSS>([&](auto ic) {
       constexpr int i = decltype(ic)::value, sl = i % RD;
       constexpr int younger = (NEXT ? PD - 1 : ((NSS - 1 - i < PD - 1) ? NSS - 1 - i : PD - 1)) * RPS;
-      if constexpr (QK && PV) {
+      if constexpr (TIGHT) {
+        if constexpr (QK) {
+          if constexpr (DUAL) lds_wait<0>(ka[sl], kb[sl]);
+          else lds_wait<0>(ka[sl]);
+        }
+        issue_v(ic);
+      } else if constexpr (QK && PV) {
         if constexpr (DUAL) lds_wait6<younger>(ka[sl], kb[sl], va[sl][0], va[sl][1], vb[sl][0], vb[sl][1]);
         else lds_wait3<younger>(ka[sl], va[sl][0], va[sl][1]);
       } else if constexpr (QK) {
@@ -466,7 +483,8 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
         if constexpr (DUAL) lds_wait<younger>(va[sl][0], va[sl][1], vb[sl][0], vb[sl][1]);
         else lds_wait<younger>(va[sl][0], va[sl][1]);
       }
-      if constexpr (i + PD < NSS || NEXT) issue(std::integral_constant<int, i + PD>{});
+      constexpr bool MORE = i + PD < NSS || NEXT;
+      if constexpr (MORE) issue(std::integral_constant<int, i + PD>{});
       if constexpr (LB >= 0) load_step(std::integral_constant<int, (LB >= 0 ? LB : 0) + i>{});
       constexpr int c = i / DB, db = i % DB;
       constexpr int G0 = i * MPS;
@@ -475,18 +493,41 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
         fa = __builtin_bit_cast(Frag<T>, ka[sl]);
         if constexpr (DUAL) fb = __builtin_bit_cast(Frag<T>, kb[sl]);
       }
-      if constexpr (PV) {
-        const u32x4 av = {va[sl][0][0], va[sl][0][1], va[sl][1][0], va[sl][1][1]};
-        fv = __builtin_bit_cast(Frag<T>, av);
-        if constexpr (DUAL) {
-          const u32x4 bv = {vb[sl][0][0], vb[sl][0][1], vb[sl][1][0], vb[sl][1][1]};
-          fw = __builtin_bit_cast(Frag<T>, bv);
+      auto take_v = [&]() {
+        constexpr int sv_ = i % RDV;
+        if constexpr (TIGHT && PV) {
+          constexpr int y = QK && MORE ? NRS : 0;  // the score fragments requested behind them
+          if constexpr (DUAL) lds_wait<y>(va[sv_][0], va[sv_][1], vb[sv_][0], vb[sv_][1]);
+          else lds_wait<y>(va[sv_][0], va[sv_][1]);
         }
-      }
+        if constexpr (PV) {
+          const u32x4 av = {va[sv_][0][0], va[sv_][0][1], va[sv_][1][0], va[sv_][1][1]};
+          fv = __builtin_bit_cast(Frag<T>, av);
+          if constexpr (DUAL) {
+            const u32x4 bv = {vb[sv_][0][0], vb[sv_][0][1], vb[sv_][1][0], vb[sv_][1][1]};
+            fw = __builtin_bit_cast(Frag<T>, bv);
+          }
+        }
+      };
+      if constexpr (!TIGHT || !QK) take_v();
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (DUAL) {
         // order: no two consecutive matrix instructions update the same tile
-        if constexpr (QK && PV) {
+        if constexpr (QK && PV && TIGHT) {
+          mfma_s<i == 0>(Spn, fa, Qtf[i]);
+          gap(std::integral_constant<int, G0 + 0>{});
+          mfma_s<i == 0>(Sn, fa, Qf[i]);
+          gap(std::integral_constant<int, G0 + 1>{});
+          mfma_s<false>(Spn, fb, Qf[i]);
+          gap(std::integral_constant<int, G0 + 2>{});
+          take_v();
+          mfma_acc(Tacc[db], fv, psfp[c]);
+          gap(std::integral_constant<int, G0 + 3>{});
+          mfma_acc(Oacc[db], fv, pfp[c]);
+          gap(std::integral_constant<int, G0 + 4>{});
+          mfma_acc(Tacc[db], fw, pfp[c]);
+          gap(std::integral_constant<int, G0 + 5>{});
+        } else if constexpr (QK && PV) {
           mfma_s<i == 0>(Spn, fa, Qtf[i]);
           gap(std::integral_constant<int, G0 + 0>{});
           mfma_acc(Oacc[db], fv, pfp[c]);
@@ -520,6 +561,7 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
           gap(std::integral_constant<int, G0 + 0>{});
         }
         if constexpr (PV) {
+          if constexpr (TIGHT && QK) take_v();
           mfma_acc(Oacc[db], fv, pfp[c]);
           gap(std::integral_constant<int, G0 + (QK ? 1 : 0)>{});
         }
@@ -730,6 +772,25 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
       if constexpr (DUAL) p.mu[(size_t)zh * L + qrow] = dead ? 0.f : mu_n + c_i;  // mu_n = rowsum(P (S' - c))
     }
   }
+}
+#endif
+template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false,
+          int WGS = (!DUAL && D <= 128 && (MASK != MASK_NONE || DROP)) ? 2 : 1>
+__global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub (and has no buffer descriptor type)
+  fwd3_body<T, D, DUAL, MASK, DROP, false>(p);
+#endif
+}
+// D = 64 with tangents: 96 accumulation registers (Q, Q', O, O'), so with 160 others two workgroups share a compute unit.  Unlike
+// fwd2_kernel, whose two waves per SIMD each alternate between matrix and vector phases (and meet in the same phase often
+// enough to take 6500 cycles for 3100 of matrix work per tile), each wave mixes them by itself.  bf16, dual forward, fwd2_kernel -> this:
+// B4 H16 L2048 191.5 -> 186.4 us, causal 112.4 -> 106.4; B2 H16 L1024 35.5 -> 32.5; B4 H16 L4096 730 -> 706, causal 389 -> 377;
+// fp16 L2048 202.7 -> 198.0.  (Without tangents, and with dropout, the same change is 1 - 4 % slower: three waves of fwd2_kernel
+// share a SIMD there.  With masks it takes 258 - 284 registers.)
+template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false>
+__global__ __launch_bounds__(256, 1) __attribute__((amdgpu_num_vgpr(160))) void fwd3_kernel_2wg(const FwdParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  fwd3_body<T, D, DUAL, MASK, DROP, true>(p);
 #endif
 }
 
