@@ -108,7 +108,7 @@ typedef struct jvpfa_fwd_args {
    * 16-byte aligned, contents don't-care.  When a launch would have fewer workgroups than the GPU has compute
    * units (one long sequence, few heads), the key tiles of every query block are then split over up to 8
    * workgroups that leave fp32 partial results there, and a second kernel merges them into o, ot, M, mu
-   * (bf16 / fp16, D = 128, no mask; ignored otherwise).  Results agree with the unsplit launch to rounding.
+   * (bf16 / fp16, D = 64 or 128, no mask; ignored otherwise).  Results agree with the unsplit launch to rounding.
    * No counterpart in the reference (one program per 32 query rows whatever the grid, JA:2474-2476). */
   void *split_workspace;
   uint64_t split_workspace_bytes;

@@ -35,7 +35,7 @@ struct Problem {
   // Split of the streamed tiles of one block of owned rows over `chunks` workgroups (1 = no split), used when
   // a launch would otherwise leave most compute units idle: workgroup c of a block takes the tiles
   // c * chunk_tiles .. (c + 1) * chunk_tiles - 1 and writes fp32 partial results to `part`, which a merge
-  // kernel adds up.  Only the kernels for 16-bit element types, D = 128, without a mask.
+  // kernel adds up.  Only the kernels for 16-bit element types, D = 64 or 128, without a mask.
   // In the backward: the query heads of a key/value head's group are dealt to `chunks` dk/dv workgroups (see
   // split.hpp), each of which leaves its share of the gradients in `part`.
   int chunks, chunk_tiles;

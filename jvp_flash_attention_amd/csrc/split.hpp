@@ -1,5 +1,5 @@
 // Small grids: when a launch has fewer workgroups than the GPU has compute units (one sequence of a few
-// thousand tokens, a handful of heads), the kernels for 16-bit element types with D = 128 and no mask split
+// thousand tokens, a handful of heads), the kernels for 16-bit element types with D = 64 or 128 and no mask split
 // the streamed tiles of every block of owned rows over several workgroups ("chunks").  Each writes fp32
 // partial results to a workspace and a merge kernel combines them with the online-softmax merge (every running
 // quantity is linear in p once the reference points m and c are made common).  The backward of such a launch runs
@@ -55,18 +55,24 @@ inline int device_cus() {
 // Workspace of the forward: per chunk and query row 2 D accumulator values (O, T, not yet divided by l) and
 // four statistics (m, l, mu_acc, c).
 inline size_t fwd_part_floats(int chunks, long long rows, int D) { return (size_t)chunks * rows * (2 * (size_t)D + 4); }
-// The kernels that can split: 16-bit element types, D = 128, no mask (the software-pipelined forward and the
-// direct-to-LDS backward kernels).  Tiles are 64 wide, blocks 128 rows.
+// The kernels that can split: 16-bit element types, D = 64 or 128, no mask (the software-pipelined forward).  Tiles are 64
+// wide, blocks 128 rows.
 template <typename P> inline bool split_capable(const P &p) {
-  return p.dtype != 2 && p.D == 128 && p.mask_kind == 0 && !(p.dropout_p > 0.f);
+  return p.dtype != 2 && (p.D == 128 || p.D == 64) && p.mask_kind == 0 && !(p.dropout_p > 0.f);
 }
-template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk) {
+template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk, bool dual) {
   SplitPlan none = {1, 0};
   if (!split_capable(p)) return none;
   const long long blocks = (long long)((p.L + 127) / 128) * p.Z * p.H;
   int keys = Lk;  // of the longest query block (causal: the last one sees keys up to its own last row)
   if (p.causal && ((p.L + 127) / 128) * 128 < keys) keys = ((p.L + 127) / 128) * 128;
-  return split_plan(blocks, (keys + 63) / 64, device_cus());
+  const int ntiles = (keys + 63) / 64;
+  // D = 64: a tile takes half the time (1.8 us with tangents, 0.9 without), so what a split costs, 8 - 10 us with the merge, is
+  // worth it from 16 or 32 tiles on (with fewer it is slower, L512 plain 10.8 -> 12.1).  Measured, bf16 B1, unsplit -> split, dual
+  // and plain: H4 L1024 34 -> 28 and 18 -> unsplit (19); H4 L2048 62 -> 33 and 32 -> 21; H8 L2048 63 -> 42 and 33 -> 26;
+  // H2 L4096 118 -> 44 and 61 -> 28; H4 L4096 119 -> 66 and 61 -> 40.
+  if (p.D == 64 && ntiles < (dual ? 16 : 32)) return none;
+  return split_plan(blocks, ntiles, device_cus());
 }
 
 // Backward with grouped heads.  A dk/dv workgroup owns 128 keys of a key/value head and works through the query heads

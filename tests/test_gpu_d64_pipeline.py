@@ -1,4 +1,6 @@
 """The pipelined forward at D = 64: rows around its shortest length, tile ends, and keys split over workgroups."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -38,3 +40,21 @@ def test_tile_ends(dt, L, Lk, causal):
     for scale in (0.125, -0.3):
         _, ref, got = run(dt, 2, 18, 9, L, Lk, causal, True, scale) if L < 200 else run(dt, 3, 16, 16, L, Lk, causal, True, scale)
         check(got, ref, True)
+
+
+@pytest.mark.parametrize("dual", [True, False])
+@pytest.mark.parametrize("Z,H,Hk,L,Lk,causal", [(1, 1, 1, 1000, 1024, False), (1, 2, 1, 300, 1025, False), (1, 2, 2, 2100, 2100, True), (2, 1, 1, 64, 4100, False)])
+def test_keys_split_over_workgroups(dual, Z, H, Hk, L, Lk, causal):
+    dev, ref, got = run("bf16", Z, H, Hk, L, Lk, causal, dual)
+    check(got, ref, dual)
+    p = _lib.make_problem(dev[0], None, _lib.MASK_NONE, causal, 0.125)
+    assert _lib.load().jvpfa_fwd_split_workspace_bytes(C.byref(p), Lk) > 0
+    _lib.set_split(False)
+    try:
+        one = _lib.backend().fwd(*dev, None, _lib.MASK_NONE, causal, 0.125)
+    finally:
+        _lib.set_split(True)
+    assert (got[2] - one[2]).abs().max().item() <= 1e-5
+    for a, b in zip(got[:2], one[:2]):
+        if a is not None:  # one rounding of the element type apart
+            assert ((a.float() - b.float()).abs() <= 2 * 2.0**-7 * b.float().abs().clamp_min(1.0)).all()
