@@ -56,6 +56,12 @@ template <int N> __device__ __forceinline__ void lds_wait(FragT &a, FragT &b, Fr
                : "+v"(a.lo), "+v"(a.hi), "+v"(b.lo), "+v"(b.hi), "+v"(c.lo), "+v"(c.hi), "+v"(d.lo), "+v"(d.hi)
                : "n"(N));
 }
+template <int N> __device__ __forceinline__ void lds_wait(FragN &a, FragN &b, FragN &c) {
+  asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(a.v), "+v"(b.v), "+v"(c.v) : "n"(N));
+}
+template <int N> __device__ __forceinline__ void lds_wait(FragT &a, FragT &b, FragT &c) {
+  asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(a.lo), "+v"(a.hi), "+v"(b.lo), "+v"(b.hi), "+v"(c.lo), "+v"(c.hi) : "n"(N));
+}
 // A score-sized tile from four quads that a wait already passed covers: tied behind it, register e = quad e / 4, entry e % 4.
 __device__ __forceinline__ f32x16 tile_of(u32x4 (&q)[4]) {
   asm volatile("" : "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3]));
@@ -589,6 +595,10 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
     }
   }
   constexpr bool has_go = GO;  // compile-time: a run-time test here would split every step into its own block
+  // Gradients of O' alone: there is no tile of gO to load or read (its slot in a stage stays empty).  With gT in its place a
+  // quarter of the loads and LDS reads fetched what no product took: bf16, backward, B1 H16 L8192 D128 causal 1804 -> 1771 us,
+  // B4 H16 L2048 D128 912 -> 892, D64 479 -> 473, D32 307 -> 297.
+  constexpr bool NO_G = DUAL && !GO;
   const uint32_t stat0 = lds0 + 2 * Cfg::STAGEB;  // row statistics, two stages of NSTAT x 64 floats
 
   Frag<T> Kf[KK], Vf[KK], Ktf[DUAL ? KK : 1], Vtf[DUAL ? KK : 1];
@@ -740,7 +750,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   auto load_any = [&](auto pc) {
     constexpr int pi = decltype(pc)::value;
     if constexpr (pi < NLOAD) {
-      load_piece(pc);
+      if constexpr (!(NO_G && pi % Cfg::NTILE == 1)) load_piece(pc);
     } else {
       constexpr int i = pi - NLOAD;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(mt_rs, (JVPFA_LDS(void))(uintptr_t)(mt_dst + i * 1024), 16, mt_o[i], 0, 0, 0);
@@ -816,13 +826,13 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
       constexpr int kk = decltype(kkc)::value, sl = SAHEAD ? kk % 2 : 0;
       const uint32_t ad = sbase + noff[kk];
       fq[sl].v = lds_b128<RO>(ad);
-      fg[sl].v = lds_b128<RO + TILEB>(ad);
+      if constexpr (!NO_G) fg[sl].v = lds_b128<RO + TILEB>(ad);
       if constexpr (DUAL) {
         fqt[sl].v = lds_b128<RO + 2 * TILEB>(ad);
         fgt[sl].v = lds_b128<RO + 3 * TILEB>(ad);
       }
     };
-    constexpr int NRN = DUAL ? 4 : 2;
+    constexpr int NRN = DUAL ? (NO_G ? 3 : 4) : 2;
     // mask values of this lane's key for the 32 queries of the half tile (register e <-> query
     // 16(e/8) + 8g + e%8): requested one half tile earlier (see fetch_mask_half), taken over here
     T mraw_a[MASK == MASK_ADD ? 16 : 1];
@@ -877,14 +887,17 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
       if constexpr (!SAHEAD) issue_n(std::integral_constant<int, kk>{});
       else if constexpr (kk + 1 < KK) issue_n(std::integral_constant<int, kk + 1>{});
       constexpr int younger_n = (SAHEAD && kk + 1 < KK) ? NRN : 0;
-      if constexpr (DUAL) lds_wait<younger_n>(fq[sl], fg[sl], fqt[sl], fgt[sl]);
+      if constexpr (NO_G) lds_wait<younger_n>(fq[sl], fqt[sl], fgt[sl]);
+      else if constexpr (DUAL) lds_wait<younger_n>(fq[sl], fg[sl], fqt[sl], fgt[sl]);
       else lds_wait<younger_n>(fq[sl], fg[sl]);
       if constexpr (INIT && F) {  // (older than the fragments just waited for)
         if constexpr (DUAL || TAN) At = tile_of(ia);
         if constexpr (DUAL || MODE == BWD_PLAIN) dP = tile_of(idp);
       }
       load_step(std::integral_constant<int, HB * KK + kk>{});
-      const Frag<T> q_ = as_frag<T>(fq[sl]), g_ = as_frag<T>(fg[sl]);
+      const Frag<T> q_ = as_frag<T>(fq[sl]);
+      Frag<T> g_;
+      if constexpr (!NO_G) g_ = as_frag<T>(fg[sl]);
       mma_vra<F>(S, q_, Kf[kk]);
       constexpr bool FI = F && !INIT;
       if constexpr (MODE == BWD_PLAIN) mma_vra<FI>(dP, g_, Vf[kk]);
@@ -940,8 +953,10 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
       const uint32_t a0 = sbase + toff[db][0], a1 = sbase + toff[db][1];
       tq[sl].lo = lds_tr64<TO>(a0);
       tq[sl].hi = lds_tr64<TO>(a1);
-      tg[sl].lo = lds_tr64<TO + TILEB>(a0);
-      tg[sl].hi = lds_tr64<TO + TILEB>(a1);
+      if constexpr (!NO_G) {
+        tg[sl].lo = lds_tr64<TO + TILEB>(a0);
+        tg[sl].hi = lds_tr64<TO + TILEB>(a1);
+      }
       if constexpr (DUAL) {
         tqt[sl].lo = lds_tr64<TO + 2 * TILEB>(a0);
         tqt[sl].hi = lds_tr64<TO + 2 * TILEB>(a1);
@@ -949,7 +964,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
         tgt[sl].hi = lds_tr64<TO + 3 * TILEB>(a1);
       }
     };
-    constexpr int NRT = DUAL ? 8 : 4;
+    constexpr int NRT = DUAL ? (NO_G ? 6 : 8) : 4;
     if constexpr (SAHEAD) issue_s(std::integral_constant<int, 0>{});
     Frag<T> mfr[2];
     if constexpr (MASK == MASK_TILE && Cfg::MTILE_SINGLE) {
@@ -1034,7 +1049,8 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
         if constexpr (!SAHEAD) issue_t(std::integral_constant<int, i>{});
         else if constexpr (db + 1 < DB) issue_t(std::integral_constant<int, i + 1>{});
         constexpr int younger = (SAHEAD && db + 1 < DB) ? NRT : 0;
-        if constexpr (DUAL) lds_wait<younger>(tq[sl], tg[sl], tqt[sl], tgt[sl]);
+        if constexpr (NO_G) lds_wait<younger>(tq[sl], tqt[sl], tgt[sl]);
+        else if constexpr (DUAL) lds_wait<younger>(tq[sl], tg[sl], tqt[sl], tgt[sl]);
         else lds_wait<younger>(tq[sl], tg[sl]);
         load_step(std::integral_constant<int, 2 * KK + HB * NPV + i>{});
         if constexpr (MODE == BWD_PLAIN) {
