@@ -100,6 +100,68 @@ template <typename T, int D, int MODE, int MASK, bool DROP> static auto pick_wid
   return bwdw_dkdv_kernel<T, D, MODE, MASK, DROP, true>;
 }
 
+// Whether dk/dv and dq go into one launch (bwd2_both_kernel): it has one end with idle compute units instead of two, and where a
+// kernel has to take both roles' registers fewer of its workgroups share a unit.  So: up to a number of blocks (in units of
+// compute units) that depends on how many do.  two_wgs: bwd2_both_kernel_2wg runs it.
+// D = 128 (one workgroup a unit either way, but for the dq kernel without tangents): causal and masked launches up to 2.5; others
+// where the launches would round up to more passes over the units than the one does, 0.6 of a pass for its end.
+// Measured, bf16, backward, two launches -> one, 288 / 544 / 704 / 1024 - 1152 blocks (dual unless said): D128 269 -> 205, 721 ->
+// 607, 490 -> 492, 1236 -> 1135 us, causal 139 -> 111, 323 -> 316, 295 -> 290; plain 123 -> 100, 332 -> 285, 233 -> 237;
+// D64 (2wg) causal 1024 blocks 314 -> 300, 1152 without a mask 731 -> 677, 1536 615 -> 602; D64 plain 69 -> 54, 164 -> 147,
+// 121 -> 118, 260 -> 245 us, 2048 blocks 471 -> 479; D32 88 -> 81, 253 -> 196, 171 -> 155, 462 -> 415, 2048 blocks 658 -> 644.
+// Where it loses: dropout at D64 plain 704 blocks, whole step 168 -> 206; D32 dual 343 -> 409; six gradients there 267 -> 299.
+template <int D, int MODE>
+static bool launch_both(long long blocks, long long kv_blocks, bool causal, bool masked, bool drop, bool six, bool grouped, bool two_wgs) {
+  const long long most = blocks > kv_blocks ? blocks : kv_blocks, cus = device_cus();
+  if (D == 32) return most <= (drop ? (MODE == BWD_DUAL ? 1.5 : 2.5) : six ? 2.2 : 8.0) * cus;
+  if (D == 64 && MODE == BWD_DUAL) return most <= (six ? 2.5 : two_wgs || drop ? 8.0 : 2.75) * cus;
+  if (D == 64) return most <= (drop ? 1.5 : grouped ? 6.0 : 4.5) * cus;
+  if (most <= cus || ((causal || masked) && most <= 2.5 * cus)) return true;
+  const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
+  return apart > (MODE == BWD_DUAL ? 1.04 : 1.08) * ((double)(blocks + kv_blocks) / cus + 0.6);
+}
+static int run_both(void (*kb)(const BwdParams, int), const BwdParams &p, long long kv_blocks, long long total, size_t lds, hipStream_t stream) {
+  if (total > 0x7fffffffLL) return -2;
+  const int rc = allow_lds(reinterpret_cast<const void *>(kb), lds);
+  if (rc != 0) return rc;
+  hipLaunchKernelGGL(kb, dim3((unsigned)total), dim3(256), lds, stream, p, (int)kv_blocks);
+  return hipGetLastError() == hipSuccess ? 0 : -6;
+}
+// The kernel for one launch of everything that is asked for (without dropout), or null where two are better or no such kernel
+// exists: six gradients and grouped heads without a mask or (six gradients) with a packed one.
+template <typename T, int D, int MODE, int MASK>
+static auto pick_both(const BwdParams &p, bool no_go, bool grouped, bool six, long long blocks, long long kv_blocks) -> void (*)(const BwdParams, int) {
+  constexpr bool NG = MODE != BWD_DUAL;
+  const bool bits = MASK == MASK_BOOL && p.pr.bits_q && p.pr.bits_k;
+  constexpr bool M = MASK != MASK_NONE;
+  const bool causal = p.pr.causal != 0, two_wgs = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits);
+  // (six: the dual and the tangent launch of a call decide alike)
+  if (!(six ? launch_both<D, BWD_DUAL>(blocks, kv_blocks, causal, M, false, true, grouped, false)
+            : launch_both<D, MODE>(blocks, kv_blocks, causal, M, false, false, grouped, two_wgs)))
+    return nullptr;
+  if constexpr (MASK == MASK_ADD) {  // (read element by element here, and as tiles by the dk/dv kernel of its own launch)
+    if (blocks >= device_cus() || kv_blocks >= device_cus()) return nullptr;
+  }
+  if (grouped) {
+    if (six) return nullptr;
+    if constexpr (MASK == MASK_NONE) return no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG, true> : bwd2_both_kernel<T, D, MODE, MASK, true, true>;
+    return nullptr;
+  }
+  if (six) {
+    if (!(MASK == MASK_NONE || bits)) return nullptr;
+    constexpr int MK = MASK == MASK_BOOL ? MASK_BITS : MASK_NONE;
+    if constexpr (D == 128) return no_go ? bwd2_all_kernel<T, D, MK, false> : bwd2_all_kernel<T, D, MK, true>;
+    else return no_go ? bwd2_both_kernel<T, D, BWD_DUAL, MK, false, false, true> : bwd2_both_kernel<T, D, BWD_DUAL, MK, true, false, true>;
+  }
+  if constexpr (D == 64 && MODE == BWD_DUAL && MASK != MASK_ADD) {
+    constexpr int MK = MASK == MASK_BOOL ? MASK_BITS : MASK_NONE;
+    if (two_wgs) return no_go ? bwd2_both_kernel_2wg<T, D, MODE, MK, NG> : bwd2_both_kernel_2wg<T, D, MODE, MK, true>;
+  } else if constexpr (MASK == MASK_BOOL) {
+    if (bits) return no_go ? bwd2_both_kernel<T, D, MODE, MASK_BITS, NG> : bwd2_both_kernel<T, D, MODE, MASK_BITS, true>;
+  }
+  return no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG> : bwd2_both_kernel<T, D, MODE, MASK, true>;
+}
+
 // Adds up the shares of dk, dv (dk', dv' of the tangent mode; all four where the dual kernel folds them in) that a
 // launch over pr.chunks query heads groups left, see split.hpp.
 template <typename T, int D> static void launch_kv_merge(const BwdParams &p, bool tangent, bool four, hipStream_t stream) {
@@ -154,6 +216,17 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       const bool no_go = MODE == BWD_DUAL && p.go == nullptr;
       constexpr bool NG = MODE != BWD_DUAL;
       const bool grouped = p.pr.Hk != p.pr.H;
+      if constexpr (MASK == MASK_NONE) {
+        if (launch_both<D, MODE>(blocks, kv_blocks, p.pr.causal != 0, false, true, false, grouped, false)) {
+          void (*kb)(const BwdParams, int);
+          if (grouped) kb = no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG, true, false, true> : bwd2_both_kernel<T, D, MODE, MASK, true, true, false, true>;
+          else kb = no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG, false, false, true> : bwd2_both_kernel<T, D, MODE, MASK, true, false, false, true>;
+          const int rc = run_both(kb, p, kv_blocks, kv_blocks + blocks, Cfg2::DKV_LDS > Cfg2::DQ_LDS ? Cfg2::DKV_LDS : Cfg2::DQ_LDS, stream);
+          if (rc != 0) return rc;
+          launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
+          return hipGetLastError() == hipSuccess ? 0 : -6;
+        }
+      }
       void (*kq)(const BwdParams) = no_go ? bwd2_dq_kernel<T, D, MODE, MASK, NG, false, true> : bwd2_dq_kernel<T, D, MODE, MASK, true, false, true>;
       size_t kv_lds = 0;
       void (*kkv)(const BwdParams) = pick_dkdv_for<T, D, MODE, MASK>(p, no_go, grouped, false, true, &kv_lds);
@@ -225,17 +298,14 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     }
     size_t kv_lds = 0;
     kkv = pick_dkdv_for<T, D, MODE, MASK>(p, no_go, grouped, MODE == BWD_DUAL && six, false, &kv_lds);
-    // a grid smaller than the GPU: both roles in one launch, side by side
-    const int cus = device_cus();
-    if (!grouped && !six && blocks < cus && kv_blocks < cus) {
-      void (*kb)(const BwdParams, int) = no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG> : bwd2_both_kernel<T, D, MODE, MASK, true>;
-      if constexpr (MASK == MASK_BOOL) {
-        if (p.pr.bits_q && p.pr.bits_k) kb = no_go ? bwd2_both_kernel<T, D, MODE, MASK_BITS, NG> : bwd2_both_kernel<T, D, MODE, MASK_BITS, true>;
+    if (auto kb = pick_both<T, D, MODE, MASK>(p, no_go, grouped, six, blocks, kv_blocks)) {
+      if constexpr (MODE == BWD_TANGENT) {
+        if (six) return 0;  // the dual launch has made all six
       }
-      constexpr size_t LDS = Cfg2::DKV_LDS > Cfg2::DQ_LDS ? Cfg2::DKV_LDS : Cfg2::DQ_LDS;
-      const int rcb = allow_lds(reinterpret_cast<const void *>(kb), LDS);
+      constexpr bool ALL = D == 128 && MODE == BWD_DUAL;  // then dk', dv' have workgroups of their own
+      const int rcb = run_both(kb, p, kv_blocks, (ALL && six ? 2 : 1) * kv_blocks + blocks, Cfg2::DKV_LDS > Cfg2::DQ_LDS ? Cfg2::DKV_LDS : Cfg2::DQ_LDS, stream);
       if (rcb != 0) return rcb;
-      hipLaunchKernelGGL(kb, dim3((unsigned)(kv_blocks + blocks)), dim3(Cfg2::NT), LDS, stream, p, (int)kv_blocks);
+      launch_kv_merge<T, D>(p, MODE == BWD_TANGENT, false, stream);
       return hipGetLastError() == hipSuccess ? 0 : -6;
     }
     int rc = allow_lds(reinterpret_cast<const void *>(kq), Cfg2::DQ_LDS);
@@ -256,6 +326,13 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     const long long kblocks = (long long)((p.pr.Lk + CfgP::BLK - 1) / CfgP::BLK) * p.pr.Z * p.pr.Hk * p.pr.chunks;
     if (qblocks > 0x7fffffffLL || kblocks > 0x7fffffffLL) return -2;
     void (*kq)(const BwdParams) = no_go ? bwdp_dq_kernel<T, D, MASK, false> : bwdp_dq_kernel<T, D, MASK, true>;
+    if (!six && launch_both<D, MODE>(qblocks, kblocks, p.pr.causal != 0, MASK != MASK_NONE, false, false, false, false)) {
+      void (*kb)(const BwdParams, int) = no_go ? bwdp_both_kernel<T, D, MASK, false> : bwdp_both_kernel<T, D, MASK, true>;
+      const int rcb = run_both(kb, p, kblocks, kblocks + qblocks, CfgP::DQ_LDS > CfgP::DKV_LDS ? CfgP::DQ_LDS : CfgP::DKV_LDS, stream);
+      if (rcb != 0) return rcb;
+      launch_kv_merge<T, D>(p, false, false, stream);
+      return hipGetLastError() == hipSuccess ? 0 : -6;
+    }
     if (six) kq = no_go ? bwdp_dq_kernel<T, D, MASK, false, true> : bwdp_dq_kernel<T, D, MASK, true, true>;
     void (*kkv)(const BwdParams) = no_go ? bwdp_dkdv_kernel<T, D, MASK, false> : bwdp_dkdv_kernel<T, D, MASK, true>;
     int rc = allow_lds(reinterpret_cast<const void *>(kq), CfgP::DQ_LDS);
@@ -269,6 +346,17 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     // without tangents in the launch two operands stay resident and one workgroup holds all 256 columns
     using CfgW = BwdWideCfg<T, D, MODE>;
     using CfgK = BwdWideKvCfg<T, D, MODE>;
+    if (MODE == BWD_PLAIN && launch_both<D, MODE>(blocks, kv_blocks, p.pr.causal != 0, MASK != MASK_NONE, false, false, false, false)) {
+      void (*kb)(const BwdParams, int) = bwdw_both_kernel<T, D, BWD_PLAIN, MASK, true>;
+      if constexpr (MASK != MASK_NONE) {
+        if (p.pr.chunks <= 1) kb = bwdw_both_kernel<T, D, BWD_PLAIN, MASK, false>;
+      }
+      using CfgKP = BwdWideKvCfg<T, D, BWD_PLAIN>;
+      const int rcb = run_both(kb, p, kv_blocks, kv_blocks + blocks, CfgKP::DKV_LDS > CfgKP::DQ_LDS ? CfgKP::DKV_LDS : CfgKP::DQ_LDS, stream);
+      if (rcb != 0) return rcb;
+      launch_kv_merge<T, D>(p, false, false, stream);
+      return hipGetLastError() == hipSuccess ? 0 : -6;
+    }
     auto kq = bwdw_dq_kernel<T, D, MODE, MASK>;
     auto kkv = pick_wide_dkdv<T, D, MODE, MASK, false>(p);
     int rc = allow_lds(reinterpret_cast<const void *>(kq), CfgW::DQ_LDS);

@@ -78,8 +78,8 @@ template <int SLOT, int N> __device__ __forceinline__ f32x16 xch_tile(const u32x
 // SIX: dq' = scale dS' K as well, from the K fragments and the dS' tiles that dq already has (a call for all six
 // gradients then needs no second launch that forms S and A again).
 // DROP: dropout (see bwd_kernel.hpp): gO V^T, gT V^T and gT V'^T reach the logits through the kept, rescaled entries.
-template <typename T, int D, int MASK, bool GO, bool SIX = false, bool DROP = false>
-__global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {
+template <typename T, int D, int MASK, bool GO, bool SIX, bool DROP>
+__device__ __forceinline__ void bwdp_dq_body(const BwdParams &p, const int bid) {
   using Cfg = BwdPairCfg<T, D>;
   constexpr int CH = Cfg::CH, ROWB = Cfg::ROWB, TILEB = Cfg::TILEB, IPW = Cfg::IPW, BT = Cfg::BT, DV = Cfg::DV;
   constexpr int KK = D / 16, DB = DV / 32, XT = Cfg::XTILE;
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L;
   const int nblk = (L + Cfg::BLK - 1) / Cfg::BLK;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.H, pr.causal != 0);
+  const int id = xcd_remap(bid, nblk, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nblk;
   const int rem = id % nblk;
   const int qb = pr.causal ? nblk - 1 - rem : rem;
@@ -409,8 +409,8 @@ __global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {
 
 // dk, dv of the dual mode: workgroup = 64 keys of a key/value head (two pairs), loop over 32-query tiles.
 // Tile slots of a stage: 0 Q, 1 gT, 2 Q', 3 gO; statistics slots M, mu, -a, -(d1 + d2).
-template <typename T, int D, int MASK, bool GO, bool DROP = false>
-__global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
+template <typename T, int D, int MASK, bool GO, bool DROP>
+__device__ __forceinline__ void bwdp_dkdv_body(const BwdParams &p, const int bid) {
   using Cfg = BwdPairCfg<T, D>;
   constexpr int CH = Cfg::CH, ROWB = Cfg::ROWB, TILEB = Cfg::TILEB, IPW = Cfg::IPW, BT = Cfg::BT;
   constexpr int KK = D / 16, DB = D / 32, XT = Cfg::XTILE;
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nblk = (Lk + Cfg::BLK - 1) / Cfg::BLK;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
+  const int id = xcd_remap(bid, nblk, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zh = id / nblk / pr.chunks, chunk = id / nblk % pr.chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nblk;
   const int z = zh / pr.Hk, hk = zh % pr.Hk, group = group_share(pr, chunk + 1) - group_share(pr, chunk);
@@ -783,11 +783,28 @@ __global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
     }
   }
 }
-#else
-template <typename T, int D, int MASK, bool GO, bool SIX = false, bool DROP = false>
-__global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {}
-template <typename T, int D, int MASK, bool GO, bool DROP = false>
-__global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {}
 #endif
+template <typename T, int D, int MASK, bool GO, bool SIX = false, bool DROP = false>
+__global__ __launch_bounds__(256, 1) void bwdp_dq_kernel(const BwdParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  bwdp_dq_body<T, D, MASK, GO, SIX, DROP>(p, blockIdx.x);
+#endif
+}
+template <typename T, int D, int MASK, bool GO, bool DROP = false>
+__global__ __launch_bounds__(256, 1) void bwdp_dkdv_kernel(const BwdParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  bwdp_dkdv_body<T, D, MASK, GO, DROP>(p, blockIdx.x);
+#endif
+}
+
+// Both roles in one launch (see bwd2_both_kernel): the first kv_blocks workgroups are dk/dv workgroups.
+template <typename T, int D, int MASK, bool GO>
+__global__ __launch_bounds__(256, 1) void bwdp_both_kernel(const BwdParams p, const int kv_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
+  if (b < kv_blocks) bwdp_dkdv_body<T, D, MASK, GO, false>(p, b);
+  else bwdp_dq_body<T, D, MASK, GO, false, false>(p, b - kv_blocks);
+#endif
+}
 
 }  // namespace jvpfa

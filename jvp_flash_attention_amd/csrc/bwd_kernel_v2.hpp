@@ -167,7 +167,8 @@ constexpr bool dq_init(int d, int mode, int mask, bool go, bool six, bool drop) 
 }
 // LEAN: one tile loop (every tile takes the limit tests) instead of an interior loop and an edge loop: less for
 // the compiler to keep in registers, for the variant that must stay within 256 of them.
-template <typename T, int D, int MODE, int MASK, bool GO, bool SIX, bool DROP = false, bool LEAN = false>
+// START: where dq_init says so.
+template <typename T, int D, int MODE, int MASK, bool GO, bool SIX, bool DROP = false, bool LEAN = false, bool START = true>
 __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) {
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
@@ -206,7 +207,7 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
 
   // INIT: A and dP start from -a and -(d1 + d2) (PLAIN -d1, TANGENT -a), which saves an addition per entry each.  A lane
   // owns one query, so a tile of either holds one number; the two tiles stay resident.
-  constexpr bool INIT = dq_init(D, MODE, MASK, GO, SIX, DROP);
+  constexpr bool INIT = START && dq_init(D, MODE, MASK, GO, SIX, DROP);
   f32x16 from_a, from_d;
   if constexpr (INIT) {
 #pragma unroll
@@ -1175,19 +1176,38 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_num_vgpr(144))) void 
 #endif
 }
 
-// Both roles in one launch, for grids smaller than the GPU: the first kv_blocks workgroups are dk/dv
-// workgroups, the others dq workgroups.  The two kernels do not depend on each other, so launched apart on a
-// stream each leaves the compute units it does not fill idle for its whole duration; together they run side
-// by side.  (For grids that fill the GPU the single launch measured the same as the two.)
+// Both roles in one launch: the first kv_blocks workgroups are dk/dv workgroups, the others dq workgroups.  The two kernels do
+// not depend on each other, but launched apart on a stream the second waits for the last workgroup of the first, so each ends
+// with compute units idle; together they have one end (launch_both says for which grids that is worth it).
 // Boolean masks of 512 and more are read from their packed copies here too: bf16 B2 H6 L577 (rows that are not aligned), first
 // order / gradients of O' / of both: D32 39.9 / 46.2 / 46.5 -> 17.2 / 24.1 / 25.3 us, D128 49.4 / 64.5 / 67.7 -> 27.7 / 44.7 / 48.6 us;
 // B2 H12 L640 (aligned): D64 31.4 / 41.2 / 43.3 -> 23.0 / 34.6 / 37.8 us.
-template <typename T, int D, int MODE, int MASK, bool GO>
+template <typename T, int D, int MODE, int MASK, bool GO, bool GROUPED = false, bool SIX = false, bool DROP = false>
 __global__ __launch_bounds__(256, 1) void bwd2_both_kernel(const BwdParams p, const int kv_blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
+  if (b < kv_blocks) bwd2_dkdv_body<T, D, MODE, MASK, GO, GROUPED, SIX, DROP>(p, b);
+  else bwd2_dq_body<T, D, MODE, MASK, GO, SIX, DROP>(p, b - kv_blocks);
+#endif
+}
+// ... with two workgroups to a compute unit (D = 64, dual): capped like bwd2_dkdv_kernel_2wg, and the dq role without the tiles
+// it starts from, which are what does not fit.
+template <typename T, int D, int MODE, int MASK, bool GO>
+__global__ __launch_bounds__(256, 1) __attribute__((amdgpu_num_vgpr(144))) void bwd2_both_kernel_2wg(const BwdParams p, const int kv_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
   if (b < kv_blocks) bwd2_dkdv_body<T, D, MODE, MASK, GO, false, false>(p, b);
-  else bwd2_dq_body<T, D, MODE, MASK, GO, false>(p, b - kv_blocks);
+  else bwd2_dq_body<T, D, MODE, MASK, GO, false, false, false, false>(p, b - kv_blocks);
+#endif
+}
+// All six gradients at D = 128: dk, dv by the first kv_blocks workgroups, dk', dv' by as many again, dq and dq' by the others.
+template <typename T, int D, int MASK, bool GO>
+__global__ __launch_bounds__(256, 1) void bwd2_all_kernel(const BwdParams p, const int kv_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
+  if (b < kv_blocks) bwd2_dkdv_body<T, D, BWD_DUAL, MASK, GO, false, false>(p, b);
+  else if (b < 2 * kv_blocks) bwd2_dkdv_body<T, D, BWD_TANGENT, MASK, true, false, false>(p, b - kv_blocks);
+  else bwd2_dq_body<T, D, BWD_DUAL, MASK, GO, true>(p, b - 2 * kv_blocks);
 #endif
 }
 

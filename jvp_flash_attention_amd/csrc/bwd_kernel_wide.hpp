@@ -38,8 +38,8 @@ __device__ __forceinline__ int swz_w(int row) { return ((row & 3) << 2) | ((row 
 
 #if defined(__HIP_DEVICE_COMPILE__)
 // DROP: dropout (see bwd_kernel.hpp): gO V^T (gT V^T) reaches the logits through the kept, rescaled entries only.
-template <typename T, int D, int MODE, int MASK, bool DROP = false>
-__global__ __launch_bounds__(256, 1) void bwdw_dq_kernel(const BwdParams p) {
+template <typename T, int D, int MODE, int MASK, bool DROP>
+__device__ __forceinline__ void bwdw_dq_body(const BwdParams &p, const int bid) {
   using Cfg = BwdWideCfg<T, D, MODE>;
   constexpr bool TAN = MODE == BWD_TANGENT;
   constexpr int CH = Cfg::CH, ROWB = Cfg::ROWB, TILEB = Cfg::TILEB, IPW = Cfg::IPW, BT = Cfg::BT;
@@ -49,7 +49,7 @@ __global__ __launch_bounds__(256, 1) void bwdw_dq_kernel(const BwdParams p) {
   const Problem &pr = p.pr;
   const int L = pr.L;
   const int nblk = (L + Cfg::BLK - 1) / Cfg::BLK;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.H, pr.causal != 0);
+  const int id = xcd_remap(bid, nblk, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nblk;
   const int rem = id % nblk;
   const int qb = pr.causal ? nblk - 1 - rem : rem;
@@ -310,10 +310,13 @@ __global__ __launch_bounds__(256, 1) void bwdw_dq_kernel(const BwdParams p) {
     }
   }
 }
-#else
-template <typename T, int D, int MODE, int MASK, bool DROP = false>
-__global__ __launch_bounds__(256, 1) void bwdw_dq_kernel(const BwdParams p) {}
 #endif
+template <typename T, int D, int MODE, int MASK, bool DROP = false>
+__global__ __launch_bounds__(256, 1) void bwdw_dq_kernel(const BwdParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  bwdw_dq_body<T, D, MODE, MASK, DROP>(p, blockIdx.x);
+#endif
+}
 
 // ------------------------------------------------------------------------------------------------
 // dk, dv (PLAIN) or dk', dv' (TANGENT) for D = 256: workgroup = 128 keys of a head, K and V resident,
@@ -329,8 +332,8 @@ template <typename T, int D, int MODE> struct BwdWideKvCfg : BwdWideCfg<T, D, MO
 // Compiled apart for masks, whose registers are full: with the shares' pointers 112 bytes are spilled, without them 80 - 96
 // (without a mask 0 and 12).
 #if defined(__HIP_DEVICE_COMPILE__)
-template <typename T, int D, int MODE, int MASK, bool DROP = false, bool SPLIT = false>
-__global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
+template <typename T, int D, int MODE, int MASK, bool DROP, bool SPLIT>
+__device__ __forceinline__ void bwdw_dkdv_body(const BwdParams &p, const int bid) {
   using Cfg = BwdWideKvCfg<T, D, MODE>;
   constexpr bool TAN = MODE == BWD_TANGENT;
   constexpr int CH = Cfg::CH, ROWB = Cfg::ROWB, TILEB = Cfg::TILEB, IPW = Cfg::IPW, BT = Cfg::BT;
@@ -341,7 +344,7 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
   const int L = pr.L, Lk = pr.Lk;  // queries, keys
   const int nblk = (Lk + Cfg::BLK - 1) / Cfg::BLK;
   const int chunks = SPLIT ? pr.chunks : 1;
-  const int id = xcd_remap(blockIdx.x, nblk, pr.Z * pr.Hk * chunks, pr.causal != 0);
+  const int id = xcd_remap(bid, nblk, pr.Z * pr.Hk * chunks, pr.causal != 0);
   const int zh = id / nblk / chunks, chunk = id / nblk % chunks;  // chunk: this workgroup's share of the query heads
   const int kb = id % nblk;  // causal: the first key blocks have the longest query loops
   const int z = zh / pr.Hk, hk = zh % pr.Hk, group = SPLIT ? group_share(pr, chunk + 1) - group_share(pr, chunk) : pr.H / pr.Hk;
@@ -682,9 +685,22 @@ __global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
     }
   }
 }
-#else
-template <typename T, int D, int MODE, int MASK, bool DROP = false, bool SPLIT = false>
-__global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {}
 #endif
+template <typename T, int D, int MODE, int MASK, bool DROP = false, bool SPLIT = false>
+__global__ __launch_bounds__(256, 1) void bwdw_dkdv_kernel(const BwdParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  bwdw_dkdv_body<T, D, MODE, MASK, DROP, SPLIT>(p, blockIdx.x);
+#endif
+}
+
+// Both roles in one launch (see bwd2_both_kernel): the first kv_blocks workgroups are dk/dv workgroups.
+template <typename T, int D, int MODE, int MASK, bool SPLIT>
+__global__ __launch_bounds__(256, 1) void bwdw_both_kernel(const BwdParams p, const int kv_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
+  if (b < kv_blocks) bwdw_dkdv_body<T, D, MODE, MASK, false, SPLIT>(p, b);
+  else bwdw_dq_body<T, D, MODE, MASK, false>(p, b - kv_blocks);
+#endif
+}
 
 }  // namespace jvpfa
