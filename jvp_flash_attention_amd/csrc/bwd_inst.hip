@@ -181,6 +181,17 @@ template <int D, int MODE, int MASK, bool GO, bool DROP> static auto pick_f32_dk
   if constexpr (D <= 64) return bwd_f32x3_dkdv_kernel<D, MODE, MASK, GO, DROP>;
   else return bwd_f32_dkdv_kernel<D, MODE, MASK, GO, DROP>;
 }
+template <int D, int MODE, int MASK, bool GO> static auto pick_f32_both() -> void (*)(const BwdParams, int) {
+  if constexpr (D <= 64) return bwd_f32x3_both_kernel<D, MODE, MASK, GO>;
+  else return bwd_f32_both_kernel<D, MODE, MASK, GO>;
+}
+// ... and whether dk/dv and dq go into one launch: by launch_both's rule for D = 128 (one workgroup a compute unit, mostly).
+static bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven) {
+  const long long most = blocks > kv_blocks ? blocks : kv_blocks, cus = device_cus();
+  if (most <= cus || (uneven && most <= 2.5 * cus)) return true;
+  const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
+  return apart > 1.04 * ((double)(blocks + kv_blocks) / cus + 0.6);
+}
 template <int D, int MODE, int MASK, bool DROP>
 static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blocks, hipStream_t stream) {
   constexpr bool NG = MODE != BWD_DUAL;  // gO may be absent only in the dual mode
@@ -191,6 +202,15 @@ static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blo
   int rc = allow_lds(reinterpret_cast<const void *>(kq), Lds::DQ);
   if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), Lds::DKV);
   if (rc != 0) return rc;
+  if constexpr (!DROP) {
+    if (launch_both_f32(blocks, kv_blocks, p.pr.causal != 0 || MASK != MASK_NONE)) {
+      void (*kb)(const BwdParams, int) = no_go ? pick_f32_both<D, MODE, MASK, NG>() : pick_f32_both<D, MODE, MASK, true>();
+      rc = run_both(kb, p, kv_blocks, kv_blocks + blocks, Lds::DKV, stream);
+      if (rc != 0) return rc;
+      launch_kv_merge<float, D>(p, MODE == BWD_TANGENT, false, stream);
+      return hipGetLastError() == hipSuccess ? 0 : -6;
+    }
+  }
   hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(BWD_NT), Lds::DKV, stream, p);
   launch_kv_merge<float, D>(p, MODE == BWD_TANGENT, false, stream);
   hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(BWD_NT), Lds::DQ, stream, p);

@@ -45,7 +45,7 @@ template <typename V> __device__ __forceinline__ void lds_done(V (&a)[4], V (&b)
 
 // dq (PLAIN / DUAL) or dq' (TANGENT): workgroup = 128 query rows, loop over key tiles K, V (, K', V').
 template <int D, int MODE, int MASK, bool GO, bool DROP>
-__device__ __forceinline__ void bwd_f32_dq_body(const BwdParams &p) {
+__device__ __forceinline__ void bwd_f32_dq_body(const BwdParams &p, const int bid) {
   using C = F32Cfg<D>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   constexpr int BT = C::BT, NJ = C::NJ, DB = C::DB, NTILE = DUAL ? 4 : 2, STAGEB = NTILE * C::TILEB;
@@ -55,7 +55,7 @@ __device__ __forceinline__ void bwd_f32_dq_body(const BwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nqb = (L + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
+  const int id = xcd_remap(bid, nqb, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nqb;
   const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
   const int z = zh / pr.H, h = zh % pr.H;
@@ -250,7 +250,7 @@ __device__ __forceinline__ void bwd_f32_dq_body(const BwdParams &p) {
 // G = gO (gT in TANGENT).  Scores are S = Q K^T (lane = key).  The query heads of a group are visited one after
 // another (this workgroup's share of them, see split.hpp).
 template <int D, int MODE, int MASK, bool GO, bool DROP>
-__device__ __forceinline__ void bwd_f32_dkdv_body(const BwdParams &p) {
+__device__ __forceinline__ void bwd_f32_dkdv_body(const BwdParams &p, const int bid) {
   using C = F32Cfg<D>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   constexpr int BT = C::BT, NJ = C::NJ, DB = C::DB, NTILE = DUAL ? 4 : 2, STAGEB = NTILE * C::TILEB;
@@ -262,7 +262,7 @@ __device__ __forceinline__ void bwd_f32_dkdv_body(const BwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nkb = (Lk + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
+  const int id = xcd_remap(bid, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zhk = id / nkb / pr.chunks, chunk = id / nkb % pr.chunks;
   const int kb = id % nkb;  // causal: the first key blocks have the longest query loops
   const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = group_share(pr, chunk + 1) - group_share(pr, chunk);
@@ -541,13 +541,23 @@ template <int D, int MODE> struct BwdF32Lds {
 template <int D, int MODE, int MASK, bool GO, bool DROP = false>
 __global__ __launch_bounds__(256, 1) void bwd_f32_dq_kernel(const BwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  bwd_f32_dq_body<D, MODE, MASK, GO, DROP>(p);
+  bwd_f32_dq_body<D, MODE, MASK, GO, DROP>(p, blockIdx.x);
 #endif
 }
 template <int D, int MODE, int MASK, bool GO, bool DROP = false>
 __global__ __launch_bounds__(256, 1) void bwd_f32_dkdv_kernel(const BwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  bwd_f32_dkdv_body<D, MODE, MASK, GO, DROP>(p);
+  bwd_f32_dkdv_body<D, MODE, MASK, GO, DROP>(p, blockIdx.x);
+#endif
+}
+
+// Both roles in one launch (see bwd2_both_kernel): the first kv_blocks workgroups are dk/dv workgroups.
+template <int D, int MODE, int MASK, bool GO>
+__global__ __launch_bounds__(256, 1) void bwd_f32_both_kernel(const BwdParams p, const int kv_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
+  if (b < kv_blocks) bwd_f32_dkdv_body<D, MODE, MASK, GO, false>(p, b);
+  else bwd_f32_dq_body<D, MODE, MASK, GO, false>(p, b - kv_blocks);
 #endif
 }
 

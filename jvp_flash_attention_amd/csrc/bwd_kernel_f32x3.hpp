@@ -135,7 +135,7 @@ template <int G, int NG, int NU, bool AFTER, typename F> __device__ __forceinlin
 }
 // dq (PLAIN / DUAL) or dq' (TANGENT).  Returns whether every output is finite.
 template <int D, int MODE, int MASK, bool GO, bool DROP>
-__device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p) {
+__device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int bid) {
   using C = X3Cfg<D>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   constexpr int BT = C::BT, KK = D / 16, DB = D / 32, NTILE = DUAL ? 4 : 2;
@@ -145,7 +145,7 @@ __device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nqb = (L + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
+  const int id = xcd_remap(bid, nqb, pr.Z * pr.H, pr.causal != 0);
   const int zh = id / nqb;
   const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
   const int z = zh / pr.H, h = zh % pr.H;
@@ -417,7 +417,7 @@ __device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p) {
 
 // dk, dv (PLAIN / DUAL) or dk', dv' (TANGENT).  Returns whether every output is finite.
 template <int D, int MODE, int MASK, bool GO, bool DROP>
-__device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p) {
+__device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p, const int bid) {
   using C = X3Cfg<D>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   constexpr int BT = C::BT, KK = D / 16, DB = D / 32, NTILE = DUAL ? 4 : 2;
@@ -430,7 +430,7 @@ __device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nkb = (Lk + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(blockIdx.x, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
+  const int id = xcd_remap(bid, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
   const int zhk = id / nkb / pr.chunks, chunk = id / nkb % pr.chunks;
   const int kb = id % nkb;  // causal: the first key blocks have the longest query loops
   const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = group_share(pr, chunk + 1) - group_share(pr, chunk);
@@ -792,13 +792,26 @@ template <int D, int MODE> struct BwdX3Lds {
 template <int D, int MODE, int MASK, bool GO, bool DROP = false, int WGS = MODE != BWD_DUAL && !DROP ? 2 : 1>
 __global__ __launch_bounds__(256, WGS) void bwd_f32x3_dq_kernel(const BwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (!bwd_f32x3_dq_body<D, MODE, MASK, GO, DROP>(p)) bwd_f32_dq_body<D, MODE, MASK, GO, DROP>(p);
+  if (!bwd_f32x3_dq_body<D, MODE, MASK, GO, DROP>(p, blockIdx.x)) bwd_f32_dq_body<D, MODE, MASK, GO, DROP>(p, blockIdx.x);
 #endif
 }
 template <int D, int MODE, int MASK, bool GO, bool DROP = false>
 __global__ __launch_bounds__(256, 1) void bwd_f32x3_dkdv_kernel(const BwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (!bwd_f32x3_dkdv_body<D, MODE, MASK, GO, DROP>(p)) bwd_f32_dkdv_body<D, MODE, MASK, GO, DROP>(p);
+  if (!bwd_f32x3_dkdv_body<D, MODE, MASK, GO, DROP>(p, blockIdx.x)) bwd_f32_dkdv_body<D, MODE, MASK, GO, DROP>(p, blockIdx.x);
+#endif
+}
+
+// Both roles in one launch (see bwd2_both_kernel): the first kv_blocks workgroups are dk/dv workgroups.
+template <int D, int MODE, int MASK, bool GO>
+__global__ __launch_bounds__(256, 1) void bwd_f32x3_both_kernel(const BwdParams p, const int kv_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
+  if (b < kv_blocks) {
+    if (!bwd_f32x3_dkdv_body<D, MODE, MASK, GO, false>(p, b)) bwd_f32_dkdv_body<D, MODE, MASK, GO, false>(p, b);
+  } else {
+    if (!bwd_f32x3_dq_body<D, MODE, MASK, GO, false>(p, b - kv_blocks)) bwd_f32_dq_body<D, MODE, MASK, GO, false>(p, b - kv_blocks);
+  }
 #endif
 }
 
