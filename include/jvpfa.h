@@ -155,10 +155,12 @@ typedef struct jvpfa_bwd_args {
                                tiles_q and tiles_k are both NULL or both set */
   int32_t Lk, Hk;           /* as in jvpfa_fwd_args; dk, dv, dkt, dvt have the shape of k */
   const uint32_t *mask_bits; /* optional, boolean masks only: the copy written by jvpfa_mask_bits(), or NULL */
-  /* optional workspace for grouped heads (Hk < p.H), or NULL: jvpfa_bwd_split_workspace_bytes() bytes of device
-   * memory, 16-byte aligned, contents don't-care.  Where one workgroup per 128 keys of a key/value head would leave
-   * compute units idle, the query heads of a group are then dealt to several workgroups that leave fp32 shares of the
-   * key and value gradients there, and a second kernel adds them up.  Results agree with the unsplit launch to rounding. */
+  /* optional workspace for grouped heads (Hk < p.H) and for small grids, or NULL: jvpfa_bwd_split_workspace_bytes() bytes
+   * of device memory, 16-byte aligned, contents don't-care.  Where one workgroup per 128 keys of a key/value head would
+   * leave compute units idle, the query heads of a group are then dealt to several workgroups that leave fp32 shares of
+   * the key and value gradients there, and a second kernel adds them up; where the whole launch would (one long
+   * sequence, few heads; bf16 / fp16, D <= 128, no mask, no dropout, Hk = p.H, dqt NULL), the tiles of every block are,
+   * for dq, dk, dv.  Results agree with the unsplit launch to rounding. */
   void *split_workspace;
   uint64_t split_workspace_bytes;
   const uint32_t *mask_bits_q; /* as in jvpfa_fwd_args (dq kernels) */

@@ -34,6 +34,8 @@ extern "C" size_t jvpfa_bwd_split_workspace_bytes(const jvpfa_problem *p, int32_
   if (!p || check_problem(*p) != JVPFA_OK || check_kv_shape(*p, Lk, Hk) != JVPFA_OK) return 0;
   Lk = Lk > 0 ? Lk : p->L;
   Hk = Hk > 0 ? Hk : p->H;
+  const BwdSplitPlan sp = bwd_split_plan_of(*p, Lk, Hk, tangent_grads != 0, true);  // (without tangents the same or none)
+  if (sp.any()) return bwd_split_floats(*p, Lk, sp) * sizeof(float);
   const int chunks = bwd_kv_chunks(*p, Lk, Hk);
   return chunks > 1 ? bwd_part_floats(*p, Lk, Hk, chunks, tangent_grads != 0) * sizeof(float) : 0;
 }
@@ -70,7 +72,12 @@ static int bwd_impl(const jvpfa_bwd_args *a, void *workspace, void *hip_stream) 
   p.go = a->go; p.gt = a->gt;
   p.dq = a->dq; p.dk = a->dk; p.dv = a->dv;
   p.dqt = a->dqt; p.dkt = a->dkt; p.dvt = a->dvt;
-  if (a->split_workspace) {  // few dk/dv workgroups: split the query heads of every group, if the workspace suffices
+  if (a->split_workspace) {  // few workgroups: split the tiles of every block, or the query heads of every group, if the workspace suffices
+    const BwdSplitPlan sp = bwd_split_plan_of(a->p, p.pr.Lk, p.pr.Hk, ntg == 3, dual);
+    if (sp.any() && aligned16(a->split_workspace) && a->split_workspace_bytes >= bwd_split_floats(a->p, p.pr.Lk, sp) * sizeof(float)) {
+      p.pr.chunk_tiles = -1;  // (the launcher makes the same plan)
+      p.pr.part = static_cast<float *>(a->split_workspace);
+    }
     const int chunks = bwd_kv_chunks(a->p, p.pr.Lk, p.pr.Hk);
     if (chunks > 1 && aligned16(a->split_workspace) &&
         a->split_workspace_bytes >= bwd_part_floats(a->p, p.pr.Lk, p.pr.Hk, chunks, ntg == 3) * sizeof(float)) {

@@ -102,7 +102,8 @@ template <typename T, int D, int MODE, int MASK, bool DROP> static auto pick_wid
 
 // Whether dk/dv and dq go into one launch (bwd2_both_kernel): it has one end with idle compute units instead of two, and where a
 // kernel has to take both roles' registers fewer of its workgroups share a unit.  So: up to a number of blocks (in units of
-// compute units) that depends on how many do.  two_wgs: bwd2_both_kernel_2wg runs it.
+// compute units) that depends on how many do.  two_wgs: bwd2_both_kernel_2wg runs it (where units get more than one workgroup;
+// below that its cap costs 4 %: B1 H8 L2048 95.1 against 91.9 us).
 // D = 128 (one workgroup a unit either way, but for the dq kernel without tangents): causal and masked launches up to 2.5; others
 // where the launches would round up to more passes over the units than the one does, 0.6 of a pass for its end.
 // Measured, bf16, backward, two launches -> one, 288 / 544 / 704 / 1024 - 1152 blocks (dual unless said): D128 269 -> 205, 721 ->
@@ -134,7 +135,7 @@ static auto pick_both(const BwdParams &p, bool no_go, bool grouped, bool six, lo
   constexpr bool NG = MODE != BWD_DUAL;
   const bool bits = MASK == MASK_BOOL && p.pr.bits_q && p.pr.bits_k;
   constexpr bool M = MASK != MASK_NONE;
-  const bool causal = p.pr.causal != 0, two_wgs = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits);
+  const bool causal = p.pr.causal != 0, two_wgs = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits) && blocks + kv_blocks > device_cus();
   // (six: the dual and the tangent launch of a call decide alike)
   if (!(six ? launch_both<D, BWD_DUAL>(blocks, kv_blocks, causal, M, false, true, grouped, false)
             : launch_both<D, MODE>(blocks, kv_blocks, causal, M, false, false, grouped, two_wgs)))
@@ -156,7 +157,8 @@ static auto pick_both(const BwdParams &p, bool no_go, bool grouped, bool six, lo
   if constexpr (D == 64 && MODE == BWD_DUAL && MASK != MASK_ADD) {
     constexpr int MK = MASK == MASK_BOOL ? MASK_BITS : MASK_NONE;
     if (two_wgs) return no_go ? bwd2_both_kernel_2wg<T, D, MODE, MK, NG> : bwd2_both_kernel_2wg<T, D, MODE, MK, true>;
-  } else if constexpr (MASK == MASK_BOOL) {
+  }
+  if constexpr (MASK == MASK_BOOL) {
     if (bits) return no_go ? bwd2_both_kernel<T, D, MODE, MASK_BITS, NG> : bwd2_both_kernel<T, D, MODE, MASK_BITS, true>;
   }
   return no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG> : bwd2_both_kernel<T, D, MODE, MASK, true>;
@@ -214,6 +216,24 @@ static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blo
   hipLaunchKernelGGL(kkv, dim3((unsigned)kv_blocks), dim3(BWD_NT), Lds::DKV, stream, p);
   launch_kv_merge<float, D>(p, MODE == BWD_TANGENT, false, stream);
   hipLaunchKernelGGL(kq, dim3((unsigned)blocks), dim3(BWD_NT), Lds::DQ, stream, p);
+  return hipGetLastError() == hipSuccess ? 0 : -6;
+}
+
+// Small grids: every block's tiles split (split.hpp).
+template <typename T, int D, int MODE> static int launch_split(const BwdParams &p, bool no_go, hipStream_t stream) {
+  using Cfg = Bwd2Cfg<T, D, MODE>;
+  const Problem &pr = p.pr;
+  const BwdSplitPlan s = bwd_split_plan(D, pr.Z, pr.H, pr.L, pr.Lk, pr.causal != 0, MODE == BWD_DUAL);
+  BwdSplit sp = {s.chunks_q, s.tiles_q, s.chunks_k, s.tiles_k, pr.part, pr.part};
+  if (s.chunks_q > 1) sp.part_k += (size_t)s.chunks_q * pr.Z * pr.H * pr.L * D;
+  const int heads = pr.Z * pr.H, kv_blocks = (pr.Lk + 127) / 128 * heads * s.chunks_k, blocks = (pr.L + 127) / 128 * heads * s.chunks_q;
+  auto kern = no_go ? bwd2_split_kernel<T, D, MODE, MODE != BWD_DUAL> : bwd2_split_kernel<T, D, MODE, true>;
+  constexpr size_t LDS = Cfg::DKV_LDS > Cfg::DQ_LDS ? Cfg::DKV_LDS : Cfg::DQ_LDS;
+  const int rc = allow_lds(reinterpret_cast<const void *>(kern), LDS);
+  if (rc != 0) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(kv_blocks + blocks)), dim3(Cfg::NT), LDS, stream, p, sp, kv_blocks);
+  const size_t elems = (size_t)heads * (pr.L > pr.Lk ? pr.L : pr.Lk) * D;
+  hipLaunchKernelGGL((bwd_split_merge_kernel<T, D>), dim3((unsigned)((elems / 8 + 255) / 256), 3), dim3(256), 0, stream, p, sp);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
@@ -318,6 +338,9 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     }
     size_t kv_lds = 0;
     kkv = pick_dkdv_for<T, D, MODE, MASK>(p, no_go, grouped, MODE == BWD_DUAL && six, false, &kv_lds);
+    if constexpr (MASK == MASK_NONE && MODE != BWD_TANGENT) {
+      if (p.pr.chunk_tiles == -1) return launch_split<T, D, MODE>(p, no_go, stream);
+    }
     if (auto kb = pick_both<T, D, MODE, MASK>(p, no_go, grouped, six, blocks, kv_blocks)) {
       if constexpr (MODE == BWD_TANGENT) {
         if (six) return 0;  // the dual launch has made all six

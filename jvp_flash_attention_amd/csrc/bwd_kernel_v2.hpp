@@ -149,6 +149,13 @@ __device__ __forceinline__ void zero_acc(f32x16 &x) {
   for (int e = 0; e < 16; ++e) x[e] = 0.f;
 }
 
+// Small grids: the streamed tiles of a block are dealt to `chunks` workgroups, tiles_x each, which leave fp32 partial results
+// where a block has more than one (bwd_split_merge_kernel adds them up).
+struct BwdSplit {
+  int chunks_q, tiles_q, chunks_k, tiles_k;
+  float *part_q, *part_k;  // [chunk][Z H L D], [chunk][dk, dv][Z H Lk D]
+};
+
 // ------------------------------------------------------------------------------------------------
 // dq (PLAIN / DUAL) or dq' (TANGENT): workgroup = 128 query rows, loop over 64-key tiles of
 // K, V (, K', V').  Scores are transposed (lane = query) so dS is the B operand of dQ^T += K^T dS^T.
@@ -168,11 +175,12 @@ constexpr bool dq_init(int d, int mode, int mask, bool go, bool six, bool drop) 
 // LEAN: one tile loop (every tile takes the limit tests) instead of an interior loop and an edge loop: less for
 // the compiler to keep in registers, for the variant that must stay within 256 of them.
 // START: where dq_init says so.
-template <typename T, int D, int MODE, int MASK, bool GO, bool SIX, bool DROP = false, bool LEAN = false, bool START = true>
-__device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) {
+template <typename T, int D, int MODE, int MASK, bool GO, bool SIX, bool DROP = false, bool LEAN = false, bool START = true, bool SPLIT = false>
+__device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid_, const BwdSplit sp = {}) {
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   static_assert(!SIX || DUAL, "dq' rides on the dual mode");
+  const int bid = SPLIT ? bid_ / sp.chunks_q : bid_, part = SPLIT ? bid_ % sp.chunks_q : 0;
   JVPFA_BWD2_COMMON(Cfg, pr.Lk, pr.L, pr.H, 1)  // owns query rows, streams key tiles
   const int qb = pr.causal ? nblk - 1 - id % nblk : id % nblk;
   const int q0 = qb * Cfg::BLK;
@@ -252,7 +260,10 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
     if (pr.tiles_q) tlist = pr.tiles_q + tile_list_offset_q(pr, z, h, qb);
   }
   const int tmax = (Lk + BT - 1) / BT - 1;  // index of the last tile of the sequence: bounds whatever a list holds
-  const int ntiles = tlist ? min(max(tlist[0], 1), tmax + 1) : (kend + BT - 1) / BT;
+  const int nall = tlist ? min(max(tlist[0], 1), tmax + 1) : (kend + BT - 1) / BT;
+  const int tb = SPLIT ? part * sp.tiles_q : 0;  // SPLIT: this workgroup's tiles are tb .. tb + ntiles - 1
+  if (SPLIT && tb > 0 && tb >= nall) return;
+  const int ntiles = SPLIT ? min(nall - tb, sp.tiles_q) : nall;
   // List elements are requested a tile ahead, unconditionally (from a harmless address when there is
   // no list: a branch around the read would split the tile loop's straight-line body).
   auto list_slot = [&](int i) { return tlist ? tlist + 1 + i : reinterpret_cast<const int *>(p.q); };
@@ -459,8 +470,8 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
     }
   };
   // the tile of this step and of the next
-  int tcur = tlist ? min(max(tlist[1], 0), tmax) : 0;
-  int tnext = tlist ? min(max(tlist[1 + min(1, ntiles - 1)], 0), tmax) : min(1, ntiles - 1);
+  int tcur = tlist ? min(max(tlist[1], 0), tmax) : tb;
+  int tnext = tlist ? min(max(tlist[1 + min(1, ntiles - 1)], 0), tmax) : tb + min(1, ntiles - 1);
   fetch_masks(tcur);
   prepare_loads(0, tcur * BT, true);
   static_for<NLOAD>([&](auto pc) { load_piece(pc); });
@@ -469,7 +480,7 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
     const int stage = t & 1;
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's share of tile t has landed
     __syncthreads();                      // ... everyone's has, and stage^1 is no longer being read
-    int tnext2 = min(t + 2, ntiles - 1), tahead = 0;
+    int tnext2 = tb + min(t + 2, ntiles - 1), tahead = 0;
     if constexpr (MASK != MASK_NONE) {
       tahead = list_request(list_slot(tnext2));
 #pragma unroll
@@ -510,7 +521,8 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid) 
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = acc[db][8 * hf + e] * pr.scale;
-        store8<T>(out + 32 * db + 16 * hf + 8 * g, x);
+        if (SPLIT && nall > sp.tiles_q) store8<float>(sp.part_q + (size_t)part * pr.Z * pr.H * L * D + head + (size_t)qrow * D + 32 * db + 16 * hf + 8 * g, x);
+        else store8<T>(out + 32 * db + 16 * hf + 8 * g, x);
         if constexpr (SIX) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) x[e] = accT[db][8 * hf + e] * pr.scale;
@@ -555,8 +567,9 @@ __global__ __launch_bounds__(256, 2) void bwd2_dq_kernel_2wg_plain(const BwdPara
 // one keeps its pointers loop-invariant).
 // SIX (dual mode only): dk' = scale dS'^T Q and dv' = P^T gT as well, from the fragments and tiles that dk, dv
 // already have (two more accumulators: fits for D <= 64).
-template <typename T, int D, int MODE, int MASK, bool GO, bool GROUPED, bool SIX, bool DROP = false>
-__device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid) {
+template <typename T, int D, int MODE, int MASK, bool GO, bool GROUPED, bool SIX, bool DROP = false, bool SPLIT = false>
+__device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid_, const BwdSplit sp = {}) {
+  const int bid = SPLIT ? bid_ / sp.chunks_k : bid_, part = SPLIT ? bid_ % sp.chunks_k : 0;
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   static_assert(!SIX || (DUAL && D <= 64), "dk', dv' ride on the dual mode, where the accumulators fit");
@@ -575,6 +588,8 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
     auto put = [&](void *dst, int t, const float *x) {
       const size_t off = head + (size_t)krow * D + d0;
       if constexpr (GROUPED) store8_or_part<T>(reinterpret_cast<T *>(dst), kv_part(pr, D, NT, t, chunk), off, x);
+      else if (SPLIT && L - (pr.causal ? (k0 / BT) * BT : 0) > sp.tiles_k * BT)
+        store8<float>(sp.part_k + ((size_t)part * 2 + t) * ((size_t)pr.Z * pr.Hk * Lk * D) + off, x);
       else store8<T>(reinterpret_cast<T *>(dst) + off, x);
     };
     put(TAN ? p.dkt : p.dk, 0, xk);
@@ -700,7 +715,10 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   // the head visited.
   const int *tlist = nullptr;
   const int tmax = (L + BT - 1) / BT - 1;  // index of the last tile of the sequence: bounds whatever a list holds
-  int ntiles = (L - istart + BT - 1) / BT;
+  const int nall = (L - istart + BT - 1) / BT;
+  const int tb = SPLIT ? part * sp.tiles_k : 0;  // SPLIT: this workgroup's tiles are tb .. tb + ntiles - 1
+  if (SPLIT && tb > 0 && tb >= nall) return;
+  int ntiles = SPLIT ? min(nall - tb, sp.tiles_k) : nall;
   auto set_list = [&](int hq_) {
     if constexpr (MASK != MASK_NONE) {
       if (pr.tiles_k) {
@@ -1098,7 +1116,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
       asm volatile("" : "+v"(bits_cur));  // taken over here, behind the wait above
       fetch_bits(tnext);
     }
-    int tnext2 = min(t + 2, ntiles - 1), tahead = 0;
+    int tnext2 = tb + min(t + 2, ntiles - 1), tahead = 0;
     if constexpr (MASK != MASK_NONE) tahead = list_request(list_slot(tnext2));
     const int i0 = istart + tcur * BT, i0n = istart + tnext * BT;
     prepare_loads(stage ^ 1, i0n, t + 1 < ntiles);
@@ -1118,7 +1136,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   };
   // Query tiles that cross the diagonal come first (causal), those that cross the end of the sequence
   // last; the tiles in between run without limit tests.
-  const int t_diag = pr.causal ? min(ntiles, (k0 + Cfg::BLK - istart + BT - 1) / BT) : 0;
+  const int t_diag = pr.causal ? min(ntiles, max((k0 + Cfg::BLK - istart + BT - 1) / BT - tb, 0)) : 0;
   const int t_end = mask_small ? max(t_diag, (L - istart) / BT) : t_diag;  // first tile that crosses the end
   for (int gi = 0; gi < group; ++gi) {
     if (gi > 0) {
@@ -1126,8 +1144,8 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
       set_query_head(hq0 + gi);
       if constexpr (GROUPED) set_list(hq0 + gi);
     }
-    tcur = tlist ? min(max(tlist[1], 0), tmax) : 0;
-    tnext = tlist ? min(max(tlist[1 + min(1, ntiles - 1)], 0), tmax) : min(1, ntiles - 1);
+    tcur = tlist ? min(max(tlist[1], 0), tmax) : tb;
+    tnext = tlist ? min(max(tlist[1 + min(1, ntiles - 1)], 0), tmax) : tb + min(1, ntiles - 1);
     if constexpr (MASK != MASK_NONE && MAHEAD) fetch_mask_half(istart + tcur * BT);
     if constexpr (MASK == MASK_BITS) fetch_bits(tcur);
     prepare_loads(0, istart + tcur * BT, true);
@@ -1209,6 +1227,39 @@ __global__ __launch_bounds__(256, 1) void bwd2_all_kernel(const BwdParams p, con
   else if (b < 2 * kv_blocks) bwd2_dkdv_body<T, D, BWD_TANGENT, MASK, true, false, false>(p, b - kv_blocks);
   else bwd2_dq_body<T, D, BWD_DUAL, MASK, GO, true>(p, b - 2 * kv_blocks);
 #endif
+}
+
+// Both roles in one launch, each block's tiles split (no mask, ungrouped).
+template <typename T, int D, int MODE, bool GO>
+__global__ __launch_bounds__(256, 1) void bwd2_split_kernel(const BwdParams p, const BwdSplit sp, const int kv_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
+  if (b < kv_blocks) bwd2_dkdv_body<T, D, MODE, MASK_NONE, GO, false, false, false, true>(p, b, sp);
+  else bwd2_dq_body<T, D, MODE, MASK_NONE, GO, false, false, false, true, true>(p, b - kv_blocks, sp);
+#endif
+}
+// Its partial results added up, in fp32 and in the order of the tiles: one thread per 8 elements of dq, dk, dv (blockIdx.y 0, 1, 2).  Blocks that
+// one workgroup did are complete.  Bound by memory: chunks * 4 + sizeof(T) bytes an element.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void bwd_split_merge_kernel(const BwdParams p, const BwdSplit sp) {
+  const Problem &pr = p.pr;
+  const int t = blockIdx.y, len = t == 0 ? pr.L : pr.Lk, other = t == 0 ? pr.Lk : pr.L;
+  const size_t elems = (size_t)pr.Z * pr.H * len * D, i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= elems) return;
+  const int row0 = (int)(i / D % len) / 128 * 128;  // first row of the block
+  // streamed rows of the block: keys up to its last row, queries from its first 64-row tile on (causal), or all
+  const int rows = !pr.causal ? other : t == 0 ? min(other, row0 + 128) : max(other - row0 / 64 * 64, 0);
+  const int tiles = (rows + 63) / 64, per = t == 0 ? sp.tiles_q : sp.tiles_k;
+  if (tiles <= per) return;
+  const float *src = t == 0 ? sp.part_q : sp.part_k + (size_t)(t - 1) * elems;
+  const size_t step = t == 0 ? elems : 2 * elems;
+  float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c * per < tiles; ++c) {
+    const f32x8 x = ld8<float>(src + c * step + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum[e] += x[e];
+  }
+  store8<T>(reinterpret_cast<T *>(t == 0 ? p.dq : t == 1 ? p.dk : p.dv) + i, sum);
 }
 
 }  // namespace jvpfa

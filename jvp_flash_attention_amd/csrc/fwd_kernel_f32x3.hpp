@@ -5,21 +5,22 @@
 // values, h = bf16(x), m = bf16(x - h), l = bf16(x - h - m) (both differences are exact; 27 bits with the signs), so
 //     x y = l h' + h l' + m m' + m h' + h m' + h h'     (left out: m l' + l m' + l l', below 2^-26 of the product)
 // is six bf16 products with fp32 accumulation: 6 x 32 cycles for 32x32x16 where the fp32 instructions take 8 x 64.
-// How the sums are formed keeps the error below that of the fp32 instructions: the small products go first where the
-// contraction is short (the scores), and into accumulators of their own where it runs over all keys (the matrix cores cut
-// off what a product has below the last place of the accumulator, in one direction, which long sums of small terms would
-// add up).  Relative error (2-norm) of one product against 64 bits, normal operands: contraction 64: 1.4e-7 (fp32
-// instructions) and 1.25e-7; contraction 8192 with two accumulators: 1.6e-6 and 5.7e-7, and for sums of one sign
-// 1.2e-6 and 4.3e-7.
+// How the sums are formed keeps the error below that of the fp32 instructions.  The matrix cores cut off what a product has
+// below the last place of the accumulator, so the small products go first where the contraction is short (the scores), and
+// into accumulators of their own where it runs over all keys; and parts are rounded to nearest, so that what is cut off has either
+// sign.  Relative error (2-norm) of one product against 64 bits, normal operands, fp32 instructions / parts in one accumulator
+// / in two: contraction 64: 1.4e-7 / 1.1e-7 / 5.0e-8; 8192: 1.6e-6 / 1.4e-6 / 5.6e-7, terms of one sign 1.2e-6 / 7.7e-7 / 4.3e-7.
 //
 // Infinities (inf = inf + nan + nan) and values that round to one are the exception: an output that is not finite makes
 // its workgroup start over with the fp32 instructions, so that every result that is not finite is theirs.
 //
 // Work split and softmax as in fwd_kernel_f32.hpp (4 waves = 128 query rows, 32-key tiles, scores transposed, lane = query).
 // Measured, dual forward at B4 H8 L1024 D64, kernel alone: key padding 201 -> 122 us, bias per head 206 -> 132 us (6 x 25.8
-// GFLOP in 16 bits: 1.2 PFLOP/s).  Q, Q' stay resident as parts.  K, V, K', V' tiles go global -> registers (a tile ahead) -> three bf16 planes each in
-// LDS; splitting there costs a tile's share of every lane once, not every wave once.  One wave per SIMD: a wave hides its
-// vector work itself, one unit of it behind each matrix instruction, in two phases per tile t with one barrier:
+// GFLOP in 16 bits: 1.2 PFLOP/s).  What bounds it: one wave per SIMD, which pays for most of its 430 vector instructions
+// beside 144 matrix instructions a tile.
+// Q, Q' stay resident as parts.  K, V, K', V' tiles go global -> registers (a tile ahead) -> three bf16 planes each in LDS;
+// splitting there costs a tile's share of every lane once, not every wave once.  A wave hides its vector work itself, one
+// unit of it behind each matrix instruction, in two phases per tile t with one barrier:
 //     A: scores of tile t + 1          with   exponentials, row sums and splitting of P, P S' of tile t
 //     B: accumulation of tile t        with   logits and row maximum of tile t + 1, splitting of K (t + 2), V (t + 1)
 #pragma once

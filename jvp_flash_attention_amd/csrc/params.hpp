@@ -37,7 +37,8 @@ struct Problem {
   // c * chunk_tiles .. (c + 1) * chunk_tiles - 1 and writes fp32 partial results to `part`, which a merge
   // kernel adds up.  Only the kernels for 16-bit element types, D = 64 or 128, without a mask.
   // In the backward: the query heads of a key/value head's group are dealt to `chunks` dk/dv workgroups (see
-  // split.hpp), each of which leaves its share of the gradients in `part`.
+  // split.hpp), each of which leaves its share of the gradients in `part`; chunk_tiles = -1: `part` is there for the shares
+  // of blocks whose tiles are split (bwd_split_plan).
   int chunks, chunk_tiles;
   float *part;
   // Dropout on the attention probabilities (0 in drop_thr: none).  Entry (z, h, query i, key j) is kept when

@@ -113,6 +113,51 @@ template <typename P> inline size_t bwd_part_floats(const P &p, int Lk, int Hk, 
   return (size_t)chunks * (tangent_grads ? 4 : 2) * ((size_t)p.Z * Hk * Lk * p.D);
 }
 
+// Backward of small grids (16-bit element types, D <= 128, no mask, no dropout, one query head per key/value head, not six
+// gradients): the tiles that a block streams are dealt to several workgroups, dq's and dk/dv's in one launch, which leave fp32
+// shares that bwd_split_merge_kernel adds up.
+//   * As many workgroups as there are compute units; causal, whose blocks have half the tiles on average, up to three a block
+//     and three a unit where that leaves 10 tiles to a share (with fewer the empty and the short ones cost more than they bring:
+//     H16 L1024 D128 60 -> 72 us, H6 L1024 42 -> 48; six for three at H2 L4096 98 -> 119).
+//   * No share under 3 tiles at D = 128, where a tile takes 4 us, 4 at D = 64, 6 at D = 32; and at D = 128 without tangents none
+//     that saves fewer than 7 tiles of 2 us (H8 L700 28 -> 31 us): the merge takes 5 - 10 us.
+//   * At D = 128 more than 8 tiles: a causal call of 512 rows then has the very sums of the first half of one of 1024 (16 heads,
+//     which fill the units unsplit).
+// Measured, bf16 B1, backward, unsplit -> split, dual / plain: D128 H1 L1024 65 -> 32 / 35 -> 23 us, H4 L1024 65 -> 38 / 36 -> 28,
+// H2 L2048 120 -> 53 / 62 -> 35, H4 L2048 121 -> 85 / 62 -> 49, H2 L4096 231 -> 147 / 116 -> 77, causal H2 L4096 228 -> 98 / 115 -> 56, H4 L4096 237 -> 156 / 117 -> 96;
+// D64 H4 L1024 49 -> 28 / 31 -> 23, H2 L2048 90 -> 38 / 55 -> 29, causal H4 L4096 173 -> 116; D32 H4 L1024 34 -> 25 / 24 -> 19,
+// H4 L2048 63 -> 41 / 44 -> 31, causal H4 L4096 121 -> 68.
+struct BwdSplitPlan {
+  int chunks_q, tiles_q, chunks_k, tiles_k;
+  bool any() const { return chunks_q > 1 || chunks_k > 1; }
+};
+inline BwdSplitPlan bwd_split_plan(int D, int Z, int H, int L, int Lk, bool causal, bool dual) {
+  const long long bq = (long long)((L + 127) / 128) * Z * H, bk = (long long)((Lk + 127) / 128) * Z * H, cus = device_cus();
+  const int reach = (L + 127) / 128 * 128, nq = ((causal && reach < Lk ? reach : Lk) + 63) / 64, nk = (L + 63) / 64;
+  const int least = D == 128 ? 3 : D == 64 ? 4 : 6;
+  BwdSplitPlan s = {1, nq, 1, nk};
+  auto deal = [&](int n, int &chunks, int &tiles) {  // n: tiles of the longest block
+    long long c = std::min<long long>(cus / (bq + bk), n / least);
+    if (causal) c = std::max(c, std::min<long long>({3, 3 * cus / (bq + bk), n / 10}));
+    c = std::min<long long>(c, 8);
+    if (c < 2 || (D == 128 && n <= 8)) return;
+    const int per = (int)((n + c - 1) / c);
+    if (D == 128 && !dual && n - per < 7) return;
+    tiles = per, chunks = (n + per - 1) / per;
+  };
+  deal(nq, s.chunks_q, s.tiles_q);
+  deal(nk, s.chunks_k, s.tiles_k);
+  return s;
+}
+template <typename P> inline BwdSplitPlan bwd_split_plan_of(const P &p, int Lk, int Hk, bool tangent_grads, bool dual) {
+  if (p.dtype == 2 || p.D > 128 || p.mask_kind != 0 || p.dropout_p > 0.f || Hk != p.H || tangent_grads) return {1, 0, 1, 0};
+  return bwd_split_plan(p.D, p.Z, p.H, p.L, Lk, p.causal != 0, dual);
+}
+template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const BwdSplitPlan &s) {
+  const size_t heads = (size_t)p.Z * p.H;
+  return heads * p.D * ((s.chunks_q > 1 ? (size_t)s.chunks_q * p.L : 0) + (s.chunks_k > 1 ? (size_t)s.chunks_k * 2 * Lk : 0));
+}
+
 // ---- merge kernels -------------------------------------------------------------------------------
 // Forward.  part = [chunk][row][2][D] accumulators, then [chunk][row][4] statistics.  One thread per (row, 8
 // columns).  With m the largest reference point of the row's chunks and w_c = 2^(m_c - m):

@@ -153,7 +153,7 @@ std::vector<Tensor> backward(const Tensor &q, const Tensor &k, const Tensor &v, 
   a.mask_bits = in<uint32_t>(c.bits_k), a.mask_bits_q = in<uint32_t>(c.bits_q);
   a.Hk = static_cast<int32_t>(k.size(1)), a.Lk = static_cast<int32_t>(k.size(2));
   Tensor shares;
-  if (c.split && a.Hk < a.p.H) {
+  if (c.split) {
     a.split_workspace_bytes = jvpfa_bwd_split_workspace_bytes(&a.p, a.Lk, a.Hk, want_tangent_grads ? 1 : 0);
     if (a.split_workspace_bytes) {
       shares = at::empty({static_cast<int64_t>(a.split_workspace_bytes)}, q.options().dtype(at::kByte).requires_grad(false));
