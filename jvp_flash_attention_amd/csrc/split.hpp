@@ -158,6 +158,37 @@ template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const B
   return heads * p.D * ((s.chunks_q > 1 ? (size_t)s.chunks_q * p.L : 0) + (s.chunks_k > 1 ? (size_t)s.chunks_k * 2 * Lk : 0));
 }
 
+// Whether dk/dv and dq go into one launch (bwd2_both_kernel): it has one end with idle compute units instead of two, and where a
+// kernel has to take both roles' registers fewer of its workgroups share a unit.  So: up to a number of blocks (in units of
+// compute units) that depends on how many do.  two_wgs: bwd2_both_kernel_2wg runs it (where units get more than one workgroup;
+// below that its cap costs 4 %: B1 H8 L2048 95.1 against 91.9 us).
+// D = 128 (one workgroup a unit either way, but for the dq kernel without tangents): causal and masked launches up to 2.5; others
+// where the launches would round up to more passes over the units than the one does, 0.6 of a pass for its end.
+// Measured, bf16, backward, two launches -> one, 288 / 544 / 704 / 1024 - 1152 blocks (dual unless said): D128 269 -> 205, 721 ->
+// 607, 490 -> 492, 1236 -> 1135 us, causal 139 -> 111, 323 -> 316, 295 -> 290; plain 123 -> 100, 332 -> 285, 233 -> 237;
+// D64 (2wg) causal 1024 blocks 314 -> 300, 1152 without a mask 731 -> 677, 1536 615 -> 602; D64 plain 69 -> 54, 164 -> 147,
+// 121 -> 118, 260 -> 245 us, 2048 blocks 471 -> 479; D32 88 -> 81, 253 -> 196, 171 -> 155, 462 -> 415, 2048 blocks 658 -> 644.
+// Where it loses: dropout at D64 plain 704 blocks, whole step 168 -> 206; D32 dual 343 -> 409; six gradients there 267 -> 299.
+template <int D, int MODE>
+inline bool launch_both(long long blocks, long long kv_blocks, bool causal, bool masked, bool drop, bool six, bool grouped, bool two_wgs) {
+  const long long most = blocks > kv_blocks ? blocks : kv_blocks, cus = device_cus();
+  if (cus <= 0) return false;  // the device cannot be asked: two launches
+  if (D == 32) return most <= (drop ? (MODE == BWD_DUAL ? 1.5 : 2.5) : six ? 2.2 : 8.0) * cus;
+  if (D == 64 && MODE == BWD_DUAL) return most <= (six ? 2.5 : two_wgs || drop ? 8.0 : 2.75) * cus;
+  if (D == 64) return most <= (drop ? 1.5 : grouped ? 6.0 : 4.5) * cus;
+  if (most <= cus || ((causal || masked) && most <= 2.5 * cus)) return true;
+  const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
+  return apart > (MODE == BWD_DUAL ? 1.04 : 1.08) * ((double)(blocks + kv_blocks) / cus + 0.6);
+}
+// ... and in fp32: by the rule for D = 128 (one workgroup a compute unit, mostly).
+inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven) {
+  const long long most = blocks > kv_blocks ? blocks : kv_blocks, cus = device_cus();
+  if (cus <= 0) return false;  // the device cannot be asked: two launches
+  if (most <= cus || (uneven && most <= 2.5 * cus)) return true;
+  const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
+  return apart > 1.04 * ((double)(blocks + kv_blocks) / cus + 0.6);
+}
+
 // ---- merge kernels -------------------------------------------------------------------------------
 // Forward.  part = [chunk][row][2][D] accumulators, then [chunk][row][4] statistics.  One thread per (row, 8
 // columns).  With m the largest reference point of the row's chunks and w_c = 2^(m_c - m):
