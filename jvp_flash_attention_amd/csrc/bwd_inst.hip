@@ -115,10 +115,11 @@ static auto pick_both(const BwdParams &p, bool no_go, bool grouped, bool six, lo
   constexpr bool NG = MODE != BWD_DUAL;
   const bool bits = MASK == MASK_BOOL && p.pr.bits_q && p.pr.bits_k;
   constexpr bool M = MASK != MASK_NONE;
+  const int kind = bits ? MASK_BITS : MASK;  // as the kernels read it
   const bool causal = p.pr.causal != 0, two_wgs = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits) && blocks + kv_blocks > device_cus();
   // (six: the dual and the tangent launch of a call decide alike)
-  if (!(six ? launch_both<D, BWD_DUAL>(blocks, kv_blocks, causal, M, false, true, grouped, false)
-            : launch_both<D, MODE>(blocks, kv_blocks, causal, M, false, false, grouped, two_wgs)))
+  if (!(six ? launch_both<D, BWD_DUAL>(blocks, kv_blocks, causal, kind, false, true, grouped, false)
+            : launch_both<D, MODE>(blocks, kv_blocks, causal, kind, false, false, grouped, two_wgs)))
     return nullptr;
   if constexpr (MASK == MASK_ADD) {  // (read element by element here, and as tiles by the dk/dv kernel of its own launch)
     if (blocks >= device_cus() || kv_blocks >= device_cus()) return nullptr;
@@ -230,7 +231,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
       constexpr bool NG = MODE != BWD_DUAL;
       const bool grouped = p.pr.Hk != p.pr.H;
       if constexpr (MASK == MASK_NONE) {
-        if (launch_both<D, MODE>(blocks, kv_blocks, p.pr.causal != 0, false, true, false, grouped, false)) {
+        if (launch_both<D, MODE>(blocks, kv_blocks, p.pr.causal != 0, MASK_NONE, true, false, grouped, false)) {
           void (*kb)(const BwdParams, int);
           if (grouped) kb = no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG, true, false, true> : bwd2_both_kernel<T, D, MODE, MASK, true, true, false, true>;
           else kb = no_go ? bwd2_both_kernel<T, D, MODE, MASK, NG, false, false, true> : bwd2_both_kernel<T, D, MODE, MASK, true, false, false, true>;
@@ -342,7 +343,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     const long long kblocks = (long long)((p.pr.Lk + CfgP::BLK - 1) / CfgP::BLK) * p.pr.Z * p.pr.Hk * p.pr.chunks;
     if (qblocks > 0x7fffffffLL || kblocks > 0x7fffffffLL) return -2;
     void (*kq)(const BwdParams) = no_go ? bwdp_dq_kernel<T, D, MASK, false> : bwdp_dq_kernel<T, D, MASK, true>;
-    if (!six && launch_both<D, MODE>(qblocks, kblocks, p.pr.causal != 0, MASK != MASK_NONE, false, false, false, false)) {
+    if (!six && launch_both<D, MODE>(qblocks, kblocks, p.pr.causal != 0, MASK, false, false, false, false)) {
       void (*kb)(const BwdParams, int) = no_go ? bwdp_both_kernel<T, D, MASK, false> : bwdp_both_kernel<T, D, MASK, true>;
       const int rcb = run_both(kb, p, kblocks, kblocks + qblocks, CfgP::DQ_LDS > CfgP::DKV_LDS ? CfgP::DQ_LDS : CfgP::DKV_LDS, stream);
       if (rcb != 0) return rcb;
@@ -362,7 +363,7 @@ static int launch_bwd_mode(const BwdParams &p, bool six, hipStream_t stream) {
     // without tangents in the launch two operands stay resident and one workgroup holds all 256 columns
     using CfgW = BwdWideCfg<T, D, MODE>;
     using CfgK = BwdWideKvCfg<T, D, MODE>;
-    if (MODE == BWD_PLAIN && launch_both<D, MODE>(blocks, kv_blocks, p.pr.causal != 0, MASK != MASK_NONE, false, false, false, false)) {
+    if (MODE == BWD_PLAIN && launch_both<D, MODE>(blocks, kv_blocks, p.pr.causal != 0, MASK, false, false, false, false)) {
       void (*kb)(const BwdParams, int) = bwdw_both_kernel<T, D, BWD_PLAIN, MASK, true>;
       if constexpr (MASK != MASK_NONE) {
         if (p.pr.chunks <= 1) kb = bwdw_both_kernel<T, D, BWD_PLAIN, MASK, false>;

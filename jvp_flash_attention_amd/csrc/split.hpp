@@ -160,23 +160,43 @@ template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const B
 
 // Whether dk/dv and dq go into one launch (bwd2_both_kernel): it has one end with idle compute units instead of two, and where a
 // kernel has to take both roles' registers fewer of its workgroups share a unit.  So: up to a number of blocks (in units of
-// compute units) that depends on how many do.  two_wgs: bwd2_both_kernel_2wg runs it (where units get more than one workgroup;
-// below that its cap costs 4 %: B1 H8 L2048 95.1 against 91.9 us).
+// compute units) that depends on how many do.  mask: as the kernels read it.  two_wgs: bwd2_both_kernel_2wg runs it (where units get
+// more than one workgroup; below that its cap costs 4 %: B1 H8 L2048 95.1 against 91.9 us).
 // D = 128 (one workgroup a unit either way, but for the dq kernel without tangents): causal and masked launches up to 2.5; others
 // where the launches would round up to more passes over the units than the one does, 0.6 of a pass for its end.
 // Measured, bf16, backward, two launches -> one, 288 / 544 / 704 / 1024 - 1152 blocks (dual unless said): D128 269 -> 205, 721 ->
 // 607, 490 -> 492, 1236 -> 1135 us, causal 139 -> 111, 323 -> 316, 295 -> 290; plain 123 -> 100, 332 -> 285, 233 -> 237;
 // D64 (2wg) causal 1024 blocks 314 -> 300, 1152 without a mask 731 -> 677, 1536 615 -> 602; D64 plain 69 -> 54, 164 -> 147,
 // 121 -> 118, 260 -> 245 us, 2048 blocks 471 -> 479; D32 88 -> 81, 253 -> 196, 171 -> 155, 462 -> 415, 2048 blocks 658 -> 644.
-// Where it loses: dropout at D64 plain 704 blocks, whole step 168 -> 206; D32 dual 343 -> 409; six gradients there 267 -> 299.
+// The lines below those, each where the quotient two / one crosses 1 (L1000, 8 blocks a head, 256 units; at 256 / 288 / 384 / 512 /
+// 640 / 1024 blocks).  Packed masks, a dense one: D32 dual 0.99 / 0.97 / 0.90 / 0.77 / 0.88 / 0.74, D64 plain 1.04 / 0.94 / 0.88 / 0.75 /
+// 0.88 / 0.72 (the separate kernels keep three workgroups on a unit there).  D64 dual on the bytes of a key padding 1.00 / 1.30 / 1.16 /
+// 0.95 / 1.08 / 0.97: past two units' worth the two launches begin a second, mostly empty pass.  Dropout: D32 dual 1.02 / 1.03 / 0.92 /
+// 0.76, causal 1.56 / 1.32 / 1.04 / 0.87; D64 plain 1.03 / 0.98 / 0.87 / 0.72, causal 1.50 / 1.30 / 1.03 / 0.86 (and
+// the tangent launch of six gradients there, which at D32 gains up to 2.5 units' worth).  Six gradients: D32 1.02 /
+// 1.01 / 0.91 / 0.81 / 0.92, causal 1.50 / 1.29 / 1.05 / 0.95, packed mask 1.36 - 1.50 ... 1.07; D64 1.00 / 1.23 / 1.11 / 0.95 / 1.08, causal
+// and packed 1.42 ... 1.01.  Grouped heads, D64 dual: 1.01 / 1.06 / 1.00 / 0.87 / 0.96 / 0.86, causal 1.40 / 1.32 / 1.09 / 0.99 / 0.88; plain
+// (1024, 1536) 1.07, 1.07, causal 1.26, 1.13.
 template <int D, int MODE>
-inline bool launch_both(long long blocks, long long kv_blocks, bool causal, bool masked, bool drop, bool six, bool grouped, bool two_wgs) {
-  const long long most = blocks > kv_blocks ? blocks : kv_blocks, cus = device_cus();
+inline bool launch_both(long long blocks, long long kv_blocks, bool causal, int mask, bool drop, bool six, bool grouped, bool two_wgs,
+                        long long cus = device_cus()) {
   if (cus <= 0) return false;  // the device cannot be asked: two launches
-  if (D == 32) return most <= (drop ? (MODE == BWD_DUAL ? 1.5 : 2.5) : six ? 2.2 : 8.0) * cus;
-  if (D == 64 && MODE == BWD_DUAL) return most <= (six ? 2.5 : two_wgs || drop ? 8.0 : 2.75) * cus;
-  if (D == 64) return most <= (drop ? 1.5 : grouped ? 6.0 : 4.5) * cus;
-  if (most <= cus || ((causal || masked) && most <= 2.5 * cus)) return true;
+  const double most = (double)(blocks > kv_blocks ? blocks : kv_blocks) / cus;
+  const bool bits = mask == MASK_BITS;
+  if (D == 32) {
+    if (MODE == BWD_PLAIN) return most <= (drop ? 2.5 : 8.0);
+    if (drop) return most <= (MODE == BWD_TANGENT ? 2.5 : causal ? 1.5 : 1.25);
+    if (six) return most <= (bits ? 2.2 : causal ? 1.5 : 1.25);
+    return most <= (bits ? 1.0 : 8.0);
+  }
+  if (D == 64 && MODE == BWD_DUAL) {
+    if (two_wgs || drop) return most <= 8.0;
+    if (six && (causal || bits)) return most <= 2.5;
+    if (grouped) return most <= (causal ? 2.0 : 1.5);
+    return most <= 1.5 || (most > 2.0 && most <= (six ? 2.5 : 2.75));
+  }
+  if (D == 64) return most <= (drop ? (causal ? 1.5 : 1.0) : bits ? 1.0 : grouped ? 6.0 : 4.5);
+  if (most <= 1.0 || ((causal || mask != MASK_NONE) && most <= 2.5)) return true;
   const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
   return apart > (MODE == BWD_DUAL ? 1.04 : 1.08) * ((double)(blocks + kv_blocks) / cus + 0.6);
 }

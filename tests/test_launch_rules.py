@@ -1,4 +1,4 @@
-"""The rules that say how a backward is launched, on the CPU: a device that cannot be asked for its compute units."""
+"""The rules that say how a backward is launched, on the CPU."""
 import os
 import subprocess
 
@@ -6,33 +6,68 @@ import pytest
 
 from jvp_flash_attention_amd import build
 
-PROGRAM = """
-#include <cstdio>
-#include "split.hpp"
-using namespace jvpfa;
-template <int D> int all(long long b) {
-  int one = 0;
-  for (int f = 0; f < 32; ++f) {
-    one += launch_both<D, BWD_PLAIN>(b, 2 * b, f & 1, f & 2, f & 4, false, f & 8, f & 16);
-    one += launch_both<D, BWD_DUAL>(2 * b, b, f & 1, f & 2, f & 4, f & 8, false, f & 16);
-    one += launch_both_f32(b, 3 * b, f & 1);
-  }
-  return one;
-}
-int main() {
-  int one = 0;
-  for (long long b : {1LL, 255LL, 300LL, 5000LL}) one += all<32>(b) + all<64>(b) + all<128>(b) + all<256>(b);
-  std::printf("%d %d\\n", device_cus(), one);
-}
-"""
+pytestmark = pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
 
 
-@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
+def run(tmp_path, text, **env):
+    """What a program with `text` in its main prints, numbers apart."""
+    src, exe = tmp_path / "rules.hip", tmp_path / "rules"
+    src.write_text('#include <cstdio>\n#include "split.hpp"\nusing namespace jvpfa;\nint main() {\n' + text + "}\n")
+    subprocess.run([build.HIPCC, *build.FLAGS, "-I", build.CSRC, str(src), "-o", str(exe)], check=True, capture_output=True)
+    r = subprocess.run([str(exe)], env={**os.environ, **env}, capture_output=True, text=True)
+    assert r.returncode == 0, r.returncode
+    return [int(x) for x in r.stdout.split()]
+
+
 def test_device_that_cannot_be_asked(tmp_path):
     """Two launches, whatever the grid (and no division by the number of units)."""
-    src, exe = tmp_path / "rules.hip", tmp_path / "rules"
-    src.write_text(PROGRAM)
-    subprocess.run([build.HIPCC, *build.FLAGS, "-I", build.CSRC, str(src), "-o", str(exe)], check=True, capture_output=True)
-    run = subprocess.run([str(exe)], env={**os.environ, "HIP_VISIBLE_DEVICES": "-1"}, capture_output=True, text=True)
-    assert run.returncode == 0, run.returncode
-    assert run.stdout.split() == ["0", "0"]
+    text = "  int one = 0;\n  for (long long b : {1LL, 255LL, 300LL, 5000LL})\n    for (int f = 0; f < 32; ++f) {\n"
+    for D in (32, 64, 128, 256):
+        text += f"""
+      one += launch_both<{D}, BWD_PLAIN>(b, 2 * b, f & 1, f & 2 ? MASK_BITS : MASK_NONE, f & 4, false, f & 8, f & 16);
+      one += launch_both<{D}, BWD_DUAL>(2 * b, b, f & 1, f & 2 ? MASK_BOOL : MASK_NONE, f & 4, f & 8, false, f & 16);
+      one += launch_both_f32(b, 3 * b, f & 1);
+"""
+    assert run(tmp_path, text + '    }\n  std::printf("%d %d", device_cus(), one);\n', HIP_VISIBLE_DEVICES="-1") == [0, 0]
+
+
+# D, mode, what the call has, and blocks of either role with what was faster on 256 compute units: 1 one launch, 0 two
+SIDES = [
+    (32, "DUAL", "bits", {256: 1, 288: 0, 512: 0, 2048: 0}),
+    (32, "DUAL", "bool", {512: 1, 2048: 1}),
+    (32, "DUAL", "", {512: 1, 2048: 1}),
+    (32, "PLAIN", "bits", {512: 1, 2048: 1}),
+    (64, "PLAIN", "bits", {256: 1, 288: 0, 1024: 0}),
+    (64, "PLAIN", "bool", {288: 1, 1024: 1}),
+    (64, "DUAL", "bits two", {512: 1, 2048: 1}),
+    (64, "DUAL", "bool", {256: 1, 384: 1, 448: 0, 512: 0, 640: 1, 1024: 0}),
+    (32, "DUAL", "drop", {320: 1, 384: 0}),
+    (32, "DUAL", "drop causal", {384: 1, 448: 0}),
+    (32, "TANGENT", "drop", {448: 1, 640: 1}),
+    (64, "PLAIN", "drop", {256: 1, 288: 0, 384: 0}),
+    (64, "PLAIN", "drop causal", {384: 1, 448: 0}),
+    (32, "DUAL", "six", {320: 1, 384: 0, 512: 0}),
+    (32, "DUAL", "six causal", {384: 1, 448: 0}),
+    (32, "DUAL", "six bits", {512: 1}),
+    (64, "DUAL", "six", {384: 1, 448: 0, 512: 0, 640: 1, 704: 0}),
+    (64, "DUAL", "six causal", {512: 1, 640: 1}),
+    (64, "DUAL", "grouped", {384: 1, 448: 0, 512: 0, 704: 0}),
+    (64, "DUAL", "grouped causal", {512: 1, 640: 0}),
+    (64, "PLAIN", "grouped", {1024: 1, 1536: 1}),
+    (128, "DUAL", "", {128: 1, 288: 1, 2048: 0}),
+    (128, "DUAL", "causal", {512: 1, 1024: 0}),
+]
+
+
+def test_one_launch_or_two(tmp_path):
+    text, want, names = "", [], []
+    for D, mode, has, sides in SIDES:
+        f = {x: str(x in has.split()).lower() for x in ("causal", "drop", "six", "grouped", "two")}
+        mask = "MASK_BITS" if "bits" in has else "MASK_BOOL" if "bool" in has else "MASK_NONE"
+        for blocks, one in sides.items():
+            call = f"launch_both<{D}, BWD_{mode}>({blocks}, {blocks}, {f['causal']}, {mask}, {f['drop']}, {f['six']}, {f['grouped']}, {f['two']}, 256)"
+            text += f'  std::printf("%d ", {call} ? 1 : 0);\n'
+            want.append(one)
+            names.append(call)
+    got = run(tmp_path, text)
+    assert [n for n, a, b in zip(names, got, want) if a != b] == []
