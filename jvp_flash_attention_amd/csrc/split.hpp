@@ -121,8 +121,9 @@ template <typename P> inline size_t bwd_part_floats(const P &p, int Lk, int Hk, 
 //     H16 L1024 D128 60 -> 72 us, H6 L1024 42 -> 48; six for three at H2 L4096 98 -> 119).
 //   * No share under 3 tiles at D = 128, where a tile takes 4 us, 4 at D = 64, 6 at D = 32; and at D = 128 without tangents none
 //     that saves fewer than 7 tiles of 2 us (H8 L700 28 -> 31 us): the merge takes 5 - 10 us.
-//   * At D = 128 more than 8 tiles: a causal call of 512 rows then has the very sums of the first half of one of 1024 (16 heads,
-//     which fill the units unsplit).
+//   * At D = 128 shares of up to 8 tiles only where they shorten the longest workgroup of the launch (a dk/dv tile takes 1.25 of
+//     a dq tile) by 3 tiles, and then, as the merge grows with what it reads, only up to a number of them: unsplit / split, dual, at 2, 8, 12, 16 heads
+//     and 512 rows 1.22, 1.06, 1.05, 0.94, causal 1.26, 1.16, 1.14, 1.09; 384 rows 1.15, 0.98, 1.01, 0.94, causal 1.16, 1.06, 1.00, 1.00.
 // Measured, bf16 B1, backward, unsplit -> split, dual / plain: D128 H1 L1024 65 -> 32 / 35 -> 23 us, H4 L1024 65 -> 38 / 36 -> 28,
 // H2 L2048 120 -> 53 / 62 -> 35, H4 L2048 121 -> 85 / 62 -> 49, H2 L4096 231 -> 147 / 116 -> 77, causal H2 L4096 228 -> 98 / 115 -> 56, H4 L4096 237 -> 156 / 117 -> 96;
 // D64 H4 L1024 49 -> 28 / 31 -> 23, H2 L2048 90 -> 38 / 55 -> 29, causal H4 L4096 173 -> 116; D32 H4 L1024 34 -> 25 / 24 -> 19,
@@ -131,8 +132,8 @@ struct BwdSplitPlan {
   int chunks_q, tiles_q, chunks_k, tiles_k;
   bool any() const { return chunks_q > 1 || chunks_k > 1; }
 };
-inline BwdSplitPlan bwd_split_plan(int D, int Z, int H, int L, int Lk, bool causal, bool dual) {
-  const long long bq = (long long)((L + 127) / 128) * Z * H, bk = (long long)((Lk + 127) / 128) * Z * H, cus = device_cus();
+inline BwdSplitPlan bwd_split_plan(int D, int Z, int H, int L, int Lk, bool causal, bool dual, long long cus = device_cus()) {
+  const long long bq = (long long)((L + 127) / 128) * Z * H, bk = (long long)((Lk + 127) / 128) * Z * H;
   const int reach = (L + 127) / 128 * 128, nq = ((causal && reach < Lk ? reach : Lk) + 63) / 64, nk = (L + 63) / 64;
   const int least = D == 128 ? 3 : D == 64 ? 4 : 6;
   BwdSplitPlan s = {1, nq, 1, nk};
@@ -140,13 +141,23 @@ inline BwdSplitPlan bwd_split_plan(int D, int Z, int H, int L, int Lk, bool caus
     long long c = std::min<long long>(cus / (bq + bk), n / least);
     if (causal) c = std::max(c, std::min<long long>({3, 3 * cus / (bq + bk), n / 10}));
     c = std::min<long long>(c, 8);
-    if (c < 2 || (D == 128 && n <= 8)) return;
+    if (c < 2) return;
     const int per = (int)((n + c - 1) / c);
     if (D == 128 && !dual && n - per < 7) return;
     tiles = per, chunks = (n + per - 1) / per;
   };
   deal(nq, s.chunks_q, s.tiles_q);
   deal(nk, s.chunks_k, s.tiles_k);
+  const bool short_q = s.chunks_q > 1 && nq <= 8, short_k = s.chunks_k > 1 && nk <= 8;
+  if (D == 128 && (short_q || short_k)) {
+    auto longest = [](int q, int k) { return std::max((double)q, 1.25 * k); };
+    const double saved = longest(short_q ? nq : s.tiles_q, short_k ? nk : s.tiles_k) - longest(s.tiles_q, s.tiles_k);
+    const double most = (saved >= 4.0 ? 0.75 : 0.3) + (causal ? 0.25 : 0.0);
+    if (saved < 3.0 || (double)(s.chunks_q * bq + s.chunks_k * bk) > most * cus) {
+      if (short_q) s.chunks_q = 1, s.tiles_q = nq;
+      if (short_k) s.chunks_k = 1, s.tiles_k = nk;
+    }
+  }
   return s;
 }
 template <typename P> inline BwdSplitPlan bwd_split_plan_of(const P &p, int Lk, int Hk, bool tangent_grads, bool dual) {

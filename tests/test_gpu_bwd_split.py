@@ -19,7 +19,17 @@ pytestmark = pytest.mark.gpu
 def test_split_blocks(dtype, D, grads, H, L, Lk, causal):
     # lengths in units of one that is split: 12 tiles into shares of no fewer than 3, 4 or 6
     unit = 64 * 12
-    L, Lk = max(1, int(unit * L)), max(1, int(unit * Lk))
+    split_or_not(dtype, D, grads, H, max(1, int(unit * L)), max(1, int(unit * Lk)), causal)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("grads", ["both", "tangent"])
+@pytest.mark.parametrize("H,L,Lk,causal", [(4, 321, 321, False), (4, 512, 512, False), (16, 512, 512, True), (2, 385, 700, False), (2, 1000, 449, True)])
+def test_split_blocks_of_up_to_eight_tiles(dtype, grads, H, L, Lk, causal):
+    split_or_not(dtype, 128, grads, H, L, Lk, causal)
+
+
+def split_or_not(dtype, D, grads, H, L, Lk, causal):
     print("case", dtype, D, grads, H, L, Lk, causal, flush=True)
     g = torch.Generator().manual_seed(L)
     q, qt, go, gt = (torch.randn(1, H, L, D, generator=g).to(dtype) for _ in range(4))

@@ -540,7 +540,7 @@ def test_config5_hvp_sweep_at_every_length(L):
         rb = dense.backward(*f64, np.zeros_like(g64), g64, mask=keep, scale=scale)
         assert _rel(dq[0, h, rows], rb["dq"][0, 0]) <= 2e-2
         assert _rel(dk[0, h, rows], rb["dk"][0, 0, rows]) <= 2e-2 and _rel(dv[0, h, rows], rb["dv"][0, 0, rows]) <= 2e-2
-    # the prefix (one workgroup per query block in both runs: a launch this small would otherwise split the key
+    # the prefix (one workgroup per block in both runs: a launch this small would otherwise split the streamed
     # tiles of a block over several workgroups, differently for the two lengths, and agree to rounding only)
     half = L // 2
     cut = [x[:, :, :half].contiguous() for x in (q, k, v, qt, kt, vt)]
@@ -554,8 +554,16 @@ def test_config5_hvp_sweep_at_every_length(L):
     assert torch.equal(M1[:, :, :half], M2) and torch.equal(mu1[:, :, :half], mu2)
     assert _rel(o, o1) <= 8e-3 and _rel(ot, ot1) <= 8e-3 and (M - M1).abs().max().item() <= 1e-5  # split or not: one ulp
     gt[:, :, half:] = 0
-    full = be.bwd(q, k, v, qt, kt, vt, o1, ot1, M1, mu1, None, gt, None, 0, True, scale)
-    part = be.bwd(*cut, o2, ot2, M2, mu2, None, gt[:, :, :half].contiguous(), None, 0, True, scale)
+    short = gt[:, :, :half].contiguous()
+    _lib.set_split(False)
+    try:
+        full = be.bwd(q, k, v, qt, kt, vt, o1, ot1, M1, mu1, None, gt, None, 0, True, scale)
+        part = be.bwd(*cut, o2, ot2, M2, mu2, None, short, None, 0, True, scale)
+    finally:
+        _lib.set_split(True)
+    again = be.bwd(*cut, o2, ot2, M2, mu2, None, short, None, 0, True, scale)
+    for n, a_, b_ in zip(("dq", "dk", "dv"), part[:3], again[:3]):
+        assert (a_.float() - b_.float()).norm() <= 2.0**-8 * a_.float().norm(), n  # split or not: one rounding of bf16
     for n, a_, b_ in zip(("dq", "dk", "dv"), full[:3], part[:3]):
         assert torch.equal(a_[:, :, :half], b_), n
     assert full[1][:, :, half:].abs().max().item() == 0.0 and full[2][:, :, half:].abs().max().item() == 0.0

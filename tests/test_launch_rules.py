@@ -71,3 +71,20 @@ def test_one_launch_or_two(tmp_path):
             names.append(call)
     got = run(tmp_path, text)
     assert [n for n, a, b in zip(names, got, want) if a != b] == []
+
+
+# D, dual, heads, queries, keys, causal, and the shares of a block of dq and of dk/dv on 256 compute units
+SHARES = [
+    # blocks of up to 8 tiles: cut where that is a tenth faster, whole where it is a tenth slower
+    (128, 1, 1, 512, 512, 0, 2, 2), (128, 1, 12, 512, 512, 0, 2, 2), (128, 1, 16, 512, 512, 0, 1, 1), (128, 1, 16, 512, 512, 1, 2, 2),
+    (128, 1, 4, 384, 384, 0, 2, 2), (128, 1, 8, 384, 384, 0, 1, 1), (128, 1, 8, 384, 384, 1, 2, 2), (128, 1, 12, 384, 384, 1, 1, 1),
+    (128, 1, 4, 320, 1500, 1, 1, 1), (128, 1, 8, 1000, 512, 0, 1, 2), (128, 1, 4, 512, 2000, 0, 3, 1), (128, 1, 2, 512, 2000, 0, 6, 2),  # one role cut is no gain if the other stays long
+    (128, 1, 1, 256, 256, 0, 1, 1), (128, 1, 4, 1024, 1024, 0, 4, 4), (128, 1, 1, 65536, 65536, 1, 1, 1),
+]
+
+
+def test_shares_of_small_backwards(tmp_path):
+    text = "".join(f'  {{ const BwdSplitPlan s = bwd_split_plan({D}, 1, {H}, {L}, {Lk}, {c}, {dual}, 256); std::printf("%d %d ", s.chunks_q, s.chunks_k); }}\n'
+                   for D, dual, H, L, Lk, c, _, _ in SHARES)
+    got = run(tmp_path, text)
+    assert [(x, got[2 * i], got[2 * i + 1]) for i, x in enumerate(SHARES) if (got[2 * i], got[2 * i + 1]) != x[-2:]] == []
