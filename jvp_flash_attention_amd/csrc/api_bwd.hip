@@ -34,8 +34,12 @@ extern "C" size_t jvpfa_bwd_split_workspace_bytes(const jvpfa_problem *p, int32_
   if (!p || check_problem(*p) != JVPFA_OK || check_kv_shape(*p, Lk, Hk) != JVPFA_OK) return 0;
   Lk = Lk > 0 ? Lk : p->L;
   Hk = Hk > 0 ? Hk : p->H;
-  const BwdSplitPlan sp = bwd_split_plan_of(*p, Lk, Hk, tangent_grads != 0, true);  // (without tangents the same or none)
-  if (sp.any()) return bwd_split_floats(*p, Lk, sp) * sizeof(float);
+  size_t floats = 0;  // of the plan with tangents or of that without, whichever takes more
+  for (const bool dual : {false, true}) {
+    const BwdSplitPlan sp = bwd_split_plan_of(*p, Lk, Hk, tangent_grads != 0, dual);
+    if (sp.any()) floats = std::max(floats, bwd_split_floats(*p, Lk, sp));
+  }
+  if (floats) return floats * sizeof(float);
   const int chunks = bwd_kv_chunks(*p, Lk, Hk);
   return chunks > 1 ? bwd_part_floats(*p, Lk, Hk, chunks, tangent_grads != 0) * sizeof(float) : 0;
 }

@@ -118,9 +118,15 @@ template <typename P> inline size_t bwd_part_floats(const P &p, int Lk, int Hk, 
 // shares that bwd_split_merge_kernel adds up.
 //   * As many workgroups as there are compute units; causal, whose blocks have half the tiles on average, up to three a block
 //     and three a unit where that leaves 10 tiles to a share (with fewer the empty and the short ones cost more than they bring:
-//     H16 L1024 D128 60 -> 72 us, H6 L1024 42 -> 48; six for three at H2 L4096 98 -> 119).
-//   * No share under 3 tiles at D = 128, where a tile takes 4 us, 4 at D = 64, 6 at D = 32; and at D = 128 without tangents none
-//     that saves fewer than 7 tiles of 2 us (H8 L700 28 -> 31 us): the merge takes 5 - 10 us.
+//     H16 L1024 D128 60 -> 72 us, H6 L1024 42 -> 48; six for three at H2 L4096 98 -> 119).  Where a unit holds one of them (D = 128;
+//     D = 64 with tangents) and both roles would be cut so, only if the blocks unsplit fit the units (D = 64: and an eighth), and at D = 128 two
+//     a block only if they fit three quarters.
+//     Causal, unsplit / split, at 192, 240 - 256, 288 - 320, 384 blocks of both roles: D128 dual 1.10, 0.93 (two), 1.17 (three), 0.83 - 0.94, 0.76 - 0.85,
+//     plain 0.99, 0.86, 1.00, 0.75 - 0.82, 0.67 - 0.79; D64 dual 1.21 - 1.46, 1.03 - 1.50, 0.85 - 1.02, 0.76 - 0.87, plain 1.27, 1.29, 1.27, 1.03 - 1.23;
+//     D32 1.44, 1.41, 1.35, 0.98 - 1.08.
+//   * No share under 3 tiles at D = 128, where a tile takes 4 us, 4 at D = 64, 6 at D = 32; and without tangents none that saves a
+//     block fewer than 7 tiles of 2 us at D = 128 (H8 L700 28 -> 31 us), the launch fewer than 6 of 1 us at D = 64 (H16 L512 19 -> 22 us): the
+//     merge takes 5 - 10 us.
 //   * At D = 128 shares of up to 8 tiles only where they shorten the longest workgroup of the launch (a dk/dv tile takes 1.25 of
 //     a dq tile) by 3 tiles, and then, as the merge grows with what it reads, only up to a number of them: unsplit / split, dual, at 2, 8, 12, 16 heads
 //     and 512 rows 1.22, 1.06, 1.05, 0.94, causal 1.26, 1.16, 1.14, 1.09; 384 rows 1.15, 0.98, 1.01, 0.94, causal 1.16, 1.06, 1.00, 1.00.
@@ -139,7 +145,12 @@ inline BwdSplitPlan bwd_split_plan(int D, int Z, int H, int L, int Lk, bool caus
   BwdSplitPlan s = {1, nq, 1, nk};
   auto deal = [&](int n, int &chunks, int &tiles) {  // n: tiles of the longest block
     long long c = std::min<long long>(cus / (bq + bk), n / least);
-    if (causal) c = std::max(c, std::min<long long>({3, 3 * cus / (bq + bk), n / 10}));
+    if (causal) {
+      const long long more = std::min<long long>({3, 3 * cus / (bq + bk), n / 10});
+      const bool alone = D == 128 || (D == 64 && dual), both = std::min(nq, nk) >= 20;
+      const bool fits = D == 64 ? 8 * (bq + bk) <= 9 * cus : (more > 2 ? 1.0 : 0.75) * cus >= bq + bk;
+      if (!alone || !both || fits) c = std::max(c, more);
+    }
     c = std::min<long long>(c, 8);
     if (c < 2) return;
     const int per = (int)((n + c - 1) / c);
@@ -148,6 +159,7 @@ inline BwdSplitPlan bwd_split_plan(int D, int Z, int H, int L, int Lk, bool caus
   };
   deal(nq, s.chunks_q, s.tiles_q);
   deal(nk, s.chunks_k, s.tiles_k);
+  if (D == 64 && !dual && std::max(nq, nk) - std::max(s.tiles_q, s.tiles_k) < 6) return {1, nq, 1, nk};
   const bool short_q = s.chunks_q > 1 && nq <= 8, short_k = s.chunks_k > 1 && nk <= 8;
   if (D == 128 && (short_q || short_k)) {
     auto longest = [](int q, int k) { return std::max((double)q, 1.25 * k); };

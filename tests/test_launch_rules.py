@@ -80,6 +80,13 @@ SHARES = [
     (128, 1, 4, 384, 384, 0, 2, 2), (128, 1, 8, 384, 384, 0, 1, 1), (128, 1, 8, 384, 384, 1, 2, 2), (128, 1, 12, 384, 384, 1, 1, 1),
     (128, 1, 4, 320, 1500, 1, 1, 1), (128, 1, 8, 1000, 512, 0, 1, 2), (128, 1, 4, 512, 2000, 0, 3, 1), (128, 1, 2, 512, 2000, 0, 6, 2),  # one role cut is no gain if the other stays long
     (128, 1, 1, 256, 256, 0, 1, 1), (128, 1, 4, 1024, 1024, 0, 4, 4), (128, 1, 1, 65536, 65536, 1, 1, 1),
+    # causal: more shares than units only while the blocks unsplit leave units idle
+    (128, 0, 16, 1500, 1500, 1, 1, 1), (128, 1, 16, 1500, 1500, 1, 1, 1), (128, 1, 10, 1500, 1500, 1, 1, 1), (128, 1, 8, 1500, 1500, 1, 2, 2),
+    (128, 1, 8, 2048, 2048, 1, 3, 3), (128, 0, 10, 2048, 2048, 1, 1, 1), (128, 1, 6, 4096, 4096, 1, 1, 1), (128, 1, 4, 4096, 4096, 1, 3, 3),
+    (128, 1, 12, 1500, 700, 1, 1, 2), (64, 1, 16, 2000, 512, 1, 1, 2),  # (one role cut is less to pay for)
+    (64, 1, 12, 2048, 2048, 1, 1, 1), (64, 1, 6, 3000, 3000, 1, 2, 2), (64, 1, 8, 2048, 2048, 1, 3, 3), (64, 0, 12, 2048, 2048, 1, 2, 2), (32, 1, 10, 2048, 2048, 1, 2, 2),
+    # D = 64 without tangents: not for four tiles
+    (64, 0, 16, 512, 512, 0, 1, 1), (64, 0, 2, 512, 512, 0, 1, 1), (64, 1, 8, 512, 512, 0, 2, 2), (64, 0, 4, 777, 777, 0, 3, 3), (64, 0, 1, 512, 2000, 0, 8, 2),
 ]
 
 
