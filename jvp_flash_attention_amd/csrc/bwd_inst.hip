@@ -116,7 +116,7 @@ static auto pick_both(const BwdParams &p, bool no_go, bool grouped, bool six, lo
   const bool bits = MASK == MASK_BOOL && p.pr.bits_q && p.pr.bits_k;
   constexpr bool M = MASK != MASK_NONE;
   const int kind = bits ? MASK_BITS : MASK;  // as the kernels read it
-  const bool causal = p.pr.causal != 0, two_wgs = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits) && blocks + kv_blocks > device_cus();
+  const bool causal = p.pr.causal != 0, two_wgs = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits) && both_two_wgs(p.pr.L, p.pr.Lk, (long long)p.pr.Z * p.pr.H, causal);
   // (six: the dual and the tangent launch of a call decide alike)
   if (!(six ? launch_both<D, BWD_DUAL>(blocks, kv_blocks, causal, kind, false, true, grouped, false)
             : launch_both<D, MODE>(blocks, kv_blocks, causal, kind, false, false, grouped, two_wgs)))

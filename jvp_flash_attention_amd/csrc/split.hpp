@@ -183,8 +183,8 @@ template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const B
 
 // Whether dk/dv and dq go into one launch (bwd2_both_kernel): it has one end with idle compute units instead of two, and where a
 // kernel has to take both roles' registers fewer of its workgroups share a unit.  So: up to a number of blocks (in units of
-// compute units) that depends on how many do.  mask: as the kernels read it.  two_wgs: bwd2_both_kernel_2wg runs it (where units get
-// more than one workgroup; below that its cap costs 4 %: B1 H8 L2048 95.1 against 91.9 us).
+// compute units) that depends on how many do.  mask: as the kernels read it.  two_wgs: bwd2_both_kernel_2wg runs it
+// (both_two_wgs).
 // D = 128 (one workgroup a unit either way, but for the dq kernel without tangents): causal and masked launches up to 2.5; others
 // where the launches would round up to more passes over the units than the one does, 0.6 of a pass for its end.
 // Measured, bf16, backward, two launches -> one, 288 / 544 / 704 / 1024 - 1152 blocks (dual unless said): D128 269 -> 205, 721 ->
@@ -222,6 +222,23 @@ inline bool launch_both(long long blocks, long long kv_blocks, bool causal, int 
   if (most <= 1.0 || ((causal || mask != MASK_NONE) && most <= 2.5)) return true;
   const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
   return apart > (MODE == BWD_DUAL ? 1.04 : 1.08) * ((double)(blocks + kv_blocks) / cus + 0.6);
+}
+// Whether bwd2_both_kernel_2wg runs a launch of D = 64, dual: two of its workgroups take longer for a pair of blocks than one uncapped for one, so it is for launches whose work, dealt
+// evenly, keeps a unit busy for longer than its longest block takes (tiles, a dk/dv tile 1.25 of a dq tile).  Uncapped / capped with that
+// quotient in brackets: causal, 140 - 250 blocks of either role, L777 - 2048 0.90 - 0.97 (0.59 - 0.95), L512 0.94 (0.70 - 0.84) and 1.04 (0.98), L340 - 640
+// 1.04 - 1.13 (1.01 - 1.13); no mask 0.96 (0.90), 1.15 - 1.25 (0.98 on), 1500 queries over 700 keys 0.93 (0.81), but
+// 512 over 1000 - 2000 1.15 - 1.3.
+inline bool both_two_wgs(int L, int Lk, long long heads, bool causal, long long cus = device_cus()) {
+  const double bq = (L + 127) / 128, bk = (Lk + 127) / 128, nq = (L + 63) / 64, nk = (Lk + 63) / 64;
+  double of_q = bq * nk, of_k = bk * nq, longest = nk;  // tiles of all query blocks, of all key blocks, of the longest query block
+  if (causal) {
+    const double whole = std::min(bq, (double)((Lk + 63) / 64 / 2)), live = std::min(bk, (double)(((L + 63) / 64 + 1) / 2));
+    of_q = whole * (whole + 1) + (bq - whole) * nk, of_k = live * nq - live * (live - 1);
+    longest = std::min(nk, 2 * bq);
+  }
+  if (causal && heads * std::max(bq, bk) >= cus) return true;
+  if (longest > 1.25 * nq) return heads * (bq + bk) > cus;  // long query blocks, which come last, must not wait for the key blocks
+  return heads * (of_q + 1.25 * of_k) > 0.97 * cus * std::max(longest, 1.25 * nq);
 }
 // ... and in fp32: by the rule for D = 128 (one workgroup a compute unit, mostly).
 inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven) {

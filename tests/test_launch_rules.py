@@ -95,3 +95,13 @@ def test_shares_of_small_backwards(tmp_path):
                    for D, dual, H, L, Lk, c, _, _ in SHARES)
     got = run(tmp_path, text)
     assert [(x, got[2 * i], got[2 * i + 1]) for i, x in enumerate(SHARES) if (got[2 * i], got[2 * i + 1]) != x[-2:]] == []
+
+
+def test_capped_kernel_for_both_roles(tmp_path):
+    """Queries, keys, heads, causal: capped where the launch has more work than its longest block for every unit."""
+    sides = {(2048, 2048, 8, 0): 0, (777, 777, 20, 0): 1, (1000, 1000, 24, 0): 1, (1500, 700, 20, 0): 0, (1000, 512, 28, 0): 0, (1000, 512, 96, 0): 1,
+             (512, 2000, 14, 0): 1, (512, 1000, 24, 0): 1, (512, 1000, 20, 0): 0,
+             (2048, 2048, 14, 1): 0, (1500, 1500, 20, 1): 0, (777, 777, 32, 1): 0, (512, 512, 48, 1): 0, (512, 512, 56, 1): 1, (340, 340, 80, 1): 1,
+             (640, 640, 48, 1): 1, (2048, 2048, 16, 1): 1, (512, 2000, 16, 1): 1, (1, 1, 1, 1): 0}
+    got = run(tmp_path, "".join(f'  std::printf("%d ", both_two_wgs({L}, {Lk}, {h}, {c}, 256) ? 1 : 0);\n' for L, Lk, h, c in sides))
+    assert [x for x, y in zip(sides, got) if y != sides[x]] == []
