@@ -118,8 +118,8 @@ static auto pick_both(const BwdParams &p, bool no_go, bool grouped, bool six, lo
   const int kind = bits ? MASK_BITS : MASK;  // as the kernels read it
   const bool causal = p.pr.causal != 0, two_wgs = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits) && both_two_wgs(p.pr.L, p.pr.Lk, (long long)p.pr.Z * p.pr.H, causal);
   // (six: the dual and the tangent launch of a call decide alike)
-  if (!(six ? launch_both<D, BWD_DUAL>(blocks, kv_blocks, causal, kind, false, true, grouped, false)
-            : launch_both<D, MODE>(blocks, kv_blocks, causal, kind, false, false, grouped, two_wgs)))
+  if (!(six ? launch_both<D, BWD_DUAL>(blocks, kv_blocks, causal, kind, false, true, grouped, false, no_go)
+            : launch_both<D, MODE>(blocks, kv_blocks, causal, kind, false, false, grouped, two_wgs, no_go)))
     return nullptr;
   if constexpr (MASK == MASK_ADD) {  // (read element by element here, and as tiles by the dk/dv kernel of its own launch)
     if (blocks >= device_cus() || kv_blocks >= device_cus()) return nullptr;

@@ -199,26 +199,28 @@ template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const B
 // the tangent launch of six gradients there, which at D32 gains up to 2.5 units' worth).  Six gradients: D32 1.02 /
 // 1.01 / 0.91 / 0.81 / 0.92, causal 1.50 / 1.29 / 1.05 / 0.95, packed mask 1.36 - 1.50 ... 1.07; D64 1.00 / 1.23 / 1.11 / 0.95 / 1.08, causal
 // and packed 1.42 ... 1.01.  Grouped heads, D64 dual: 1.01 / 1.06 / 1.00 / 0.87 / 0.96 / 0.86, causal 1.40 / 1.32 / 1.09 / 0.99 / 0.88; plain
-// (1024, 1536) 1.07, 1.07, causal 1.26, 1.13.
+// (1024, 1536) 1.07, 1.07, causal 1.26, 1.13; gradients of O' alone, dual, at 448 / 512 / 640 1.02 / 1.04 / 1.18, causal 1.00 / 1.00 / 1.08.
+// Documents in a packed mask differ with what is drawn: D32 dual 1.05 - 1.28 at 280 - 336 blocks, 0.9 - 1.4 at 384, 0.75 - 1.0 past that; D64
+// plain 0.9 - 1.15 at 280 - 336.  Where they gain what a dense mask loses they have the line.  Padding by batch entry as bytes, D64 dual, at 392 1.12 - 1.16.
 template <int D, int MODE>
 inline bool launch_both(long long blocks, long long kv_blocks, bool causal, int mask, bool drop, bool six, bool grouped, bool two_wgs,
-                        long long cus = device_cus()) {
+                        bool no_go = false, long long cus = device_cus()) {
   if (cus <= 0) return false;  // the device cannot be asked: two launches
   const double most = (double)(blocks > kv_blocks ? blocks : kv_blocks) / cus;
   const bool bits = mask == MASK_BITS;
   if (D == 32) {
     if (MODE == BWD_PLAIN) return most <= (drop ? 2.5 : 8.0);
     if (drop) return most <= (MODE == BWD_TANGENT ? 2.5 : causal ? 1.5 : 1.25);
-    if (six) return most <= (bits ? 2.2 : causal ? 1.5 : 1.25);
-    return most <= (bits ? 1.0 : 8.0);
+    if (six) return most <= (bits ? 2.2 : causal ? 1.5 : 1.35);
+    return most <= (bits ? 1.35 : 8.0);
   }
   if (D == 64 && MODE == BWD_DUAL) {
     if (two_wgs || drop) return most <= 8.0;
     if (six && (causal || bits)) return most <= 2.5;
-    if (grouped) return most <= (causal ? 2.0 : 1.5);
-    return most <= 1.5 || (most > 2.0 && most <= (six ? 2.5 : 2.75));
+    if (grouped) return most <= (no_go ? 2.75 : causal ? 2.0 : 1.5);
+    return most <= 1.6 || (most > 2.0 && most <= (six ? 2.5 : 2.75));
   }
-  if (D == 64) return most <= (drop ? (causal ? 1.5 : 1.0) : bits ? 1.0 : grouped ? 6.0 : 4.5);
+  if (D == 64) return most <= (drop ? (causal ? 1.5 : 1.0) : bits ? 1.3 : grouped ? 6.0 : 4.5);
   if (most <= 1.0 || ((causal || mask != MASK_NONE) && most <= 2.5)) return true;
   const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
   return apart > (MODE == BWD_DUAL ? 1.04 : 1.08) * ((double)(blocks + kv_blocks) / cus + 0.6);

@@ -33,26 +33,27 @@ def test_device_that_cannot_be_asked(tmp_path):
 
 # D, mode, what the call has, and blocks of either role with what was faster on 256 compute units: 1 one launch, 0 two
 SIDES = [
-    (32, "DUAL", "bits", {256: 1, 288: 0, 512: 0, 2048: 0}),
+    (32, "DUAL", "bits", {256: 1, 336: 1, 384: 0, 512: 0, 2048: 0}),
     (32, "DUAL", "bool", {512: 1, 2048: 1}),
     (32, "DUAL", "", {512: 1, 2048: 1}),
     (32, "PLAIN", "bits", {512: 1, 2048: 1}),
-    (64, "PLAIN", "bits", {256: 1, 288: 0, 1024: 0}),
+    (64, "PLAIN", "bits", {256: 1, 320: 1, 384: 0, 1024: 0}),
     (64, "PLAIN", "bool", {288: 1, 1024: 1}),
     (64, "DUAL", "bits two", {512: 1, 2048: 1}),
-    (64, "DUAL", "bool", {256: 1, 384: 1, 448: 0, 512: 0, 640: 1, 1024: 0}),
+    (64, "DUAL", "bool", {256: 1, 392: 1, 448: 0, 512: 0, 640: 1, 1024: 0}),
     (32, "DUAL", "drop", {320: 1, 384: 0}),
     (32, "DUAL", "drop causal", {384: 1, 448: 0}),
     (32, "TANGENT", "drop", {448: 1, 640: 1}),
     (64, "PLAIN", "drop", {256: 1, 288: 0, 384: 0}),
     (64, "PLAIN", "drop causal", {384: 1, 448: 0}),
-    (32, "DUAL", "six", {320: 1, 384: 0, 512: 0}),
+    (32, "DUAL", "six", {336: 1, 384: 0, 512: 0}),
     (32, "DUAL", "six causal", {384: 1, 448: 0}),
     (32, "DUAL", "six bits", {512: 1}),
     (64, "DUAL", "six", {384: 1, 448: 0, 512: 0, 640: 1, 704: 0}),
     (64, "DUAL", "six causal", {512: 1, 640: 1}),
     (64, "DUAL", "grouped", {384: 1, 448: 0, 512: 0, 704: 0}),
     (64, "DUAL", "grouped causal", {512: 1, 640: 0}),
+    (64, "DUAL", "grouped alone", {512: 1, 640: 1, 768: 0}),  # gradients of O' alone
     (64, "PLAIN", "grouped", {1024: 1, 1536: 1}),
     (128, "DUAL", "", {128: 1, 288: 1, 2048: 0}),
     (128, "DUAL", "causal", {512: 1, 1024: 0}),
@@ -62,10 +63,10 @@ SIDES = [
 def test_one_launch_or_two(tmp_path):
     text, want, names = "", [], []
     for D, mode, has, sides in SIDES:
-        f = {x: str(x in has.split()).lower() for x in ("causal", "drop", "six", "grouped", "two")}
+        f = {x: str(x in has.split()).lower() for x in ("causal", "drop", "six", "grouped", "two", "alone")}
         mask = "MASK_BITS" if "bits" in has else "MASK_BOOL" if "bool" in has else "MASK_NONE"
         for blocks, one in sides.items():
-            call = f"launch_both<{D}, BWD_{mode}>({blocks}, {blocks}, {f['causal']}, {mask}, {f['drop']}, {f['six']}, {f['grouped']}, {f['two']}, 256)"
+            call = f"launch_both<{D}, BWD_{mode}>({blocks}, {blocks}, {f['causal']}, {mask}, {f['drop']}, {f['six']}, {f['grouped']}, {f['two']}, {f['alone']}, 256)"
             text += f'  std::printf("%d ", {call} ? 1 : 0);\n'
             want.append(one)
             names.append(call)
