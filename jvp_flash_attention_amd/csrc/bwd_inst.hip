@@ -179,7 +179,7 @@ static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blo
   if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), Lds::DKV);
   if (rc != 0) return rc;
   if constexpr (!DROP) {
-    if (launch_both_f32(blocks, kv_blocks, p.pr.causal != 0 || MASK != MASK_NONE)) {
+    if (launch_both_f32<D, MODE>(blocks, kv_blocks, p.pr.causal != 0 || MASK == MASK_BOOL)) {
       void (*kb)(const BwdParams, int) = no_go ? pick_f32_both<D, MODE, MASK, NG>() : pick_f32_both<D, MODE, MASK, true>();
       rc = run_both(kb, p, kv_blocks, kv_blocks + blocks, Lds::DKV, stream);
       if (rc != 0) return rc;

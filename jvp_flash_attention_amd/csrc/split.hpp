@@ -242,13 +242,22 @@ inline bool both_two_wgs(int L, int Lk, long long heads, bool causal, long long 
   if (longest > 1.25 * nq) return heads * (bq + bk) > cus;  // long query blocks, which come last, must not wait for the key blocks
   return heads * (of_q + 1.25 * of_k) > 0.97 * cus * std::max(longest, 1.25 * nq);
 }
-// ... and in fp32: by the rule for D = 128 (one workgroup a compute unit, mostly).
-inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven) {
-  const long long most = blocks > kv_blocks ? blocks : kv_blocks, cus = device_cus();
+// ... and in fp32 (one workgroup a compute unit but at D = 32 without tangents, and the separate dq kernel without tangents at D = 64).
+// uneven: causal, or a boolean mask, which may leave blocks little to do.  Measured as above, two / one at 136 - 160, 168 - 192, 224 -
+// 256, 416, 448 - 512, 640 blocks (L1000): no mask, D64 dual 0.99 - 1.01, 0.90 - 0.94, 1.01, 1.00, 0.98 - 1.01, 1.10, plain 1.13 - 1.19, 0.96, 1.02, 1.03,
+// 0.96 - 0.99, 1.09; D128 1.15, 0.99, 1.01, 1.08, 1.01, 1.16; a bias D64 dual 1.05, 0.93, 1.00, 1.01, 0.98 - 1.01, 1.10, plain at 448 0.96.  Padding by
+// batch entry D64 1.10 - 1.28, 0.97 - 1.09, 1.02, 1.07, 0.98 - 1.02, 1.10; documents 1.14 - 1.23, 1.34 - 1.41, 1.02 - 1.29, 1.13, 1.01 - 1.14, 1.08; a dense
+// mask as a bias; causal 1.5 at 192, 1.02 at 640.  D32 plain, whatever the mask, 1.00 - 1.57, 1.01 - 1.04 at 2048 blocks (and the tangent
+// launch of six gradients alike).
+template <int D, int MODE>
+inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven, long long cus = device_cus()) {
   if (cus <= 0) return false;  // the device cannot be asked: two launches
-  if (most <= cus || (uneven && most <= 2.5 * cus)) return true;
+  const double most = (double)(blocks > kv_blocks ? blocks : kv_blocks) / cus, together = (double)(blocks + kv_blocks) / cus;
+  if (D == 32 && MODE != BWD_DUAL) return most <= 8.0;
+  if (uneven && most <= 2.5) return true;
+  if (most <= 1.0 && (D > 64 || MODE != BWD_DUAL || together <= 1.3 || most > 0.85)) return true;
   const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
-  return apart > 1.04 * ((double)(blocks + kv_blocks) / cus + 0.6);
+  return apart > together + 0.7;
 }
 
 // ---- merge kernels -------------------------------------------------------------------------------

@@ -26,7 +26,7 @@ def test_device_that_cannot_be_asked(tmp_path):
         text += f"""
       one += launch_both<{D}, BWD_PLAIN>(b, 2 * b, f & 1, f & 2 ? MASK_BITS : MASK_NONE, f & 4, false, f & 8, f & 16);
       one += launch_both<{D}, BWD_DUAL>(2 * b, b, f & 1, f & 2 ? MASK_BOOL : MASK_NONE, f & 4, f & 8, false, f & 16);
-      one += launch_both_f32(b, 3 * b, f & 1);
+      one += launch_both_f32<{D}, BWD_PLAIN>(b, 3 * b, f & 1) + launch_both_f32<{D}, BWD_DUAL>(3 * b, b, f & 2);
 """
     assert run(tmp_path, text + '    }\n  std::printf("%d %d", device_cus(), one);\n', HIP_VISIBLE_DEVICES="-1") == [0, 0]
 
@@ -72,6 +72,25 @@ def test_one_launch_or_two(tmp_path):
             names.append(call)
     got = run(tmp_path, text)
     assert [n for n, a, b in zip(names, got, want) if a != b] == []
+
+
+# the same in fp32; "uneven": causal or a boolean mask
+SIDES_F32 = [
+    (32, "PLAIN", "", {168: 1, 448: 1, 2048: 1}),
+    (32, "TANGENT", "", {168: 1, 448: 1}),
+    (32, "DUAL", "", {160: 1, 176: 0, 208: 0, 224: 1, 256: 1, 416: 1, 448: 0, 640: 1, 768: 0}),
+    (64, "DUAL", "", {136: 1, 168: 0, 192: 0, 240: 1, 256: 1, 288: 1, 384: 1, 480: 0, 640: 1, 768: 0}),
+    (64, "PLAIN", "", {160: 1, 192: 1, 224: 1, 448: 0, 2048: 0}),
+    (64, "DUAL", "uneven", {160: 1, 256: 1, 448: 1, 512: 1, 640: 1, 768: 0}),
+    (128, "DUAL", "", {144: 1, 192: 1, 256: 1, 320: 1, 416: 1, 576: 1, 640: 1, 1024: 0}),
+]
+
+
+def test_one_launch_or_two_in_fp32(tmp_path):
+    calls = {f"launch_both_f32<{D}, BWD_{mode}>({n}, {n}, {str(has == 'uneven').lower()}, 256)": one
+             for D, mode, has, sides in SIDES_F32 for n, one in sides.items()}
+    got = run(tmp_path, "".join(f'  std::printf("%d ", {c} ? 1 : 0);\n' for c in calls))
+    assert [c for c, a in zip(calls, got) if a != calls[c]] == []
 
 
 # D, dual, heads, queries, keys, causal, and the shares of a block of dq and of dk/dv on 256 compute units
