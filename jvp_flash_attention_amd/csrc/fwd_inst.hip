@@ -56,7 +56,7 @@ static int launch_fwd2_one(const FwdParams &p, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
-// ... and its software-pipelined form (D = 128).
+// ... and its software-pipelined form (D = 128; D = 64 with tangents or split keys, two workgroups to a compute unit with tangents).
 template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false>
 static int launch_fwd3_one(const FwdParams &p, hipStream_t stream) {
   using Cfg = Fwd2Cfg<T, D, DUAL>;
@@ -167,10 +167,12 @@ static int launch_fwd_mask(const FwdParams &p, int mask, hipStream_t stream) {
   } else if constexpr (sizeof(T) == 2 && D < 128) {
     switch (mask) {
       case MASK_NONE:
-        // D = 64: the pipelined kernel with tangents, from 8 key tiles on (filling and draining it costs two of them), and
-        // wherever the keys are split, which it alone can.  Two workgroups of either share a compute unit.
+        // D = 64: the pipelined kernel with tangents, from 8 key tiles in the longest block on (filling and draining it costs two
+        // of them: causal, 128 queries over 1024 keys, 1.05 of the other's time), and wherever the keys are split, which it alone can.
+        // Two workgroups of either share a compute unit.
         if constexpr (D == 64) {
-          if (p.pr.chunks > 1 || (DUAL && p.pr.Lk >= 512)) return launch_fwd3_one<T, D, DUAL, MASK_NONE>(p, stream);
+          const int reach = p.pr.causal ? (p.pr.L + 127) / 128 * 128 : p.pr.Lk;
+          if (p.pr.chunks > 1 || (DUAL && p.pr.Lk >= 512 && reach >= 512)) return launch_fwd3_one<T, D, DUAL, MASK_NONE>(p, stream);
         }
         return launch_fwd2_one<T, D, DUAL, MASK_NONE>(p, stream);
       case MASK_BOOL: return p.pr.bits_q ? launch_fwd2_one<T, D, DUAL, MASK_BITS>(p, stream) : launch_fwd2_one<T, D, DUAL, MASK_BOOL>(p, stream);
