@@ -94,6 +94,26 @@ __device__ __forceinline__ bool x3_any(bool mine, uint32_t lds0, int wave, int l
   return __builtin_amdgcn_readfirstlane(all ? 1 : 0) != 0;
 }
 
+// A bias is loaded as vectors from rows that start anywhere (an address that is a multiple of 4 is enough for one); element by element
+// the plain kernel at D = 32 spent most of its time on it: B1 H24 L577 81 -> 27 us (fp32 instructions with such loads: 52).
+template <int MASK> __device__ __forceinline__ bool x3_mask_rows(const Problem &pr) {
+  if constexpr (MASK == MASK_ADD) return pr.ms[3] == 1 && (reinterpret_cast<uintptr_t>(pr.mask) & 3) == 0;
+  else return mask_rows_aligned<float, MASK>(pr);
+}
+template <int MASK> __device__ __forceinline__ MaskAhead<float, MASK> x3_mask_fetch8(const Problem &pr, int64_t rowoff, int key0) {
+  if constexpr (MASK == MASK_ADD) {
+    typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+    const f32x4_any *src = reinterpret_cast<const f32x4_any *>(reinterpret_cast<const float *>(pr.mask) + rowoff + key0);
+    const f32x4 lo = src[0], hi = src[1];
+    MaskAhead<float, MASK> m;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m.f[e] = lo[e], m.f[e + 4] = hi[e];
+    return m;
+  } else {
+    return mask_fetch8<float, MASK>(pr, rowoff, key0);
+  }
+}
+
 // Returns whether every output is finite.
 template <int D, bool DUAL, int MASK, bool DROP>
 __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
@@ -157,7 +177,7 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
   const int64_t mrow = MASK != MASK_NONE ? z * pr.ms[0] + h * pr.ms[1] + (int64_t)qld * pr.ms[2] : 0;
   const uint32_t drop_row = DROP ? drop_row_word(pr, zh, qld) : 0u;
   bool mask_al = false;
-  if constexpr (MASK != MASK_NONE) mask_al = mask_rows_aligned<float, MASK>(pr);
+  if constexpr (MASK != MASK_NONE) mask_al = x3_mask_rows<MASK>(pr);
   int kend = pr.causal ? min(Lk, q0 + C::BLK) : Lk;
   TileWalk<BT> walk;  // key tiles visited: up to kend, or the caller's list of those that hold an attended entry
   {
@@ -245,7 +265,7 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
     if constexpr (MASK != MASK_NONE) {
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        mk[c] = (mask_al && jn + BT <= Lk) ? mask_fetch8<float, MASK>(pr, mrow, jn + 16 * c + 8 * g) : mask_fetch8_lim<float, MASK>(pr, mrow, jn + 16 * c + 8 * g);
+        mk[c] = (mask_al && jn + BT <= Lk) ? x3_mask_fetch8<MASK>(pr, mrow, jn + 16 * c + 8 * g) : mask_fetch8_lim<float, MASK>(pr, mrow, jn + 16 * c + 8 * g);
     }
   };
   const int klim = min(pr.causal ? qrow : 0x7fffffff, Lk - 1);

@@ -36,6 +36,32 @@ def test_tile_edges(D, L, Lk, mask):
         assert np.abs(got.double().cpu().numpy() - want).max() <= 1e-4 * max(1.0, np.abs(want).max()), name
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("grads", ["plain", "six"])
+@pytest.mark.parametrize("first,row", [(0, 255), (1, 256), (2, 257), (3, 258), (1, 259)])
+def test_bias_rows_wherever_they_start(D, grads, first, row):
+    """Vector loads of a bias take rows and planes at any element: the same bits as from rows on 16-byte boundaries."""
+    print("case", D, grads, first, row, flush=True)
+    L, Lk, H = 131, 255, 2
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rand = lambda n: torch.randn(1, H, n, D, generator=g, device="cuda")  # noqa: E731
+    a = [rand(L), rand(Lk), rand(Lk), rand(L), rand(Lk), rand(Lk), rand(L), rand(L)]
+    if grads == "plain":
+        a[3:6], a[7] = [None] * 3, None
+    bias = torch.randn(1, H, L, Lk, generator=g, device="cuda")
+    be = _lib.backend()
+
+    def step(first, row):
+        flat = torch.full((first + H * L * row,), float("nan"), device="cuda")
+        mask = flat[first:].as_strided((1, H, L, Lk), (H * L * row, L * row, row, 1))
+        mask.copy_(bias)
+        o, ot, M, mu = be.fwd(*a[:6], mask, _lib.MASK_ADD, False, D**-0.5)
+        return o, ot, *be.bwd(*a[:6], o, ot, M, mu, *a[6:], mask, _lib.MASK_ADD, False, D**-0.5, grads == "six")
+
+    for x, y in zip(step(first, row), step(0, 256)):
+        assert x is y is None or torch.equal(x, y)
+
+
 def test_key_rows_past_32_bits_of_bytes():
     """One query over 2^23 + 70 keys of 512 bytes: one of the first keys, then the last, has a logit of 64, all others 0, and so
     all the weight but e^-64 each.  The exponent 64 log2(e) = 92 is rounded to 92 * 2^-24 on either side of its difference
