@@ -682,7 +682,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   }
   // The query heads that read this key/value head are visited one after another (one, h itself, for
   // the shapes the reference admits); hq is the current one, and what depends on it is set per head:
-  // tile slots 0 Q, 1 G (gO; gT in TANGENT; gT again in DUAL without gO), 2 Q', 3 gT, and the
+  // tile slots 0 Q, 1 G (gO; gT in TANGENT; empty in DUAL without gO), 2 Q', 3 gT, and the
   // statistics slots PLAIN M, -d1 | DUAL M, mu, -a, -(d1 + d2) | TANGENT M, -a
   const int group = GROUPED ? group_share(pr, chunk + 1) - group_share(pr, chunk) : 1;  // ... of this workgroup's share
   const int hq0 = GROUPED ? h * (pr.H / pr.Hk) + group_share(pr, chunk) : h;
@@ -695,7 +695,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
     const size_t qhead = ((size_t)z * pr.H + hq) * L * D * sizeof(T), qrow0 = ((size_t)z * pr.H + hq) * L;
     Qb = reinterpret_cast<const char *>(p.q) + qhead;
     gTb = (DUAL || TAN) ? reinterpret_cast<const char *>(p.gt) + qhead : nullptr;
-    Gb = TAN ? gTb : (has_go ? reinterpret_cast<const char *>(p.go) + qhead : gTb);
+    Gb = TAN ? gTb : NO_G ? nullptr : reinterpret_cast<const char *>(p.go) + qhead;
     Qtb = DUAL ? reinterpret_cast<const char *>(p.qt) + qhead : nullptr;
     st_p[0] = p.M + qrow0;
     st_p[1] = MODE == BWD_PLAIN ? p.neg_d1 + qrow0 : (DUAL ? p.mu + qrow0 : p.neg_a + qrow0);
@@ -739,7 +739,7 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   auto prepare_loads = [&](int stage, int i0, bool on) {
     ld_dst = lds0 + stage * Cfg::STAGEB + (wave * IPW) * 1024;
     ld_rs[0] = tile_rsrc(Qb, i0, on);
-    ld_rs[1] = tile_rsrc(Gb, i0, on);
+    if constexpr (!NO_G) ld_rs[1] = tile_rsrc(Gb, i0, on);
     if constexpr (DUAL) {
       ld_rs[2] = tile_rsrc(Qtb, i0, on);
       ld_rs[3] = tile_rsrc(gTb, i0, on);
