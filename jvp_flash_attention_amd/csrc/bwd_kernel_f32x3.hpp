@@ -11,7 +11,7 @@
 // 1.4e-6 (2-norm, signs mixed; 0.77e-6 for terms of one sign) where the fp32 instructions are by 1.6e-6 (1.2e-6).
 // What bounds them: one wave per SIMD, which pays most of an issue slot for each vector instruction between the matrix ones.
 // Measured, B4 H8 L1024 D64 dual, kernels alone: key padding dq 251 -> 153 us, dk/dv 326 -> 200 us; bias per head dq 263 ->
-// 172 us, dk/dv 339 -> 228 us (its 16 mask values per lane are single loads).
+// 172 us, dk/dv 339 -> 228 us (without a mask the whole backward takes as long).
 #pragma once
 #include "bwd_kernel_f32.hpp"
 #include "fwd_kernel_f32x3.hpp"

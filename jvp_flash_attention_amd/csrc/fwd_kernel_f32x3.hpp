@@ -2,7 +2,8 @@
 //
 // An fp32 matrix instruction does 1/16 of the work of a bf16 one in the same time, and fwd_kernel_f32.hpp keeps the fp32
 // ones busy for 80 - 85 % of its time: what is left to gain is the rate itself.  An fp32 value x is the sum of three bf16
-// values, h = bf16(x), m = bf16(x - h), l = bf16(x - h - m) (both differences are exact; 27 bits with the signs), so
+// values, h = bf16(x), m = bf16(x - h), l = bf16(x - h - m) (both differences are exact; 27 bits with the signs; for |x| from 2^-108 on:
+// below it l is subnormal and its last bits are lost), so
 //     x y = l h' + h l' + m m' + m h' + h m' + h h'     (left out: m l' + l m' + l l', below 2^-26 of the product)
 // is six bf16 products with fp32 accumulation: 6 x 32 cycles for 32x32x16 where the fp32 instructions take 8 x 64.
 // How the sums are formed keeps the error below that of the fp32 instructions.  The matrix cores cut off what a product has

@@ -1,10 +1,11 @@
 // Small grids: when a launch has fewer workgroups than the GPU has compute units (one sequence of a few
-// thousand tokens, a handful of heads), the kernels for 16-bit element types with D = 64 or 128 and no mask split
-// the streamed tiles of every block of owned rows over several workgroups ("chunks").  Each writes fp32
-// partial results to a workspace and a merge kernel combines them with the online-softmax merge (every running
-// quantity is linear in p once the reference points m and c are made common).  The backward of such a launch runs
-// its dk/dv and dq workgroups side by side in one launch instead (bwd2_both_kernel); what it splits is grouped heads
-// (bwd_kv_chunks below).  The reference has nothing like it (one program per 32 query rows, jvp_attention.py:2474).
+// thousand tokens, a handful of heads), the kernels for 16-bit element types without a mask (forward: D = 64 or 128,
+// backward: D <= 128) split the streamed tiles of every block of owned rows over several workgroups ("chunks").  Each writes
+// fp32 partial results to a workspace; the forward's merge kernel combines them with the online-softmax merge (every running
+// quantity is linear in p once the reference points m and c are made common), the backward's adds them up.  Where key/value heads
+// are few (grouped heads), the backward deals the query heads of each to several workgroups (bwd_kv_chunks).  And it runs its dk/dv and
+// dq workgroups in one launch where that leaves fewer units idle (launch_both).  The reference has nothing like it (one
+// program per 32 query rows, jvp_attention.py:2474).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
