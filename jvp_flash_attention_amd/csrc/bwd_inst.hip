@@ -116,10 +116,10 @@ static auto pick_both(const BwdParams &p, bool no_go, bool grouped, bool six, lo
   const bool bits = MASK == MASK_BOOL && p.pr.bits_q && p.pr.bits_k;
   constexpr bool M = MASK != MASK_NONE;
   const int kind = bits ? MASK_BITS : MASK;  // as the kernels read it
-  const bool causal = p.pr.causal != 0, two_wgs = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits) && both_two_wgs(p.pr.L, p.pr.Lk, (long long)p.pr.Z * p.pr.H, causal);
+  const bool causal = p.pr.causal != 0, twin = D == 64 && MODE == BWD_DUAL && !grouped && !six && (!M || bits);
   // (six: the dual and the tangent launch of a call decide alike)
   if (!(six ? launch_both<D, BWD_DUAL>(blocks, kv_blocks, causal, kind, false, true, grouped, false, no_go)
-            : launch_both<D, MODE>(blocks, kv_blocks, causal, kind, false, false, grouped, two_wgs, no_go)))
+            : launch_both<D, MODE>(blocks, kv_blocks, causal, kind, false, false, grouped, twin, no_go)))
     return nullptr;
   if constexpr (MASK == MASK_ADD) {  // (read element by element here, and as tiles by the dk/dv kernel of its own launch)
     if (blocks >= device_cus() || kv_blocks >= device_cus()) return nullptr;
@@ -137,7 +137,8 @@ static auto pick_both(const BwdParams &p, bool no_go, bool grouped, bool six, lo
   }
   if constexpr (D == 64 && MODE == BWD_DUAL && MASK != MASK_ADD) {
     constexpr int MK = MASK == MASK_BOOL ? MASK_BITS : MASK_NONE;
-    if (two_wgs) return no_go ? bwd2_both_kernel_2wg<T, D, MODE, MK, NG> : bwd2_both_kernel_2wg<T, D, MODE, MK, true>;
+    if (twin && both_two_wgs(p.pr.L, p.pr.Lk, (long long)p.pr.Z * p.pr.H, causal))
+      return no_go ? bwd2_both_kernel_2wg<T, D, MODE, MK, NG> : bwd2_both_kernel_2wg<T, D, MODE, MK, true>;
   }
   if constexpr (MASK == MASK_BOOL) {
     if (bits) return no_go ? bwd2_both_kernel<T, D, MODE, MASK_BITS, NG> : bwd2_both_kernel<T, D, MODE, MASK_BITS, true>;

@@ -184,8 +184,8 @@ template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const B
 
 // Whether dk/dv and dq go into one launch (bwd2_both_kernel): it has one end with idle compute units instead of two, and where a
 // kernel has to take both roles' registers fewer of its workgroups share a unit.  So: up to a number of blocks (in units of
-// compute units) that depends on how many do.  mask: as the kernels read it.  two_wgs: bwd2_both_kernel_2wg runs it
-// (both_two_wgs).
+// compute units) that depends on how many do.  mask: as the kernels read it.  twin: the launch has a capped
+// kernel (both_two_wgs says which of the two runs it).
 // D = 128 (one workgroup a unit either way, but for the dq kernel without tangents): causal and masked launches up to 2.5; others
 // where the launches would round up to more passes over the units than the one does, 0.6 of a pass for its end.
 // Measured, bf16, backward, two launches -> one, 288 / 544 / 704 / 1024 - 1152 blocks (dual unless said): D128 269 -> 205, 721 ->
@@ -200,11 +200,15 @@ template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const B
 // the tangent launch of six gradients there, which at D32 gains up to 2.5 units' worth).  Six gradients: D32 1.02 /
 // 1.01 / 0.91 / 0.81 / 0.92, causal 1.50 / 1.29 / 1.05 / 0.95, packed mask 1.36 - 1.50 ... 1.07; D64 1.00 / 1.23 / 1.11 / 0.95 / 1.08, causal
 // and packed 1.42 ... 1.01.  Grouped heads, D64 dual: 1.01 / 1.06 / 1.00 / 0.87 / 0.96 / 0.86, causal 1.40 / 1.32 / 1.09 / 0.99 / 0.88; plain
-// (1024, 1536) 1.07, 1.07, causal 1.26, 1.13; gradients of O' alone, dual, at 448 / 512 / 640 1.02 / 1.04 / 1.18, causal 1.00 / 1.00 / 1.08.
+// (448, 512, 640, 1024, 1536) 0.94 - 0.99, 1.07, 1.10, 1.05, 1.07, causal (1024, 1536) 1.26, 1.13; gradients of O' alone, dual, at 448 / 512 / 640 1.02 / 1.04 / 1.18, causal 1.00 / 1.00 / 1.08.
 // Documents in a packed mask differ with what is drawn: D32 dual 1.05 - 1.28 at 280 - 336 blocks, 0.9 - 1.4 at 384, 0.75 - 1.0 past that; D64
-// plain 0.9 - 1.15 at 280 - 336.  Where they gain what a dense mask loses they have the line.  Padding by batch entry as bytes, D64 dual, at 392 1.12 - 1.16.
+// plain 0.9 - 1.15 at 280 - 336.  Where they gain what a dense mask loses they have the line.  Padding by batch entry as bytes, D64 dual, at 392 1.12 - 1.16,
+// with 512 blocks of one role and 64 - 96 of the other 1.10 - 1.27.
+// D = 128 plain, masked, 448 / 512 blocks: padding 0.97 - 1.06 / 0.98, dense 0.94 / 0.96, documents 1.02 - 1.10 / 1.02 - 1.08.
+// D = 256, whose blocks with tangents have 64 rows, by the same rule: dual 272 / 384 / 448 / 512 / 640 / 896 / 1024 blocks 1.32 / 1.21 / 0.98 / 1.01 / 1.14 / 1.13 /
+// 1.01, causal 1.39 / 1.04 / 1.01 / 1.00 / 1.08 / 1.03 / 1.03, masked 1.34 - 1.45 / 1.22 - 1.26 / 1.00 - 1.20 / 1.01 - 1.09 / 1.13 - 1.16; plain alike.
 template <int D, int MODE>
-inline bool launch_both(long long blocks, long long kv_blocks, bool causal, int mask, bool drop, bool six, bool grouped, bool two_wgs,
+inline bool launch_both(long long blocks, long long kv_blocks, bool causal, int mask, bool drop, bool six, bool grouped, bool twin,
                         bool no_go = false, long long cus = device_cus()) {
   if (cus <= 0) return false;  // the device cannot be asked: two launches
   const double most = (double)(blocks > kv_blocks ? blocks : kv_blocks) / cus;
@@ -216,10 +220,11 @@ inline bool launch_both(long long blocks, long long kv_blocks, bool causal, int 
     return most <= (bits ? 1.35 : 8.0);
   }
   if (D == 64 && MODE == BWD_DUAL) {
-    if (two_wgs || drop) return most <= 8.0;
+    if (twin || drop) return most <= 8.0;
     if (six && (causal || bits)) return most <= 2.5;
     if (grouped) return most <= (no_go ? 2.75 : causal ? 2.0 : 1.5);
-    return most <= 1.6 || (most > 2.0 && most <= (six ? 2.5 : 2.75));
+    const double least = (double)(blocks < kv_blocks ? blocks : kv_blocks) / cus;
+    return (least <= 1.6 || most > 2.0) && most <= (six ? 2.5 : 2.75);
   }
   if (D == 64) return most <= (drop ? (causal ? 1.5 : 1.0) : bits ? 1.3 : grouped ? 6.0 : 4.5);
   if (most <= 1.0 || ((causal || mask != MASK_NONE) && most <= 2.5)) return true;

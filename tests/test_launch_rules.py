@@ -86,6 +86,15 @@ SIDES_F32 = [
 ]
 
 
+def test_one_launch_for_roles_of_unequal_length(tmp_path):
+    """D = 64, dual: few blocks of one role fit beside many of the other, where as many again of them would not."""
+    calls = {f"launch_both<64, BWD_DUAL>({a}, {b}, false, MASK_BOOL, false, false, false, false, false, 256)": one
+             for a, b, one in ((512, 64, 1), (96, 512, 1), (512, 512, 0), (512, 420, 0), (640, 64, 1), (768, 64, 0))}
+    calls["launch_both<64, BWD_DUAL>(512, 16, false, MASK_NONE, false, false, false, true, false, 256)"] = 1  # 4000 queries over 64 keys, uncapped
+    got = run(tmp_path, "".join(f'  std::printf("%d ", {c} ? 1 : 0);\n' for c in calls))
+    assert [c for c, a in zip(calls, got) if a != calls[c]] == []
+
+
 def test_one_launch_or_two_in_fp32(tmp_path):
     calls = {f"launch_both_f32<{D}, BWD_{mode}>({n}, {n}, {str(has == 'uneven').lower()}, 256)": one
              for D, mode, has, sides in SIDES_F32 for n, one in sides.items()}
