@@ -85,13 +85,11 @@ ALONE = {"q": ("k", "kt"), "k": ("q", "qt"), "v": ("go", "gt"), "qt": ("k",), "k
 
 
 @pytest.mark.parametrize("D", [32, 64])
-@pytest.mark.parametrize("where", list(ALONE))
-@pytest.mark.parametrize("call", ["dual", "plain", "mask", "causal", "grouped", "dropout"])
+@pytest.mark.parametrize("where,call", [(w, c) for c in ("dual", "plain", "mask", "causal", "grouped", "dropout") for w in ALONE
+                                        if c != "plain" or w in ("q", "k", "v", "go")])
 def test_a_finite_value_whose_first_part_is_not(D, where, call):
     """3.4e38 rounds to infinity in bf16, and no result may show it: the sums it has a share in start over with the fp32
     instructions.  Bound: that of fp32 sums (above), column by column."""
-    if call == "plain" and where not in ("q", "k", "v", "go"):
-        return
     print("case", D, where, call, flush=True)
     names, L, Lk, H = ("q", "k", "v", "qt", "kt", "vt", "go", "gt"), 200, 150, 4 if call == "grouped" else 1
     x = dict(zip(names, inputs(D, L, Lk, H, 1, 9)))
