@@ -70,6 +70,39 @@ def test_gradients_of_constants_are_constants_under_create_graph(dual):
     assert torch.equal(w.grad, dq)
 
 
+@pytest.mark.parametrize("tangents_require_grad", [False, True])
+def test_dual_tensors_of_any_origin_get_their_gradients(tangents_require_grad):
+    """Leaves, results of other operators and transposed views, dual or not, against the same values as contiguous leaves."""
+    cpu = _inputs(64, torch.bfloat16)
+    go, gt = cpu[6].cuda(), cpu[7].cuda()
+
+    def step(lay, back):
+        leaves = [lay(x.cuda()).requires_grad_(i < 3 or tangents_require_grad) for i, x in enumerate(cpu[:6])]
+        with fwAD.dual_level():
+            q, k, v, qt, kt, _ = (back(x) for x in leaves)
+            v = v * 1  # a result, without a tangent
+            out = JVPAttn.fwd_dual(fwAD.make_dual(q, qt), fwAD.make_dual(k, kt), v)
+            o, ot = fwAD.unpack_dual(out)
+            grads = torch.autograd.grad((o, ot), leaves[: 5 if tangents_require_grad else 3], (go, gt))
+        assert fwAD._current_level < 0 and out.shape == go.shape
+        return [o.detach(), ot.detach(), *(back(g) for g in grads)]
+
+    want = step(lambda x: x, lambda x: x)
+    got = step(lambda x: x.transpose(1, 2).contiguous(), lambda x: x.transpose(1, 2))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_a_primal_changed_in_place_before_its_backward_is_noticed():
+    q, k, v, qt, kt, vt, go, _ = (x.cuda() for x in _inputs(64, torch.bfloat16))
+    q.requires_grad_()
+    with fwAD.dual_level():
+        out = JVPAttn.fwd_dual(*(fwAD.make_dual(a, b) for a, b in zip((q, k, v), (qt, kt, vt))))
+        o, _ = fwAD.unpack_dual(out)
+        k.mul_(2)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(o, q, go)
+
+
 def test_arguments_are_refused_with_the_reason():
     q, k, v = (x.cuda() for x in _inputs(64, torch.bfloat16)[:3])
     with pytest.raises(AssertionError, match="one dtype"):
