@@ -36,7 +36,7 @@ extern "C" size_t jvpfa_bwd_split_workspace_bytes(const jvpfa_problem *p, int32_
   Hk = Hk > 0 ? Hk : p->H;
   size_t floats = 0;  // of the plan with tangents or of that without, whichever takes more
   for (const bool dual : {false, true}) {
-    const BwdSplitPlan sp = bwd_split_plan_of(*p, Lk, Hk, tangent_grads != 0, dual);
+    const BwdDeal sp = bwd_deal_of(*p, Lk, Hk, tangent_grads != 0, dual);
     if (sp.any()) floats = std::max(floats, bwd_split_floats(*p, Lk, sp));
   }
   if (floats) return floats * sizeof(float);
@@ -77,7 +77,7 @@ static int bwd_impl(const jvpfa_bwd_args *a, void *workspace, void *hip_stream) 
   p.dq = a->dq; p.dk = a->dk; p.dv = a->dv;
   p.dqt = a->dqt; p.dkt = a->dkt; p.dvt = a->dvt;
   if (a->split_workspace) {  // few workgroups: split the tiles of every block, or the query heads of every group, if the workspace suffices
-    const BwdSplitPlan sp = bwd_split_plan_of(a->p, p.pr.Lk, p.pr.Hk, ntg == 3, dual);
+    const BwdDeal sp = bwd_deal_of(a->p, p.pr.Lk, p.pr.Hk, ntg == 3, dual);
     if (sp.any() && aligned16(a->split_workspace) && a->split_workspace_bytes >= bwd_split_floats(a->p, p.pr.Lk, sp) * sizeof(float)) {
       p.pr.chunk_tiles = -1;  // (the launcher makes the same plan)
       p.pr.part = static_cast<float *>(a->split_workspace);

@@ -194,21 +194,23 @@ static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blo
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
-// Small grids: every block's tiles split (split.hpp).
+// Small grids: blocks' tiles split (split.hpp).
 template <typename T, int D, int MODE> static int launch_split(const BwdParams &p, bool no_go, hipStream_t stream) {
   using Cfg = Bwd2Cfg<T, D, MODE>;
   const Problem &pr = p.pr;
-  const BwdSplitPlan s = bwd_split_plan(D, pr.Z, pr.H, pr.L, pr.Lk, pr.causal != 0, MODE == BWD_DUAL);
-  BwdSplit sp = {s.chunks_q, s.tiles_q, s.chunks_k, s.tiles_k, pr.part, pr.part};
-  if (s.chunks_q > 1) sp.part_k += (size_t)s.chunks_q * pr.Z * pr.H * pr.L * D;
-  const int heads = pr.Z * pr.H, kv_blocks = (pr.Lk + 127) / 128 * heads * s.chunks_k, blocks = (pr.L + 127) / 128 * heads * s.chunks_q;
+  const BwdDeal d = bwd_deal(D, pr.Z, pr.H, pr.L, pr.Lk, pr.causal != 0, MODE == BWD_DUAL);
+  BwdSplit sp = {d.q, d.k, pr.part, pr.part};
+  if (d.q.most > 1) sp.part_k += (size_t)d.q.most * pr.Z * pr.H * pr.L * D;
+  const int heads = pr.Z * pr.H, bq = (pr.L + 127) / 128, bk = (pr.Lk + 127) / 128;
+  const int kv_blocks = heads * (d.k.step > 0 ? d.k.workgroups() + std::max(bk - bq, 0) : bk * d.k.most);
+  const int blocks = heads * (d.q.step > 0 ? d.q.workgroups() : bq * d.q.most);
   auto kern = no_go ? bwd2_split_kernel<T, D, MODE, MODE != BWD_DUAL> : bwd2_split_kernel<T, D, MODE, true>;
   constexpr size_t LDS = Cfg::DKV_LDS > Cfg::DQ_LDS ? Cfg::DKV_LDS : Cfg::DQ_LDS;
   const int rc = allow_lds(reinterpret_cast<const void *>(kern), LDS);
   if (rc != 0) return rc;
   hipLaunchKernelGGL(kern, dim3((unsigned)(kv_blocks + blocks)), dim3(Cfg::NT), LDS, stream, p, sp, kv_blocks);
-  const size_t elems = (size_t)heads * (pr.L > pr.Lk ? pr.L : pr.Lk) * D;
-  hipLaunchKernelGGL((bwd_split_merge_kernel<T, D>), dim3((unsigned)((elems / 8 + 255) / 256), 3), dim3(256), 0, stream, p, sp);
+  constexpr int RPB = 2048 / D;
+  hipLaunchKernelGGL((bwd_split_merge_kernel<T, D>), dim3((unsigned)((std::max(pr.L, pr.Lk) + RPB - 1) / RPB), heads, 3), dim3(256), 0, stream, p, sp);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 

@@ -78,7 +78,7 @@ template <int N> __device__ __forceinline__ void lds_wait4(u32x4 &a, u32x4 &b, u
 // SLOTn are LDS tile slots inside a stage; a tile is BT rows, row-major, chunks swizzled by swz_u.
 // the loads of the next tile are spread over the first three quarters of a tile's steps
 constexpr int bwd_spread(int nstep) { return 3 * nstep / 4; }
-#define JVPFA_BWD2_COMMON(Cfg, STREAMED_ROWS, OWN_ROWS, OWN_HEADS, CHUNKS)                                                                                      \
+#define JVPFA_BWD2_COMMON(Cfg, STREAMED_ROWS, OWN_ROWS, OWN_HEADS, CHUNKS, DEALT)                                                                                 \
   constexpr int CH = Cfg::CH, ROWB = Cfg::ROWB, TILEB = Cfg::TILEB, IPW = Cfg::IPW, BT = Cfg::BT;                   \
   constexpr int KK = D / 16, DB = D / 32;                                                                           \
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];                                        \
@@ -87,7 +87,7 @@ constexpr int bwd_spread(int nstep) { return 3 * nstep / 4; }
   const int L = pr.L;                                                                                               \
   /* a workgroup owns 128 of the OWN_ROWS rows of one (z, head out of OWN_HEADS), or one of CHUNKS shares of it */ \
   const int nblk = ((OWN_ROWS) + Cfg::BLK - 1) / Cfg::BLK;                                                          \
-  const int id = xcd_remap(bid, nblk, pr.Z * (OWN_HEADS) * (CHUNKS), pr.causal != 0);                                               \
+  const int id = (DEALT) >= 0 ? (DEALT) : xcd_remap(bid, nblk, pr.Z * (OWN_HEADS) * (CHUNKS), pr.causal != 0);                      \
   const int zh = id / nblk / (CHUNKS), chunk = id / nblk % (CHUNKS);                                                \
   const int z = zh / (OWN_HEADS), h = zh % (OWN_HEADS);                                                             \
   const int tid = threadIdx.x;                                                                                      \
@@ -149,11 +149,11 @@ __device__ __forceinline__ void zero_acc(f32x16 &x) {
   for (int e = 0; e < 16; ++e) x[e] = 0.f;
 }
 
-// Small grids: the streamed tiles of a block are dealt to `chunks` workgroups, tiles_x each, which leave fp32 partial results
-// where a block has more than one (bwd_split_merge_kernel adds them up).
+// Small grids: the streamed tiles of a block are dealt to several workgroups (Deal), which leave fp32 partial results where a block
+// has more than one (bwd_split_merge_kernel adds them up).
 struct BwdSplit {
-  int chunks_q, tiles_q, chunks_k, tiles_k;
-  float *part_q, *part_k;  // [chunk][Z H L D], [chunk][dk, dv][Z H Lk D]
+  Deal q, k;
+  float *part_q, *part_k;  // [share][Z H L D], [share][dk, dv][Z H Lk D]
 };
 
 // ------------------------------------------------------------------------------------------------
@@ -176,12 +176,22 @@ constexpr bool dq_init(int d, int mode, int mask, bool go, bool six, bool drop) 
 // the compiler to keep in registers, for the variant that must stay within 256 of them.
 // START: where dq_init says so.
 template <typename T, int D, int MODE, int MASK, bool GO, bool SIX, bool DROP = false, bool LEAN = false, bool START = true, bool SPLIT = false>
-__device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid_, const BwdSplit sp = {}) {
+__device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid_, const BwdSplit sp = {}, const int total = 0) {
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   static_assert(!SIX || DUAL, "dq' rides on the dual mode");
-  const int bid = SPLIT ? bid_ / sp.chunks_q : bid_, part = SPLIT ? bid_ % sp.chunks_q : 0;
-  JVPFA_BWD2_COMMON(Cfg, pr.Lk, pr.L, pr.H, 1)  // owns query rows, streams key tiles
+  int bid = bid_, dealt = -1;
+  Share share = {0, 1, 0};
+  if constexpr (SPLIT) {
+    if (sp.q.step > 0) {  // (the id of a causal block counts from the last one)
+      const HeadRank hr = deal_heads(bid_, p.pr.Z * p.pr.H, total, more_than_units());
+      share = share_of(sp.q, hr.rank);
+      dealt = hr.head * sp.q.last + sp.q.last - 1 - share.order;
+    } else {
+      share.count = sp.q.most, share.index = bid_ % sp.q.most, bid = bid_ / sp.q.most;
+    }
+  }
+  JVPFA_BWD2_COMMON(Cfg, pr.Lk, pr.L, pr.H, 1, dealt)  // owns query rows, streams key tiles
   const int qb = pr.causal ? nblk - 1 - id % nblk : id % nblk;
   const int q0 = qb * Cfg::BLK;
   const int qrow = q0 + wave * 32 + r;
@@ -261,9 +271,10 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid_,
   }
   const int tmax = (Lk + BT - 1) / BT - 1;  // index of the last tile of the sequence: bounds whatever a list holds
   const int nall = tlist ? min(max(tlist[0], 1), tmax + 1) : (kend + BT - 1) / BT;
-  const int tb = SPLIT ? part * sp.tiles_q : 0;  // SPLIT: this workgroup's tiles are tb .. tb + ntiles - 1
+  const int per = SPLIT && share.count > 1 ? (nall + share.count - 1) / share.count : nall;
+  const int tb = SPLIT ? share.index * per : 0;  // SPLIT: this workgroup's tiles are tb .. tb + ntiles - 1
   if (SPLIT && tb > 0 && tb >= nall) return;
-  const int ntiles = SPLIT ? min(nall - tb, sp.tiles_q) : nall;
+  const int ntiles = SPLIT ? min(nall - tb, per) : nall;
   // List elements are requested a tile ahead, unconditionally (from a harmless address when there is
   // no list: a branch around the read would split the tile loop's straight-line body).
   auto list_slot = [&](int i) { return tlist ? tlist + 1 + i : reinterpret_cast<const int *>(p.q); };
@@ -521,7 +532,7 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid_,
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = acc[db][8 * hf + e] * pr.scale;
-        if (SPLIT && nall > sp.tiles_q) store8<float>(sp.part_q + (size_t)part * pr.Z * pr.H * L * D + head + (size_t)qrow * D + 32 * db + 16 * hf + 8 * g, x);
+        if (SPLIT && share.count > 1) store8<float>(sp.part_q + (size_t)share.index * pr.Z * pr.H * L * D + head + (size_t)qrow * D + 32 * db + 16 * hf + 8 * g, x);
         else store8<T>(out + 32 * db + 16 * hf + 8 * g, x);
         if constexpr (SIX) {
 #pragma unroll
@@ -568,12 +579,24 @@ __global__ __launch_bounds__(256, 2) void bwd2_dq_kernel_2wg_plain(const BwdPara
 // SIX (dual mode only): dk' = scale dS'^T Q and dv' = P^T gT as well, from the fragments and tiles that dk, dv
 // already have (two more accumulators: fits for D <= 64).
 template <typename T, int D, int MODE, int MASK, bool GO, bool GROUPED, bool SIX, bool DROP = false, bool SPLIT = false>
-__device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid_, const BwdSplit sp = {}) {
-  const int bid = SPLIT ? bid_ / sp.chunks_k : bid_, part = SPLIT ? bid_ % sp.chunks_k : 0;
+__device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid_, const BwdSplit sp = {}, const int total = 0) {
+  int bid = bid_, dealt = -1;
+  Share share = {0, 1, 0};
+  if constexpr (SPLIT) {
+    if (sp.k.step > 0) {
+      const HeadRank hr = deal_heads(bid_, p.pr.Z * p.pr.H, total, more_than_units());
+      const int seen = sp.k.workgroups();  // ... then the key blocks behind the last query, which have zero gradients
+      if (hr.rank < seen) share = share_of(sp.k, hr.rank);
+      const int block = hr.rank < seen ? sp.k.last - 1 - share.order : sp.k.last + hr.rank - seen;
+      dealt = hr.head * ((p.pr.Lk + 127) / 128) + block;
+    } else {
+      share.count = sp.k.most, share.index = bid_ % sp.k.most, bid = bid_ / sp.k.most;
+    }
+  }
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   static_assert(!SIX || (DUAL && D <= 64), "dk', dv' ride on the dual mode, where the accumulators fit");
-  JVPFA_BWD2_COMMON(Cfg, pr.L, pr.Lk, pr.Hk, GROUPED ? pr.chunks : 1)  // owns key rows (h: key/value head), streams query tiles
+  JVPFA_BWD2_COMMON(Cfg, pr.L, pr.Lk, pr.Hk, GROUPED ? pr.chunks : 1, dealt)  // owns key rows (h: key/value head), streams query tiles
   const int kb = id % nblk;  // causal: the first key blocks have the longest query loops
   const int k0 = kb * Cfg::BLK;
   const int krow = k0 + wave * 32 + r;
@@ -588,8 +611,8 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
     auto put = [&](void *dst, int t, const float *x) {
       const size_t off = head + (size_t)krow * D + d0;
       if constexpr (GROUPED) store8_or_part<T>(reinterpret_cast<T *>(dst), kv_part(pr, D, NT, t, chunk), off, x);
-      else if (SPLIT && L - (pr.causal ? (k0 / BT) * BT : 0) > sp.tiles_k * BT)
-        store8<float>(sp.part_k + ((size_t)part * 2 + t) * ((size_t)pr.Z * pr.Hk * Lk * D) + off, x);
+      else if (SPLIT && share.count > 1)
+        store8<float>(sp.part_k + ((size_t)share.index * 2 + t) * ((size_t)pr.Z * pr.Hk * Lk * D) + off, x);
       else store8<T>(reinterpret_cast<T *>(dst) + off, x);
     };
     put(TAN ? p.dkt : p.dk, 0, xk);
@@ -716,9 +739,10 @@ __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid
   const int *tlist = nullptr;
   const int tmax = (L + BT - 1) / BT - 1;  // index of the last tile of the sequence: bounds whatever a list holds
   const int nall = (L - istart + BT - 1) / BT;
-  const int tb = SPLIT ? part * sp.tiles_k : 0;  // SPLIT: this workgroup's tiles are tb .. tb + ntiles - 1
+  const int per = SPLIT && share.count > 1 ? (nall + share.count - 1) / share.count : nall;
+  const int tb = SPLIT ? share.index * per : 0;  // SPLIT: this workgroup's tiles are tb .. tb + ntiles - 1
   if (SPLIT && tb > 0 && tb >= nall) return;
-  int ntiles = SPLIT ? min(nall - tb, sp.tiles_k) : nall;
+  int ntiles = SPLIT ? min(nall - tb, per) : nall;
   auto set_list = [&](int hq_) {
     if constexpr (MASK != MASK_NONE) {
       if (pr.tiles_k) {
@@ -1229,32 +1253,34 @@ __global__ __launch_bounds__(256, 1) void bwd2_all_kernel(const BwdParams p, con
 #endif
 }
 
-// Both roles in one launch, each block's tiles split (no mask, ungrouped).
+// Both roles in one launch, blocks' tiles split (no mask, ungrouped).
 template <typename T, int D, int MODE, bool GO>
 __global__ __launch_bounds__(256, 1) void bwd2_split_kernel(const BwdParams p, const BwdSplit sp, const int kv_blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
-  if (b < kv_blocks) bwd2_dkdv_body<T, D, MODE, MASK_NONE, GO, false, false, false, true>(p, b, sp);
-  else bwd2_dq_body<T, D, MODE, MASK_NONE, GO, false, false, false, true, true>(p, b - kv_blocks, sp);
+  if (b < kv_blocks) bwd2_dkdv_body<T, D, MODE, MASK_NONE, GO, false, false, false, true>(p, b, sp, kv_blocks);
+  else bwd2_dq_body<T, D, MODE, MASK_NONE, GO, false, false, false, true, true>(p, b - kv_blocks, sp, gridDim.x - kv_blocks);
 #endif
 }
-// Its partial results added up, in fp32 and in the order of the tiles: one thread per 8 elements of dq, dk, dv (blockIdx.y 0, 1, 2).  Blocks that
-// one workgroup did are complete.  Bound by memory: chunks * 4 + sizeof(T) bytes an element.
+// Its partial results added up, in fp32 and in the order of the tiles: one thread per 8 elements of dq, dk, dv (blockIdx.z 0, 1, 2)
+// of head blockIdx.y.  Blocks that one workgroup did are complete.  Bound by memory: shares * 4 + sizeof(T) bytes an element.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void bwd_split_merge_kernel(const BwdParams p, const BwdSplit sp) {
   const Problem &pr = p.pr;
-  const int t = blockIdx.y, len = t == 0 ? pr.L : pr.Lk, other = t == 0 ? pr.Lk : pr.L;
-  const size_t elems = (size_t)pr.Z * pr.H * len * D, i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
-  if (i >= elems) return;
-  const int row0 = (int)(i / D % len) / 128 * 128;  // first row of the block
+  constexpr int RPB = 2048 / D;  // rows of a workgroup
+  const int t = blockIdx.z, len = t == 0 ? pr.L : pr.Lk, other = t == 0 ? pr.Lk : pr.L;
+  const int first = blockIdx.x * RPB, block = first / 128;  // (uniform: RPB divides 128)
   // streamed rows of the block: keys up to its last row, queries from its first 64-row tile on (causal), or all
-  const int rows = !pr.causal ? other : t == 0 ? min(other, row0 + 128) : max(other - row0 / 64 * 64, 0);
-  const int tiles = (rows + 63) / 64, per = t == 0 ? sp.tiles_q : sp.tiles_k;
-  if (tiles <= per) return;
+  const int rows = !pr.causal ? other : t == 0 ? min(other, block * 128 + 128) : max(other - block * 128, 0);
+  const Deal &d = t == 0 ? sp.q : sp.k;
+  const int tiles = (rows + 63) / 64, dealt = d.step > 0 ? d.shares(t == 0 ? block : d.last - 1 - block) : d.most;
+  if (dealt == 1 || first + (int)threadIdx.x / (D / 8) >= len) return;
+  const int per = (tiles + dealt - 1) / dealt;
+  const size_t elems = (size_t)pr.Z * pr.H * len * D, i = ((size_t)blockIdx.y * len + first) * D + threadIdx.x * 8;
   const float *src = t == 0 ? sp.part_q : sp.part_k + (size_t)(t - 1) * elems;
   const size_t step = t == 0 ? elems : 2 * elems;
   float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int c = 0; c * per < tiles; ++c) {
+  for (int c = 0; c == 0 || c * per < tiles; ++c) {
     const f32x8 x = ld8<float>(src + c * step + i);
 #pragma unroll
     for (int e = 0; e < 8; ++e) sum[e] += x[e];

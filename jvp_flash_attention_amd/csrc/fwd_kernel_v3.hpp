@@ -69,12 +69,22 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L;
   const int nqb = (L + Cfg::BM - 1) / Cfg::BM;
-  // small grids: the key tiles of a query block are split over pr.chunks workgroups (see split.hpp)
-  const int chunks = pr.chunks;
-  const int chunk = chunks > 1 ? (int)(blockIdx.x % chunks) : 0;
-  const int id = xcd_remap(chunks > 1 ? blockIdx.x / chunks : blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
-  const int zh = id / nqb;
-  const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
+  // small grids: the key tiles of query blocks are split over workgroups (see split.hpp), of every block alike or as Deal says
+  constexpr bool DEALT = MASK == MASK_NONE && !DROP && D <= 128;
+  const int chunks = DEALT ? pr.chunks : 1;
+  int zh, qb;
+  Share share = {0, 1, 0};
+  if (chunks > 1 && pr.chunk_tiles > 0) {
+    const HeadRank hr = deal_heads(blockIdx.x, pr.Z * pr.H, gridDim.x, more_than_units());
+    share = share_of(Deal{chunks, pr.chunk_tiles, 0, nqb}, hr.rank);
+    zh = hr.head, qb = share.order;
+  } else {
+    share.count = chunks, share.index = chunks > 1 ? (int)(blockIdx.x % chunks) : 0;
+    const int id = xcd_remap(chunks > 1 ? blockIdx.x / chunks : blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
+    zh = id / nqb;
+    qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
+  }
+  const bool split = share.count > 1;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
@@ -96,7 +106,7 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
     if (pr.klimit) kend = min(kend, max(__builtin_amdgcn_readfirstlane(pr.klimit[zh / pr.H]), 1));
   }
   const int nt_all = (kend + BN - 1) / BN;
-  const int t_first = chunks > 1 ? min(chunk * pr.chunk_tiles, nt_all) : 0;
+  const int share_tiles = split ? (nt_all + share.count - 1) / share.count : nt_all, t_first = split ? share.index * share_tiles : 0;
   // Tiles visited: t_first .. t_first + ntiles - 1, or (with a mask) the caller's list of the tiles of this query
   // block that hold an attended entry (ascending; a tile left out would have contributed exact zeros).
   const int *tlist = nullptr;
@@ -106,13 +116,13 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   const int tmax = (pr.Lk + BN - 1) / BN - 1;  // index of the last tile of the sequence: bounds whatever a list holds
   // (what is read from a list is the same in every lane; saying so keeps the tile pointers in scalar registers)
   const int ntiles = tlist ? __builtin_amdgcn_readfirstlane(min(max(tlist[0], 1), tmax + 1))
-                           : (chunks > 1 ? min(nt_all - t_first, pr.chunk_tiles) : nt_all);  // 0: nothing for this chunk
+                           : min(nt_all - t_first, share_tiles);
   const int k0 = t_first * BN;
   const int Lk = pr.Lk - k0;
   // partial results of a chunk: [chunk][row][O | T][D] floats, then [chunk][row][m, l, mu_acc, c]
-  const size_t nrows = (size_t)pr.Z * pr.H * L, prow = (size_t)chunk * nrows + (size_t)zh * L + qrow;
-  float *part_stat = pr.part + (size_t)chunks * nrows * 2 * D + prow * 4;
-  if (chunks > 1 && ntiles <= 0) {  // no tile falls to this chunk (short causal rows): it weighs nothing
+  const size_t nrows = (size_t)pr.Z * pr.H * L, prow = (size_t)share.index * nrows + (size_t)zh * L + qrow;
+  float *part_stat = pr.part + (size_t)pr.chunks * nrows * 2 * D + prow * 4;
+  if (split && ntiles <= 0) {  // fewer tiles than shares would take: this one weighs nothing
     if (qrow < L && g == 0) {
       const f32x4 none = {-__builtin_inff(), 0.f, 0.f, 0.f};
       *reinterpret_cast<f32x4 *>(part_stat) = none;
@@ -720,7 +730,7 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   // ---- epilogue ---------------------------------------------------------------------------------
   l_i += xor32(l_i);
   if constexpr (DUAL) mu_i += xor32(mu_i);
-  if (chunks > 1) {  // this chunk's share, left as it stands for the merge kernel
+  if (split) {  // this chunk's share, left as it stands for the merge kernel
     if (qrow < L) {
       float *pa = pr.part + prow * 2 * D;
 #pragma unroll

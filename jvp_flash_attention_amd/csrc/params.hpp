@@ -32,9 +32,8 @@ struct Problem {
   // of word hf being the entry of (query, key 64 * tile + 32 * hf + i); keys past Lk are zero bits.  For the forward and
   // dq kernels, whose lanes own a query.
   const uint32_t *bits_q;
-  // Split of the streamed tiles of one block of owned rows over `chunks` workgroups (1 = no split), used when
-  // a launch would otherwise leave most compute units idle: workgroup c of a block takes the tiles
-  // c * chunk_tiles .. (c + 1) * chunk_tiles - 1 and writes fp32 partial results to `part`, which a merge
+  // Forward: how the key tiles of query blocks are split over workgroups (Deal; 1 = no split), used when a launch would
+  // otherwise leave most compute units idle.  A share of a split block leaves fp32 partial results in `part`, which a merge
   // kernel adds up.  Only the kernels for 16-bit element types, D = 64 or 128, without a mask.
   // In the backward: the query heads of a key/value head's group are dealt to `chunks` dk/dv workgroups (see
   // split.hpp), each of which leaves its share of the gradients in `part`; chunk_tiles = -1: `part` is there for the shares
@@ -105,6 +104,47 @@ __host__ __device__ inline size_t mask_bits_q_offset(const Problem &pr, int z, i
 }
 __host__ __device__ inline size_t mask_bits_offset(const Problem &pr, int z, int h) {
   return tile_list_plane(pr, z, h) * (size_t)((pr.L + 63) / 64) * (size_t)pr.Lk * 2;
+}
+
+// How a head's causal blocks are dealt to workgroups that share their streamed tiles.  Blocks are counted by length: each block
+// streams two tiles more than the one before in that `order`, so the orders below `step` get one workgroup, the next `step` two,
+// and so on up to `most`: every share is then about as long.  (step 0, host only: every block gets `most`.)  A head's blocks are
+// the orders first .. last - 1.
+struct Deal {
+  int most, step, first, last;
+  __host__ __device__ int shares(int order) const {
+    int c = 1;
+    while (c < most && order >= c * step) ++c;
+    return c;
+  }
+  __host__ __device__ int workgroups() const {
+    int n = 0, hi = last;
+    for (int c = most; c > 0; --c) {
+      const int from = (c - 1) * step, lo = from > first ? from : first;
+      if (lo < hi) n += (hi - lo) * c, hi = lo;
+    }
+    return n;
+  }
+};
+struct Share {
+  int order, count, index;
+};
+// Workgroup `rank` of a head, roughly longest first: the longer half of the whole blocks and all shares (which are about as long:
+// none is shorter than half of the longest), then the shorter half of the whole blocks.
+__host__ __device__ inline Share share_of(const Deal &d, int rank) {
+  const int top = d.most > 1 && d.step < d.last ? d.step : d.last, whole = top > d.first ? top - d.first : 0;
+  const int early = d.most > 1 ? (whole + 1) / 2 : whole;
+  if (rank < early) return {top - 1 - rank, 1, 0};
+  rank -= early;
+  int hi = d.last;
+  for (int c = d.most; c > 1; --c) {
+    const int from = (c - 1) * d.step, lo = from > d.first ? from : d.first;
+    if (lo >= hi) continue;
+    if (rank < (hi - lo) * c) return {hi - 1 - rank / c, c, rank % c};
+    rank -= (hi - lo) * c;
+    hi = lo;
+  }
+  return {top - 1 - early - rank, 1, 0};
 }
 
 struct FwdParams {

@@ -20,12 +20,12 @@
 namespace jvpfa {
 
 struct SplitPlan {
-  int chunks, chunk_tiles;
+  int chunks, chunk_tiles;  // as in Problem: Deal::most, Deal::step
 };
 
 // blocks: workgroups of the launch without a split; ntiles_max: streamed tiles of its longest block.
 inline SplitPlan split_plan(long long blocks, int ntiles_max, int cus) {
-  SplitPlan s = {1, ntiles_max};
+  SplitPlan s = {1, 0};
   if (cus <= 0 || blocks <= 0 || 2 * blocks > cus) return s;
   // one workgroup per compute unit at most: a workgroup has a fixed cost of about three tiles (its first loads,
   // filling and draining the pipeline), so a second round of short chunks costs more than it saves
@@ -33,10 +33,57 @@ inline SplitPlan split_plan(long long blocks, int ntiles_max, int cus) {
   if (want > 8) want = 8;
   if (want > ntiles_max / 2) want = ntiles_max / 2;    // a chunk is at least two tiles
   if (want < 2) return s;
-  s.chunk_tiles = (int)((ntiles_max + want - 1) / want);
-  s.chunks = (ntiles_max + s.chunk_tiles - 1) / s.chunk_tiles;
+  const int tiles = (int)((ntiles_max + want - 1) / want);
+  s.chunks = (ntiles_max + tiles - 1) / tiles;
   return s;
 }
+
+// What a launch takes whose blocks differ in length (causal) and are dealt as Deal says, in us, with the longest workgroups first:
+// what the longest takes; where there are more workgroups than places for them also their sum dealt out and a share of the longest
+// for the end, and two of the length at which the places run out.  The constants of a kernel fit what its shares of 1/2 ... 1/8 of the
+// longest block took (17 shapes of 32 - 512 blocks for each of the backward's, within 7 %; what is picked by them is within 8 % of the
+// best of those shares, 1 % on average).
+struct DealCost {
+  double tile;     // of 64 streamed rows
+  double start;    // a workgroup's first loads, filling and draining its pipeline
+  double merge;    // the launch that adds the shares up
+  double traffic;  // a share of weight 1 for every unit, written and read again
+  double end;      // of the longest, see above
+  int places;      // workgroups that share a compute unit without taking longer
+  double pair;     // of two workgroups in turn, see above
+};
+class DealTime {
+ public:
+  DealTime(long long cus, const DealCost &cost) : cus_(cus), c_(cost) { std::fill(of_length_, of_length_ + TOP + 1, 0); }
+  // scale: a tile of this role in tiles; weight: of its shares
+  template <typename N> void add(const Deal &d, long long heads, double scale, double weight, N tiles_of) {
+    for (int order = d.first; order < d.last; ++order) {
+      const int n = tiles_of(order), count = d.shares(order);
+      const double length = (n + count - 1) / count * scale;
+      const long long w = count * heads;
+      sum_ += length * c_.tile * w + w * c_.start, workgroups_ += w, longest_ = std::max(longest_, length * c_.tile);
+      of_length_[std::min((int)length, TOP)] += w;
+      if (count > 1) parts_ += weight * w;
+    }
+  }
+  double total() const {
+    const long long places = cus_ * c_.places;
+    double time = longest_ + c_.start;
+    if (workgroups_ > places) {
+      int length = TOP;
+      for (long long n = of_length_[TOP]; n <= places && length > 0; n += of_length_[length]) --length;
+      time = std::max({time, sum_ / places + c_.end * longest_, 2.0 * (c_.pair * length * c_.tile + c_.start)});
+    }
+    return time + (parts_ > 0.0 ? c_.merge + c_.traffic * parts_ / cus_ : 0.0);
+  }
+
+ private:
+  static constexpr int TOP = 512;
+  long long cus_;
+  DealCost c_;
+  double sum_ = 0.0, longest_ = 0.0, parts_ = 0.0;
+  long long workgroups_ = 0, of_length_[TOP + 1];
+};
 
 // Compute units of the current device (0 if it cannot be asked), looked up once per device.  Callable from any
 // thread: the cache is atomic, and two threads that both find it empty store the same value.
@@ -62,7 +109,7 @@ template <typename P> inline bool split_capable(const P &p) {
   return p.dtype != 2 && (p.D == 128 || p.D == 64) && p.mask_kind == 0 && !(p.dropout_p > 0.f);
 }
 template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk, bool dual) {
-  SplitPlan none = {1, 0};
+  const SplitPlan none = {1, 0};
   if (!split_capable(p)) return none;
   const long long blocks = (long long)((p.L + 127) / 128) * p.Z * p.H;
   int keys = Lk;  // of the longest query block (causal: the last one sees keys up to its own last row)
@@ -73,7 +120,33 @@ template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk, bool d
   // and plain: H4 L1024 34 -> 28 and 18 -> unsplit (19); H4 L2048 62 -> 33 and 32 -> 21; H8 L2048 63 -> 42 and 33 -> 26;
   // H2 L4096 118 -> 44 and 61 -> 28; H4 L4096 119 -> 66 and 61 -> 40.
   if (p.D == 64 && ntiles < (dual ? 16 : 32)) return none;
-  return split_plan(blocks, ntiles, device_cus());
+  const int cus = device_cus();
+  const SplitPlan even = split_plan(blocks, ntiles, cus);
+  if (!p.causal || blocks >= cus || ntiles < 12) return even;
+  // Causal: shares of one length for all blocks (Deal), where the account of DealTime says that it is worth a twentieth; fewer
+  // blocks than there are units, whose longest ones alone set the time otherwise.  (Some launches of up to half as many again would gain as
+  // well, 1.1 - 1.3 times; there every block is one workgroup's, so that the rows of a causal call do not depend on its length in any bit.)
+  // The costs fit what was measured of shares of 1/2 ... 1/8.  Causal, bf16, B1, dual forward / without tangents, before -> this: D128 H8
+  // L2048 57 -> 49 / 34 -> 29 us, H12 L2048 81 -> 64 / 42 -> 34, H6 L4096 148 -> 100 / 77 -> 51, H2 L8192
+  // 162 -> 125 / 85 -> 64; D64 H12 L1500 43 -> 31, H6 L4096 102 -> 64 / 61 -> 39, H2 L8192 111 -> 80 / 66 -> 47, H1 L16384 208 -> 130 /
+  // 121 -> 73; none of 60 shapes slower.
+  const bool wide = p.D == 128;
+  const DealCost cost = {wide ? (dual ? 2.45 : 1.2) : (dual ? 1.6 : 0.85), wide && dual ? 6.0 : 5.0, 7.0, 11.0 * p.D / 128 * (dual ? 1.0 : 0.5), 0.25, 1, 1.0};
+  const int nblk = (p.L + 127) / 128;
+  auto time = [&](int most, int step) {
+    DealTime t(cus, cost);
+    t.add({most, step, 0, nblk}, (long long)p.Z * p.H, 1.0, 1.0, [&](int order) { return (std::min((order + 1) * 128, Lk) + 63) / 64; });
+    return t.total();
+  };
+  SplitPlan best = none;
+  double least = time(1, 0) / 1.06;
+  for (int most = 2; most <= 8; ++most) {
+    const int step = ((ntiles + 1) / 2 + most - 1) / most;  // the longest block, of ntiles, gets `most` shares
+    if (step < 2 || blocks * most > 3 * cus) break;
+    const double t = time(most, step);
+    if (t < least) least = t, best = {most, step};
+  }
+  return best;
 }
 
 // Backward with grouped heads.  A dk/dv workgroup owns 128 keys of a key/value head and works through the query heads
@@ -173,13 +246,59 @@ inline BwdSplitPlan bwd_split_plan(int D, int Z, int H, int L, int Lk, bool caus
   }
   return s;
 }
-template <typename P> inline BwdSplitPlan bwd_split_plan_of(const P &p, int Lk, int Hk, bool tangent_grads, bool dual) {
-  if (p.dtype == 2 || p.D > 128 || p.mask_kind != 0 || p.dropout_p > 0.f || Hk != p.H || tangent_grads) return {1, 0, 1, 0};
-  return bwd_split_plan(p.D, p.Z, p.H, p.L, Lk, p.causal != 0, dual);
+// The deal of either role's blocks that a launch goes by.  Causal, from 12 tiles on, where the account of DealTime says that it is
+// shorter than with whole blocks: shares of one length for all blocks of both roles, so that the long ones get most of them.
+// Causal, bf16, B1, backward with tangents / without, before -> this: D128 H12 L1024 68 -> 57 us, H16 L1024 69 -> 65, H9 L2048 127 -> 108 / 64 -> 60,
+// H7 L2500 154 -> 122 / 78 -> 67, H2 L12000 719 -> 588 / 331 -> 266; D64 H16 L1024 50 -> 43 / 31 -> 29, H6 L4096 173 -> 140 / 83 -> 69, H1 L30000 1227 ->
+// 1101 / 713 -> 458; D32 H12 L1024 35 -> 24 / 24 -> 20, H6 L4096 115 -> 88 / 50 -> 44, H1 L8192 91 -> 60 / 63 -> 36; of 250 shapes the slowest
+// 6 % slower (D64 H3 L5000 without tangents 58 -> 62).
+// Otherwise shares of the length that bwd_split_plan says.
+struct BwdDeal {
+  Deal q, k;
+  bool any() const { return q.most > 1 || k.most > 1; }
+};
+inline BwdDeal bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bool dual, long long cus = device_cus()) {
+  const int bq = (L + 127) / 128, bk = (Lk + 127) / 128;
+  const BwdSplitPlan even = bwd_split_plan(D, Z, H, L, Lk, causal, dual, cus);
+  if (!causal) return {{even.chunks_q, 0, 0, bq}, {even.chunks_k, 0, 0, bk}};
+  auto step_of = [](int chunks, int tiles) { return chunks > 1 ? (tiles + 1) / 2 : 0; };
+  const long long heads = (long long)Z * H;
+  const int nq = (std::min(bq * 128, Lk) + 63) / 64, nk = (L + 63) / 64, live = std::min(bk, bq);  // tiles of the longest blocks; key blocks that a query sees
+  const BwdDeal alike = {{even.chunks_q, step_of(even.chunks_q, even.tiles_q), 0, bq}, {even.chunks_k, step_of(even.chunks_k, even.tiles_k), bq - live, bq}};
+  if ( cus <= 0 || std::max(nq, nk) < 12 || heads * (bq + bk) >= 2 * cus) return alike;
+  const DealCost cost = D == 128 ? (dual ? DealCost{3.0, 2.9, 6.4, 9.9, 0.34, 1, 1.0} : DealCost{1.5, 3.9, 7.0, 6.1, 0.14, 1, 1.0})
+                        : D == 64 ? (dual ? DealCost{2.0, 6.0, 4.2, 3.4, 0.2, 1, 1.0} : DealCost{1.2, 9.0, 3.6, 2.3, 0.4, 2, 0.7})
+                                  : (dual ? DealCost{1.5, 5.5, 5.0, 2.1, 0.57, 2, 0.5} : DealCost{1.0, 4.5, 3.0, 1.8, 0.15, 2, 0.7});
+  constexpr double KEYS = 1.25;  // a dk/dv tile in dq tiles
+  auto time = [&](const BwdDeal &d) {
+    DealTime t(cus, cost);
+    t.add(d.q, heads, 1.0, 1.0, [&](int order) { return (std::min((order + 1) * 128, Lk) + 63) / 64; });
+    t.add(d.k, heads, KEYS, 2.0, [&](int order) { return (L - 128 * (bq - 1 - order) + 63) / 64; });
+    return t.total();
+  };
+  BwdDeal best = {{1, 0, 0, bq}, {1, 0, bq - live, bq}};
+  double least = time(best) * (dual ? 1.07 : 1.0);  // (the account is fitted to shares; of whole blocks with tangents it makes 7 % too little)
+  const double longest = std::max((double)nq, KEYS * nk);
+  for (const int j : {4, 5, 6, 8, 12, 16}) {  // shares of 1/2 ... 1/8 of the longest block
+    const double share = longest * 2 / j;
+    auto deal = [&](int n, double t, int first, int last) {
+      const int most = std::min(8, std::max(1, (int)(n * t / share + 0.99)));
+      return Deal{most, most > 1 ? ((n + 1) / 2 + most - 1) / most : 0, first, last};
+    };
+    const BwdDeal d = {deal(nq, 1.0, 0, bq), deal(nk, KEYS, bq - live, bq)};
+    if ((d.q.most > 1 && d.q.step < 2) || (d.k.most > 1 && d.k.step < 2) || heads * (d.q.most * bq + 2 * d.k.most * bk) > 6 * cus) break;
+    const double t = time(d);
+    if (t < least) least = t, best = d;
+  }
+  return best.any() ? best : alike;
 }
-template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const BwdSplitPlan &s) {
+template <typename P> inline BwdDeal bwd_deal_of(const P &p, int Lk, int Hk, bool tangent_grads, bool dual) {
+  if (p.dtype == 2 || p.D > 128 || p.mask_kind != 0 || p.dropout_p > 0.f || Hk != p.H || tangent_grads) return {{1, 0, 0, 0}, {1, 0, 0, 0}};
+  return bwd_deal(p.D, p.Z, p.H, p.L, Lk, p.causal != 0, dual);
+}
+template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const BwdDeal &d) {
   const size_t heads = (size_t)p.Z * p.H;
-  return heads * p.D * ((s.chunks_q > 1 ? (size_t)s.chunks_q * p.L : 0) + (s.chunks_k > 1 ? (size_t)s.chunks_k * 2 * Lk : 0));
+  return heads * p.D * ((d.q.most > 1 ? (size_t)d.q.most * p.L : 0) + (d.k.most > 1 ? (size_t)d.k.most * 2 * Lk : 0));
 }
 
 // Whether dk/dv and dq go into one launch (bwd2_both_kernel): it has one end with idle compute units instead of two, and where a
@@ -268,18 +387,18 @@ inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven, 
 
 // ---- merge kernels -------------------------------------------------------------------------------
 // Forward.  part = [chunk][row][2][D] accumulators, then [chunk][row][4] statistics.  One thread per (row, 8
-// columns).  With m the largest reference point of the row's chunks and w_c = 2^(m_c - m):
+// columns), a grid of (rows of a head, heads).  With m the largest reference point of the row's chunks and w_c = 2^(m_c - m):
 //   l = sum w_c l_c,  O = sum w_c O_c,  and, with c the reference of S' of the heaviest chunk,
 //   T = sum w_c (T_c + (c_c - c) O_c),  mu_acc = sum w_c (mu_c + (c_c - c) l_c);
 // then the epilogue of the forward kernels: O / l, O' = T / l - (mu_acc / l) O, M = m + log2 l, mu = mu_acc / l + c.
 template <typename T, int D, bool DUAL>
-__global__ __launch_bounds__(256) void fwd_merge_kernel(const float *part, int chunks, long long rows, T *o, T *ot,
-                                                        float *M, float *mu) {
-  constexpr int LPR = D / 8;
-  const long long row = (long long)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+__global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, T *ot, float *M, float *mu) {
+  constexpr int LPR = D / 8, RPB = 256 / LPR;
+  const int in_head = blockIdx.x * RPB, chunks = Deal{pr.chunks, pr.chunk_tiles, 0, 0}.shares(in_head / 128);  // (uniform: RPB divides 128)
+  if (chunks == 1 || in_head + (int)threadIdx.x / LPR >= pr.L) return;  // a block that one workgroup did is finished
+  const size_t rows = (size_t)pr.Z * pr.H * pr.L, row = (size_t)blockIdx.y * pr.L + in_head + threadIdx.x / LPR;
   const int d0 = (threadIdx.x % LPR) * 8;
-  if (row >= rows) return;
-  const float *stat = part + (size_t)chunks * rows * 2 * D;
+  const float *part = pr.part, *stat = part + (size_t)pr.chunks * rows * 2 * D;
   float m = -__builtin_inff();
   for (int c = 0; c < chunks; ++c) m = fmaxf(m, stat[((size_t)c * rows + row) * 4]);
   float l = 0.f, best = -1.f, cref = 0.f;

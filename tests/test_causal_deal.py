@@ -1,0 +1,102 @@
+"""Causal blocks dealt to workgroups by length: the deal itself on the CPU, and forwards and backwards that go by it on the GPU."""
+import ctypes as C
+import os
+
+import pytest
+import torch
+
+from jvp_flash_attention_amd import _lib, build
+from oracle import dense
+
+from .test_launch_rules import run
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
+def test_every_share_is_dealt_once(tmp_path):
+    """Ranks 0 .. workgroups() - 1 of a head are the shares of its orders, each once; shares() of an order agrees."""
+    text = """
+  int bad = 0;
+  for (int most = 1; most <= 8; ++most)
+    for (int step = most > 1; step <= 9; ++step)
+      for (int first = 0; first < 20; first += 3)
+        for (int last = first + 1; last < 41; ++last) {
+          const Deal d = {most, step, first, last};
+          int n = 0, seen[41][8] = {};
+          for (int o = first; o < last; ++o) n += d.shares(o);
+          bad += n != d.workgroups();
+          for (int r = 0; r < n; ++r) {
+            const Share s = share_of(d, r);
+            const bool in = s.order >= first && s.order < last && s.index >= 0 && s.index < s.count;
+            bad += !in || s.count != d.shares(s.order) || seen[s.order][s.index]++ != 0;
+          }
+        }
+  std::printf("%d ", bad);
+"""
+    assert run(tmp_path, text) == [0]
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
+def test_deals_of_backwards(tmp_path):
+    """Whole blocks where they fill the units or are short, more shares the longer a block is, and bounded partial results."""
+    shapes = [(D, dual, H, L, Lk) for D in (32, 64, 128) for dual in (0, 1) for H in (1, 3, 16, 40) for L in (100, 777, 3000, 30000) for Lk in (64, 1000, 30000)]
+    text = "  int bad = 0, split = 0;\n"
+    for D, dual, H, L, Lk in shapes:
+        text += f"""  {{ const BwdDeal d = bwd_deal({D}, 1, {H}, {L}, {Lk}, true, {dual}, 256);
+    const int bq = {(L + 127) // 128}, bk = {(Lk + 127) // 128};
+    bad += d.q.most < 1 || d.q.most > 8 || d.k.most < 1 || d.k.most > 8 || (d.q.most > 1 && d.q.step < 1) || (d.k.most > 1 && d.k.step < 1);
+    bad += d.q.last != bq || d.k.last != bq || d.k.first != bq - std::min(bq, bk);
+    bad += d.any() && {H} * (d.q.most * bq + 2 * d.k.most * bk) > 6 * 256 + 2 * 256 * 8;
+    split += d.any(); }}
+"""
+    bad, split = run(tmp_path, text + '  std::printf("%d %d", bad, split);\n')
+    assert bad == 0 and 0 < split < len(shapes)
+    whole = ", ".join(f"bwd_deal({D}, 4, 16, 2048, 2048, true, true, 256).any()" for D in (32, 64, 128))
+    assert run(tmp_path, f'  for (bool b : {{{whole}}}) std::printf("%d ", b ? 1 : 0);\n') == [0, 0, 0]
+
+
+# few workgroups, more than there are units (heads that are and are not a multiple of 8), keys and queries of unequal number
+SHAPES = [(1, 4, 1100, 1100), (1, 3, 4200, 4200), (2, 4, 2100, 2100), (1, 2, 900, 2000), (1, 3, 2000, 900)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Z,H,L,Lk", SHAPES)
+@pytest.mark.parametrize("grads", ["plain", "both", "tangent"])
+def test_dealt_blocks_agree_with_whole_ones(dtype, D, Z, H, L, Lk, grads):
+    """Against the same kernels on whole blocks, and a slab of rows of O, O' against the dense oracle."""
+    print("case", dtype, D, Z, H, L, Lk, grads, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(L + D)
+    rand = lambda n: torch.randn(Z, H, n, D, generator=g, device="cuda").to(dtype)  # noqa: E731
+    q, qt, go, gt, k, v, kt, vt = rand(L), rand(L), rand(L), rand(L), rand(Lk), rand(Lk), rand(Lk), rand(Lk)
+    t = (None,) * 3 if grads == "plain" else (qt, kt, vt)
+    be, scale = _lib.backend(), D**-0.5
+    p = _lib.make_problem(q, None, _lib.MASK_NONE, True, scale)
+    assert _lib.load().jvpfa_bwd_split_workspace_bytes(C.byref(p), Lk, H, 0) > 0
+    fwd = lambda: be.fwd(q, k, v, *t, None, _lib.MASK_NONE, True, scale)  # noqa: E731
+    got = fwd()
+    _lib.set_split(False)
+    try:
+        one = fwd()
+        bwd = lambda: be.bwd(q, k, v, *t, *one, go if grads != "tangent" else None, gt if grads != "plain" else None,  # noqa: E731
+                             None, _lib.MASK_NONE, True, scale)
+        whole = bwd()
+    finally:
+        _lib.set_split(True)
+    dealt = bwd()
+    ulp = 2.0**-7 if dtype == torch.bfloat16 else 2.0**-10
+    for a, b in zip(got[2:], one[2:]):
+        assert b is None or (a - b).abs().max().item() <= 1e-5 * max(1.0, b.abs().max().item())
+    for a, b in zip(got[:2], one[:2]):  # P is rounded against another reference point in each share: one unit, two for O'
+        assert b is None or ((a.float() - b.float()).abs() <= 2 * ulp * b.float().abs().clamp_min(1.0)).all()
+    for a, b in zip(dealt[:3], whole[:3]):  # the same P and dS, sums in fp32 in another order, each rounded once
+        assert (a.float() - b.float()).norm() <= ulp / 2 * b.float().norm()
+        assert ((a.float() - b.float()).abs() <= ulp * b.float().abs() + 1e-5 * b.float().abs().max()).all()
+    rows = slice(max(0, L - 70), L)  # the last rows: the block with most shares
+    f = [x[:1, :1].double().cpu().numpy() for x in (q, k, v, qt, kt, vt)]
+    keep = torch.arange(Lk)[None, :] <= torch.arange(L)[rows][:, None]
+    ref = dense.forward(f[0][:, :, rows], f[1], f[2], f[3][:, :, rows], f[4], f[5], mask=keep[None, None].numpy(), scale=scale)
+    for x, name in ((got[0], "O"), (got[1], "Ot")):
+        if x is not None:
+            want = ref[name]
+            assert abs(x[:1, :1, rows].double().cpu().numpy() - want).max() <= 2e-2 * abs(want).max()
