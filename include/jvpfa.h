@@ -106,9 +106,10 @@ typedef struct jvpfa_fwd_args {
   int32_t Lk, Hk;
   /* optional workspace for small grids, or NULL: jvpfa_fwd_split_workspace_bytes(&p, Lk) bytes of device memory,
    * 16-byte aligned, contents don't-care.  When a launch would have fewer workgroups than the GPU has compute
-   * units (one long sequence, few heads), the key tiles of every query block are then split over up to 8
+   * units (one long sequence, few heads), the key tiles of query blocks are then split over up to 8
    * workgroups that leave fp32 partial results there, and a second kernel merges them into o, ot, M, mu
-   * (bf16 / fp16, D = 64 or 128, no mask; ignored otherwise).  Results agree with the unsplit launch to rounding.
+   * (bf16 / fp16, D = 64 or 128, no mask; fp32, D <= 128, without dropout and grouped heads; ignored otherwise).  Results agree
+   * with the unsplit launch to rounding.
    * No counterpart in the reference (one program per 32 query rows whatever the grid, JA:2474-2476). */
   void *split_workspace;
   uint64_t split_workspace_bytes;
@@ -159,8 +160,8 @@ typedef struct jvpfa_bwd_args {
    * of device memory, 16-byte aligned, contents don't-care.  Where one workgroup per 128 keys of a key/value head would
    * leave compute units idle, the query heads of a group are then dealt to several workgroups that leave fp32 shares of
    * the key and value gradients there, and a second kernel adds them up; where the whole launch would (one long
-   * sequence, few heads; bf16 / fp16, D <= 128, no mask, no dropout, Hk = p.H, dqt NULL), the tiles of every block are,
-   * for dq, dk, dv.  Results agree with the unsplit launch to rounding. */
+   * sequence, few heads; D <= 128, no dropout, Hk = p.H; bf16 / fp16: no mask, dqt NULL), the tiles of blocks are, for dq as
+   * well as for dk, dv.  Results agree with the unsplit launch to rounding. */
   void *split_workspace;
   uint64_t split_workspace_bytes;
   const uint32_t *mask_bits_q; /* as in jvpfa_fwd_args (dq kernels) */

@@ -39,7 +39,9 @@ extern "C" int jvpfa_fwd(const jvpfa_fwd_args *a, void *hip_stream) {
   p.q = a->q; p.k = a->k; p.v = a->v;
   p.qt = a->qt; p.kt = a->kt; p.vt = a->vt;
   p.o = a->o; p.ot = a->ot; p.M = a->M; p.mu = a->mu;
-  if (a->split_workspace) {  // small grid: split the key tiles of every query block, if the workspace suffices
+  // Small grid: split the key tiles of query blocks, if the workspace suffices.  (fp32 with grouped heads: blocks stay whole, as they do
+  // in its backward, so that the gradients of a head do not depend on how many others there are.)
+  if (a->split_workspace && !(a->p.dtype == JVPFA_FP32 && p.pr.Hk != p.pr.H)) {
     const SplitPlan sp = fwd_split_plan(a->p, p.pr.Lk, dual);
     if (sp.chunks > 1 && aligned16(a->split_workspace) &&
         a->split_workspace_bytes >= fwd_part_floats(sp.chunks, (long long)a->p.Z * a->p.H * a->p.L, a->p.D) * sizeof(float)) {
@@ -53,8 +55,9 @@ extern "C" int jvpfa_fwd(const jvpfa_fwd_args *a, void *hip_stream) {
 
 extern "C" size_t jvpfa_fwd_split_workspace_bytes(const jvpfa_problem *p, int32_t Lk) {
   if (!p || check_problem(*p) != JVPFA_OK) return 0;
-  const SplitPlan sp = fwd_split_plan(*p, Lk > 0 ? Lk : p->L, true);  // (a plan without tangents takes no more)
-  return sp.chunks > 1 ? fwd_part_floats(sp.chunks, (long long)p->Z * p->H * p->L, p->D) * sizeof(float) : 0;
+  int chunks = 1;  // of the plan with tangents or of that without, whichever takes more
+  for (const bool dual : {false, true}) chunks = std::max(chunks, fwd_split_plan(*p, Lk > 0 ? Lk : p->L, dual).chunks);
+  return chunks > 1 ? fwd_part_floats(chunks, (long long)p->Z * p->H * p->L, p->D) * sizeof(float) : 0;
 }
 
 extern "C" int jvpfa_abi_version(void) { return JVPFA_ABI_VERSION; }

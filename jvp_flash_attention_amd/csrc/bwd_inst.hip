@@ -156,6 +156,21 @@ template <typename T, int D> static void launch_kv_merge(const BwdParams &p, boo
                      p.pr.chunks, elems, tangent ? dkt : dk, tangent ? dvt : dv, dkt, dvt);
 }
 
+// The deal of a launch whose blocks' tiles are split (what jvpfa_bwd found worth it), and the workgroups of either role.
+template <int D, bool F32> static BwdSplit split_of(const Problem &pr, bool dual, long long *kv_blocks, long long *blocks) {
+  const BwdDeal d = bwd_deal(F32, D, pr.Z, pr.H, pr.L, pr.Lk, pr.causal != 0, dual);
+  const long long heads = (long long)pr.Z * pr.H;
+  const int bq = (pr.L + 127) / 128, bk = (pr.Lk + 127) / 128;
+  *kv_blocks = heads * (d.k.step > 0 ? d.k.workgroups() + std::max(bk - bq, 0) : bk * d.k.most);
+  *blocks = heads * (d.q.step > 0 ? d.q.workgroups() : bq * d.q.most);
+  return {d.q, d.k, pr.part, pr.part + (d.q.most > 1 ? (size_t)d.q.most * heads * pr.L * D : 0)};
+}
+template <typename T, int D> static void launch_split_merge(const BwdParams &p, const BwdSplit &sp, bool tangent, hipStream_t stream) {
+  constexpr int RPB = 2048 / D;
+  hipLaunchKernelGGL((bwd_split_merge_kernel<T, D>), dim3((unsigned)((std::max(p.pr.L, p.pr.Lk) + RPB - 1) / RPB), p.pr.Z * p.pr.H, 3), dim3(256), 0,
+                     stream, p, sp, tangent ? 1 : 0);
+}
+
 // The dq and dk/dv kernels for fp32 with D <= 128: up to D = 64 as three bf16 parts.
 template <int D, int MODE, int MASK, bool GO, bool DROP> static auto pick_f32_dq() -> void (*)(const BwdParams) {
   if constexpr (D <= 64) return bwd_f32x3_dq_kernel<D, MODE, MASK, GO, DROP>;
@@ -165,9 +180,9 @@ template <int D, int MODE, int MASK, bool GO, bool DROP> static auto pick_f32_dk
   if constexpr (D <= 64) return bwd_f32x3_dkdv_kernel<D, MODE, MASK, GO, DROP>;
   else return bwd_f32_dkdv_kernel<D, MODE, MASK, GO, DROP>;
 }
-template <int D, int MODE, int MASK, bool GO> static auto pick_f32_both() -> void (*)(const BwdParams, int) {
-  if constexpr (D <= 64) return bwd_f32x3_both_kernel<D, MODE, MASK, GO>;
-  else return bwd_f32_both_kernel<D, MODE, MASK, GO>;
+template <int D, int MODE, int MASK, bool GO> static auto pick_f32_both(bool split) -> void (*)(const BwdParams, const BwdSplit, int) {
+  if constexpr (D <= 64) return split ? bwd_f32x3_both_kernel<D, MODE, MASK, GO, true> : bwd_f32x3_both_kernel<D, MODE, MASK, GO, false>;
+  else return split ? bwd_f32_both_kernel<D, MODE, MASK, GO, true> : bwd_f32_both_kernel<D, MODE, MASK, GO, false>;
 }
 template <int D, int MODE, int MASK, bool DROP>
 static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blocks, hipStream_t stream) {
@@ -180,11 +195,18 @@ static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blo
   if (rc == 0) rc = allow_lds(reinterpret_cast<const void *>(kkv), Lds::DKV);
   if (rc != 0) return rc;
   if constexpr (!DROP) {
-    if (launch_both_f32<D, MODE>(blocks, kv_blocks, p.pr.causal != 0 || MASK == MASK_BOOL)) {
-      void (*kb)(const BwdParams, int) = no_go ? pick_f32_both<D, MODE, MASK, NG>() : pick_f32_both<D, MODE, MASK, true>();
-      rc = run_both(kb, p, kv_blocks, kv_blocks + blocks, Lds::DKV, stream);
+    const bool split = p.pr.chunk_tiles == -1;
+    if (split || launch_both_f32<D, MODE>(blocks, kv_blocks, p.pr.causal != 0 || MASK == MASK_BOOL)) {
+      void (*kb)(const BwdParams, const BwdSplit, int) = no_go ? pick_f32_both<D, MODE, MASK, NG>(split) : pick_f32_both<D, MODE, MASK, true>(split);
+      const Problem &pr = p.pr;
+      BwdSplit sp = {{1, 0, 0, 0}, {1, 0, 0, 0}, nullptr, nullptr};
+      if (split) sp = split_of<D, true>(pr, MODE != BWD_PLAIN, &kv_blocks, &blocks);
+      if (kv_blocks + blocks > 0x7fffffffLL) return -2;
+      rc = allow_lds(reinterpret_cast<const void *>(kb), Lds::DKV);
       if (rc != 0) return rc;
-      launch_kv_merge<float, D>(p, MODE == BWD_TANGENT, false, stream);
+      hipLaunchKernelGGL(kb, dim3((unsigned)(kv_blocks + blocks)), dim3(256), Lds::DKV, stream, p, sp, (int)kv_blocks);
+      if (split) launch_split_merge<float, D>(p, sp, MODE == BWD_TANGENT, stream);
+      else launch_kv_merge<float, D>(p, MODE == BWD_TANGENT, false, stream);
       return hipGetLastError() == hipSuccess ? 0 : -6;
     }
   }
@@ -197,20 +219,14 @@ static int launch_bwd_f32(const BwdParams &p, long long blocks, long long kv_blo
 // Small grids: blocks' tiles split (split.hpp).
 template <typename T, int D, int MODE> static int launch_split(const BwdParams &p, bool no_go, hipStream_t stream) {
   using Cfg = Bwd2Cfg<T, D, MODE>;
-  const Problem &pr = p.pr;
-  const BwdDeal d = bwd_deal(D, pr.Z, pr.H, pr.L, pr.Lk, pr.causal != 0, MODE == BWD_DUAL);
-  BwdSplit sp = {d.q, d.k, pr.part, pr.part};
-  if (d.q.most > 1) sp.part_k += (size_t)d.q.most * pr.Z * pr.H * pr.L * D;
-  const int heads = pr.Z * pr.H, bq = (pr.L + 127) / 128, bk = (pr.Lk + 127) / 128;
-  const int kv_blocks = heads * (d.k.step > 0 ? d.k.workgroups() + std::max(bk - bq, 0) : bk * d.k.most);
-  const int blocks = heads * (d.q.step > 0 ? d.q.workgroups() : bq * d.q.most);
+  long long kv_blocks, blocks;
+  const BwdSplit sp = split_of<D, false>(p.pr, MODE == BWD_DUAL, &kv_blocks, &blocks);
   auto kern = no_go ? bwd2_split_kernel<T, D, MODE, MODE != BWD_DUAL> : bwd2_split_kernel<T, D, MODE, true>;
   constexpr size_t LDS = Cfg::DKV_LDS > Cfg::DQ_LDS ? Cfg::DKV_LDS : Cfg::DQ_LDS;
   const int rc = allow_lds(reinterpret_cast<const void *>(kern), LDS);
   if (rc != 0) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(kv_blocks + blocks)), dim3(Cfg::NT), LDS, stream, p, sp, kv_blocks);
-  constexpr int RPB = 2048 / D;
-  hipLaunchKernelGGL((bwd_split_merge_kernel<T, D>), dim3((unsigned)((std::max(pr.L, pr.Lk) + RPB - 1) / RPB), heads, 3), dim3(256), 0, stream, p, sp);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(kv_blocks + blocks)), dim3(Cfg::NT), LDS, stream, p, sp, (int)kv_blocks);
+  launch_split_merge<T, D>(p, sp, false, stream);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 

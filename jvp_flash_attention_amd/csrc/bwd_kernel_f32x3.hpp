@@ -134,8 +134,8 @@ template <int G, int NG, int NU, bool AFTER, typename F> __device__ __forceinlin
   __builtin_amdgcn_sched_barrier(0);
 }
 // dq (PLAIN / DUAL) or dq' (TANGENT).  Returns whether every output is finite.
-template <int D, int MODE, int MASK, bool GO, bool DROP>
-__device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int bid) {
+template <int D, int MODE, int MASK, bool GO, bool DROP, bool SPLIT = false>
+__device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int bid, const BwdSplit sp = {}, const int total = 0) {
   using C = X3Cfg<D>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   constexpr int BT = C::BT, KK = D / 16, DB = D / 32, NTILE = DUAL ? 4 : 2;
@@ -145,9 +145,10 @@ __device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int 
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nqb = (L + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(bid, nqb, pr.Z * pr.H, pr.causal != 0);
-  const int zh = id / nqb;
-  const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
+  const Dealt share = SPLIT ? deal_query_block(sp.q, bid, total, nqb, pr.Z * pr.H, pr.causal != 0) : Dealt{xcd_remap(bid, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
+  const bool split = SPLIT && share.count > 1;
+  const int zh = share.id / nqb;
+  const int qb = pr.causal ? nqb - 1 - share.id % nqb : share.id % nqb;
   const int z = zh / pr.H, h = zh % pr.H;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
@@ -185,6 +186,7 @@ __device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int 
       if (pr.tiles_q) tl = pr.tiles_q + tile_list_offset_q(pr, z, h, qb);
     }
     walk.init(tl, 0, kend, Lk);
+    if (split) walk.take(share.index, share.count, ((pr.causal ? min(Lk, q0 + C::BLK) : Lk) + TILE_W - 1) / TILE_W);
   }
   const int ntiles = __builtin_amdgcn_readfirstlane(walk.n);
   auto tile_at = [&](int it) { return __builtin_amdgcn_readfirstlane(walk.at(min(it, max(ntiles - 1, 0)))); };
@@ -389,6 +391,7 @@ __device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int 
   if constexpr (MASK == MASK_NONE) {  // the causal diagonal and the end form the tail of the walk
     int t_lim = Lk / BT;
     if (pr.causal) t_lim = min(t_lim, q0 / BT);
+    t_lim -= walk.first;
     for (; t < min(t_lim, ntiles); ++t) step(t, std::false_type{});
     for (; t < ntiles; ++t) step(t, std::true_type{});
   } else {
@@ -397,7 +400,7 @@ __device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int 
   accs_ready(acc);
   float check = 0.f;  // not zero once an output is not finite
   if (qrow < L) {
-    float *out = reinterpret_cast<float *>(TAN ? p.dqt : p.dq) + head + (size_t)qrow * D;
+    float *out = (split ? sp.part_q + (size_t)share.index * pr.Z * pr.H * L * D : reinterpret_cast<float *>(TAN ? p.dqt : p.dq)) + head + (size_t)qrow * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
 #pragma unroll
@@ -416,8 +419,8 @@ __device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int 
 }
 
 // dk, dv (PLAIN / DUAL) or dk', dv' (TANGENT).  Returns whether every output is finite.
-template <int D, int MODE, int MASK, bool GO, bool DROP>
-__device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p, const int bid) {
+template <int D, int MODE, int MASK, bool GO, bool DROP, bool SPLIT = false>
+__device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p, const int bid, const BwdSplit sp = {}, const int total = 0) {
   using C = X3Cfg<D>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   constexpr int BT = C::BT, KK = D / 16, DB = D / 32, NTILE = DUAL ? 4 : 2;
@@ -430,9 +433,11 @@ __device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p, const in
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nkb = (Lk + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(bid, nkb, pr.Z * pr.Hk * pr.chunks, pr.causal != 0);
-  const int zhk = id / nkb / pr.chunks, chunk = id / nkb % pr.chunks;
-  const int kb = id % nkb;  // causal: the first key blocks have the longest query loops
+  const int shares = pr.Z * pr.Hk * pr.chunks;
+  const Dealt share = SPLIT ? deal_key_block(sp.k, bid, total, nkb, shares, pr.causal != 0) : Dealt{xcd_remap(bid, nkb, shares, pr.causal != 0), 1, 0};
+  const bool split = SPLIT && share.count > 1;
+  const int zhk = share.id / nkb / pr.chunks, chunk = share.id / nkb % pr.chunks;
+  const int kb = share.id % nkb;  // causal: the first key blocks have the longest query loops
   const int z = zhk / pr.Hk, hk = zhk % pr.Hk, group = group_share(pr, chunk + 1) - group_share(pr, chunk);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
@@ -483,6 +488,7 @@ __device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p, const in
       if constexpr (MASK != MASK_NONE) {
         if (pr.klimit && k0 >= pr.klimit[z]) walk.n = 0;  // a key block the caller's hint declares fully masked: zeros
       }
+      if (split) walk.take(share.index, share.count, (max(L - istart, 0) + TILE_W - 1) / TILE_W);
     }
     const int ntiles = __builtin_amdgcn_readfirstlane(walk.n);
     auto tile_at = [&](int it) { return __builtin_amdgcn_readfirstlane(walk.at(min(it, max(ntiles - 1, 0)))); };
@@ -752,7 +758,7 @@ __device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p, const in
     };
     int t = 0;
     if constexpr (MASK == MASK_NONE) {  // the tiles of the causal diagonal come first
-      const int t_lim = pr.causal ? min(C::BLK / BT, ntiles) : 0;
+      const int t_lim = pr.causal ? min(C::BLK / BT - walk.first, ntiles) : 0;
       for (; t < t_lim; ++t) step(t, std::true_type{});
     }
     for (; t < ntiles; ++t) step(t, std::false_type{});
@@ -760,7 +766,8 @@ __device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p, const in
   accs_ready(dK, dV);
   float check = 0.f;  // not zero once an output is not finite
   if (krow < Lk) {
-    float *partk = kv_part(pr, D, 2, 0, chunk), *partv = kv_part(pr, D, 2, 1, chunk);
+    const size_t elems = (size_t)pr.Z * pr.Hk * Lk * D;
+    float *partk = split ? sp.part_k + share.index * 2 * elems : kv_part(pr, D, 2, 0, chunk), *partv = split ? partk + elems : kv_part(pr, D, 2, 1, chunk);
     const size_t off = kvhead + (size_t)krow * D;
     float *outk = (partk ? partk : reinterpret_cast<float *>(TAN ? p.dkt : p.dk)) + off;
     float *outv = (partv ? partv : reinterpret_cast<float *>(TAN ? p.dvt : p.dv)) + off;
@@ -802,15 +809,17 @@ __global__ __launch_bounds__(256, 1) void bwd_f32x3_dkdv_kernel(const BwdParams 
 #endif
 }
 
-// Both roles in one launch (see bwd2_both_kernel): the first kv_blocks workgroups are dk/dv workgroups.
-template <int D, int MODE, int MASK, bool GO>
-__global__ __launch_bounds__(256, 1) void bwd_f32x3_both_kernel(const BwdParams p, const int kv_blocks) {
+// Both roles in one launch (see bwd2_both_kernel): the first kv_blocks workgroups are dk/dv workgroups.  SPLIT: blocks' tiles split
+// (split.hpp), compiled apart: what it needs takes 15 - 80 scalar registers that the others' loops have to spill (B2 H6 L777 D64 first
+// order with a bias, whose rows are not aligned: 124 -> 159 us).
+template <int D, int MODE, int MASK, bool GO, bool SPLIT>
+__global__ __launch_bounds__(256, 1) void bwd_f32x3_both_kernel(const BwdParams p, const BwdSplit sp, const int kv_blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const int b = __builtin_amdgcn_readfirstlane(blockIdx.x);
   if (b < kv_blocks) {
-    if (!bwd_f32x3_dkdv_body<D, MODE, MASK, GO, false>(p, b)) bwd_f32_dkdv_body<D, MODE, MASK, GO, false>(p, b);
+    if (!bwd_f32x3_dkdv_body<D, MODE, MASK, GO, false, SPLIT>(p, b, sp, kv_blocks)) bwd_f32_dkdv_body<D, MODE, MASK, GO, false, SPLIT>(p, b, sp, kv_blocks);
   } else {
-    if (!bwd_f32x3_dq_body<D, MODE, MASK, GO, false>(p, b - kv_blocks)) bwd_f32_dq_body<D, MODE, MASK, GO, false>(p, b - kv_blocks);
+    if (!bwd_f32x3_dq_body<D, MODE, MASK, GO, false, SPLIT>(p, b - kv_blocks, sp, gridDim.x - kv_blocks)) bwd_f32_dq_body<D, MODE, MASK, GO, false, SPLIT>(p, b - kv_blocks, sp, gridDim.x - kv_blocks);
   }
 #endif
 }

@@ -149,13 +149,6 @@ __device__ __forceinline__ void zero_acc(f32x16 &x) {
   for (int e = 0; e < 16; ++e) x[e] = 0.f;
 }
 
-// Small grids: the streamed tiles of a block are dealt to several workgroups (Deal), which leave fp32 partial results where a block
-// has more than one (bwd_split_merge_kernel adds them up).
-struct BwdSplit {
-  Deal q, k;
-  float *part_q, *part_k;  // [share][Z H L D], [share][dk, dv][Z H Lk D]
-};
-
 // ------------------------------------------------------------------------------------------------
 // dq (PLAIN / DUAL) or dq' (TANGENT): workgroup = 128 query rows, loop over 64-key tiles of
 // K, V (, K', V').  Scores are transposed (lane = query) so dS is the B operand of dQ^T += K^T dS^T.
@@ -176,22 +169,12 @@ constexpr bool dq_init(int d, int mode, int mask, bool go, bool six, bool drop) 
 // the compiler to keep in registers, for the variant that must stay within 256 of them.
 // START: where dq_init says so.
 template <typename T, int D, int MODE, int MASK, bool GO, bool SIX, bool DROP = false, bool LEAN = false, bool START = true, bool SPLIT = false>
-__device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid_, const BwdSplit sp = {}, const int total = 0) {
+__device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid, const BwdSplit sp = {}, const int total = 0) {
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   static_assert(!SIX || DUAL, "dq' rides on the dual mode");
-  int bid = bid_, dealt = -1;
-  Share share = {0, 1, 0};
-  if constexpr (SPLIT) {
-    if (sp.q.step > 0) {  // (the id of a causal block counts from the last one)
-      const HeadRank hr = deal_heads(bid_, p.pr.Z * p.pr.H, total, more_than_units());
-      share = share_of(sp.q, hr.rank);
-      dealt = hr.head * sp.q.last + sp.q.last - 1 - share.order;
-    } else {
-      share.count = sp.q.most, share.index = bid_ % sp.q.most, bid = bid_ / sp.q.most;
-    }
-  }
-  JVPFA_BWD2_COMMON(Cfg, pr.Lk, pr.L, pr.H, 1, dealt)  // owns query rows, streams key tiles
+  const Dealt share = SPLIT ? deal_query_block(sp.q, bid, total, (p.pr.L + Cfg::BLK - 1) / Cfg::BLK, p.pr.Z * p.pr.H, p.pr.causal != 0) : Dealt{-1, 1, 0};
+  JVPFA_BWD2_COMMON(Cfg, pr.Lk, pr.L, pr.H, 1, share.id)  // owns query rows, streams key tiles
   const int qb = pr.causal ? nblk - 1 - id % nblk : id % nblk;
   const int q0 = qb * Cfg::BLK;
   const int qrow = q0 + wave * 32 + r;
@@ -579,24 +562,12 @@ __global__ __launch_bounds__(256, 2) void bwd2_dq_kernel_2wg_plain(const BwdPara
 // SIX (dual mode only): dk' = scale dS'^T Q and dv' = P^T gT as well, from the fragments and tiles that dk, dv
 // already have (two more accumulators: fits for D <= 64).
 template <typename T, int D, int MODE, int MASK, bool GO, bool GROUPED, bool SIX, bool DROP = false, bool SPLIT = false>
-__device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid_, const BwdSplit sp = {}, const int total = 0) {
-  int bid = bid_, dealt = -1;
-  Share share = {0, 1, 0};
-  if constexpr (SPLIT) {
-    if (sp.k.step > 0) {
-      const HeadRank hr = deal_heads(bid_, p.pr.Z * p.pr.H, total, more_than_units());
-      const int seen = sp.k.workgroups();  // ... then the key blocks behind the last query, which have zero gradients
-      if (hr.rank < seen) share = share_of(sp.k, hr.rank);
-      const int block = hr.rank < seen ? sp.k.last - 1 - share.order : sp.k.last + hr.rank - seen;
-      dealt = hr.head * ((p.pr.Lk + 127) / 128) + block;
-    } else {
-      share.count = sp.k.most, share.index = bid_ % sp.k.most, bid = bid_ / sp.k.most;
-    }
-  }
+__device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid, const BwdSplit sp = {}, const int total = 0) {
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
+  const Dealt share = SPLIT ? deal_key_block(sp.k, bid, total, (p.pr.Lk + Cfg::BLK - 1) / Cfg::BLK, p.pr.Z * p.pr.H, p.pr.causal != 0) : Dealt{-1, 1, 0};
   static_assert(!SIX || (DUAL && D <= 64), "dk', dv' ride on the dual mode, where the accumulators fit");
-  JVPFA_BWD2_COMMON(Cfg, pr.L, pr.Lk, pr.Hk, GROUPED ? pr.chunks : 1, dealt)  // owns key rows (h: key/value head), streams query tiles
+  JVPFA_BWD2_COMMON(Cfg, pr.L, pr.Lk, pr.Hk, GROUPED ? pr.chunks : 1, share.id)  // owns key rows (h: key/value head), streams query tiles
   const int kb = id % nblk;  // causal: the first key blocks have the longest query loops
   const int k0 = kb * Cfg::BLK;
   const int krow = k0 + wave * 32 + r;
@@ -1262,30 +1233,4 @@ __global__ __launch_bounds__(256, 1) void bwd2_split_kernel(const BwdParams p, c
   else bwd2_dq_body<T, D, MODE, MASK_NONE, GO, false, false, false, true, true>(p, b - kv_blocks, sp, gridDim.x - kv_blocks);
 #endif
 }
-// Its partial results added up, in fp32 and in the order of the tiles: one thread per 8 elements of dq, dk, dv (blockIdx.z 0, 1, 2)
-// of head blockIdx.y.  Blocks that one workgroup did are complete.  Bound by memory: shares * 4 + sizeof(T) bytes an element.
-template <typename T, int D>
-__global__ __launch_bounds__(256) void bwd_split_merge_kernel(const BwdParams p, const BwdSplit sp) {
-  const Problem &pr = p.pr;
-  constexpr int RPB = 2048 / D;  // rows of a workgroup
-  const int t = blockIdx.z, len = t == 0 ? pr.L : pr.Lk, other = t == 0 ? pr.Lk : pr.L;
-  const int first = blockIdx.x * RPB, block = first / 128;  // (uniform: RPB divides 128)
-  // streamed rows of the block: keys up to its last row, queries from its first 64-row tile on (causal), or all
-  const int rows = !pr.causal ? other : t == 0 ? min(other, block * 128 + 128) : max(other - block * 128, 0);
-  const Deal &d = t == 0 ? sp.q : sp.k;
-  const int tiles = (rows + 63) / 64, dealt = d.step > 0 ? d.shares(t == 0 ? block : d.last - 1 - block) : d.most;
-  if (dealt == 1 || first + (int)threadIdx.x / (D / 8) >= len) return;
-  const int per = (tiles + dealt - 1) / dealt;
-  const size_t elems = (size_t)pr.Z * pr.H * len * D, i = ((size_t)blockIdx.y * len + first) * D + threadIdx.x * 8;
-  const float *src = t == 0 ? sp.part_q : sp.part_k + (size_t)(t - 1) * elems;
-  const size_t step = t == 0 ? elems : 2 * elems;
-  float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int c = 0; c == 0 || c * per < tiles; ++c) {
-    const f32x8 x = ld8<float>(src + c * step + i);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sum[e] += x[e];
-  }
-  store8<T>(reinterpret_cast<T *>(t == 0 ? p.dq : t == 1 ? p.dk : p.dv) + i, sum);
-}
-
 }  // namespace jvpfa

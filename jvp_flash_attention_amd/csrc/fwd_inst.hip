@@ -25,6 +25,13 @@ static int launch_fwd_one(const FwdParams &p, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
+// The partial results of blocks that several workgroups did become o, ot, M, mu.
+template <typename T, int D, bool DUAL> static void launch_fwd_merge(const FwdParams &p, hipStream_t stream) {
+  constexpr int RPB = 256 / (D / 8);
+  hipLaunchKernelGGL((fwd_merge_kernel<T, D, DUAL>), dim3((p.pr.L + RPB - 1) / RPB, p.pr.Z * p.pr.H), dim3(256), 0, stream, p.pr,
+                     reinterpret_cast<T *>(p.o), reinterpret_cast<T *>(p.ot), p.M, p.mu);
+}
+
 // fp32 with D <= 128: direct-to-LDS as well; up to D = 64 as three bf16 parts.
 template <int D, bool DUAL, int MASK, bool DROP = false>
 static int launch_fwd_f32_one(const FwdParams &p, hipStream_t stream) {
@@ -32,13 +39,16 @@ static int launch_fwd_f32_one(const FwdParams &p, hipStream_t stream) {
   constexpr bool X3 = D <= 64;
   constexpr size_t LDS = X3 ? X3Lds<D, DUAL>::FWD : 2 * (DUAL ? 4 : 2) * (size_t)C::TILEB;
   void (*kern)(const FwdParams);
-  if constexpr (X3) kern = fwd_f32x3_kernel<D, DUAL, MASK, DROP>;
-  else kern = fwd_f32_kernel<D, DUAL, MASK, DROP>;
+  const bool split = p.pr.chunks > 1;
+  if constexpr (X3) kern = split ? fwd_f32x3_kernel<D, DUAL, MASK, DROP, !DROP> : fwd_f32x3_kernel<D, DUAL, MASK, DROP, false>;
+  else kern = split ? fwd_f32_kernel<D, DUAL, MASK, DROP, !DROP> : fwd_f32_kernel<D, DUAL, MASK, DROP, false>;
   int rc = allow_lds(reinterpret_cast<const void *>(kern), LDS);
   if (rc != 0) return rc;
-  const long long blocks = (long long)((p.pr.L + C::BLK - 1) / C::BLK) * p.pr.Z * p.pr.H;
+  const int nqb = (p.pr.L + C::BLK - 1) / C::BLK;
+  const long long blocks = (long long)(split ? Deal{p.pr.chunks, p.pr.chunk_tiles, 0, nqb}.workgroups() : nqb) * p.pr.Z * p.pr.H;
   if (blocks > 0x7fffffffLL) return -2;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::NT), LDS, stream, p);
+  if (split) launch_fwd_merge<float, D, DUAL>(p, stream);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 
@@ -69,11 +79,7 @@ static int launch_fwd3_one(const FwdParams &p, hipStream_t stream) {
   const long long blocks = (long long)(p.pr.chunks > 1 ? Deal{p.pr.chunks, p.pr.chunk_tiles, 0, nqb}.workgroups() : nqb) * p.pr.Z * p.pr.H;
   if (blocks > 0x7fffffffLL) return -2;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, p);
-  if (p.pr.chunks > 1) {  // the chunks' partial results become o, ot, M, mu
-    constexpr int RPB = 256 / (D / 8);
-    hipLaunchKernelGGL((fwd_merge_kernel<T, D, DUAL>), dim3((p.pr.L + RPB - 1) / RPB, p.pr.Z * p.pr.H), dim3(256), 0, stream, p.pr,
-                       reinterpret_cast<T *>(p.o), reinterpret_cast<T *>(p.ot), p.M, p.mu);
-  }
+  if (p.pr.chunks > 1) launch_fwd_merge<T, D, DUAL>(p, stream);
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 

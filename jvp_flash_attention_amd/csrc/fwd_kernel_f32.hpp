@@ -112,7 +112,7 @@ template <int D, int NTILE> struct F32Tiles {
   }
 };
 
-template <int D, bool DUAL, int MASK, bool DROP>
+template <int D, bool DUAL, int MASK, bool DROP, bool SPLIT = false>
 __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
   using C = F32Cfg<D>;
   constexpr int BT = C::BT, NJ = C::NJ, DB = C::DB, NTILE = DUAL ? 4 : 2, STAGEB = NTILE * C::TILEB;
@@ -123,9 +123,12 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nqb = (L + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
-  const int zh = id / nqb;
-  const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;  // causal: the longest key loops first
+  // SPLIT, small grids: the key tiles of query blocks are split over workgroups (see split.hpp)
+  const Dealt share = SPLIT ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0)
+                            : Dealt{xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
+  const bool split = SPLIT && share.count > 1;
+  const int zh = share.id / nqb;
+  const int qb = pr.causal ? nqb - 1 - share.id % nqb : share.id % nqb;  // causal: the longest key loops first
   const int z = zh / pr.H, h = zh % pr.H;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
@@ -173,9 +176,18 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
       if (pr.klimit) kend = min(kend, max(pr.klimit[z], 1));
       if (pr.tiles_q) tl = pr.tiles_q + tile_list_offset_q(pr, z, h, qb);
     }
+    const int whole = ((pr.causal ? min(Lk, q0 + C::BLK) : Lk) + TILE_W - 1) / TILE_W;
     walk.init(tl, 0, kend, Lk);
+    if (split) walk.take(share.index, share.count, whole);
   }
   const int ntiles = __builtin_amdgcn_readfirstlane(walk.n);
+  // partial results of a share: [share][row][O | T][D], then [share][row][m, l, mu_acc, c]
+  const size_t nrows = (size_t)pr.Z * pr.H * L, prow = (size_t)share.index * nrows + (size_t)zh * L + qrow;
+  float *part_stat = pr.part + (size_t)pr.chunks * nrows * 2 * D + prow * 4;
+  if (split && ntiles <= 0) {  // none of its tiles is visited: it weighs nothing
+    if (qrow < L && g == 0) *reinterpret_cast<f32x4 *>(part_stat) = f32x4{NEG_INF, 0.f, 0.f, 0.f};
+    return;
+  }
   auto tile_at = [&](int it) { return __builtin_amdgcn_readfirstlane(walk.at(min(it, max(ntiles - 1, 0)))); };
 
   F32Tiles<D, NTILE> tiles;
@@ -339,11 +351,11 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
   // ---- epilogue ------------------------------------------------------------------------------------
   l_i += xor32(l_i);
   if constexpr (DUAL) mu_i += xor32(mu_i);
-  const bool dead = !(l_i > 0.f);
-  const float inv = dead ? 0.f : 1.f / l_i, mu_n = mu_i * inv;
+  const bool dead = !split && !(l_i > 0.f);
+  const float inv = split ? 1.f : dead ? 0.f : 1.f / l_i, mu_n = split ? 0.f : mu_i * inv;  // a share is left as it stands for the merge kernel
   if (qrow < L) {
-    float *Og = reinterpret_cast<float *>(p.o) + head + (size_t)qrow * D;
-    float *Otg = DUAL ? reinterpret_cast<float *>(p.ot) + head + (size_t)qrow * D : nullptr;
+    float *Og = split ? pr.part + prow * 2 * D : reinterpret_cast<float *>(p.o) + head + (size_t)qrow * D;
+    float *Otg = split ? Og + D : DUAL ? reinterpret_cast<float *>(p.ot) + head + (size_t)qrow * D : nullptr;
     // registers 4q .. 4q + 3 are rows 8q + 4g + 0..3: 4 DB consecutive columns
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -360,7 +372,9 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
         if constexpr (DUAL) *reinterpret_cast<f32x4 *>(Otg + d0 + x) = f32x4{ot[x], ot[x + 1], ot[x + 2], ot[x + 3]};
       }
     }
-    if (g == 0) {
+    if (split) {
+      if (g == 0) *reinterpret_cast<f32x4 *>(part_stat) = f32x4{m_i, l_i, mu_i, 0.f};
+    } else if (g == 0) {
       p.M[(size_t)zh * L + qrow] = dead ? __builtin_inff() : m_i + __builtin_amdgcn_logf(l_i);
       if constexpr (DUAL) p.mu[(size_t)zh * L + qrow] = mu_n;
     }
@@ -368,10 +382,10 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
 }
 #endif
 
-template <int D, bool DUAL, int MASK, bool DROP>
+template <int D, bool DUAL, int MASK, bool DROP, bool SPLIT>
 __global__ __launch_bounds__(256, 1) void fwd_f32_kernel(const FwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  fwd_f32_body<D, DUAL, MASK, DROP>(p);
+  fwd_f32_body<D, DUAL, MASK, DROP, SPLIT>(p);
 #endif
 }
 

@@ -116,7 +116,7 @@ template <int MASK> __device__ __forceinline__ MaskAhead<float, MASK> x3_mask_fe
 }
 
 // Returns whether every output is finite.
-template <int D, bool DUAL, int MASK, bool DROP>
+template <int D, bool DUAL, int MASK, bool DROP, bool SPLIT>
 __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
   using C = X3Cfg<D>;
   constexpr int BT = C::BT, CH = C::CH, ROWB = C::ROWB, PLANE = C::PLANE, OPB = C::OPB;
@@ -128,9 +128,12 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nqb = (L + C::BLK - 1) / C::BLK;
-  const int id = xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
-  const int zh = id / nqb;
-  const int qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;  // causal: the longest key loops first
+  // SPLIT, small grids: the key tiles of query blocks are split over workgroups (see split.hpp)
+  const Dealt share = SPLIT ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0)
+                            : Dealt{xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
+  const bool split = SPLIT && share.count > 1;
+  const int zh = share.id / nqb;
+  const int qb = pr.causal ? nqb - 1 - share.id % nqb : share.id % nqb;  // causal: the longest key loops first
   const int z = zh / pr.H, h = zh % pr.H;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
@@ -187,9 +190,18 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
       if (pr.klimit) kend = min(kend, max(pr.klimit[z], 1));
       if (pr.tiles_q) tl = pr.tiles_q + tile_list_offset_q(pr, z, h, qb);
     }
+    const int whole = ((pr.causal ? min(Lk, q0 + C::BLK) : Lk) + TILE_W - 1) / TILE_W;
     walk.init(tl, 0, kend, Lk);
+    if (split) walk.take(share.index, share.count, whole);
   }
   const int ntiles = __builtin_amdgcn_readfirstlane(walk.n);
+  // partial results of a share: [share][row][O | T][D], then [share][row][m, l, mu_acc, c]
+  const size_t nrows = (size_t)pr.Z * pr.H * L, prow = (size_t)share.index * nrows + (size_t)zh * L + qrow;
+  float *part_stat = pr.part + (size_t)pr.chunks * nrows * 2 * D + prow * 4;
+  if (split && ntiles <= 0) {  // none of its tiles is visited: it weighs nothing
+    if (qrow < L && g == 0) *reinterpret_cast<f32x4 *>(part_stat) = f32x4{NEG_INF, 0.f, 0.f, 0.f};
+    return true;
+  }
   auto tile_at = [&](int it) { return __builtin_amdgcn_readfirstlane(walk.at(min(it, max(ntiles - 1, 0)))); };
 
   // ---- staging: task i of a lane is eight consecutive elements of a row of tensor op (K, K', V, V') --------
@@ -508,6 +520,7 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
   // the limits of the causal diagonal and of the end: from tile t_lim on (no lists without a mask)
   int t_lim = Lk / BT;
   if (pr.causal) t_lim = min(t_lim, q0 / BT);
+  t_lim -= walk.first;
   constexpr bool LIMITS = MASK == MASK_NONE;
   using LimB = std::integral_constant<bool, LIMITS>;
   phase_a(B1{}, B0{}, 0u, 0u, 0);
@@ -536,12 +549,12 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
   // ---- epilogue ------------------------------------------------------------------------------------
   l_i += xor32(l_i);
   if constexpr (DUAL) mu_i += xor32(mu_i);
-  const bool dead = !(l_i > 0.f);
-  const float inv = dead ? 0.f : 1.f / l_i, mu_n = mu_i * inv;
+  const bool dead = !split && !(l_i > 0.f);
+  const float inv = split ? 1.f : dead ? 0.f : 1.f / l_i, mu_n = split ? 0.f : mu_i * inv;  // a share is left as it stands for the merge kernel
   float check = l_i * 0.f;  // not zero once an output is not finite (a row sum that is not a number makes its row 0)
   if (qrow < L) {
-    float *Og = reinterpret_cast<float *>(p.o) + head + (size_t)qrow * D;
-    float *Otg = DUAL ? reinterpret_cast<float *>(p.ot) + head + (size_t)qrow * D : nullptr;
+    float *Og = split ? pr.part + prow * 2 * D : reinterpret_cast<float *>(p.o) + head + (size_t)qrow * D;
+    float *Otg = split ? Og + D : DUAL ? reinterpret_cast<float *>(p.ot) + head + (size_t)qrow * D : nullptr;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
 #pragma unroll
@@ -561,7 +574,9 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
         if constexpr (DUAL) store8<float>(Otg + d0, t8);
       }
     }
-    if (g == 0) {
+    if (split) {
+      if (g == 0) *reinterpret_cast<f32x4 *>(part_stat) = f32x4{m_i, l_i, mu_i, 0.f};
+    } else if (g == 0) {
       p.M[(size_t)zh * L + qrow] = dead ? __builtin_inff() : m_i + __builtin_amdgcn_logf(l_i);
       if constexpr (DUAL) p.mu[(size_t)zh * L + qrow] = mu_n;
     }
@@ -573,10 +588,10 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
 template <int D, bool DUAL> struct X3Lds {
   static constexpr size_t FWD = 2 * (size_t)(DUAL ? 4 : 2) * X3Cfg<D>::OPB;  // (more than the fp32 tiles take)
 };
-template <int D, bool DUAL, int MASK, bool DROP, int WGS = DUAL ? 1 : 2>
+template <int D, bool DUAL, int MASK, bool DROP, bool SPLIT, int WGS = DUAL ? 1 : 2>
 __global__ __launch_bounds__(256, WGS) void fwd_f32x3_kernel(const FwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if (!fwd_f32x3_body<D, DUAL, MASK, DROP>(p)) fwd_f32_body<D, DUAL, MASK, DROP>(p);
+  if (!fwd_f32x3_body<D, DUAL, MASK, DROP, SPLIT>(p)) fwd_f32_body<D, DUAL, MASK, DROP, SPLIT>(p);
 #endif
 }
 

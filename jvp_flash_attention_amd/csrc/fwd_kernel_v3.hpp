@@ -71,19 +71,10 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   const int nqb = (L + Cfg::BM - 1) / Cfg::BM;
   // small grids: the key tiles of query blocks are split over workgroups (see split.hpp), of every block alike or as Deal says
   constexpr bool DEALT = MASK == MASK_NONE && !DROP && D <= 128;
-  const int chunks = DEALT ? pr.chunks : 1;
-  int zh, qb;
-  Share share = {0, 1, 0};
-  if (chunks > 1 && pr.chunk_tiles > 0) {
-    const HeadRank hr = deal_heads(blockIdx.x, pr.Z * pr.H, gridDim.x, more_than_units());
-    share = share_of(Deal{chunks, pr.chunk_tiles, 0, nqb}, hr.rank);
-    zh = hr.head, qb = share.order;
-  } else {
-    share.count = chunks, share.index = chunks > 1 ? (int)(blockIdx.x % chunks) : 0;
-    const int id = xcd_remap(chunks > 1 ? blockIdx.x / chunks : blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0);
-    zh = id / nqb;
-    qb = pr.causal ? nqb - 1 - id % nqb : id % nqb;
-  }
+  const Dealt share = DEALT && pr.chunks > 1 ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0)
+                                             : Dealt{xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
+  const int zh = share.id / nqb;
+  const int qb = pr.causal ? nqb - 1 - share.id % nqb : share.id % nqb;
   const bool split = share.count > 1;
 
   const int tid = threadIdx.x;

@@ -161,7 +161,7 @@ template <int W> struct TileWalk {
   static_assert(W == 32 || W == 64);
   static constexpr int SUB = TILE_W / W;
   const int *list = nullptr;
-  int n = 0, start = 0, tmax = 0;
+  int n = 0, start = 0, tmax = 0, first = 0;
   __device__ __forceinline__ void init(const int *l, int start_, int end, int len) {
     list = l;
     start = start_;
@@ -174,7 +174,24 @@ template <int W> struct TileWalk {
     const int last = min(max(l[cnt], 0), tmax);
     n = SUB * cnt - ((SUB == 2 && last * TILE_W + W >= len) ? 1 : 0);
   }
-  __device__ __forceinline__ int at(int it) const {
+  // Share `index` out of `count` of a walk that would have `whole` 64-wide tiles without a mask: those of an equal part of them, so
+  // that the shares do not depend on what a list or a limit leaves out.
+  __device__ __forceinline__ void take(int index, int count, int whole) {
+    const int per = (whole + count - 1) / count, lo = index * per, hi = lo + per;
+    int from = lo, to = hi;  // (walk positions, 64 wide)
+    if (list) {  // ascending: as many entries as lie below either end
+      const int cnt = min(max(list[0], 1), tmax + 1), lane = threadIdx.x % 64;
+      from = to = 0;
+      for (int i0 = 0; i0 < cnt; i0 += 64) {
+        const int e = i0 + lane < cnt ? list[1 + i0 + lane] : 0x7fffffff;
+        from += __popcll(__ballot(e < lo)), to += __popcll(__ballot(e < hi));
+      }
+    }
+    first = min(SUB * from, max(n - 1, 0));
+    n = max(min(n, SUB * to) - SUB * from, 0);
+  }
+  __device__ __forceinline__ int at(int it_) const {
+    const int it = it_ + first;
     if (!list) return start + it * W;
     return min(max(list[1 + it / SUB], 0), tmax) * TILE_W + (it % SUB) * W;
   }

@@ -147,6 +147,13 @@ __host__ __device__ inline Share share_of(const Deal &d, int rank) {
   return {top - 1 - early - rank, 1, 0};
 }
 
+// Backward: the streamed tiles of blocks are dealt to several workgroups, which leave fp32 partial results where a block has more
+// than one (bwd_split_merge_kernel adds them up).
+struct BwdSplit {
+  Deal q, k;
+  float *part_q, *part_k;  // [share][Z H L D], [share][two gradients][Z H Lk D]
+};
+
 struct FwdParams {
   Problem pr;
   const void *q, *k, *v, *qt, *kt, *vt;

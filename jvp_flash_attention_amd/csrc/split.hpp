@@ -12,12 +12,30 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 
 #include "common.hpp"
 #include "params.hpp"
 
 namespace jvpfa {
+
+// make() of these sizes, from the last few that this thread asked for: a plan is a function of sizes alone, a call asks for it up to
+// four times, and each time takes 1 - 3 us.
+template <typename Plan, int N, typename Make> inline Plan remembered(const std::array<int, N> &sizes, Make make) {
+  struct Entry {
+    std::array<int, N> sizes;
+    Plan plan;
+    bool used;
+  };
+  static thread_local Entry entries[8];
+  static thread_local int next;
+  for (const Entry &e : entries)
+    if (e.used && e.sizes == sizes) return e.plan;
+  Entry &e = entries[next++ % 8];
+  e = {sizes, make(), true};
+  return e.plan;
+}
 
 struct SplitPlan {
   int chunks, chunk_tiles;  // as in Problem: Deal::most, Deal::step
@@ -52,6 +70,10 @@ struct DealCost {
   int places;      // workgroups that share a compute unit without taking longer
   double pair;     // of two workgroups in turn, see above
 };
+// A second launch and its workspace take 7 us on the host, and a step of forward and backward that takes the GPU less than some 110 us is
+// bound by the host: a split that adds a launch is for forwards and backwards that take at least this long, and saves at least so much.
+// (B1 H2 L300 D64 fp32, both outputs' gradients: 57 -> 47 us on the GPU, 112 -> 127 us a step.)
+constexpr double SPLIT_LAUNCH_US = 7.0, SPLIT_FORWARD_US = 40.0, SPLIT_BACKWARD_US = 65.0;
 class DealTime {
  public:
   DealTime(long long cus, const DealCost &cost) : cus_(cus), c_(cost) { std::fill(of_length_, of_length_ + TOP + 1, 0); }
@@ -62,6 +84,7 @@ class DealTime {
       const double length = (n + count - 1) / count * scale;
       const long long w = count * heads;
       sum_ += length * c_.tile * w + w * c_.start, workgroups_ += w, longest_ = std::max(longest_, length * c_.tile);
+      alike_ = alike_ && (workgroups_ == w || length == last_), last_ = length;
       of_length_[std::min((int)length, TOP)] += w;
       if (count > 1) parts_ += weight * w;
     }
@@ -73,6 +96,7 @@ class DealTime {
       int length = TOP;
       for (long long n = of_length_[TOP]; n <= places && length > 0; n += of_length_[length]) --length;
       time = std::max({time, sum_ / places + c_.end * longest_, 2.0 * (c_.pair * length * c_.tile + c_.start)});
+      if (alike_) time = std::max(time, (double)((workgroups_ + places - 1) / places) * (longest_ + c_.start));
     }
     return time + (parts_ > 0.0 ? c_.merge + c_.traffic * parts_ / cus_ : 0.0);
   }
@@ -81,7 +105,8 @@ class DealTime {
   static constexpr int TOP = 512;
   long long cus_;
   DealCost c_;
-  double sum_ = 0.0, longest_ = 0.0, parts_ = 0.0;
+  bool alike_ = true;  // one length: whole passes over the places
+  double sum_ = 0.0, longest_ = 0.0, parts_ = 0.0, last_ = 0.0;
   long long workgroups_ = 0, of_length_[TOP + 1];
 };
 
@@ -108,7 +133,36 @@ inline size_t fwd_part_floats(int chunks, long long rows, int D) { return (size_
 template <typename P> inline bool split_capable(const P &p) {
   return p.dtype != 2 && (p.D == 128 || p.D == 64) && p.mask_kind == 0 && !(p.dropout_p > 0.f);
 }
-template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk, bool dual) {
+// fp32 at D <= 128 (without dropout): a tile takes three to nine times as long as in 16 bits, so that a split is worth it for any grid that
+// leaves units idle, also by a second pass that is not full: 192 blocks in quarters are three passes of a quarter.  Dual / without
+// tangents, whole blocks -> this: D64 B1 H8 L512 51 -> 32 us, H2 L4096 causal 342 -> 82 / 153 -> 50, B2 H6 L777 with a bias 79 -> 48; D128 H8 L512
+// 187 -> 55 / 70 -> 33, H16 L1024 366 -> 209 / 135 -> 84, H40 L1000 733 -> 601 / 255 -> 216; D32 H12 L1024 causal 58 -> 29.
+template <typename P> inline SplitPlan fwd_split_plan_f32(const P &p, int Lk, bool dual, int cus) {
+  SplitPlan best = {1, 0};
+  const int nblk = (p.L + 127) / 128;
+  const long long heads = (long long)p.Z * p.H, blocks = heads * nblk;
+  if (p.D > 128 || p.dropout_p > 0.f || cus <= 0 || blocks >= 2 * cus) return best;
+  const bool shared = !dual && p.D <= 64;  // two workgroups to a unit, so only as many as there are units
+  const double tile = p.D == 128 ? (dual ? 22.4 : 8.1) : p.D == 64 ? (dual ? 5.6 : 2.4) : (dual ? 3.3 : 1.75);
+  const DealCost cost = {tile, 6.0, 6.0, 8.4 * p.D / 64 * (dual ? 1.0 : 0.5), 0.25, 1, 1.0};
+  auto n = [&](int order) { return ((p.causal ? std::min((order + 1) * 128, Lk) : Lk) + 63) / 64; };
+  auto time = [&](const SplitPlan &s) {
+    DealTime t(cus, cost);
+    t.add({s.chunks, s.chunk_tiles, 0, nblk}, heads, 1.0, 1.0, n);
+    return t.total();
+  };
+  const int longest = n(nblk - 1);
+  if (time(best) < SPLIT_FORWARD_US) return best;
+  double least = std::min(time(best) / 1.05, time(best) - SPLIT_LAUNCH_US);
+  for (int most = 2; most <= 8 && most <= longest; ++most) {
+    const SplitPlan s = {most, p.causal ? ((longest + 1) / 2 + most - 1) / most : 0};
+    if (blocks * most > (shared ? 1 : 4) * cus) break;
+    const double t = time(s);
+    if (t < least) least = t, best = s;
+  }
+  return best;
+}
+template <typename P> inline SplitPlan fwd_split_plan_16(const P &p, int Lk, bool dual, int cus) {
   const SplitPlan none = {1, 0};
   if (!split_capable(p)) return none;
   const long long blocks = (long long)((p.L + 127) / 128) * p.Z * p.H;
@@ -120,7 +174,6 @@ template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk, bool d
   // and plain: H4 L1024 34 -> 28 and 18 -> unsplit (19); H4 L2048 62 -> 33 and 32 -> 21; H8 L2048 63 -> 42 and 33 -> 26;
   // H2 L4096 118 -> 44 and 61 -> 28; H4 L4096 119 -> 66 and 61 -> 40.
   if (p.D == 64 && ntiles < (dual ? 16 : 32)) return none;
-  const int cus = device_cus();
   const SplitPlan even = split_plan(blocks, ntiles, cus);
   if (!p.causal || blocks >= cus || ntiles < 12) return even;
   // Causal: shares of one length for all blocks (Deal), where the account of DealTime says that it is worth a twentieth; fewer
@@ -139,7 +192,8 @@ template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk, bool d
     return t.total();
   };
   SplitPlan best = none;
-  double least = time(1, 0) / 1.06;
+  if (even.chunks == 1 && time(1, 0) < SPLIT_FORWARD_US) return none;
+  double least = std::min(time(1, 0) / 1.06, time(1, 0) - (even.chunks == 1 ? SPLIT_LAUNCH_US : 0.0));
   for (int most = 2; most <= 8; ++most) {
     const int step = ((ntiles + 1) / 2 + most - 1) / most;  // the longest block, of ntiles, gets `most` shares
     if (step < 2 || blocks * most > 3 * cus) break;
@@ -147,6 +201,12 @@ template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk, bool d
     if (t < least) least = t, best = {most, step};
   }
   return best;
+}
+
+template <typename P> inline SplitPlan fwd_split_plan(const P &p, int Lk, bool dual) {
+  const int cus = device_cus(), kind = (p.dtype == 2) | (p.causal != 0) << 1 | dual << 2 | (p.mask_kind != 0) << 3 | (p.dropout_p > 0.f) << 4;
+  return remembered<SplitPlan, 7>({p.D, p.Z, p.H, p.L, Lk, kind, cus},
+                                  [&] { return p.dtype == 2 ? fwd_split_plan_f32(p, Lk, dual, cus) : fwd_split_plan_16(p, Lk, dual, cus); });
 }
 
 // Backward with grouped heads.  A dk/dv workgroup owns 128 keys of a key/value head and works through the query heads
@@ -257,7 +317,7 @@ struct BwdDeal {
   Deal q, k;
   bool any() const { return q.most > 1 || k.most > 1; }
 };
-inline BwdDeal bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bool dual, long long cus = device_cus()) {
+inline BwdDeal make_bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bool dual, long long cus = device_cus()) {
   const int bq = (L + 127) / 128, bk = (Lk + 127) / 128;
   const BwdSplitPlan even = bwd_split_plan(D, Z, H, L, Lk, causal, dual, cus);
   if (!causal) return {{even.chunks_q, 0, 0, bq}, {even.chunks_k, 0, 0, bk}};
@@ -277,7 +337,9 @@ inline BwdDeal bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bool du
     return t.total();
   };
   BwdDeal best = {{1, 0, 0, bq}, {1, 0, bq - live, bq}};
-  double least = time(best) * (dual ? 1.07 : 1.0);  // (the account is fitted to shares; of whole blocks with tangents it makes 7 % too little)
+  double least = time(best) * (dual && D == 64 ? 1.07 : 1.0);  // (the account is fitted to shares; of whole blocks with tangents it makes 7 % too little at D = 64)
+  if (!alike.any() && least < SPLIT_BACKWARD_US) return alike;
+  if (alike.any()) least = std::min(least, 0.92 * time(alike));  // (closer than that the account does not tell them apart)
   const double longest = std::max((double)nq, KEYS * nk);
   for (const int j : {4, 5, 6, 8, 12, 16}) {  // shares of 1/2 ... 1/8 of the longest block
     const double share = longest * 2 / j;
@@ -292,9 +354,53 @@ inline BwdDeal bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bool du
   }
   return best.any() ? best : alike;
 }
+// ... and in fp32 at D <= 128 (without dropout, one query head per key/value head; any mask, six gradients as well), by the same
+// reasons as the forward.  With tangents / without, whole blocks -> this: D64 B1 H8 L512 83 -> 41 us, H12 L1024 causal 160 -> 108 / 78 -> 53, B3 H4 L640
+// padded 115 -> 70 / 65 -> 44; D128 H8 L512 337 -> 113 / 133 -> 56, H12 L1024 causal 673 -> 336 / 256 -> 149; D32 H2 L4096 causal 362 -> 142 /
+// 203 -> 59; six gradients D64 H4 L900 208 -> 93.
+inline BwdDeal make_bwd_deal_f32(int D, int Z, int H, int L, int Lk, bool causal, bool dual, long long cus = device_cus()) {
+  const int bq = (L + 127) / 128, bk = (Lk + 127) / 128, live = causal ? std::min(bk, bq) : bk;
+  const long long heads = (long long)Z * H;
+  auto nq = [&](int order) { return ((causal ? std::min((order + 1) * 128, Lk) : Lk) + 63) / 64; };
+  auto nk = [&](int order) { return (L - (causal ? 128 * (bq - 1 - order) : 0) + 63) / 64; };
+  const int k0 = causal ? bq - live : 0, k1 = causal ? bq : bk;  // orders of the key blocks that a query sees
+  BwdDeal best = {{1, 0, 0, bq}, {1, 0, k0, k1}};
+  if (cus <= 0 || heads * (bq + bk) >= 4 * cus) return best;
+  constexpr double KEYS = 1.3;  // a dk/dv tile in dq tiles
+  const double tile = D == 128 ? (dual ? 32.0 : 12.5) : D == 64 ? (dual ? 7.5 : 3.4) : (dual ? 4.6 : 2.4);
+  const DealCost cost = {tile, 6.0, 6.0, 4.2 * D / 64, 0.12, D == 32 && !dual ? 2 : 1, 1.0};
+  auto time = [&](const BwdDeal &d) {
+    DealTime t(cus, cost);
+    t.add(d.k, heads, KEYS, 2.0, nk);
+    t.add(d.q, heads, 1.0, 1.0, nq);
+    return t.total();
+  };
+  const int longest_q = nq(bq - 1), longest_k = nk(k1 - 1);
+  // whole blocks: in one launch, or in two that each end with units idle
+  const double apart = (double)((heads * bq + cus - 1) / cus) * (longest_q * tile + cost.start) + (double)((heads * live + cus - 1) / cus) * (longest_k * KEYS * tile + cost.start);
+  double least = std::min(time(best), apart) / 1.06;
+  if (least < SPLIT_BACKWARD_US) return best;
+  const double longest = std::max((double)longest_q, KEYS * longest_k);
+  for (const int j : {3, 4, 5, 6, 8, 10, 12, 16}) {
+    auto deal = [&](int n, double scale, int first, int last) {
+      const int most = std::min({8, n, std::max(1, (int)(n * scale * j / (2 * longest) + 0.99))});
+      return Deal{most, causal && most > 1 ? ((n + 1) / 2 + most - 1) / most : 0, first, last};
+    };
+    const BwdDeal d = {deal(longest_q, 1.0, 0, bq), deal(longest_k, KEYS, k0, k1)};
+    if (heads * (d.q.most * bq + 2 * d.k.most * bk) > 8 * cus) break;
+    const double t = time(d);
+    if (d.any() && t < least) least = t, best = d;
+  }
+  return best;
+}
+inline BwdDeal bwd_deal(bool f32, int D, int Z, int H, int L, int Lk, bool causal, bool dual, long long cus = device_cus()) {
+  return remembered<BwdDeal, 7>({D, Z, H, L, Lk, f32 | causal << 1 | dual << 2, (int)cus},
+                                [&] { return f32 ? make_bwd_deal_f32(D, Z, H, L, Lk, causal, dual, cus) : make_bwd_deal(D, Z, H, L, Lk, causal, dual, cus); });
+}
 template <typename P> inline BwdDeal bwd_deal_of(const P &p, int Lk, int Hk, bool tangent_grads, bool dual) {
+  if (p.dtype == 2 && p.D <= 128 && !(p.dropout_p > 0.f) && Hk == p.H) return bwd_deal(true, p.D, p.Z, p.H, p.L, Lk, p.causal != 0, dual);
   if (p.dtype == 2 || p.D > 128 || p.mask_kind != 0 || p.dropout_p > 0.f || Hk != p.H || tangent_grads) return {{1, 0, 0, 0}, {1, 0, 0, 0}};
-  return bwd_deal(p.D, p.Z, p.H, p.L, Lk, p.causal != 0, dual);
+  return bwd_deal(false, p.D, p.Z, p.H, p.L, Lk, p.causal != 0, dual);
 }
 template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const BwdDeal &d) {
   const size_t heads = (size_t)p.Z * p.H;
@@ -458,6 +564,32 @@ __global__ __launch_bounds__(256) void bwd_kv_merge_kernel(const float *part, in
     for (int e = 0; e < 8; ++e) sum[e] += x[e];
   }
   store8<T>((t == 0 ? g0 : t == 1 ? g1 : t == 2 ? g2 : g3) + i, sum);
+}
+
+// ---- the merge of a launch whose blocks are dealt to several workgroups: their partial results added up, in fp32 and in the order of the tiles: one thread per 8 elements of dq, dk, dv (blockIdx.z 0, 1, 2)
+// of head blockIdx.y (tangent: dq', dk', dv').  Blocks that one workgroup did are complete.  Bound by memory: shares * 4 + sizeof(T) bytes an element.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void bwd_split_merge_kernel(const BwdParams p, const BwdSplit sp, const int tangent) {
+  const Problem &pr = p.pr;
+  constexpr int RPB = 2048 / D;  // rows of a workgroup
+  const int t = blockIdx.z, len = t == 0 ? pr.L : pr.Lk, other = t == 0 ? pr.Lk : pr.L;
+  const int first = blockIdx.x * RPB, block = first / 128;  // (uniform: RPB divides 128)
+  // streamed rows of the block: keys up to its last row, queries from its first 64-row tile on (causal), or all
+  const int rows = !pr.causal ? other : t == 0 ? min(other, block * 128 + 128) : max(other - block * 128, 0);
+  const Deal &d = t == 0 ? sp.q : sp.k;
+  const int tiles = (rows + 63) / 64, dealt = d.step > 0 ? d.shares(t == 0 ? block : d.last - 1 - block) : d.most;
+  if (dealt == 1 || first + (int)threadIdx.x / (D / 8) >= len) return;
+  const int per = (tiles + dealt - 1) / dealt;
+  const size_t elems = (size_t)pr.Z * pr.H * len * D, i = ((size_t)blockIdx.y * len + first) * D + threadIdx.x * 8;
+  const float *src = t == 0 ? sp.part_q : sp.part_k + (size_t)(t - 1) * elems;
+  const size_t step = t == 0 ? elems : 2 * elems;
+  float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c == 0 || c * per < tiles; ++c) {
+    const f32x8 x = ld8<float>(src + c * step + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum[e] += x[e];
+  }
+  store8<T>(reinterpret_cast<T *>(t == 0 ? (tangent ? p.dqt : p.dq) : t == 1 ? (tangent ? p.dkt : p.dk) : (tangent ? p.dvt : p.dv)) + i, sum);
 }
 
 }  // namespace jvpfa

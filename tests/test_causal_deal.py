@@ -41,7 +41,7 @@ def test_deals_of_backwards(tmp_path):
     shapes = [(D, dual, H, L, Lk) for D in (32, 64, 128) for dual in (0, 1) for H in (1, 3, 16, 40) for L in (100, 777, 3000, 30000) for Lk in (64, 1000, 30000)]
     text = "  int bad = 0, split = 0;\n"
     for D, dual, H, L, Lk in shapes:
-        text += f"""  {{ const BwdDeal d = bwd_deal({D}, 1, {H}, {L}, {Lk}, true, {dual}, 256);
+        text += f"""  {{ const BwdDeal d = bwd_deal(false, {D}, 1, {H}, {L}, {Lk}, true, {dual}, 256);
     const int bq = {(L + 127) // 128}, bk = {(Lk + 127) // 128};
     bad += d.q.most < 1 || d.q.most > 8 || d.k.most < 1 || d.k.most > 8 || (d.q.most > 1 && d.q.step < 1) || (d.k.most > 1 && d.k.step < 1);
     bad += d.q.last != bq || d.k.last != bq || d.k.first != bq - std::min(bq, bk);
@@ -50,7 +50,7 @@ def test_deals_of_backwards(tmp_path):
 """
     bad, split = run(tmp_path, text + '  std::printf("%d %d", bad, split);\n')
     assert bad == 0 and 0 < split < len(shapes)
-    whole = ", ".join(f"bwd_deal({D}, 4, 16, 2048, 2048, true, true, 256).any()" for D in (32, 64, 128))
+    whole = ", ".join(f"bwd_deal(false, {D}, 4, 16, 2048, 2048, true, true, 256).any()" for D in (32, 64, 128))
     assert run(tmp_path, f'  for (bool b : {{{whole}}}) std::printf("%d ", b ? 1 : 0);\n') == [0, 0, 0]
 
 
