@@ -71,15 +71,19 @@ template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false>
 static int launch_fwd3_one(const FwdParams &p, hipStream_t stream) {
   using Cfg = Fwd2Cfg<T, D, DUAL>;
   void (*kern)(const FwdParams);
-  if constexpr (D == 64 && DUAL) kern = fwd3_kernel_2wg<T, D, DUAL, MASK, DROP>;
-  else kern = fwd3_kernel<T, D, DUAL, MASK, DROP>;
+  constexpr bool CAN = MASK == MASK_NONE && !DROP;  // split its blocks' keys, see split_capable
+  const bool split = CAN && p.pr.chunks > 1;
+  if constexpr (D == 64 && DUAL) kern = split ? fwd3_kernel_2wg<T, D, DUAL, MASK, DROP, CAN> : fwd3_kernel_2wg<T, D, DUAL, MASK, DROP>;
+  else kern = split ? fwd3_kernel<T, D, DUAL, MASK, DROP, CAN> : fwd3_kernel<T, D, DUAL, MASK, DROP>;
   int rc = allow_lds(reinterpret_cast<const void *>(kern), Cfg::LDS_BYTES);
   if (rc != 0) return rc;
   const int nqb = (p.pr.L + Cfg::BM - 1) / Cfg::BM;
-  const long long blocks = (long long)(p.pr.chunks > 1 ? Deal{p.pr.chunks, p.pr.chunk_tiles, 0, nqb}.workgroups() : nqb) * p.pr.Z * p.pr.H;
+  const long long blocks = (long long)(split ? Deal{p.pr.chunks, p.pr.chunk_tiles, 0, nqb}.workgroups() : nqb) * p.pr.Z * p.pr.H;
   if (blocks > 0x7fffffffLL) return -2;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, p);
-  if (p.pr.chunks > 1) launch_fwd_merge<T, D, DUAL>(p, stream);
+  if constexpr (CAN) {
+    if (split) launch_fwd_merge<T, D, DUAL>(p, stream);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -6;
 }
 

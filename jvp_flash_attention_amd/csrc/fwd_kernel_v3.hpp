@@ -53,7 +53,7 @@ template <int N> __device__ __forceinline__ void lds_wait3(u32x4 &a, u32x2 &c, u
 // TIGHT: a third fewer registers for fragments.  Score fragments are read one super-step ahead instead of three, V fragments at
 // the top of their own super-step, behind whose score products they arrive.  For two workgroups on a compute unit, each of
 // which covers the other's waits.
-template <typename T, int D, bool DUAL, int MASK, bool DROP, bool TIGHT>
+template <typename T, int D, bool DUAL, int MASK, bool DROP, bool TIGHT, bool SPLIT>
 __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   using Cfg = Fwd2Cfg<T, D, DUAL>;
   constexpr int BN = Cfg::BN, CH = Cfg::CH, ROWB = Cfg::ROWB, TILEB = Cfg::TILEB, IPW = Cfg::IPW;
@@ -69,13 +69,15 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   const Problem &pr = p.pr;
   const int L = pr.L;
   const int nqb = (L + Cfg::BM - 1) / Cfg::BM;
-  // small grids: the key tiles of query blocks are split over workgroups (see split.hpp), of every block alike or as Deal says
-  constexpr bool DEALT = MASK == MASK_NONE && !DROP && D <= 128;
-  const Dealt share = DEALT && pr.chunks > 1 ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0)
-                                             : Dealt{xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
+  // SPLIT, small grids: the key tiles of query blocks are split over workgroups (see split.hpp), of every block alike or as Deal says.
+  // Compiled apart: with the shares as a branch of every launch B4 H16 L4096 D128 took 1384 us for 1370, B1 H16 L32768 causal with its
+  // backward 37.09 ms for 36.94; without it both are within 0.2 % of a kernel that knows no shares.
+  static_assert(!SPLIT || (MASK == MASK_NONE && !DROP && D <= 128));
+  const Dealt share = SPLIT ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0)
+                            : Dealt{xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
   const int zh = share.id / nqb;
   const int qb = pr.causal ? nqb - 1 - share.id % nqb : share.id % nqb;
-  const bool split = share.count > 1;
+  const bool split = SPLIT && share.count > 1;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
@@ -775,11 +777,11 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   }
 }
 #endif
-template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false,
+template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false, bool SPLIT = false,
           int WGS = (!DUAL && D <= 128 && (MASK != MASK_NONE || DROP)) ? 2 : 1>
 __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub (and has no buffer descriptor type)
-  fwd3_body<T, D, DUAL, MASK, DROP, false>(p);
+  fwd3_body<T, D, DUAL, MASK, DROP, false, SPLIT>(p);
 #endif
 }
 // D = 64 with tangents: 96 accumulation registers (Q, Q', O, O'), so with 160 others two workgroups share a compute unit.  Unlike
@@ -788,10 +790,10 @@ __global__ __launch_bounds__(256, WGS) void fwd3_kernel(const FwdParams p) {
 // B4 H16 L2048 191.5 -> 186.4 us, causal 112.4 -> 106.4; B2 H16 L1024 35.5 -> 32.5; B4 H16 L4096 730 -> 706, causal 389 -> 377;
 // fp16 L2048 202.7 -> 198.0.  (Without tangents, and with dropout, the same change is 1 - 4 % slower: three waves of fwd2_kernel
 // share a SIMD there.  With masks it takes 258 - 284 registers.)
-template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false>
+template <typename T, int D, bool DUAL, int MASK = MASK_NONE, bool DROP = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_num_vgpr(160))) void fwd3_kernel_2wg(const FwdParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  fwd3_body<T, D, DUAL, MASK, DROP, true>(p);
+  fwd3_body<T, D, DUAL, MASK, DROP, true, SPLIT>(p);
 #endif
 }
 
