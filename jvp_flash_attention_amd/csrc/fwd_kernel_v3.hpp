@@ -71,7 +71,8 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   const int nqb = (L + Cfg::BM - 1) / Cfg::BM;
   // SPLIT, small grids: the key tiles of query blocks are split over workgroups (see split.hpp), of every block alike or as Deal says.
   // Compiled apart: with the shares as a branch of every launch B4 H16 L4096 D128 took 1384 us for 1370, B1 H16 L32768 causal with its
-  // backward 37.09 ms for 36.94; without it both are within 0.2 % of a kernel that knows no shares.
+  // backward 37.09 ms for 36.94; without it both are 0.2 - 0.5 % off (1428 for 1424 us, 38.72 for 38.59 ms on another card): within what
+  // two runs of one build differ by.
   static_assert(!SPLIT || (MASK == MASK_NONE && !DROP && D <= 128));
   const Dealt share = SPLIT ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0)
                             : Dealt{xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
