@@ -497,6 +497,9 @@ inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven, 
 //   l = sum w_c l_c,  O = sum w_c O_c,  and, with c the reference of S' of the heaviest chunk,
 //   T = sum w_c (T_c + (c_c - c) O_c),  mu_acc = sum w_c (mu_c + (c_c - c) l_c);
 // then the epilogue of the forward kernels: O / l, O' = T / l - (mu_acc / l) O, M = m + log2 l, mu = mu_acc / l + c.
+// A share that visited nothing says so by l = -1 and is left out.  All others are added up, however small their weight: that of a
+// share whose scores are all NaN, which no reference point is taken from, or -inf is 0, and 0 times what it holds is what one
+// workgroup's rescaling makes of it.  So the outputs that are not numbers are those of whole blocks.
 template <typename T, int D, bool DUAL>
 __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, T *ot, float *M, float *mu) {
   constexpr int LPR = D / 8, RPB = 256 / LPR;
@@ -507,10 +510,12 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, 
   const float *part = pr.part, *stat = part + (size_t)pr.chunks * rows * 2 * D;
   float m = -__builtin_inff();
   for (int c = 0; c < chunks; ++c) m = fmaxf(m, stat[((size_t)c * rows + row) * 4]);
+  const float m_use = m == -__builtin_inff() ? 0.f : m;
   float l = 0.f, best = -1.f, cref = 0.f;
   for (int c = 0; c < chunks; ++c) {
     const float *st = stat + ((size_t)c * rows + row) * 4;
-    const float w = (st[0] == -__builtin_inff()) ? 0.f : __builtin_amdgcn_exp2f(st[0] - m);
+    if (st[1] < 0.f) continue;
+    const float w = __builtin_amdgcn_exp2f(st[0] - m_use);
     l += w * st[1];
     if (w * st[1] > best) {
       best = w * st[1];
@@ -522,8 +527,8 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, 
   for (int e = 0; e < 8; ++e) O[e] = Tt[e] = 0.f;
   for (int c = 0; c < chunks; ++c) {
     const float *st = stat + ((size_t)c * rows + row) * 4;
-    const float w = (st[0] == -__builtin_inff()) ? 0.f : __builtin_amdgcn_exp2f(st[0] - m);
-    if (w == 0.f) continue;
+    if (st[1] < 0.f) continue;
+    const float w = __builtin_amdgcn_exp2f(st[0] - m_use);
     const float *acc = part + ((size_t)c * rows + row) * 2 * D + d0;
     const float dc = st[3] - cref;
     mua += w * (st[2] + dc * st[1]);
@@ -546,7 +551,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, 
   if constexpr (DUAL) store8<T>(ot + (size_t)row * D + d0, t8);
   if (d0 == 0) {
     M[row] = dead ? __builtin_inff() : m + __builtin_amdgcn_logf(l);
-    if constexpr (DUAL) mu[row] = dead ? 0.f : mu_n + cref;
+    if constexpr (DUAL) mu[row] = !dead ? mu_n + cref : sizeof(T) == 4 ? mu_n : 0.f;  // (as the kernels of either type leave it)
   }
 }
 
