@@ -29,10 +29,11 @@ template <typename Plan, int N, typename Make> inline Plan remembered(const std:
     bool used;
   };
   static thread_local Entry entries[8];
-  static thread_local int next;
+  static thread_local int next;  // (0 .. 7: a count of all plans would overflow in a long run)
   for (const Entry &e : entries)
     if (e.used && e.sizes == sizes) return e.plan;
-  Entry &e = entries[next++ % 8];
+  Entry &e = entries[next];
+  next = (next + 1) % 8;
   e = {sizes, make(), true};
   return e.plan;
 }

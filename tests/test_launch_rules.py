@@ -134,3 +134,23 @@ def test_capped_kernel_for_both_roles(tmp_path):
              (640, 640, 48, 1): 1, (2048, 2048, 16, 1): 1, (512, 2000, 16, 1): 1, (1, 1, 1, 1): 0}
     got = run(tmp_path, "".join(f'  std::printf("%d ", both_two_wgs({L}, {Lk}, {h}, {c}, 256) ? 1 : 0);\n' for L, Lk, h, c in sides))
     assert [x for x, y in zip(sides, got) if y != sides[x]] == []
+
+
+PLANS = """
+  long long made = 0;
+  auto plan = [&](int size) { return remembered<int, 1>({size}, [&] { ++made; return 3 * size; }); };
+"""
+
+
+def test_plans_are_remembered_however_many_were_made(tmp_path):
+    """More plans than a 32-bit count holds, each of another size: the last one is still found where it was put."""
+    text = PLANS + """
+  const long long many = (1LL << 31) + 19;
+  long long sum = 0;
+  for (long long i = 0; i < many; ++i) sum += plan((int)(unsigned)i) != 3 * (int)(unsigned)i;
+  const long long before = made;
+  const int size = 12345;
+  sum += plan(size) != 3 * size, sum += plan(size) != 3 * size;
+  std::printf("%d %d", (int)sum, (int)(made - before));
+"""
+    assert run(tmp_path, text) == [0, 1]
