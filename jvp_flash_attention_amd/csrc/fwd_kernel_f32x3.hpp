@@ -199,7 +199,7 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
   const size_t nrows = (size_t)pr.Z * pr.H * L, prow = (size_t)share.index * nrows + (size_t)zh * L + qrow;
   float *part_stat = pr.part + (size_t)pr.chunks * nrows * 2 * D + prow * 4;
   if (split && ntiles <= 0) {  // none of its tiles is visited: it weighs nothing
-    if (qrow < L && g == 0) *reinterpret_cast<f32x4 *>(part_stat) = f32x4{NEG_INF, -1.f, 0.f, 0.f};
+    if (qrow < L && g == 0) *reinterpret_cast<f32x4 *>(part_stat) = f32x4{NEG_INF, -0.f, 0.f, 0.f};
     return true;
   }
   auto tile_at = [&](int it) { return __builtin_amdgcn_readfirstlane(walk.at(min(it, max(ntiles - 1, 0)))); };

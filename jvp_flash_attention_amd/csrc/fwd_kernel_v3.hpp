@@ -118,7 +118,7 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   float *part_stat = pr.part + (size_t)pr.chunks * nrows * 2 * D + prow * 4;
   if (split && ntiles <= 0) {  // fewer tiles than shares would take: this one weighs nothing
     if (qrow < L && g == 0) {
-      const f32x4 none = {-__builtin_inff(), -1.f, 0.f, 0.f};
+      const f32x4 none = {-__builtin_inff(), -0.f, 0.f, 0.f};
       *reinterpret_cast<f32x4 *>(part_stat) = none;
     }
     return;

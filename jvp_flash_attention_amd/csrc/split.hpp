@@ -498,7 +498,7 @@ inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven, 
 //   l = sum w_c l_c,  O = sum w_c O_c,  and, with c the reference of S' of the heaviest chunk,
 //   T = sum w_c (T_c + (c_c - c) O_c),  mu_acc = sum w_c (mu_c + (c_c - c) l_c);
 // then the epilogue of the forward kernels: O / l, O' = T / l - (mu_acc / l) O, M = m + log2 l, mu = mu_acc / l + c.
-// A share that visited nothing says so by l = -1 and is left out.  All others are added up, however small their weight: that of a
+// A share that visited nothing says so by l = -0 (a sum is never that) and is left out.  All others are added up, however small their weight: that of a
 // share whose scores are all NaN, which no reference point is taken from, or -inf is 0, and 0 times what it holds is what one
 // workgroup's rescaling makes of it.  So the outputs that are not numbers are those of whole blocks.
 template <typename T, int D, bool DUAL>
@@ -515,9 +515,8 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, 
   float l = 0.f, best = -1.f, cref = 0.f;
   for (int c = 0; c < chunks; ++c) {
     const float *st = stat + ((size_t)c * rows + row) * 4;
-    if (st[1] < 0.f) continue;
     const float w = __builtin_amdgcn_exp2f(st[0] - m_use);
-    l += w * st[1];
+    l += w * st[1];  // (no branch on what is loaded: it would put the shares' loads behind one another)
     if (w * st[1] > best) {
       best = w * st[1];
       cref = st[3];
@@ -528,7 +527,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, 
   for (int e = 0; e < 8; ++e) O[e] = Tt[e] = 0.f;
   for (int c = 0; c < chunks; ++c) {
     const float *st = stat + ((size_t)c * rows + row) * 4;
-    if (st[1] < 0.f) continue;
+    if (__builtin_bit_cast(uint32_t, st[1]) == 0x80000000u) continue;
     const float w = __builtin_amdgcn_exp2f(st[0] - m_use);
     const float *acc = part + ((size_t)c * rows + row) * 2 * D + d0;
     const float dc = st[3] - cref;
