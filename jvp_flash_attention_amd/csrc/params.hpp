@@ -107,20 +107,20 @@ __host__ __device__ inline size_t mask_bits_offset(const Problem &pr, int z, int
 }
 
 // How a head's causal blocks are dealt to workgroups that share their streamed tiles.  Blocks are counted by length: each block
-// streams two tiles more than the one before in that `order`, so the orders below `step` get one workgroup, the next `step` two,
-// and so on up to `most`: every share is then about as long.  (step 0, host only: every block gets `most`.)  A head's blocks are
-// the orders first .. last - 1.
+// streams two tiles more than the one before in that `order`, 2 (order + 1) at most, and gets a workgroup for every `step` of them,
+// up to `most`: every share is then about as long.  (step 0: every block gets `most`.)  A head's blocks are the orders first .. last - 1.
 struct Deal {
   int most, step, first, last;
+  __host__ __device__ int first_of(int count) const { return (count - 1) * step >> 1; }  // the shortest block of so many workgroups
   __host__ __device__ int shares(int order) const {
     int c = 1;
-    while (c < most && order >= c * step) ++c;
+    while (c < most && order >= first_of(c + 1)) ++c;
     return c;
   }
   __host__ __device__ int workgroups() const {
     int n = 0, hi = last;
     for (int c = most; c > 0; --c) {
-      const int from = (c - 1) * step, lo = from > first ? from : first;
+      const int from = first_of(c), lo = from > first ? from : first;
       if (lo < hi) n += (hi - lo) * c, hi = lo;
     }
     return n;
@@ -132,13 +132,13 @@ struct Share {
 // Workgroup `rank` of a head, roughly longest first: the longer half of the whole blocks and all shares (which are about as long:
 // none is shorter than half of the longest), then the shorter half of the whole blocks.
 __host__ __device__ inline Share share_of(const Deal &d, int rank) {
-  const int top = d.most > 1 && d.step < d.last ? d.step : d.last, whole = top > d.first ? top - d.first : 0;
+  const int top = d.most > 1 && d.first_of(2) < d.last ? d.first_of(2) : d.last, whole = top > d.first ? top - d.first : 0;
   const int early = d.most > 1 ? (whole + 1) / 2 : whole;
   if (rank < early) return {top - 1 - rank, 1, 0};
   rank -= early;
   int hi = d.last;
   for (int c = d.most; c > 1; --c) {
-    const int from = (c - 1) * d.step, lo = from > d.first ? from : d.first;
+    const int from = d.first_of(c), lo = from > d.first ? from : d.first;
     if (lo >= hi) continue;
     if (rank < (hi - lo) * c) return {hi - 1 - rank / c, c, rank % c};
     rank -= (hi - lo) * c;

@@ -156,7 +156,7 @@ template <typename P> inline SplitPlan fwd_split_plan_f32(const P &p, int Lk, bo
   if (time(best) < SPLIT_FORWARD_US) return best;
   double least = std::min(time(best) / 1.05, time(best) - SPLIT_LAUNCH_US);
   for (int most = 2; most <= 8 && most <= longest; ++most) {
-    const SplitPlan s = {most, p.causal ? ((longest + 1) / 2 + most - 1) / most : 0};
+    const SplitPlan s = {most, p.causal ? ((longest + 1) / 2 + most - 1) / most * 2 : 0};
     if (blocks * most > (shared ? 1 : 4) * cus) break;
     const double t = time(s);
     if (t < least) least = t, best = s;
@@ -175,7 +175,9 @@ template <typename P> inline SplitPlan fwd_split_plan_16(const P &p, int Lk, boo
   // and plain: H4 L1024 34 -> 28 and 18 -> unsplit (19); H4 L2048 62 -> 33 and 32 -> 21; H8 L2048 63 -> 42 and 33 -> 26;
   // H2 L4096 118 -> 44 and 61 -> 28; H4 L4096 119 -> 66 and 61 -> 40.
   if (p.D == 64 && ntiles < (dual ? 16 : 32)) return none;
-  const SplitPlan even = split_plan(blocks, ntiles, cus);
+  SplitPlan even = split_plan(blocks, ntiles, cus);
+  // causal: shares of that length for the shorter blocks, too (all blocks in as many: H12 L693 D128 without tangents 18.8 -> 20.6 us)
+  if (p.causal && even.chunks > 1) even.chunk_tiles = (ntiles + even.chunks - 1) / even.chunks;
   if (!p.causal || blocks >= cus || ntiles < 12) return even;
   // Causal: shares of one length for all blocks (Deal), where the account of DealTime says that it is worth a twentieth; fewer
   // blocks than there are units, whose longest ones alone set the time otherwise.  (Some launches of up to half as many again would gain as
@@ -196,8 +198,8 @@ template <typename P> inline SplitPlan fwd_split_plan_16(const P &p, int Lk, boo
   if (even.chunks == 1 && time(1, 0) < SPLIT_FORWARD_US) return none;
   double least = std::min(time(1, 0) / 1.06, time(1, 0) - (even.chunks == 1 ? SPLIT_LAUNCH_US : 0.0));
   for (int most = 2; most <= 8; ++most) {
-    const int step = ((ntiles + 1) / 2 + most - 1) / most;  // the longest block, of ntiles, gets `most` shares
-    if (step < 2 || blocks * most > 3 * cus) break;
+    const int step = ((ntiles + 1) / 2 + most - 1) / most * 2;  // the longest block, of ntiles, gets `most` shares
+    if (step < 4 || blocks * most > 3 * cus) break;
     const double t = time(most, step);
     if (t < least) least = t, best = {most, step};
   }
@@ -322,7 +324,9 @@ inline BwdDeal make_bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bo
   const int bq = (L + 127) / 128, bk = (Lk + 127) / 128;
   const BwdSplitPlan even = bwd_split_plan(D, Z, H, L, Lk, causal, dual, cus);
   if (!causal) return {{even.chunks_q, 0, 0, bq}, {even.chunks_k, 0, 0, bk}};
-  auto step_of = [](int chunks, int tiles) { return chunks > 1 ? (tiles + 1) / 2 : 0; };
+  auto step_of = [](int chunks, int tiles) { return chunks > 1 ? tiles : 0; };
+  // (in the account with shares of whole blocks, two tiles: what its pick was measured with)
+  auto rounded = [](const BwdDeal &d) { return BwdDeal{{d.q.most, (d.q.step + 1) / 2 * 2, d.q.first, d.q.last}, {d.k.most, (d.k.step + 1) / 2 * 2, d.k.first, d.k.last}}; };
   const long long heads = (long long)Z * H;
   const int nq = (std::min(bq * 128, Lk) + 63) / 64, nk = (L + 63) / 64, live = std::min(bk, bq);  // tiles of the longest blocks; key blocks that a query sees
   const BwdDeal alike = {{even.chunks_q, step_of(even.chunks_q, even.tiles_q), 0, bq}, {even.chunks_k, step_of(even.chunks_k, even.tiles_k), bq - live, bq}};
@@ -340,16 +344,16 @@ inline BwdDeal make_bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bo
   BwdDeal best = {{1, 0, 0, bq}, {1, 0, bq - live, bq}};
   double least = time(best) * (dual && D == 64 ? 1.07 : 1.0);  // (the account is fitted to shares; of whole blocks with tangents it makes 7 % too little at D = 64)
   if (!alike.any() && least < SPLIT_BACKWARD_US) return alike;
-  if (alike.any()) least = std::min(least, 0.92 * time(alike));  // (closer than that the account does not tell them apart)
+  if (alike.any()) least = std::min(least, 0.92 * time(rounded(alike)));  // (closer than that the account does not tell them apart)
   const double longest = std::max((double)nq, KEYS * nk);
   for (const int j : {4, 5, 6, 8, 12, 16}) {  // shares of 1/2 ... 1/8 of the longest block
     const double share = longest * 2 / j;
     auto deal = [&](int n, double t, int first, int last) {
       const int most = std::min(8, std::max(1, (int)(n * t / share + 0.99)));
-      return Deal{most, most > 1 ? ((n + 1) / 2 + most - 1) / most : 0, first, last};
+      return Deal{most, most > 1 ? ((n + 1) / 2 + most - 1) / most * 2 : 0, first, last};
     };
     const BwdDeal d = {deal(nq, 1.0, 0, bq), deal(nk, KEYS, bq - live, bq)};
-    if ((d.q.most > 1 && d.q.step < 2) || (d.k.most > 1 && d.k.step < 2) || heads * (d.q.most * bq + 2 * d.k.most * bk) > 6 * cus) break;
+    if ((d.q.most > 1 && d.q.step < 4) || (d.k.most > 1 && d.k.step < 4) || heads * (d.q.most * bq + 2 * d.k.most * bk) > 6 * cus) break;
     const double t = time(d);
     if (t < least) least = t, best = d;
   }
@@ -385,7 +389,7 @@ inline BwdDeal make_bwd_deal_f32(int D, int Z, int H, int L, int Lk, bool causal
   for (const int j : {3, 4, 5, 6, 8, 10, 12, 16}) {
     auto deal = [&](int n, double scale, int first, int last) {
       const int most = std::min({8, n, std::max(1, (int)(n * scale * j / (2 * longest) + 0.99))});
-      return Deal{most, causal && most > 1 ? ((n + 1) / 2 + most - 1) / most : 0, first, last};
+      return Deal{most, causal && most > 1 ? ((n + 1) / 2 + most - 1) / most * 2 : 0, first, last};
     };
     const BwdDeal d = {deal(longest_q, 1.0, 0, bq), deal(longest_k, KEYS, k0, k1)};
     if (heads * (d.q.most * bq + 2 * d.k.most * bk) > 8 * cus) break;

@@ -54,6 +54,25 @@ def test_deals_of_backwards(tmp_path):
     assert run(tmp_path, f'  for (bool b : {{{whole}}}) std::printf("%d ", b ? 1 : 0);\n') == [0, 0, 0]
 
 
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
+def test_equal_shares_are_as_long_as_planned(tmp_path):
+    """Odd lengths, too: no share of any block is longer, and no block is cut into more than it needs."""
+    text = "  int bad = 0, odd = 0;\n  struct P { int D, Z, H, L, dtype, causal, mask_kind; float dropout_p; };\n"
+    for D, dual, H, L in [(128, 1, 3, 728), (128, 1, 7, 1635), (64, 0, 3, 5000), (128, 0, 12, 1997), (128, 1, 2, 6201), (64, 1, 5, 3427)]:
+        text += f"""  {{ const BwdSplitPlan e = bwd_split_plan({D}, 1, {H}, {L}, {L}, true, {dual}, 256);
+    const BwdDeal d = make_bwd_deal({D}, 1, {H}, {L}, {L}, true, {dual}, 256);
+    odd += e.tiles_q % 2;
+    for (int o = 0; o < d.q.last; ++o) bad += d.q.shares(o) != (2 * o + 2 + e.tiles_q - 1) / e.tiles_q; }}
+"""
+    for H, L in [(12, 693), (12, 651), (5, 676), (3, 680)]:
+        text += f"""  {{ const P p = {{128, 1, {H}, {L}, 0, 1, 0, 0.f}}; const SplitPlan s = fwd_split_plan_16(p, {L}, false, 256);
+    const int n = {(L + 63) // 64}, per = (n + s.chunks - 1) / s.chunks;
+    for (int o = 0; o < {(L + 127) // 128}; ++o) bad += s.chunks < 2 || Deal{{s.chunks, s.chunk_tiles, 0, {(L + 127) // 128}}}.shares(o) != (std::min(2 * o + 2, n) + per - 1) / per; }}
+"""
+    bad, odd = run(tmp_path, text + '  std::printf("%d %d", bad, odd);\n')
+    assert bad == 0 and odd > 3
+
+
 # few workgroups, more than there are units (heads that are and are not a multiple of 8), keys and queries of unequal number
 SHAPES = [(1, 4, 1100, 1100), (1, 3, 4200, 4200), (2, 4, 2100, 2100), (1, 2, 900, 2000), (1, 3, 2000, 900)]
 
