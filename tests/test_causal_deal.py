@@ -73,6 +73,19 @@ def test_equal_shares_are_as_long_as_planned(tmp_path):
     assert bad == 0 and odd > 3
 
 
+# D, tangents, heads, rows of a causal forward, and the shares of its longest block on 256 compute units
+FORWARDS = [(128, 0, 6, 1111, 3), (128, 0, 4, 1111, 3), (128, 0, 3, 1667, 5), (128, 0, 6, 1484, 4), (64, 0, 5, 1985, 4), (64, 0, 3, 1985, 4), (64, 1, 8, 1103, 3),
+            (128, 1, 8, 2048, 3), (128, 1, 2, 8192, 3), (64, 0, 3, 7421, 4), (64, 0, 1, 14336, 4), (128, 1, 6, 4096, 2)]
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
+def test_no_more_shares_than_the_merge_is_worth(tmp_path):
+    text = "  struct P { int D, Z, H, L, dtype, causal, mask_kind; float dropout_p; };\n"
+    for D, dual, H, L, _ in FORWARDS:
+        text += f'  {{ const P p = {{{D}, 1, {H}, {L}, 0, 1, 0, 0.f}}; std::printf("%d ", fwd_split_plan_16(p, {L}, {dual}, 256).chunks); }}\n'
+    assert [(x, y) for x, y in zip(FORWARDS, run(tmp_path, text)) if x[-1] != y] == []
+
+
 # few workgroups, more than there are units (heads that are and are not a multiple of 8), keys and queries of unequal number
 SHAPES = [(1, 4, 1100, 1100), (1, 3, 4200, 4200), (2, 4, 2100, 2100), (1, 2, 900, 2000), (1, 3, 2000, 900)]
 
