@@ -120,9 +120,12 @@ typedef struct jvpfa_fwd_args {
 
 int jvpfa_fwd(const jvpfa_fwd_args *args, void *hip_stream);
 
-/* Bytes of split_workspace with which jvpfa_fwd would split this problem on the current device; 0 if it would
- * not (grid large enough, or a kernel that does not split). */
+/* Bytes of split_workspace with which jvpfa_fwd would split this problem on the current device, with tangents or without, whichever takes
+ * more, and with as many key/value heads as query heads; 0 if it would not (grid large enough, or a kernel that does not split). */
 size_t jvpfa_fwd_split_workspace_bytes(const jvpfa_problem *p, int32_t Lk);
+/* ... with which jvpfa_fwd would split the call that these arguments make (split_workspace and its size are not looked at, the other pointers
+ * only for NULL); 0 if it would not use any. */
+size_t jvpfa_fwd_split_needed(const jvpfa_fwd_args *args);
 
 /*
  * Backward of  Loss = <go, o> + <gt, ot>.  Replaces the device work of
@@ -172,8 +175,10 @@ int jvpfa_bwd(const jvpfa_bwd_args *args, void *hip_stream);
 size_t jvpfa_bwd_workspace_bytes(int32_t Z, int32_t H, int32_t L);
 
 /* Bytes of split_workspace with which jvpfa_bwd would split this problem on the current device (tangent_grads: dqt,
- * dkt, dvt are asked for too); 0 if it would not. */
+ * dkt, dvt are asked for too), with a gradient of ot or without, whichever takes more; 0 if it would not. */
 size_t jvpfa_bwd_split_workspace_bytes(const jvpfa_problem *p, int32_t Lk, int32_t Hk, int32_t tangent_grads);
+/* ... with which jvpfa_bwd would split the call that these arguments make, as jvpfa_fwd_split_needed(). */
+size_t jvpfa_bwd_split_needed(const jvpfa_bwd_args *args);
 
 /*
  * jvpfa_bwd for callers that cannot hand over a workspace because they cannot allocate one: code

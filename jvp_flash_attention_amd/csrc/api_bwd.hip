@@ -44,6 +44,16 @@ extern "C" size_t jvpfa_bwd_split_workspace_bytes(const jvpfa_problem *p, int32_
   return chunks > 1 ? bwd_part_floats(*p, Lk, Hk, chunks, tangent_grads != 0) * sizeof(float) : 0;
 }
 
+extern "C" size_t jvpfa_bwd_split_needed(const jvpfa_bwd_args *a) {
+  if (!a || a->struct_size != sizeof(jvpfa_bwd_args) || check_problem(a->p) != JVPFA_OK || check_kv_shape(a->p, a->Lk, a->Hk) != JVPFA_OK) return 0;
+  const int Lk = a->Lk > 0 ? a->Lk : a->p.L, Hk = a->Hk > 0 ? a->Hk : a->p.H;
+  const bool six = a->dqt != nullptr;
+  const BwdDeal sp = bwd_deal_of(a->p, Lk, Hk, six, a->gt != nullptr);
+  if (sp.any()) return bwd_split_floats(a->p, Lk, sp) * sizeof(float);
+  const int chunks = bwd_kv_chunks(a->p, Lk, Hk);
+  return chunks > 1 ? bwd_part_floats(a->p, Lk, Hk, chunks, six) * sizeof(float) : 0;
+}
+
 // Everything jvpfa_bwd does, with the row statistics of the pre-pass in `workspace`.
 static int bwd_impl(const jvpfa_bwd_args *a, void *workspace, void *hip_stream) {
   if (!a) return JVPFA_E_NULL;

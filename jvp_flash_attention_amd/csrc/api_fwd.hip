@@ -18,6 +18,17 @@ static const fwd_launcher kFwd[12] = {fwd_bf16_32, fwd_bf16_64, fwd_bf16_128, fw
 
 using namespace jvpfa;
 
+// How a valid call's blocks are split if its workspace suffices, and what that takes.  (fp32 with grouped heads: blocks stay whole, as they
+// do in its backward, so that the gradients of a head do not depend on how many others there are.)
+static SplitPlan fwd_plan_of(const jvpfa_fwd_args &a) {
+  const int Lk = a.Lk > 0 ? a.Lk : a.p.L, Hk = a.Hk > 0 ? a.Hk : a.p.H;
+  if (a.p.dtype == JVPFA_FP32 && Hk != a.p.H) return {1, 0};
+  return fwd_split_plan(a.p, Lk, a.qt != nullptr);
+}
+static size_t fwd_part_bytes(const jvpfa_problem &p, const SplitPlan &s, bool dual) {
+  return s.chunks > 1 ? fwd_part_floats(s.chunks, (long long)p.Z * p.H * p.L, p.D, dual) * sizeof(float) : 0;
+}
+
 extern "C" int jvpfa_fwd(const jvpfa_fwd_args *a, void *hip_stream) {
   if (!a) return JVPFA_E_NULL;
   if (a->struct_size != sizeof(jvpfa_fwd_args)) return JVPFA_E_ABI;
@@ -39,12 +50,9 @@ extern "C" int jvpfa_fwd(const jvpfa_fwd_args *a, void *hip_stream) {
   p.q = a->q; p.k = a->k; p.v = a->v;
   p.qt = a->qt; p.kt = a->kt; p.vt = a->vt;
   p.o = a->o; p.ot = a->ot; p.M = a->M; p.mu = a->mu;
-  // Small grid: split the key tiles of query blocks, if the workspace suffices.  (fp32 with grouped heads: blocks stay whole, as they do
-  // in its backward, so that the gradients of a head do not depend on how many others there are.)
-  if (a->split_workspace && !(a->p.dtype == JVPFA_FP32 && p.pr.Hk != p.pr.H)) {
-    const SplitPlan sp = fwd_split_plan(a->p, p.pr.Lk, dual);
-    if (sp.chunks > 1 && aligned16(a->split_workspace) &&
-        a->split_workspace_bytes >= fwd_part_floats(sp.chunks, (long long)a->p.Z * a->p.H * a->p.L, a->p.D) * sizeof(float)) {
+  if (a->split_workspace) {  // small grid: split the key tiles of query blocks, if the workspace suffices
+    const SplitPlan sp = fwd_plan_of(*a);
+    if (sp.chunks > 1 && aligned16(a->split_workspace) && a->split_workspace_bytes >= fwd_part_bytes(a->p, sp, dual)) {
       p.pr.chunks = sp.chunks;
       p.pr.chunk_tiles = sp.chunk_tiles;
       p.pr.part = static_cast<float *>(a->split_workspace);
@@ -55,9 +63,14 @@ extern "C" int jvpfa_fwd(const jvpfa_fwd_args *a, void *hip_stream) {
 
 extern "C" size_t jvpfa_fwd_split_workspace_bytes(const jvpfa_problem *p, int32_t Lk) {
   if (!p || check_problem(*p) != JVPFA_OK) return 0;
-  int chunks = 1;  // of the plan with tangents or of that without, whichever takes more
-  for (const bool dual : {false, true}) chunks = std::max(chunks, fwd_split_plan(*p, Lk > 0 ? Lk : p->L, dual).chunks);
-  return chunks > 1 ? fwd_part_floats(chunks, (long long)p->Z * p->H * p->L, p->D) * sizeof(float) : 0;
+  size_t most = 0;
+  for (const bool dual : {false, true}) most = std::max(most, fwd_part_bytes(*p, fwd_split_plan(*p, Lk > 0 ? Lk : p->L, dual), dual));
+  return most;
+}
+
+extern "C" size_t jvpfa_fwd_split_needed(const jvpfa_fwd_args *a) {
+  if (!a || a->struct_size != sizeof(jvpfa_fwd_args) || check_problem(a->p) != JVPFA_OK || check_kv_shape(a->p, a->Lk, a->Hk) != JVPFA_OK) return 0;
+  return fwd_part_bytes(a->p, fwd_plan_of(*a), a->qt != nullptr);
 }
 
 extern "C" int jvpfa_abi_version(void) { return JVPFA_ABI_VERSION; }

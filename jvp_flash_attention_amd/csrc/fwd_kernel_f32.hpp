@@ -183,7 +183,7 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
   const int ntiles = __builtin_amdgcn_readfirstlane(walk.n);
   // partial results of a share: [share][row][O | T][D], then [share][row][m, l, mu_acc, c]
   const size_t nrows = (size_t)pr.Z * pr.H * L, prow = (size_t)share.index * nrows + (size_t)zh * L + qrow;
-  float *part_stat = pr.part + (size_t)pr.chunks * nrows * 2 * D + prow * 4;
+  float *part_stat = pr.part + (size_t)pr.chunks * nrows * ((DUAL ? 2 : 1) * D) + prow * 4;
   if (split && ntiles <= 0) {  // none of its tiles is visited: it weighs nothing
     if (qrow < L && g == 0) *reinterpret_cast<f32x4 *>(part_stat) = f32x4{NEG_INF, -0.f, 0.f, 0.f};
     return;
@@ -354,7 +354,7 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
   const bool dead = !split && !(l_i > 0.f);
   const float inv = split ? 1.f : dead ? 0.f : 1.f / l_i, mu_n = split ? 0.f : mu_i * inv;  // a share is left as it stands for the merge kernel
   if (qrow < L) {
-    float *Og = split ? pr.part + prow * 2 * D : reinterpret_cast<float *>(p.o) + head + (size_t)qrow * D;
+    float *Og = split ? pr.part + prow * ((DUAL ? 2 : 1) * D) : reinterpret_cast<float *>(p.o) + head + (size_t)qrow * D;
     float *Otg = split ? Og + D : DUAL ? reinterpret_cast<float *>(p.ot) + head + (size_t)qrow * D : nullptr;
     // registers 4q .. 4q + 3 are rows 8q + 4g + 0..3: 4 DB consecutive columns
 #pragma unroll

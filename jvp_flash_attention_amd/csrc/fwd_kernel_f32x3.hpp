@@ -197,7 +197,7 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
   const int ntiles = __builtin_amdgcn_readfirstlane(walk.n);
   // partial results of a share: [share][row][O | T][D], then [share][row][m, l, mu_acc, c]
   const size_t nrows = (size_t)pr.Z * pr.H * L, prow = (size_t)share.index * nrows + (size_t)zh * L + qrow;
-  float *part_stat = pr.part + (size_t)pr.chunks * nrows * 2 * D + prow * 4;
+  float *part_stat = pr.part + (size_t)pr.chunks * nrows * ((DUAL ? 2 : 1) * D) + prow * 4;
   if (split && ntiles <= 0) {  // none of its tiles is visited: it weighs nothing
     if (qrow < L && g == 0) *reinterpret_cast<f32x4 *>(part_stat) = f32x4{NEG_INF, -0.f, 0.f, 0.f};
     return true;
@@ -553,7 +553,7 @@ __device__ __forceinline__ bool fwd_f32x3_body(const FwdParams &p) {
   const float inv = split ? 1.f : dead ? 0.f : 1.f / l_i, mu_n = split ? 0.f : mu_i * inv;  // a share is left as it stands for the merge kernel
   float check = l_i * 0.f;  // not zero once an output is not finite (a row sum that is not a number makes its row 0)
   if (qrow < L) {
-    float *Og = split ? pr.part + prow * 2 * D : reinterpret_cast<float *>(p.o) + head + (size_t)qrow * D;
+    float *Og = split ? pr.part + prow * ((DUAL ? 2 : 1) * D) : reinterpret_cast<float *>(p.o) + head + (size_t)qrow * D;
     float *Otg = split ? Og + D : DUAL ? reinterpret_cast<float *>(p.ot) + head + (size_t)qrow * D : nullptr;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {

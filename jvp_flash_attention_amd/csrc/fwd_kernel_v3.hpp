@@ -115,7 +115,7 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   const int Lk = pr.Lk - k0;
   // partial results of a chunk: [chunk][row][O | T][D] floats, then [chunk][row][m, l, mu_acc, c]
   const size_t nrows = (size_t)pr.Z * pr.H * L, prow = (size_t)share.index * nrows + (size_t)zh * L + qrow;
-  float *part_stat = pr.part + (size_t)pr.chunks * nrows * 2 * D + prow * 4;
+  float *part_stat = pr.part + (size_t)pr.chunks * nrows * ((DUAL ? 2 : 1) * D) + prow * 4;
   if (split && ntiles <= 0) {  // fewer tiles than shares would take: this one weighs nothing
     if (qrow < L && g == 0) {
       const f32x4 none = {-__builtin_inff(), -0.f, 0.f, 0.f};
@@ -726,7 +726,7 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   if constexpr (DUAL) mu_i += xor32(mu_i);
   if (split) {  // this chunk's share, left as it stands for the merge kernel
     if (qrow < L) {
-      float *pa = pr.part + prow * 2 * D;
+      float *pa = pr.part + prow * ((DUAL ? 2 : 1) * D);
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
 #pragma unroll

@@ -128,7 +128,7 @@ inline int device_cus() {
 
 // Workspace of the forward: per chunk and query row 2 D accumulator values (O, T, not yet divided by l) and
 // four statistics (m, l, mu_acc, c).
-inline size_t fwd_part_floats(int chunks, long long rows, int D) { return (size_t)chunks * rows * (2 * (size_t)D + 4); }
+inline size_t fwd_part_floats(int chunks, long long rows, int D, bool dual) { return (size_t)chunks * rows * ((dual ? 2 : 1) * (size_t)D + 4); }
 // The kernels that can split: 16-bit element types, D = 64 or 128, no mask (the software-pipelined forward).  Tiles are 64
 // wide, blocks 128 rows.
 template <typename P> inline bool split_capable(const P &p) {
@@ -501,7 +501,7 @@ inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven, 
 }
 
 // ---- merge kernels -------------------------------------------------------------------------------
-// Forward.  part = [chunk][row][2][D] accumulators, then [chunk][row][4] statistics.  One thread per (row, 8
+// Forward.  part = [chunk][row][O, with tangents T][D] accumulators, then [chunk][row][4] statistics.  One thread per (row, 8
 // columns), a grid of (rows of a head, heads).  With m the largest reference point of the row's chunks and w_c = 2^(m_c - m):
 //   l = sum w_c l_c,  O = sum w_c O_c,  and, with c the reference of S' of the heaviest chunk,
 //   T = sum w_c (T_c + (c_c - c) O_c),  mu_acc = sum w_c (mu_c + (c_c - c) l_c);
@@ -511,12 +511,12 @@ inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven, 
 // workgroup's rescaling makes of it.  So the outputs that are not numbers are those of whole blocks.
 template <typename T, int D, bool DUAL>
 __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, T *ot, float *M, float *mu) {
-  constexpr int LPR = D / 8, RPB = 256 / LPR;
+  constexpr int LPR = D / 8, RPB = 256 / LPR, ROW = DUAL ? 2 * D : D;
   const int in_head = blockIdx.x * RPB, chunks = Deal{pr.chunks, pr.chunk_tiles, 0, 0}.shares(in_head / 128);  // (uniform: RPB divides 128)
   if (chunks == 1 || in_head + (int)threadIdx.x / LPR >= pr.L) return;  // a block that one workgroup did is finished
   const size_t rows = (size_t)pr.Z * pr.H * pr.L, row = (size_t)blockIdx.y * pr.L + in_head + threadIdx.x / LPR;
   const int d0 = (threadIdx.x % LPR) * 8;
-  const float *part = pr.part, *stat = part + (size_t)pr.chunks * rows * 2 * D;
+  const float *part = pr.part, *stat = part + (size_t)pr.chunks * rows * ROW;
   float m = -__builtin_inff();
   for (int c = 0; c < chunks; ++c) m = fmaxf(m, stat[((size_t)c * rows + row) * 4]);
   const float m_use = m == -__builtin_inff() ? 0.f : m;
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, 
     const float *st = stat + ((size_t)c * rows + row) * 4;
     if (__builtin_bit_cast(uint32_t, st[1]) == 0x80000000u) continue;
     const float w = __builtin_amdgcn_exp2f(st[0] - m_use);
-    const float *acc = part + ((size_t)c * rows + row) * 2 * D + d0;
+    const float *acc = part + ((size_t)c * rows + row) * ROW + d0;
     const float dc = st[3] - cref;
     mua += w * (st[2] + dc * st[1]);
 #pragma unroll

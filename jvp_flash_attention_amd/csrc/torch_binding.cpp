@@ -114,7 +114,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> forward(const Tensor &q, const Tensor
   a.Hk = static_cast<int32_t>(k.size(1)), a.Lk = static_cast<int32_t>(k.size(2));  // may differ from q's
   Tensor workspace;
   if (c.split) {
-    a.split_workspace_bytes = jvpfa_fwd_split_workspace_bytes(&a.p, a.Lk);
+    a.split_workspace_bytes = jvpfa_fwd_split_needed(&a);
     if (a.split_workspace_bytes) {
       workspace = at::empty({static_cast<int64_t>(a.split_workspace_bytes)}, q.options().dtype(at::kByte).requires_grad(false));
       a.split_workspace = out(workspace);
@@ -155,7 +155,7 @@ std::vector<Tensor> backward(const Tensor &q, const Tensor &k, const Tensor &v, 
   a.Hk = static_cast<int32_t>(k.size(1)), a.Lk = static_cast<int32_t>(k.size(2));
   Tensor shares;
   if (c.split) {
-    a.split_workspace_bytes = jvpfa_bwd_split_workspace_bytes(&a.p, a.Lk, a.Hk, want_tangent_grads ? 1 : 0);
+    a.split_workspace_bytes = jvpfa_bwd_split_needed(&a);
     if (a.split_workspace_bytes) {
       shares = at::empty({static_cast<int64_t>(a.split_workspace_bytes)}, q.options().dtype(at::kByte).requires_grad(false));
       a.split_workspace = out(shares);

@@ -1,4 +1,4 @@
-"""Forwards whose blocks' keys are dealt to several workgroups: what is not a number comes out where whole blocks have it."""
+"""Calls whose blocks' tiles are dealt to several workgroups: what is not a number comes out where whole blocks have it, and the workspace is the one in use."""
 import ctypes as C
 
 import pytest
@@ -92,3 +92,84 @@ def test_masked_shares_of_values_that_are_not_numbers(D):
         alive = torch.isfinite(b)
         assert torch.equal(alive, torch.isfinite(a)) and torch.equal(torch.isnan(a), torch.isnan(b)), i
         assert (a[alive] - b[alive]).norm() <= 1e-5 * b[alive].norm(), i
+
+
+def _fwd_args(dev, o, ot, M, mu, causal, scale):
+    a = _lib.FwdArgs()
+    a.struct_size = C.sizeof(_lib.FwdArgs)
+    a.p = _lib.make_problem(dev[0], None, _lib.MASK_NONE, causal, scale)
+    for name, x in zip(("q", "k", "v", "qt", "kt", "vt", "o", "ot", "M", "mu"), (*dev, o, ot, M, mu)):
+        setattr(a, name, None if x is None else x.data_ptr())
+    a.Hk, a.Lk = dev[1].shape[1], dev[1].shape[2]
+    return a
+
+
+@pytest.mark.parametrize("dtype,D,H,Hk,L,causal", [(torch.float32, 128, 8, 8, 512, False), (torch.float32, 64, 2, 2, 2048, True), (torch.float32, 128, 16, 4, 1024, True),
+                                                   (torch.bfloat16, 128, 2, 2, 2048, False), (torch.float16, 64, 3, 3, 3000, True), (torch.bfloat16, 128, 8, 2, 1500, True)])
+@pytest.mark.parametrize("dual", [False, True])
+def test_a_call_takes_the_workspace_that_it_uses(dtype, D, H, Hk, L, causal, dual):
+    """What is asked for is what is written and allocated: nothing behind it, nothing for a call that stays whole, no half for tangents that are not there."""
+    print("case", dtype, D, H, Hk, L, causal, dual, flush=True)
+    g = torch.Generator().manual_seed(L)
+    dev = [torch.randn(1, h, L, D, generator=g).to(dtype).cuda() for h in (H, Hk, Hk, H, Hk, Hk)]
+    if not dual:
+        dev[3:] = [None] * 3
+    be, lib, scale, rows = _lib.backend(), _lib.load(), D**-0.5, H * L
+    want = be.fwd(*dev, None, _lib.MASK_NONE, causal, scale)
+    outputs = sum(x.numel() * x.element_size() for x in want if x is not None)
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    again = be.fwd(*dev, None, _lib.MASK_NONE, causal, scale)
+    taken = torch.cuda.max_memory_allocated() - base - outputs
+    slack = 5 << 20  # blocks of the allocator that were not worth splitting, at most 1 MiB each
+    if dtype == torch.float32 and Hk != H:
+        assert taken <= slack
+    a = _fwd_args(dev, *again, causal, scale)
+    needed = lib.jvpfa_fwd_split_needed(C.byref(a))
+    assert needed % (rows * ((2 if dual else 1) * D + 4) * 4) == 0 and taken <= needed + slack
+    assert (needed == 0) == (dtype == torch.float32 and Hk != H)
+    assert needed <= lib.jvpfa_fwd_split_workspace_bytes(C.byref(a.p), L)
+    if not needed:
+        return
+    assert needed // (rows * ((2 if dual else 1) * D + 4) * 4) in range(2, 9)
+    space = torch.full((needed + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    for x in again:
+        if x is not None:
+            x.fill_(float("nan"))
+    a.split_workspace, a.split_workspace_bytes = space.data_ptr(), needed
+    _lib.check(lib.jvpfa_fwd(C.byref(a), torch.cuda.current_stream().cuda_stream))
+    assert all(torch.equal(x, y) for x, y in zip(again, want) if y is not None)
+    assert (space[needed:] == 0x5A).all() and not (space[:needed] == 0x5A).all()
+    a.split_workspace_bytes = needed - 1  # too little: whole blocks
+    space.fill_(0x5A)
+    _lib.check(lib.jvpfa_fwd(C.byref(a), torch.cuda.current_stream().cuda_stream))
+    assert (space == 0x5A).all() and torch.isfinite(again[0]).all()
+
+
+@pytest.mark.parametrize("dtype,D,H,Hk,L", [(torch.float32, 64, 8, 8, 700), (torch.float32, 128, 8, 2, 512), (torch.bfloat16, 128, 4, 4, 1024), (torch.bfloat16, 64, 3, 3, 3000)])
+@pytest.mark.parametrize("grads", ["plain", "both", "six"])
+def test_a_backward_takes_the_workspace_that_it_uses(dtype, D, H, Hk, L, grads):
+    print("case", dtype, D, H, Hk, L, grads, flush=True)
+    g = torch.Generator().manual_seed(L)
+    dev = [torch.randn(1, h, L, D, generator=g).to(dtype).cuda() for h in (H, Hk, Hk, H, Hk, Hk, H, H)]
+    if grads == "plain":
+        dev[3:6], dev[7] = [None] * 3, None
+    be, lib, scale = _lib.backend(), _lib.load(), D**-0.5
+    o, ot, M, mu = be.fwd(*dev[:6], None, _lib.MASK_NONE, True, scale)
+    want = be.bwd(*dev[:6], o, ot, M, mu, *dev[6:], None, _lib.MASK_NONE, True, scale, grads == "six")
+    got = [None if x is None else torch.full_like(x, float("nan")) for x in want]
+    rows = torch.empty(lib.jvpfa_bwd_workspace_bytes(1, H, L), dtype=torch.uint8, device="cuda")
+    a = _lib.BwdArgs()
+    a.struct_size = C.sizeof(_lib.BwdArgs)
+    a.p = _lib.make_problem(dev[0], None, _lib.MASK_NONE, True, scale)
+    names = ("q", "k", "v", "qt", "kt", "vt", "o", "ot", "M", "mu", "go", "gt", "dq", "dk", "dv", "dqt", "dkt", "dvt", "workspace")
+    for name, x in zip(names, (*dev[:6], o, ot, M, mu, *dev[6:], *got, rows)):
+        setattr(a, name, None if x is None else x.data_ptr())
+    a.Hk, a.Lk = Hk, L
+    needed = lib.jvpfa_bwd_split_needed(C.byref(a))
+    assert needed <= lib.jvpfa_bwd_split_workspace_bytes(C.byref(a.p), L, Hk, int(grads == "six"))
+    space = torch.full((needed + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    a.split_workspace, a.split_workspace_bytes = space.data_ptr(), needed
+    _lib.check(lib.jvpfa_bwd(C.byref(a), torch.cuda.current_stream().cuda_stream))
+    assert all(torch.equal(x, y) for x, y in zip(got, want) if y is not None)
+    assert (space[needed:] == 0x5A).all() and (needed == 0 or not (space[:needed] == 0x5A).all())
