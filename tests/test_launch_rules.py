@@ -142,6 +142,18 @@ PLANS = """
 """
 
 
+def test_plans_are_remembered_for_as_many_shapes_as_a_model_has(tmp_path):
+    """Sixteen shapes in turn, again and again: each is planned once, and every answer is that of its sizes."""
+    text = PLANS + """
+  int bad = 0;
+  for (int i = 0; i < 1600; ++i) bad += plan(100 + i % 16 * 37) != 3 * (100 + i % 16 * 37);
+  const int first = made;
+  for (int i = -1000; i < 1000; ++i) bad += plan(i * 7919) != 3 * (i * 7919) || plan(i * 7919) != 3 * (i * 7919);
+  std::printf("%d %d %d", bad, first, (int)(made - first));
+"""
+    assert run(tmp_path, text) == [0, 16, 2000]
+
+
 def test_plans_are_remembered_however_many_were_made(tmp_path):
     """More plans than a 32-bit count holds, each of another size: the last one is still found where it was put."""
     text = PLANS + """
