@@ -90,6 +90,7 @@ static int bwd_impl(const jvpfa_bwd_args *a, void *workspace, void *hip_stream) 
     const BwdDeal sp = bwd_deal_of(a->p, p.pr.Lk, p.pr.Hk, ntg == 3, dual);
     if (sp.any() && aligned16(a->split_workspace) && a->split_workspace_bytes >= bwd_split_floats(a->p, p.pr.Lk, sp) * sizeof(float)) {
       p.pr.chunk_tiles = -1;  // (the launcher makes the same plan)
+      p.pr.units = device_cus();
       p.pr.part = static_cast<float *>(a->split_workspace);
     }
     const int chunks = bwd_kv_chunks(a->p, p.pr.Lk, p.pr.Hk);

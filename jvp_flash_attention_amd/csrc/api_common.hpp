@@ -48,6 +48,7 @@ inline Problem to_problem(const jvpfa_problem &p, const int32_t *key_limit, cons
   r.chunks = 1;
   r.chunk_tiles = 0;
   r.part = nullptr;
+  r.units = 0;
   r.drop_thr = 0;
   r.drop_s0 = r.drop_s1 = 0;
   r.drop_rinv = 1.f;

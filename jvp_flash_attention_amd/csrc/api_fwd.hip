@@ -55,6 +55,7 @@ extern "C" int jvpfa_fwd(const jvpfa_fwd_args *a, void *hip_stream) {
     if (sp.chunks > 1 && aligned16(a->split_workspace) && a->split_workspace_bytes >= fwd_part_bytes(a->p, sp, dual)) {
       p.pr.chunks = sp.chunks;
       p.pr.chunk_tiles = sp.chunk_tiles;
+      p.pr.units = device_cus();
       p.pr.part = static_cast<float *>(a->split_workspace);
     }
   }

@@ -145,7 +145,7 @@ __device__ __forceinline__ bool bwd_f32x3_dq_body(const BwdParams &p, const int 
   const Problem &pr = p.pr;
   const int L = pr.L, Lk = pr.Lk;
   const int nqb = (L + C::BLK - 1) / C::BLK;
-  const Dealt share = SPLIT ? deal_query_block(sp.q, bid, total, nqb, pr.Z * pr.H, pr.causal != 0) : Dealt{xcd_remap(bid, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
+  const Dealt share = SPLIT ? deal_query_block(sp.q, bid, total, nqb, pr.Z * pr.H, pr.causal != 0, more_than_units(gridDim.x, pr.units)) : Dealt{xcd_remap(bid, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
   const bool split = SPLIT && share.count > 1;
   const int zh = share.id / nqb;
   const int qb = pr.causal ? nqb - 1 - share.id % nqb : share.id % nqb;
@@ -434,7 +434,7 @@ __device__ __forceinline__ bool bwd_f32x3_dkdv_body(const BwdParams &p, const in
   const int L = pr.L, Lk = pr.Lk;
   const int nkb = (Lk + C::BLK - 1) / C::BLK;
   const int shares = pr.Z * pr.Hk * pr.chunks;
-  const Dealt share = SPLIT ? deal_key_block(sp.k, bid, total, nkb, shares, pr.causal != 0) : Dealt{xcd_remap(bid, nkb, shares, pr.causal != 0), 1, 0};
+  const Dealt share = SPLIT ? deal_key_block(sp.k, bid, total, nkb, shares, pr.causal != 0, more_than_units(gridDim.x, pr.units)) : Dealt{xcd_remap(bid, nkb, shares, pr.causal != 0), 1, 0};
   const bool split = SPLIT && share.count > 1;
   const int zhk = share.id / nkb / pr.chunks, chunk = share.id / nkb % pr.chunks;
   const int kb = share.id % nkb;  // causal: the first key blocks have the longest query loops

@@ -173,7 +173,7 @@ __device__ __forceinline__ void bwd2_dq_body(const BwdParams &p, const int bid, 
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
   static_assert(!SIX || DUAL, "dq' rides on the dual mode");
-  const Dealt share = SPLIT ? deal_query_block(sp.q, bid, total, (p.pr.L + Cfg::BLK - 1) / Cfg::BLK, p.pr.Z * p.pr.H, p.pr.causal != 0) : Dealt{-1, 1, 0};
+  const Dealt share = SPLIT ? deal_query_block(sp.q, bid, total, (p.pr.L + Cfg::BLK - 1) / Cfg::BLK, p.pr.Z * p.pr.H, p.pr.causal != 0, more_than_units(gridDim.x, p.pr.units)) : Dealt{-1, 1, 0};
   JVPFA_BWD2_COMMON(Cfg, pr.Lk, pr.L, pr.H, 1, share.id)  // owns query rows, streams key tiles
   const int qb = pr.causal ? nblk - 1 - id % nblk : id % nblk;
   const int q0 = qb * Cfg::BLK;
@@ -565,7 +565,7 @@ template <typename T, int D, int MODE, int MASK, bool GO, bool GROUPED, bool SIX
 __device__ __forceinline__ void bwd2_dkdv_body(const BwdParams &p, const int bid, const BwdSplit sp = {}, const int total = 0) {
   using Cfg = Bwd2Cfg<T, D, MODE>;
   constexpr bool DUAL = MODE == BWD_DUAL, TAN = MODE == BWD_TANGENT;
-  const Dealt share = SPLIT ? deal_key_block(sp.k, bid, total, (p.pr.Lk + Cfg::BLK - 1) / Cfg::BLK, p.pr.Z * p.pr.H, p.pr.causal != 0) : Dealt{-1, 1, 0};
+  const Dealt share = SPLIT ? deal_key_block(sp.k, bid, total, (p.pr.Lk + Cfg::BLK - 1) / Cfg::BLK, p.pr.Z * p.pr.H, p.pr.causal != 0, more_than_units(gridDim.x, p.pr.units)) : Dealt{-1, 1, 0};
   static_assert(!SIX || (DUAL && D <= 64), "dk', dv' ride on the dual mode, where the accumulators fit");
   JVPFA_BWD2_COMMON(Cfg, pr.L, pr.Lk, pr.Hk, GROUPED ? pr.chunks : 1, share.id)  // owns key rows (h: key/value head), streams query tiles
   const int kb = id % nblk;  // causal: the first key blocks have the longest query loops

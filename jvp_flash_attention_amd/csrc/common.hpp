@@ -170,7 +170,7 @@ __device__ __forceinline__ int xcd_remap(int bid, int per_head, int heads, bool 
 struct HeadRank {
   int head, rank;
 };
-__device__ __forceinline__ HeadRank deal_heads(int bid, int heads, int total, bool ordered) {
+__host__ __device__ __forceinline__ HeadRank deal_heads(int bid, int heads, int total, bool ordered) {
   constexpr int NXCD = 8;
   if (!ordered) {
     const int per_head = total / heads;
@@ -180,7 +180,7 @@ __device__ __forceinline__ HeadRank deal_heads(int bid, int heads, int total, bo
   const int mine = heads / NXCD, j = bid / NXCD;
   return {(j % mine) * NXCD + bid % NXCD, j / mine};
 }
-__device__ __forceinline__ bool more_than_units() { return gridDim.x > 256; }
+__host__ __device__ __forceinline__ bool more_than_units(int workgroups, int units) { return workgroups > units; }
 
 // Store 8 consecutive elements of type T converted from fp32.
 template <typename T> __device__ __forceinline__ void store8(T *dst, const float *x) {

@@ -124,7 +124,7 @@ __device__ __forceinline__ void fwd_f32_body(const FwdParams &p) {
   const int L = pr.L, Lk = pr.Lk;
   const int nqb = (L + C::BLK - 1) / C::BLK;
   // SPLIT, small grids: the key tiles of query blocks are split over workgroups (see split.hpp)
-  const Dealt share = SPLIT ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0)
+  const Dealt share = SPLIT ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0, more_than_units(gridDim.x, pr.units))
                             : Dealt{xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
   const bool split = SPLIT && share.count > 1;
   const int zh = share.id / nqb;

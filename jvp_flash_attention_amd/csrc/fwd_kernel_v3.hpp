@@ -74,7 +74,7 @@ __device__ __forceinline__ void fwd3_body(const FwdParams &p) {
   // backward 37.09 ms for 36.94; without it both are 0.2 - 0.5 % off (1428 for 1424 us, 38.72 for 38.59 ms on another card): within what
   // two runs of one build differ by.
   static_assert(!SPLIT || (MASK == MASK_NONE && !DROP && D <= 128));
-  const Dealt share = SPLIT ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0)
+  const Dealt share = SPLIT ? deal_query_block({pr.chunks, pr.chunk_tiles, 0, nqb}, blockIdx.x, gridDim.x, nqb, pr.Z * pr.H, pr.causal != 0, more_than_units(gridDim.x, pr.units))
                             : Dealt{xcd_remap(blockIdx.x, nqb, pr.Z * pr.H, pr.causal != 0), 1, 0};
   const int zh = share.id / nqb;
   const int qb = pr.causal ? nqb - 1 - share.id % nqb : share.id % nqb;

@@ -45,6 +45,7 @@ struct Problem {
   // (seed, z, h, i, j) in the forward, both backward kernels and jvpfa_dropout_keep.
   uint32_t drop_thr, drop_s0, drop_s1;
   float drop_rinv;
+  int units;  // compute units of the device, where blocks are split
 };
 
 // Counter-based keep decision, shaped so that a kernel pays a handful of vector instructions per entry whichever

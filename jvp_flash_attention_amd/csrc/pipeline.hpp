@@ -9,21 +9,21 @@
 
 namespace jvpfa {
 
-// What workgroup bid of a launch of `total` does that goes by a deal: a share of block `id` (as xcd_remap counts them).
+// What workgroup bid of a launch of `total` does that goes by a deal: a share of block `id` (as xcd_remap counts them).  ordered: see deal_heads.
 struct Dealt {
   int id, count, index;
 };
-__device__ __forceinline__ Dealt deal_query_block(const Deal &d, int bid, int total, int blocks, int heads, bool causal) {
+__device__ __forceinline__ Dealt deal_query_block(const Deal &d, int bid, int total, int blocks, int heads, bool causal, bool ordered) {
   if (d.step > 0) {  // (the id of a causal block counts from the last one)
-    const HeadRank hr = deal_heads(bid, heads, total, more_than_units());
+    const HeadRank hr = deal_heads(bid, heads, total, ordered);
     const Share s = share_of(d, hr.rank);
     return {hr.head * blocks + blocks - 1 - s.order, s.count, s.index};
   }
   return {xcd_remap(d.most > 1 ? bid / d.most : bid, blocks, heads, causal), d.most, d.most > 1 ? bid % d.most : 0};
 }
-__device__ __forceinline__ Dealt deal_key_block(const Deal &d, int bid, int total, int blocks, int heads, bool causal) {
+__device__ __forceinline__ Dealt deal_key_block(const Deal &d, int bid, int total, int blocks, int heads, bool causal, bool ordered) {
   if (d.step > 0) {
-    const HeadRank hr = deal_heads(bid, heads, total, more_than_units());
+    const HeadRank hr = deal_heads(bid, heads, total, ordered);
     const int seen = d.workgroups();  // ... then the key blocks behind the last query, which have zero gradients
     if (hr.rank >= seen) return {hr.head * blocks + d.last + hr.rank - seen, 1, 0};
     const Share s = share_of(d, hr.rank);

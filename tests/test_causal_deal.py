@@ -86,6 +86,21 @@ def test_no_more_shares_than_the_merge_is_worth(tmp_path):
     assert [(x, y) for x, y in zip(FORWARDS, run(tmp_path, text)) if x[-1] != y] == []
 
 
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
+def test_order_of_a_launch_goes_by_the_units_of_the_device(tmp_path):
+    """280 workgroups of 4 heads: heads side by side on 256 units, the shares of a block on 304; either way each once."""
+    text = """  for (int units : {256, 304}) {
+    int seen[4][70] = {}, bad = 0;
+    for (int b = 0; b < 280; ++b) {
+      const HeadRank r = deal_heads(b, 4, 280, more_than_units(280, units));
+      bad += r.head < 0 || r.head > 3 || r.rank < 0 || r.rank > 69 || seen[r.head][r.rank]++;
+    }
+    std::printf("%d %d ", bad, deal_heads(1, 4, 280, more_than_units(280, units)).head);
+  }
+"""
+    assert run(tmp_path, text) == [0, 1, 0, 0]
+
+
 # few workgroups, more than there are units (heads that are and are not a multiple of 8), keys and queries of unequal number
 SHAPES = [(1, 4, 1100, 1100), (1, 3, 4200, 4200), (2, 4, 2100, 2100), (1, 2, 900, 2000), (1, 3, 2000, 900)]
 
