@@ -192,10 +192,12 @@ template <typename P> inline SplitPlan fwd_split_plan_16(const P &p, int Lk, boo
   const DealCost cost = {wide ? (dual ? 2.45 : 1.2) : (dual ? 1.6 : 0.85), wide && dual ? 6.0 : 5.0, 7.0, 11.0 * p.D / 128 * (dual ? 1.0 : 0.5), 0.25, 1, 1.0};
   const int nblk = (p.L + 127) / 128;
   auto time = [&](int most, int step) {
-    // The merge reads a row's shares one after another.  Counted where equal shares are the alternative, whose number this one is measured
-    // against: H3 L1990 D64 without tangents in 4, 5, 8 shares 19.0, 19.2, 20.8 us; H6 L1111 D128 in 3, 5 shares 20.9, 22.6 (equal ones 21.5).
+    // The merge reads a row's shares one after another.  Counted where three or more equal shares are the alternative and blocks are short:
+    // H3 L1990 D64 without tangents in 4, 5, 8 shares 19.0, 19.2, 20.8 us; H6 L1111 D128 in 3, 5 shares 20.9, 22.6 (equal ones 21.5).  Over a hundred
+    // such launches 2.3 % less, 5 % more at worst.  In others the account is too coarse for it (H1 L16384 D64, two equal shares: 67.5 us in 6, but
+    // 84 in the 3 that it would pick; H1 L8483 D64, three: 32.6 us in 7, 34.9 in 6).
     DealCost with_merge = cost;
-    if (even.chunks > 1) with_merge.merge = 3.5 + 1.0 * most;
+    if (even.chunks > 2 && ntiles <= 64) with_merge.merge = 3.5 + 1.0 * most;
     DealTime t(cus, with_merge);
     t.add({most, step, 0, nblk}, (long long)p.Z * p.H, 1.0, 1.0, [&](int order) { return (std::min((order + 1) * 128, Lk) + 63) / 64; });
     return t.total();

@@ -75,7 +75,7 @@ def test_equal_shares_are_as_long_as_planned(tmp_path):
 
 # D, tangents, heads, rows of a causal forward, and the shares of its longest block on 256 compute units
 FORWARDS = [(128, 0, 6, 1111, 3), (128, 0, 4, 1111, 3), (128, 0, 3, 1667, 5), (128, 0, 6, 1484, 4), (64, 0, 5, 1985, 4), (64, 0, 3, 1985, 4), (64, 1, 8, 1103, 3),
-            (128, 1, 8, 2048, 3), (128, 1, 2, 8192, 3), (64, 0, 3, 7421, 4), (64, 0, 1, 14336, 4), (128, 1, 6, 4096, 2)]
+            (128, 1, 8, 2048, 3), (128, 1, 2, 8192, 3), (64, 0, 3, 7421, 4), (64, 0, 1, 14336, 4), (128, 1, 6, 4096, 2), (64, 0, 1, 16384, 6), (64, 0, 1, 8483, 7), (64, 1, 10, 1400, 4)]
 
 
 @pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
