@@ -1,5 +1,4 @@
 """Causal blocks dealt to workgroups by length: the deal itself on the CPU, and forwards and backwards that go by it on the GPU."""
-import ctypes as C
 import os
 
 import pytest
@@ -8,6 +7,7 @@ import torch
 from jvp_flash_attention_amd import _lib, build
 from oracle import dense
 
+from .test_gpu_split_merge import dealt_parts
 from .test_launch_rules import run
 
 
@@ -105,6 +105,10 @@ def test_order_of_a_launch_goes_by_the_units_of_the_device(tmp_path):
 SHAPES = [(1, 4, 1100, 1100), (1, 3, 4200, 4200), (2, 4, 2100, 2100), (1, 2, 900, 2000), (1, 3, 2000, 900)]
 
 
+# ... whose forwards stay whole on 256 compute units: always at D = 32, which has no kernel for it; at D = 64 head dim, queries, keys, tangents
+WHOLE_FORWARDS = {(64, 1100, 1100, False), (64, 2100, 2100, False), (64, 900, 2000, False), (64, 2000, 900, False), (64, 2000, 900, True)}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D", [32, 64, 128])
@@ -118,8 +122,8 @@ def test_dealt_blocks_agree_with_whole_ones(dtype, D, Z, H, L, Lk, grads):
     q, qt, go, gt, k, v, kt, vt = rand(L), rand(L), rand(L), rand(L), rand(Lk), rand(Lk), rand(Lk), rand(Lk)
     t = (None,) * 3 if grads == "plain" else (qt, kt, vt)
     be, scale = _lib.backend(), D**-0.5
-    p = _lib.make_problem(q, None, _lib.MASK_NONE, True, scale)
-    assert _lib.load().jvpfa_bwd_split_workspace_bytes(C.byref(p), Lk, H, 0) > 0
+    parts = dealt_parts((q, k, v, *t), (go, gt if grads != "plain" else None), None, _lib.MASK_NONE, True, scale)
+    assert parts == (D > 32 and (D, L, Lk, grads != "plain") not in WHOLE_FORWARDS, True)
     fwd = lambda: be.fwd(q, k, v, *t, None, _lib.MASK_NONE, True, scale)  # noqa: E731
     got = fwd()
     _lib.set_split(False)
@@ -134,8 +138,14 @@ def test_dealt_blocks_agree_with_whole_ones(dtype, D, Z, H, L, Lk, grads):
     ulp = 2.0**-7 if dtype == torch.bfloat16 else 2.0**-10
     for a, b in zip(got[2:], one[2:]):
         assert b is None or (a - b).abs().max().item() <= 1e-5 * max(1.0, b.abs().max().item())
-    for a, b in zip(got[:2], one[:2]):  # P is rounded against another reference point in each share: one unit, two for O'
-        assert b is None or ((a.float() - b.float()).abs() <= 2 * ulp * b.float().abs().clamp_min(1.0)).all()
+    # P is rounded against another reference point in each share, so either side has for every key an error of its own of up to half a unit of p, as
+    # good as independent: 0.3 units of the entry's size by root mean square (0.2 for a uniform error, times the square root of 2), and the result's own
+    # rounding.  O' has two products that are rounded so.  Five times that for the worst of 2 million entries, against its row's root mean square.
+    for a, b, products in zip(got[:2], one[:2], (1, 2)):
+        if b is not None:
+            a, b = a.double(), b.double()
+            assert (a - b).norm() <= products * ulp / 2 * b.norm()
+            assert ((a - b).abs() <= ulp * b.abs() + products * 2 * ulp * b.square().mean(-1, keepdim=True).sqrt()).all()
     for a, b in zip(dealt[:3], whole[:3]):  # the same P and dS, sums in fp32 in another order, each rounded once
         assert (a.float() - b.float()).norm() <= ulp / 2 * b.float().norm()
         assert ((a.float() - b.float()).abs() <= ulp * b.float().abs() + 1e-5 * b.float().abs().max()).all()

@@ -1,12 +1,12 @@
 """The pipelined forward at D = 64: rows around its shortest length, tile ends, and keys split over workgroups."""
-import ctypes as C
-
 import numpy as np
 import pytest
 import torch
 
 from jvp_flash_attention_amd import _lib
 from oracle import dense
+
+from .test_gpu_split_merge import dealt_parts
 
 pytestmark = pytest.mark.gpu
 
@@ -47,8 +47,7 @@ def test_tile_ends(dt, L, Lk, causal):
 def test_keys_split_over_workgroups(dual, Z, H, Hk, L, Lk, causal):
     dev, ref, got = run("bf16", Z, H, Hk, L, Lk, causal, dual)
     check(got, ref, dual)
-    p = _lib.make_problem(dev[0], None, _lib.MASK_NONE, causal, 0.125)
-    assert _lib.load().jvpfa_fwd_split_workspace_bytes(C.byref(p), Lk) > 0
+    assert dealt_parts(dev, (None, None), None, _lib.MASK_NONE, causal, 0.125)[0] == (dual or Lk >= 32 * 64)  # (short calls without tangents stay whole)
     _lib.set_split(False)
     try:
         one = _lib.backend().fwd(*dev, None, _lib.MASK_NONE, causal, 0.125)

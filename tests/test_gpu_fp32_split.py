@@ -1,12 +1,12 @@
 """fp32 calls whose blocks' tiles are dealt to several workgroups: against the same calls on whole blocks and the dense oracle."""
-import ctypes as C
-
 import numpy as np
 import pytest
 import torch
 
 from jvp_flash_attention_amd import _lib
 from oracle import dense
+
+from .test_gpu_split_merge import dealt_parts
 
 pytestmark = pytest.mark.gpu
 
@@ -35,6 +35,13 @@ SHAPES = [(1, 2, 900, 900, "causal"), (2, 3, 130, 2000, "none"), (1, 2, 2000, 13
           (3, 2, 1025, 1025, "padding"), (2, 2, 1200, 1104, "documents"), (1, 2, 1040, 1040, "bias"), (1, 2, 1033, 901, "bias"), (1, 1, 3300, 3300, "causal")]
 
 
+# ... of which stay whole, as too short to be worth another launch on 256 compute units: head dim, queries, keys, tangents
+WHOLE_FORWARDS = {(D, 2000, 130, dual) for D in (32, 64, 128) for dual in (False, True)} - {(128, 2000, 130, True)}
+WHOLE_FORWARDS |= {(32, 1400, 400, True), (32, 1400, 400, False), (64, 1400, 400, False)}
+WHOLE_BACKWARDS = {(32, *n, False) for n in ((900, 900), (1100, 2000), (1025, 1025), (1200, 1104), (1040, 1040), (1033, 901))}
+WHOLE_FORWARDS |= WHOLE_BACKWARDS
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Z,H,L,Lk,kind", SHAPES)
 @pytest.mark.parametrize("grads", ["plain", "both", "tangent", "six"])
@@ -50,12 +57,9 @@ def test_dealt_tiles_agree_with_whole_blocks(D, Z, H, L, Lk, kind, grads):
     if grads == "tangent":
         dev[6] = None
     dmask = None if mask is None else mask.cuda()
-    p = _lib.make_problem(dev[0], dmask, mk, causal, scale)
-    lib = _lib.load()
-    if D == 128 or grads != "plain" or max(L, Lk) >= 2000:  # (short first-order calls at small head dims stay whole)
-        six = int(grads == "six")
-        assert max(lib.jvpfa_fwd_split_workspace_bytes(C.byref(p), Lk), lib.jvpfa_bwd_split_workspace_bytes(C.byref(p), Lk, H, six)) > 0
     args = (dev[:6], dev[6:], dmask, mk, causal, scale, grads == "six")
+    what = (D, L, Lk, grads != "plain")
+    assert dealt_parts(*args) == (what not in WHOLE_FORWARDS, what not in WHOLE_BACKWARDS)
     got = _step(*args)
     _lib.set_split(False)
     try:

@@ -9,6 +9,19 @@ from jvp_flash_attention_amd import _lib
 pytestmark = pytest.mark.gpu
 
 
+def dealt_parts(dev, gs, mask, kind, causal, scale, six=False):
+    """Whether the forward and the backward of exactly this call go over blocks that several workgroups share."""
+    lib, (q, k, _, qt, _, _) = _lib.load(), dev
+    f, b = _lib.FwdArgs(), _lib.BwdArgs()
+    for a in (f, b):
+        a.struct_size, a.p = C.sizeof(type(a)), _lib.make_problem(q, mask, kind, causal, scale)
+        a.Hk, a.Lk = k.shape[1], k.shape[2]
+    f.qt = None if qt is None else qt.data_ptr()
+    b.gt = None if gs[1] is None else gs[1].data_ptr()
+    b.dqt = q.data_ptr() if six else None
+    return lib.jvpfa_fwd_split_needed(C.byref(f)) > 0, lib.jvpfa_bwd_split_needed(C.byref(b)) > 0
+
+
 def _step(dev, gs, mask, kind, causal, scale):
     be = _lib.backend()
     o, ot, M, mu = be.fwd(*dev, mask, kind, causal, scale)
@@ -45,9 +58,8 @@ def test_what_is_not_a_number_stays_where_it_is(dtype, D, dual, where, causal):
     if not dual:
         dev[3:6], dev[7] = [None] * 3, None
     kind, scale = _lib.MASK_NONE, D**-0.5
-    p = _lib.make_problem(dev[0], None, kind, causal, scale)
-    assert _lib.load().jvpfa_fwd_split_workspace_bytes(C.byref(p), L) > 0
     args = (dev[:6], dev[6:], None, kind, causal, scale)
+    assert dealt_parts(*args)[0]
     got = _step(*args)
     _lib.set_split(False)
     try:
@@ -78,8 +90,7 @@ def test_masked_shares_of_values_that_are_not_numbers(D):
     dev[2][1, 1, 600] = float("nan")
     dev[1][0, 1, 900] = float("nan")  # in a tile that no row visits
     args = (dev[:6], dev[6:], mask.cuda(), _lib.MASK_BOOL, False, D**-0.5)
-    p = _lib.make_problem(dev[0], args[2], _lib.MASK_BOOL, False, D**-0.5)
-    assert _lib.load().jvpfa_fwd_split_workspace_bytes(C.byref(p), L) > 0
+    assert dealt_parts(*args)[0]
     got = _step(*args)
     _lib.set_split(False)
     try:
