@@ -32,12 +32,12 @@ struct Problem {
   // of word hf being the entry of (query, key 64 * tile + 32 * hf + i); keys past Lk are zero bits.  For the forward and
   // dq kernels, whose lanes own a query.
   const uint32_t *bits_q;
-  // Forward: how the key tiles of query blocks are split over workgroups (Deal; 1 = no split), used when a launch would
-  // otherwise leave most compute units idle.  A share of a split block leaves fp32 partial results in `part`, which a merge
-  // kernel adds up.  Only the kernels for 16-bit element types, D = 64 or 128, without a mask.
+  // Forward: how the key tiles of query blocks are split over workgroups (Deal::most and Deal::step; 1 = no split), used when a
+  // launch would otherwise leave compute units idle.  A share of a split block leaves fp32 partial results in `part`, which a
+  // merge kernel adds up.  The kernels for 16-bit element types at D = 64 or 128 without a mask, and for fp32 at D <= 128.
   // In the backward: the query heads of a key/value head's group are dealt to `chunks` dk/dv workgroups (see
   // split.hpp), each of which leaves its share of the gradients in `part`; chunk_tiles = -1: `part` is there for the shares
-  // of blocks whose tiles are split (bwd_split_plan).
+  // of blocks whose tiles are split (bwd_deal).
   int chunks, chunk_tiles;
   float *part;
   // Dropout on the attention probabilities (0 in drop_thr: none).  Entry (z, h, query i, key j) is kept when

@@ -1,11 +1,12 @@
-// Small grids: when a launch has fewer workgroups than the GPU has compute units (one sequence of a few
-// thousand tokens, a handful of heads), the kernels for 16-bit element types without a mask (forward: D = 64 or 128,
-// backward: D <= 128) split the streamed tiles of every block of owned rows over several workgroups ("chunks").  Each writes
-// fp32 partial results to a workspace; the forward's merge kernel combines them with the online-softmax merge (every running
-// quantity is linear in p once the reference points m and c are made common), the backward's adds them up.  Where key/value heads
-// are few (grouped heads), the backward deals the query heads of each to several workgroups (bwd_kv_chunks).  And it runs its dk/dv and
-// dq workgroups in one launch where that leaves fewer units idle (launch_both).  The reference has nothing like it (one
-// program per 32 query rows, jvp_attention.py:2474).
+// Small grids: when a launch has fewer workgroups than the GPU has compute units (one sequence of a few thousand tokens, a
+// handful of heads), or causal ones of very different length, the streamed tiles of blocks of owned rows are dealt to several
+// workgroups ("shares", Deal).  Each leaves fp32 partial results in a workspace; the forward's merge kernel combines them with
+// the online-softmax merge (every running quantity is linear in p once the reference points m and c are made common), the
+// backward's adds them up.  The kernels that can: 16-bit element types without a mask (forward D = 64 or 128, backward D <= 128)
+// and fp32 at D <= 128 with any mask, all without dropout.  Non-causal blocks get as many workgroups each, causal ones by their length.
+// Where key/value heads are few (grouped heads), the backward deals the query heads of each to several workgroups (bwd_kv_chunks).
+// And it runs its dk/dv and dq workgroups in one launch where that leaves fewer units idle (launch_both).  The reference has
+// nothing like it (one program per 32 query rows, jvp_attention.py:2474).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -20,9 +21,9 @@
 
 namespace jvpfa {
 
-// make() of these sizes, from the last ones that this thread asked for: a plan is a function of sizes alone, a call asks for it twice (its
-// workspace and its launch), and making it takes 1 - 3 us.  As many as the attention shapes of a large model; looking through them takes
-// 0.02 us, where eight, in turn over nine shapes, were made anew on every call.
+// make() of these sizes, from the last ones that this thread asked for: a plan is a function of sizes alone, a call asks for it
+// twice (its workspace and its launch), and making it takes 1 - 3 us.  As many as the attention shapes of a large model; looking
+// through them takes 0.02 us, where eight, in turn over nine shapes, were made anew on every call.
 template <typename Plan, int N, typename Make> inline Plan remembered(const std::array<int, N> &sizes, Make make) {
   constexpr int SLOTS = 32;
   struct Entry {
@@ -73,9 +74,11 @@ struct DealCost {
   int places;      // workgroups that share a compute unit without taking longer
   double pair;     // of two workgroups in turn, see above
 };
-// A second launch and its workspace take 7 us on the host, and a step of forward and backward that takes the GPU less than some 110 us is
-// bound by the host: a split that adds a launch is for forwards and backwards that take at least this long, and saves at least so much.
-// (B1 H2 L300 D64 fp32, both outputs' gradients: 57 -> 47 us on the GPU, 112 -> 127 us a step.)
+// A second launch and its workspace take 7 us on the host, and an eager step of forward and backward that takes the GPU less than
+// some 110 us is bound by the host (B1 H2 L300 D64 fp32, both outputs' gradients, in shares: 57 -> 47 us on the GPU, 112 -> 127 us a
+// step).  So a split that adds a launch is for forwards and backwards that take at least this long by the account, and a forward
+// has to save what the launch costs; a backward of that length, which the host does not bound, has to be faster by its account
+// alone.  A caller without that host time (a captured graph, the C ABI) has the same plans: that backward stays at 57 us there.
 constexpr double SPLIT_LAUNCH_US = 7.0, SPLIT_FORWARD_US = 40.0, SPLIT_BACKWARD_US = 65.0;
 class DealTime {
  public:
@@ -131,15 +134,16 @@ inline int device_cus() {
 // Workspace of the forward: per chunk and query row 2 D accumulator values (O, T, not yet divided by l) and
 // four statistics (m, l, mu_acc, c).
 inline size_t fwd_part_floats(int chunks, long long rows, int D, bool dual) { return (size_t)chunks * rows * ((dual ? 2 : 1) * (size_t)D + 4); }
-// The kernels that can split: 16-bit element types, D = 64 or 128, no mask (the software-pipelined forward).  Tiles are 64
-// wide, blocks 128 rows.
+// The 16-bit kernels that can split: D = 64 or 128, no mask (the software-pipelined forward).  Tiles are 64 wide, blocks 128 rows.
 template <typename P> inline bool split_capable(const P &p) {
   return p.dtype != 2 && (p.D == 128 || p.D == 64) && p.mask_kind == 0 && !(p.dropout_p > 0.f);
 }
-// fp32 at D <= 128 (without dropout): a tile takes three to nine times as long as in 16 bits, so that a split is worth it for any grid that
-// leaves units idle, also by a second pass that is not full: 192 blocks in quarters are three passes of a quarter.  Dual / without
-// tangents, whole blocks -> this: D64 B1 H8 L512 51 -> 32 us, H2 L4096 causal 342 -> 82 / 153 -> 50, B2 H6 L777 with a bias 79 -> 48; D128 H8 L512
-// 187 -> 55 / 70 -> 33, H16 L1024 366 -> 209 / 135 -> 84, H40 L1000 733 -> 601 / 255 -> 216; D32 H12 L1024 causal 58 -> 29.
+// fp32 at D <= 128 (without dropout): a tile takes three to nine times as long as in 16 bits, so that a split is worth it for
+// any grid that leaves units idle, also by a second pass that is not full: 192 blocks in quarters are three passes of a quarter.
+// Whole blocks -> this, us, dual / without tangents:
+//   D64  B1 H8 L512 51 -> 33 / whole (24); H2 L4096 causal 342 -> 82 / 153 -> 49; B2 H6 L777 with a bias 79 -> 49 / whole (39)
+//   D128 B1 H8 L512 186 -> 55 / 70 -> 33; H16 L1024 366 -> 208 / 135 -> 83; H40 L1000 732 -> 599 / 254 -> 214
+//   D32  B1 H12 L1024 causal 58 -> 29 / whole (33)
 template <typename P> inline SplitPlan fwd_split_plan_f32(const P &p, int Lk, bool dual, int cus) {
   SplitPlan best = {1, 0};
   const int nblk = (p.L + 127) / 128;
@@ -182,20 +186,20 @@ template <typename P> inline SplitPlan fwd_split_plan_16(const P &p, int Lk, boo
   if (p.causal && even.chunks > 1) even.chunk_tiles = (ntiles + even.chunks - 1) / even.chunks;
   if (!p.causal || blocks >= cus || ntiles < 12) return even;
   // Causal: shares of one length for all blocks (Deal), where the account of DealTime says that it is worth a twentieth; fewer
-  // blocks than there are units, whose longest ones alone set the time otherwise.  (Some launches of up to half as many again would gain as
-  // well, 1.1 - 1.3 times; there every block is one workgroup's, so that the rows of a causal call do not depend on its length in any bit.)
-  // The costs fit what was measured of shares of 1/2 ... 1/8.  Causal, bf16, B1, dual forward / without tangents, before -> this: D128 H8
-  // L2048 57 -> 49 / 34 -> 29 us, H12 L2048 81 -> 64 / 42 -> 34, H6 L4096 148 -> 100 / 77 -> 51, H2 L8192
-  // 162 -> 125 / 85 -> 64; D64 H12 L1500 43 -> 31, H6 L4096 102 -> 64 / 61 -> 39, H2 L8192 111 -> 80 / 66 -> 47, H1 L16384 208 -> 130 /
-  // 121 -> 73; none of 60 shapes slower.
+  // blocks than there are units, whose longest ones alone set the time otherwise.  From as many blocks as units on every block
+  // is one workgroup's (some launches of up to half as many again would gain as well, 1.1 - 1.3 times).
+  // The costs fit what was measured of shares of 1/2 ... 1/8.  Causal, bf16, B1, us, before -> this, dual / without tangents:
+  //   D128 H8 L2048 56 -> 49 / 34 -> 29; H12 L2048 80 -> 65 / whole (42); H6 L4096 146 -> 99 / 77 -> 50; H2 L8192 159 -> 123 / 84 -> 64
+  //   D64  H12 L1500 43 -> 32 / whole (26); H6 L4096 103 -> 65 / 62 -> 38; H2 L8192 111 -> 80 / 66 -> 49; H1 L16384 207 -> 129 / 121 -> 67
+  // Slower than equal shares of every block: a few of one to three heads, by 2 - 5 % and less than 1 us (D64 H1 L3128 19.9 -> 20.8).
   const bool wide = p.D == 128;
   const DealCost cost = {wide ? (dual ? 2.45 : 1.2) : (dual ? 1.6 : 0.85), wide && dual ? 6.0 : 5.0, 7.0, 11.0 * p.D / 128 * (dual ? 1.0 : 0.5), 0.25, 1, 1.0};
   const int nblk = (p.L + 127) / 128;
   auto time = [&](int most, int step) {
-    // The merge reads a row's shares one after another.  Counted where three or more equal shares are the alternative and blocks are short:
-    // H3 L1990 D64 without tangents in 4, 5, 8 shares 19.0, 19.2, 20.8 us; H6 L1111 D128 in 3, 5 shares 20.9, 22.6 (equal ones 21.5).  Over a hundred
-    // such launches 2.3 % less, 5 % more at worst.  In others the account is too coarse for it (H1 L16384 D64, two equal shares: 67.5 us in 6, but
-    // 84 in the 3 that it would pick; H1 L8483 D64, three: 32.6 us in 7, 34.9 in 6).
+    // The merge reads a row's shares one after another.  Counted where three or more equal shares are the alternative and blocks
+    // are short: H3 L1990 D64 without tangents in 4, 5, 8 shares 19.0, 19.2, 20.8 us; H6 L1111 D128 in 3, 5 shares 20.9, 22.6
+    // (equal ones 21.5); over a hundred such launches 2.3 % less, 5 % more at worst.  In others the account is too coarse for it
+    // (H1 L16384 D64, two equal shares: 67.5 us in 6, but 84 in the 3 that it would pick; H1 L8483, three: 32.6 in 7, 34.9 in 6).
     DealCost with_merge = cost;
     if (even.chunks > 2 && ntiles <= 64) with_merge.merge = 3.5 + 1.0 * most;
     DealTime t(cus, with_merge);
@@ -261,24 +265,25 @@ template <typename P> inline size_t bwd_part_floats(const P &p, int Lk, int Hk, 
 // Backward of small grids (16-bit element types, D <= 128, no mask, no dropout, one query head per key/value head, not six
 // gradients): the tiles that a block streams are dealt to several workgroups, dq's and dk/dv's in one launch, which leave fp32
 // shares that bwd_split_merge_kernel adds up.
-//   * As many workgroups as there are compute units; causal, whose blocks have half the tiles on average, up to three a block
-//     and three a unit where that leaves 10 tiles to a share (with fewer the empty and the short ones cost more than they bring:
-//     H16 L1024 D128 60 -> 72 us, H6 L1024 42 -> 48; six for three at H2 L4096 98 -> 119).  Where a unit holds one of them (D = 128;
-//     D = 64 with tangents) and both roles would be cut so, only if the blocks unsplit fit the units (D = 64: and an eighth), and at D = 128 two
-//     a block only if they fit three quarters.
-//     Causal, unsplit / split, at 192, 240 - 256, 288 - 320, 384 blocks of both roles: D128 dual 1.10, 0.93 (two), 1.17 (three), 0.83 - 0.94, 0.76 - 0.85,
-//     plain 0.99, 0.86, 1.00, 0.75 - 0.82, 0.67 - 0.79; D64 dual 1.21 - 1.46, 1.03 - 1.50, 0.85 - 1.02, 0.76 - 0.87, plain 1.27, 1.29, 1.27, 1.03 - 1.23;
-//     D32 1.44, 1.41, 1.35, 0.98 - 1.08.
-//   * No share under 3 tiles at D = 128, where a tile takes 4 us, 4 at D = 64, 6 at D = 32; and without tangents none that saves a
-//     block fewer than 7 tiles of 2 us at D = 128 (H8 L700 28 -> 31 us), the launch fewer than 6 of 1 us at D = 64 (H16 L512 19 -> 22 us): the
-//     merge takes 5 - 10 us.
+//   * As many workgroups as there are compute units; causal, whose blocks have half the tiles on average, up to three a block and
+//     three a unit where that leaves 10 tiles to a share (with fewer the empty and the short ones cost more than they bring: H16
+//     L1024 D128 60 -> 72 us, H6 L1024 42 -> 48; six for three at H2 L4096 98 -> 119).  Where a unit holds one of them (D = 128;
+//     D = 64 with tangents) and both roles would be cut so, only if the blocks unsplit fit the units (D = 64: and an eighth), and
+//     at D = 128 two a block only if they fit three quarters. Causal, unsplit / split, at 192, 240 - 256, 288 - 320, 384 blocks
+//     of both roles: D128 dual 1.10, 0.93 (two), 1.17 (three), 0.83 - 0.94, 0.76 - 0.85, plain 0.99, 0.86, 1.00, 0.75 - 0.82,
+//     0.67 - 0.79; D64 dual 1.21 - 1.46, 1.03 - 1.50, 0.85 - 1.02, 0.76 - 0.87, plain 1.27, 1.29, 1.27, 1.03 - 1.23; D32 1.44,
+//     1.41, 1.35, 0.98 - 1.08.
+//   * No share under 3 tiles at D = 128, where a tile takes 4 us, 4 at D = 64, 6 at D = 32; and without tangents none that saves
+//     a block fewer than 7 tiles of 2 us at D = 128 (H8 L700 28 -> 31 us), the launch fewer than 6 of 1 us at D = 64 (H16 L512 19
+//     -> 22 us): the merge takes 5 - 10 us.
 //   * At D = 128 shares of up to 8 tiles only where they shorten the longest workgroup of the launch (a dk/dv tile takes 1.25 of
-//     a dq tile) by 3 tiles, and then, as the merge grows with what it reads, only up to a number of them: unsplit / split, dual, at 2, 8, 12, 16 heads
-//     and 512 rows 1.22, 1.06, 1.05, 0.94, causal 1.26, 1.16, 1.14, 1.09; 384 rows 1.15, 0.98, 1.01, 0.94, causal 1.16, 1.06, 1.00, 1.00.
-// Measured, bf16 B1, backward, unsplit -> split, dual / plain: D128 H1 L1024 65 -> 32 / 35 -> 23 us, H4 L1024 65 -> 38 / 36 -> 28,
-// H2 L2048 120 -> 53 / 62 -> 35, H4 L2048 121 -> 85 / 62 -> 49, H2 L4096 231 -> 147 / 116 -> 77, causal H2 L4096 228 -> 98 / 115 -> 56, H4 L4096 237 -> 156 / 117 -> 96;
-// D64 H4 L1024 49 -> 28 / 31 -> 23, H2 L2048 90 -> 38 / 55 -> 29, causal H4 L4096 173 -> 116; D32 H4 L1024 34 -> 25 / 24 -> 19,
-// H4 L2048 63 -> 41 / 44 -> 31, causal H4 L4096 121 -> 68.
+//     a dq tile) by 3 tiles, and then, as the merge grows with what it reads, only up to a number of them: unsplit / split, dual,
+//     at 2, 8, 12, 16 heads and 512 rows 1.22, 1.06, 1.05, 0.94, causal 1.26, 1.16, 1.14, 1.09; 384 rows 1.15, 0.98, 1.01, 0.94,
+//     causal 1.16, 1.06, 1.00, 1.00.
+// Measured, bf16 B1, backward, unsplit -> split, dual / plain: D128 H1 L1024 65 -> 32 / 35 -> 23 us, H4 L1024 65 -> 38 / 36 ->
+// 28, H2 L2048 120 -> 53 / 62 -> 35, H4 L2048 121 -> 85 / 62 -> 49, H2 L4096 231 -> 147 / 116 -> 77, causal H2 L4096 228 -> 98 /
+// 115 -> 56, H4 L4096 237 -> 156 / 117 -> 96; D64 H4 L1024 49 -> 28 / 31 -> 23, H2 L2048 90 -> 38 / 55 -> 29, causal H4 L4096 173
+// -> 116; D32 H4 L1024 34 -> 25 / 24 -> 19, H4 L2048 63 -> 41 / 44 -> 31, causal H4 L4096 121 -> 68.
 struct BwdSplitPlan {
   int chunks_q, tiles_q, chunks_k, tiles_k;
   bool any() const { return chunks_q > 1 || chunks_k > 1; }
@@ -319,10 +324,12 @@ inline BwdSplitPlan bwd_split_plan(int D, int Z, int H, int L, int Lk, bool caus
 }
 // The deal of either role's blocks that a launch goes by.  Causal, from 12 tiles on, where the account of DealTime says that it is
 // shorter than with whole blocks: shares of one length for all blocks of both roles, so that the long ones get most of them.
-// Causal, bf16, B1, backward with tangents / without, before -> this: D128 H12 L1024 68 -> 57 us, H16 L1024 69 -> 65, H9 L2048 127 -> 108 / 64 -> 60,
-// H7 L2500 154 -> 122 / 78 -> 67, H2 L12000 719 -> 588 / 331 -> 266; D64 H16 L1024 50 -> 43 / 31 -> 29, H6 L4096 173 -> 140 / 83 -> 69, H1 L30000 1227 ->
-// 1101 / 713 -> 458; D32 H12 L1024 35 -> 24 / 24 -> 20, H6 L4096 115 -> 88 / 50 -> 44, H1 L8192 91 -> 60 / 63 -> 36; of 250 shapes the slowest
-// 6 % slower (D64 H3 L5000 without tangents 58 -> 62).
+// Causal, bf16, B1, us, before -> this, with tangents / without:
+//   D128 H9 L2048 129 -> 109 / whole (65); H7 L2500 156 -> 124 / 78 -> 67; H2 L12000 717 -> 598 / 334 -> 265
+//   D64  H6 L4096 174 -> 142 / 85 -> 70; H1 L30000 1218 -> 1109 / 712 -> 458; H3 L5000 136 -> 122 / 58 -> 60
+//   D32  H6 L4096 118 -> 86 / 50 -> 44; H1 L8192 91 -> 60 / 63 -> 36
+// H12 and H16 L1024 at any D stay whole, though shares would take D128 68 -> 57 and 69 -> 65, D64 50 -> 43 / 31 -> 29, D32 35 -> 24 / 24 -> 20:
+// they are shorter than SPLIT_BACKWARD_US.  Slower: D64 H3 L4700 - L5100 without tangents, by 1 - 3 %.
 // Otherwise shares of the length that bwd_split_plan says.
 struct BwdDeal {
   Deal q, k;
@@ -336,9 +343,10 @@ inline BwdDeal make_bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bo
   // (in the account with shares of whole blocks, two tiles: what its pick was measured with)
   auto rounded = [](const BwdDeal &d) { return BwdDeal{{d.q.most, (d.q.step + 1) / 2 * 2, d.q.first, d.q.last}, {d.k.most, (d.k.step + 1) / 2 * 2, d.k.first, d.k.last}}; };
   const long long heads = (long long)Z * H;
-  const int nq = (std::min(bq * 128, Lk) + 63) / 64, nk = (L + 63) / 64, live = std::min(bk, bq);  // tiles of the longest blocks; key blocks that a query sees
+  // tiles of the longest blocks; key blocks that a query sees
+  const int nq = (std::min(bq * 128, Lk) + 63) / 64, nk = (L + 63) / 64, live = std::min(bk, bq);
   const BwdDeal alike = {{even.chunks_q, step_of(even.chunks_q, even.tiles_q), 0, bq}, {even.chunks_k, step_of(even.chunks_k, even.tiles_k), bq - live, bq}};
-  if ( cus <= 0 || std::max(nq, nk) < 12 || heads * (bq + bk) >= 2 * cus) return alike;
+  if (cus <= 0 || std::max(nq, nk) < 12 || heads * (bq + bk) >= 2 * cus) return alike;
   const DealCost cost = D == 128 ? (dual ? DealCost{3.0, 2.9, 6.4, 9.9, 0.34, 1, 1.0} : DealCost{1.5, 3.9, 7.0, 6.1, 0.14, 1, 1.0})
                         : D == 64 ? (dual ? DealCost{2.0, 6.0, 4.2, 3.4, 0.2, 1, 1.0} : DealCost{1.2, 9.0, 3.6, 2.3, 0.4, 2, 0.7})
                                   : (dual ? DealCost{1.5, 5.5, 5.0, 2.1, 0.57, 2, 0.5} : DealCost{1.0, 4.5, 3.0, 1.8, 0.15, 2, 0.7});
@@ -368,9 +376,11 @@ inline BwdDeal make_bwd_deal(int D, int Z, int H, int L, int Lk, bool causal, bo
   return best.any() ? best : alike;
 }
 // ... and in fp32 at D <= 128 (without dropout, one query head per key/value head; any mask, six gradients as well), by the same
-// reasons as the forward.  With tangents / without, whole blocks -> this: D64 B1 H8 L512 83 -> 41 us, H12 L1024 causal 160 -> 108 / 78 -> 53, B3 H4 L640
-// padded 115 -> 70 / 65 -> 44; D128 H8 L512 337 -> 113 / 133 -> 56, H12 L1024 causal 673 -> 336 / 256 -> 149; D32 H2 L4096 causal 362 -> 142 /
-// 203 -> 59; six gradients D64 H4 L900 208 -> 93.
+// reasons as the forward.  Whole blocks -> this, us, with tangents / without:
+//   D64  B1 H8 L512 82 -> 41 / whole (43); H12 L1024 causal 159 -> 104 / 78 -> 53; B3 H4 L640 padded 115 -> 72 / whole (65);
+//        H2 L4096 causal 584 -> 249 / 278 -> 118; six gradients H4 L900 208 -> 93
+//   D128 B1 H8 L512 336 -> 113 / 133 -> 55; H12 L1024 causal 670 -> 334 / 255 -> 146
+//   D32  B1 H2 L4096 causal 361 -> 145 / 204 -> 63
 inline BwdDeal make_bwd_deal_f32(int D, int Z, int H, int L, int Lk, bool causal, bool dual, long long cus = device_cus()) {
   const int bq = (L + 127) / 128, bk = (Lk + 127) / 128, live = causal ? std::min(bk, bq) : bk;
   const long long heads = (long long)Z * H;
@@ -422,29 +432,30 @@ template <typename P> inline size_t bwd_split_floats(const P &p, int Lk, const B
 
 // Whether dk/dv and dq go into one launch (bwd2_both_kernel): it has one end with idle compute units instead of two, and where a
 // kernel has to take both roles' registers fewer of its workgroups share a unit.  So: up to a number of blocks (in units of
-// compute units) that depends on how many do.  mask: as the kernels read it.  twin: the launch has a capped
-// kernel (both_two_wgs says which of the two runs it).
-// D = 128 (one workgroup a unit either way, but for the dq kernel without tangents): causal and masked launches up to 2.5; others
-// where the launches would round up to more passes over the units than the one does, 0.6 of a pass for its end.
-// Measured, bf16, backward, two launches -> one, 288 / 544 / 704 / 1024 - 1152 blocks (dual unless said): D128 269 -> 205, 721 ->
-// 607, 490 -> 492, 1236 -> 1135 us, causal 139 -> 111, 323 -> 316, 295 -> 290; plain 123 -> 100, 332 -> 285, 233 -> 237;
-// D64 (2wg) causal 1024 blocks 314 -> 300, 1152 without a mask 731 -> 677, 1536 615 -> 602; D64 plain 69 -> 54, 164 -> 147,
-// 121 -> 118, 260 -> 245 us, 2048 blocks 471 -> 479; D32 88 -> 81, 253 -> 196, 171 -> 155, 462 -> 415, 2048 blocks 658 -> 644.
-// The lines below those, each where the quotient two / one crosses 1 (L1000, 8 blocks a head, 256 units; at 256 / 288 / 384 / 512 /
-// 640 / 1024 blocks).  Packed masks, a dense one: D32 dual 0.99 / 0.97 / 0.90 / 0.77 / 0.88 / 0.74, D64 plain 1.04 / 0.94 / 0.88 / 0.75 /
-// 0.88 / 0.72 (the separate kernels keep three workgroups on a unit there).  D64 dual on the bytes of a key padding 1.00 / 1.30 / 1.16 /
-// 0.95 / 1.08 / 0.97: past two units' worth the two launches begin a second, mostly empty pass.  Dropout: D32 dual 1.02 / 1.03 / 0.92 /
-// 0.76, causal 1.56 / 1.32 / 1.04 / 0.87; D64 plain 1.03 / 0.98 / 0.87 / 0.72, causal 1.50 / 1.30 / 1.03 / 0.86 (and
-// the tangent launch of six gradients there, which at D32 gains up to 2.5 units' worth).  Six gradients: D32 1.02 /
-// 1.01 / 0.91 / 0.81 / 0.92, causal 1.50 / 1.29 / 1.05 / 0.95, packed mask 1.36 - 1.50 ... 1.07; D64 1.00 / 1.23 / 1.11 / 0.95 / 1.08, causal
-// and packed 1.42 ... 1.01.  Grouped heads, D64 dual: 1.01 / 1.06 / 1.00 / 0.87 / 0.96 / 0.86, causal 1.40 / 1.32 / 1.09 / 0.99 / 0.88; plain
-// (448, 512, 640, 1024, 1536) 0.94 - 0.99, 1.07, 1.10, 1.05, 1.07, causal (1024, 1536) 1.26, 1.13; gradients of O' alone, dual, at 448 / 512 / 640 1.02 / 1.04 / 1.18, causal 1.00 / 1.00 / 1.08.
-// Documents in a packed mask differ with what is drawn: D32 dual 1.05 - 1.28 at 280 - 336 blocks, 0.9 - 1.4 at 384, 0.75 - 1.0 past that; D64
-// plain 0.9 - 1.15 at 280 - 336.  Where they gain what a dense mask loses they have the line.  Padding by batch entry as bytes, D64 dual, at 392 1.12 - 1.16,
-// with 512 blocks of one role and 64 - 96 of the other 1.10 - 1.27.
-// D = 128 plain, masked, 448 / 512 blocks: padding 0.97 - 1.06 / 0.98, dense 0.94 / 0.96, documents 1.02 - 1.10 / 1.02 - 1.08.
-// D = 256, whose blocks with tangents have 64 rows, by the same rule: dual 272 / 384 / 448 / 512 / 640 / 896 / 1024 blocks 1.32 / 1.21 / 0.98 / 1.01 / 1.14 / 1.13 /
-// 1.01, causal 1.39 / 1.04 / 1.01 / 1.00 / 1.08 / 1.03 / 1.03, masked 1.34 - 1.45 / 1.22 - 1.26 / 1.00 - 1.20 / 1.01 - 1.09 / 1.13 - 1.16; plain alike.
+// compute units) that depends on how many do.  mask: as the kernels read it.  twin: the launch has a capped kernel (both_two_wgs
+// says which of the two runs it). D = 128 (one workgroup a unit either way, but for the dq kernel without tangents): causal and
+// masked launches up to 2.5; others where the launches would round up to more passes over the units than the one does, 0.6 of a
+// pass for its end. Measured, bf16, backward, two launches -> one, 288 / 544 / 704 / 1024 - 1152 blocks (dual unless said): D128
+// 269 -> 205, 721 -> 607, 490 -> 492, 1236 -> 1135 us, causal 139 -> 111, 323 -> 316, 295 -> 290; plain 123 -> 100, 332 -> 285,
+// 233 -> 237; D64 (2wg) causal 1024 blocks 314 -> 300, 1152 without a mask 731 -> 677, 1536 615 -> 602; D64 plain 69 -> 54, 164
+// -> 147, 121 -> 118, 260 -> 245 us, 2048 blocks 471 -> 479; D32 88 -> 81, 253 -> 196, 171 -> 155, 462 -> 415, 2048 blocks 658 ->
+// 644. The lines below those, each where the quotient two / one crosses 1 (L1000, 8 blocks a head, 256 units; at 256 / 288 / 384
+// / 512 / 640 / 1024 blocks).  Packed masks, a dense one: D32 dual 0.99 / 0.97 / 0.90 / 0.77 / 0.88 / 0.74, D64 plain 1.04 / 0.94
+// / 0.88 / 0.75 / 0.88 / 0.72 (the separate kernels keep three workgroups on a unit there).  D64 dual on the bytes of a key
+// padding 1.00 / 1.30 / 1.16 / 0.95 / 1.08 / 0.97: past two units' worth the two launches begin a second, mostly empty pass.
+// Dropout: D32 dual 1.02 / 1.03 / 0.92 / 0.76, causal 1.56 / 1.32 / 1.04 / 0.87; D64 plain 1.03 / 0.98 / 0.87 / 0.72, causal 1.50
+// / 1.30 / 1.03 / 0.86 (and the tangent launch of six gradients there, which at D32 gains up to 2.5 units' worth).  Six
+// gradients: D32 1.02 / 1.01 / 0.91 / 0.81 / 0.92, causal 1.50 / 1.29 / 1.05 / 0.95, packed mask 1.36 - 1.50 ... 1.07; D64 1.00 /
+// 1.23 / 1.11 / 0.95 / 1.08, causal and packed 1.42 ... 1.01.  Grouped heads, D64 dual: 1.01 / 1.06 / 1.00 / 0.87 / 0.96 / 0.86,
+// causal 1.40 / 1.32 / 1.09 / 0.99 / 0.88; plain (448, 512, 640, 1024, 1536) 0.94 - 0.99, 1.07, 1.10, 1.05, 1.07, causal (1024,
+// 1536) 1.26, 1.13; gradients of O' alone, dual, at 448 / 512 / 640 1.02 / 1.04 / 1.18, causal 1.00 / 1.00 / 1.08. Documents in a
+// packed mask differ with what is drawn: D32 dual 1.05 - 1.28 at 280 - 336 blocks, 0.9 - 1.4 at 384, 0.75 - 1.0 past that; D64
+// plain 0.9 - 1.15 at 280 - 336.  Where they gain what a dense mask loses they have the line.  Padding by batch entry as bytes,
+// D64 dual, at 392 1.12 - 1.16, with 512 blocks of one role and 64 - 96 of the other 1.10 - 1.27. D = 128 plain, masked, 448 /
+// 512 blocks: padding 0.97 - 1.06 / 0.98, dense 0.94 / 0.96, documents 1.02 - 1.10 / 1.02 - 1.08. D = 256, whose blocks with
+// tangents have 64 rows, by the same rule: dual 272 / 384 / 448 / 512 / 640 / 896 / 1024 blocks 1.32 / 1.21 / 0.98 / 1.01 / 1.14
+// / 1.13 / 1.01, causal 1.39 / 1.04 / 1.01 / 1.00 / 1.08 / 1.03 / 1.03, masked 1.34 - 1.45 / 1.22 - 1.26 / 1.00 - 1.20 / 1.01 -
+// 1.09 / 1.13 - 1.16; plain alike.
 template <int D, int MODE>
 inline bool launch_both(long long blocks, long long kv_blocks, bool causal, int mask, bool drop, bool six, bool grouped, bool twin,
                         bool no_go = false, long long cus = device_cus()) {
@@ -469,11 +480,11 @@ inline bool launch_both(long long blocks, long long kv_blocks, bool causal, int 
   const double apart = (double)((blocks + cus - 1) / cus + (kv_blocks + cus - 1) / cus);
   return apart > (MODE == BWD_DUAL ? 1.04 : 1.08) * ((double)(blocks + kv_blocks) / cus + 0.6);
 }
-// Whether bwd2_both_kernel_2wg runs a launch of D = 64, dual: two of its workgroups take longer for a pair of blocks than one uncapped for one, so it is for launches whose work, dealt
-// evenly, keeps a unit busy for longer than its longest block takes (tiles, a dk/dv tile 1.25 of a dq tile).  Uncapped / capped with that
-// quotient in brackets: causal, 140 - 250 blocks of either role, L777 - 2048 0.90 - 0.97 (0.59 - 0.95), L512 0.94 (0.70 - 0.84) and 1.04 (0.98), L340 - 640
-// 1.04 - 1.13 (1.01 - 1.13); no mask 0.96 (0.90), 1.15 - 1.25 (0.98 on), 1500 queries over 700 keys 0.93 (0.81), but
-// 512 over 1000 - 2000 1.15 - 1.3.
+// Whether bwd2_both_kernel_2wg runs a launch of D = 64, dual: two of its workgroups take longer for a pair of blocks than one
+// uncapped for one, so it is for launches whose work, dealt evenly, keeps a unit busy for longer than its longest block takes
+// (tiles, a dk/dv tile 1.25 of a dq tile).  Uncapped / capped with that quotient in brackets: causal, 140 - 250 blocks of either
+// role, L777 - 2048 0.90 - 0.97 (0.59 - 0.95), L512 0.94 (0.70 - 0.84) and 1.04 (0.98), L340 - 640 1.04 - 1.13 (1.01 - 1.13); no
+// mask 0.96 (0.90), 1.15 - 1.25 (0.98 on), 1500 queries over 700 keys 0.93 (0.81), but 512 over 1000 - 2000 1.15 - 1.3.
 inline bool both_two_wgs(int L, int Lk, long long heads, bool causal, long long cus = device_cus()) {
   const double bq = (L + 127) / 128, bk = (Lk + 127) / 128, nq = (L + 63) / 64, nk = (Lk + 63) / 64;
   double of_q = bq * nk, of_k = bk * nq, longest = nk;  // tiles of all query blocks, of all key blocks, of the longest query block
@@ -486,13 +497,14 @@ inline bool both_two_wgs(int L, int Lk, long long heads, bool causal, long long 
   if (longest > 1.25 * nq) return heads * (bq + bk) > cus;  // long query blocks, which come last, must not wait for the key blocks
   return heads * (of_q + 1.25 * of_k) > 0.97 * cus * std::max(longest, 1.25 * nq);
 }
-// ... and in fp32 (one workgroup a compute unit but at D = 32 without tangents, and the separate dq kernel without tangents at D = 64).
-// uneven: causal, or a boolean mask, which may leave blocks little to do.  Measured as above, two / one at 136 - 160, 168 - 192, 224 -
-// 256, 416, 448 - 512, 640 blocks (L1000): no mask, D64 dual 0.99 - 1.01, 0.90 - 0.94, 1.01, 1.00, 0.98 - 1.01, 1.10, plain 1.13 - 1.19, 0.96, 1.02, 1.03,
-// 0.96 - 0.99, 1.09; D128 1.15, 0.99, 1.01, 1.08, 1.01, 1.16; a bias D64 dual 1.05, 0.93, 1.00, 1.01, 0.98 - 1.01, 1.10, plain at 448 0.96.  Padding by
-// batch entry D64 1.10 - 1.28, 0.97 - 1.09, 1.02, 1.07, 0.98 - 1.02, 1.10; documents 1.14 - 1.23, 1.34 - 1.41, 1.02 - 1.29, 1.13, 1.01 - 1.14, 1.08; a dense
-// mask as a bias; causal 1.5 at 192, 1.02 at 640.  D32 plain, whatever the mask, 1.00 - 1.57, 1.01 - 1.04 at 2048 blocks (and the tangent
-// launch of six gradients alike).
+// ... and in fp32 (one workgroup a compute unit but at D = 32 without tangents, and the separate dq kernel without tangents at D
+// = 64). uneven: causal, or a boolean mask, which may leave blocks little to do.  Measured as above, two / one at 136 - 160, 168
+// - 192, 224 - 256, 416, 448 - 512, 640 blocks (L1000): no mask, D64 dual 0.99 - 1.01, 0.90 - 0.94, 1.01, 1.00, 0.98 - 1.01,
+// 1.10, plain 1.13 - 1.19, 0.96, 1.02, 1.03, 0.96 - 0.99, 1.09; D128 1.15, 0.99, 1.01, 1.08, 1.01, 1.16; a bias D64 dual 1.05,
+// 0.93, 1.00, 1.01, 0.98 - 1.01, 1.10, plain at 448 0.96.  Padding by batch entry D64 1.10 - 1.28, 0.97 - 1.09, 1.02, 1.07, 0.98
+// - 1.02, 1.10; documents 1.14 - 1.23, 1.34 - 1.41, 1.02 - 1.29, 1.13, 1.01 - 1.14, 1.08; a dense mask as a bias; causal 1.5 at
+// 192, 1.02 at 640.  D32 plain, whatever the mask, 1.00 - 1.57, 1.01 - 1.04 at 2048 blocks (and the tangent launch of six
+// gradients alike).
 template <int D, int MODE>
 inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven, long long cus = device_cus()) {
   if (cus <= 0) return false;  // the device cannot be asked: two launches
@@ -504,15 +516,14 @@ inline bool launch_both_f32(long long blocks, long long kv_blocks, bool uneven, 
   return apart > together + 0.7;
 }
 
-// ---- merge kernels -------------------------------------------------------------------------------
-// Forward.  part = [chunk][row][O, with tangents T][D] accumulators, then [chunk][row][4] statistics.  One thread per (row, 8
-// columns), a grid of (rows of a head, heads).  With m the largest reference point of the row's chunks and w_c = 2^(m_c - m):
-//   l = sum w_c l_c,  O = sum w_c O_c,  and, with c the reference of S' of the heaviest chunk,
-//   T = sum w_c (T_c + (c_c - c) O_c),  mu_acc = sum w_c (mu_c + (c_c - c) l_c);
-// then the epilogue of the forward kernels: O / l, O' = T / l - (mu_acc / l) O, M = m + log2 l, mu = mu_acc / l + c.
-// A share that visited nothing says so by l = -0 (a sum is never that) and is left out.  All others are added up, however small their weight: that of a
-// share whose scores are all NaN, which no reference point is taken from, or -inf is 0, and 0 times what it holds is what one
-// workgroup's rescaling makes of it.  So the outputs that are not numbers are those of whole blocks.
+// ---- merge kernels ------------------------------------------------------------------------------- Forward.  part =
+// [chunk][row][O, with tangents T][D] accumulators, then [chunk][row][4] statistics.  One thread per (row, 8 columns), a grid of
+// (rows of a head, heads).  With m the largest reference point of the row's chunks and w_c = 2^(m_c - m): l = sum w_c l_c,  O =
+// sum w_c O_c,  and, with c the reference of S' of the heaviest chunk, T = sum w_c (T_c + (c_c - c) O_c),  mu_acc = sum w_c (mu_c
+// + (c_c - c) l_c); then the epilogue of the forward kernels: O / l, O' = T / l - (mu_acc / l) O, M = m + log2 l, mu = mu_acc / l
+// + c. A share that visited nothing says so by l = -0 (a sum is never that) and is left out.  All others are added up, however
+// small their weight: that of a share whose scores are all NaN, which no reference point is taken from, or -inf is 0, and 0 times
+// what it holds is what one workgroup's rescaling makes of it.  So the outputs that are not numbers are those of whole blocks.
 template <typename T, int D, bool DUAL>
 __global__ __launch_bounds__(256) void fwd_merge_kernel(const Problem pr, T *o, T *ot, float *M, float *mu) {
   constexpr int LPR = D / 8, RPB = 256 / LPR, ROW = DUAL ? 2 * D : D;
@@ -583,8 +594,9 @@ __global__ __launch_bounds__(256) void bwd_kv_merge_kernel(const float *part, in
   store8<T>((t == 0 ? g0 : t == 1 ? g1 : t == 2 ? g2 : g3) + i, sum);
 }
 
-// ---- the merge of a launch whose blocks are dealt to several workgroups: their partial results added up, in fp32 and in the order of the tiles: one thread per 8 elements of dq, dk, dv (blockIdx.z 0, 1, 2)
-// of head blockIdx.y (tangent: dq', dk', dv').  Blocks that one workgroup did are complete.  Bound by memory: shares * 4 + sizeof(T) bytes an element.
+// Backward whose blocks' tiles are dealt to several workgroups: their partial results added up, in fp32 and in the order of the
+// tiles: one thread per 8 elements of dq, dk, dv (blockIdx.z 0, 1, 2) of head blockIdx.y (tangent: dq', dk', dv').  Blocks that one
+// workgroup did are complete.  Bound by memory: shares * 4 + sizeof(T) bytes an element.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void bwd_split_merge_kernel(const BwdParams p, const BwdSplit sp, const int tangent) {
   const Problem &pr = p.pr;

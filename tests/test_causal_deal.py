@@ -86,6 +86,33 @@ def test_no_more_shares_than_the_merge_is_worth(tmp_path):
     assert [(x, y) for x, y in zip(FORWARDS, run(tmp_path, text)) if x[-1] != y] == []
 
 
+# calls that comments quote a time for, in shares or whole, on 256 compute units: direction, type (2: fp32), D, tangents, batch, heads, rows, causal, dealt
+QUOTED = [
+    *((0, "fwd", 128, d, 1, h, n, 1, x) for h, n, x2 in ((8, 2048, (1, 1)), (12, 2048, (0, 1)), (6, 4096, (1, 1)), (2, 8192, (1, 1))) for d, x in enumerate(x2)),
+    *((0, "fwd", 64, d, 1, h, n, 1, x) for h, n, x2 in ((12, 1500, (0, 1)), (6, 4096, (1, 1)), (2, 8192, (1, 1)), (1, 16384, (1, 1))) for d, x in enumerate(x2)),
+    *((0, "bwd", 128, d, 1, h, n, 1, x) for h, n, x2 in ((12, 1024, (0, 0)), (16, 1024, (0, 0)), (9, 2048, (0, 1)), (7, 2500, (1, 1)), (2, 12000, (1, 1))) for d, x in enumerate(x2)),
+    *((0, "bwd", 64, d, 1, h, n, 1, x) for h, n, x2 in ((16, 1024, (0, 0)), (6, 4096, (1, 1)), (1, 30000, (1, 1)), (3, 5000, (1, 1))) for d, x in enumerate(x2)),
+    *((0, "bwd", 32, d, 1, h, n, 1, x) for h, n, x2 in ((12, 1024, (0, 0)), (6, 4096, (1, 1)), (1, 8192, (1, 1))) for d, x in enumerate(x2)),
+    *((2, "fwd", D, d, z, h, n, c, x) for D, z, h, n, c, x2 in ((64, 1, 8, 512, 0, (0, 1)), (64, 1, 2, 4096, 1, (1, 1)), (64, 2, 6, 777, 0, (0, 1)), (128, 1, 8, 512, 0, (1, 1)),
+                                                          (128, 1, 16, 1024, 0, (1, 1)), (128, 1, 40, 1000, 0, (1, 1)), (32, 1, 12, 1024, 1, (0, 1))) for d, x in enumerate(x2)),
+    *((2, "bwd", D, d, z, h, n, c, x) for D, z, h, n, c, x2 in ((64, 1, 8, 512, 0, (0, 1)), (64, 1, 12, 1024, 1, (1, 1)), (64, 3, 4, 640, 0, (0, 1)), (64, 1, 2, 4096, 1, (1, 1)),
+                                                          (128, 1, 8, 512, 0, (1, 1)), (128, 1, 12, 1024, 1, (1, 1)), (32, 1, 2, 4096, 1, (1, 1))) for d, x in enumerate(x2)),
+    (2, "bwd", 64, 1, 1, 4, 900, 0, 1), (2, "bwd", 64, 1, 1, 2, 300, 0, 0),
+]
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
+def test_calls_with_a_quoted_time_are_dealt_or_whole(tmp_path):
+    text = "  struct P { int D, Z, H, L, dtype, causal, mask_kind; float dropout_p; };\n"
+    for kind, way, D, dual, Z, H, L, causal, _ in QUOTED:
+        if way == "fwd":
+            plan = f"fwd_split_plan_{'f32' if kind else 16}(p, {L}, {dual}, 256).chunks > 1"
+        else:
+            plan = f"make_bwd_deal{'_f32' if kind else ''}({D}, {Z}, {H}, {L}, {L}, {causal}, {dual}, 256).any()"
+        text += f'  {{ const P p = {{{D}, {Z}, {H}, {L}, {kind}, {causal}, 0, 0.f}}; (void)p; std::printf("%d ", {plan} ? 1 : 0); }}\n'
+    assert [x for x, y in zip(QUOTED, run(tmp_path, text)) if x[-1] != y] == []
+
+
 @pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no HIP compiler")
 def test_order_of_a_launch_goes_by_the_units_of_the_device(tmp_path):
     """280 workgroups of 4 heads: heads side by side on 256 units, the shares of a block on 304; either way each once."""
